@@ -26,8 +26,6 @@
 // operation rounds once, as in the CPU oracle.
 #include <hip/hip_runtime.h>
 
-#include <mutex>
-
 #include "../../include/aslhip.h"
 #include "kernels.hpp"
 
@@ -46,6 +44,14 @@ __device__ __forceinline__ const __attribute__((address_space(1))) T *gload(cons
 template <class T>
 __device__ __forceinline__ __attribute__((address_space(1))) T *gstore(char *p) {
   return (__attribute__((address_space(1))) T *)p;
+}
+
+// A wavefront-uniform address kept in scalar registers: without this the
+// compiler adds the lane's offset first and carries one 64-bit vector address
+// per direction (D3Q19: 90 instead of 64 VGPRs).
+__device__ __forceinline__ char *scalar_base(char *p) {
+  asm("" : "+s"(p));
+  return p;
 }
 
 // ---------------------------------------------------------------------------
@@ -254,16 +260,35 @@ __device__ __forceinline__ void collide(C (&v)[Q], C w, bool compressible, bool 
   for (int d = 0; d < 3; ++d) m_o[d] = m[d];
 }
 
+// n / d for a divisor known to the host, M = floor(2^64 / d) + 1 (0: d = 1).
+// n M / 2^64 lies above n / d by at most n / 2^64 < 1 / d, so the floor is
+// exact for all 32-bit n and d.  Uniform operands: a few scalar instructions.
+__device__ __forceinline__ unsigned udivm(unsigned n, unsigned long long M) {
+  const unsigned long long lo = static_cast<unsigned long long>(n) * static_cast<unsigned>(M);
+  const unsigned long long hi = static_cast<unsigned long long>(n) * static_cast<unsigned>(M >> 32);
+  const unsigned q = static_cast<unsigned>((hi + (lo >> 32)) >> 32);
+  return M == 0 ? n : q;
+}
+
+// n / d per lane for n < 2^21: (n + 1/2) / d is at least 1 / (2 d) from the
+// next integer and its FP32 product with the rounded 1 / d is off by at most
+// 2^-23 (n + 1/2) / d, so the truncation is exact.  Three full-rate
+// instructions instead of a 64-bit multiplication's quarter-rate ones.
+__device__ __forceinline__ unsigned lane_div(unsigned n, float inv) {
+  return static_cast<unsigned>((static_cast<float>(n) + 0.5f) * inv);
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs (id % 8).  With a
 // group size g > 1, each XCD takes runs of g consecutive chunks (workgroup b
 // of a group of 8 g works on chunk  group * 8g + (b % 8) * g + (b % 8g) / 8),
 // so that neighbouring chunks, which share cache lines at their edges, meet
 // in the same L2; the last, partial group keeps the hardware order.
-__device__ __forceinline__ int xcd_remap(int L, int n, int g) {
-  const int span = 8 * g, grp = L / span;
-  if ((grp + 1) * span > n) return L;
+// m = floor(2^64 / 8g) + 1.
+__device__ __forceinline__ int xcd_remap(int L, int n, int g, unsigned long long m) {
+  const int span = 8 * g, grp = static_cast<int>(udivm(static_cast<unsigned>(L), m));
   const int r = L - grp * span;
-  return grp * span + (r & 7) * g + (r >> 3);
+  const int c = grp * span + (r & 7) * g + (r >> 3);
+  return (grp + 1) * span > n ? L : c;
 }
 
 // Workgroup b of n taking the chunks in reverse order within its XCD's share:
@@ -275,145 +300,230 @@ __device__ __forceinline__ int xcd_reverse(int b, int n) {
   return r + 8 * (nr - 1 - (b >> 3));
 }
 
+// The chunk of workgroup b in a launch of n.
+template <bool ODD>
+__device__ __forceinline__ int chunk_of(const StepHot &g, int b, int n) {
+  if (ODD) b = xcd_reverse(b, n);
+  return xcd_remap(b, n, g.remap, g.mspan);
+}
+
 __device__ __forceinline__ int wrap1(int v, int n) { return v < 1 ? n : (v > n ? 1 : v); }
 
-template <class C>
-__device__ __forceinline__ C face_val(const StepArgs &a, int f, int k);
-template <>
-__device__ __forceinline__ float face_val<float>(const StepArgs &a, int f, int k) {
-  return a.fval32[f][k];
-}
-template <>
-__device__ __forceinline__ double face_val<double>(const StepArgs &a, int f, int k) {
-  return a.fval64[f][k];
+// The item of work of one lane (StepHot).
+struct Item {
+  unsigned row;   // ghost-inclusive index of the row's cell z = 0
+  int x, y, z;    // 1-based interior coordinates (runs of cells: z counts runs)
+  bool act;       // false: past the end of the launch (stands in for the chunk's first item)
+};
+
+// No branches: each scalar load of g would sink into the branch that uses it
+// and wait there, one memory latency after the other before the first load.
+// Rows hold fewer than 2^20 cells (aslhip_lattice_create); only ny may be
+// large, so rows are counted from the end of the plane the chunk starts in.
+__device__ __forceinline__ Item item_of(const StepHot &g, int chunk) {
+  // the chunk's first item, in scalar registers
+  const unsigned rowi = static_cast<unsigned>(g.rowi), ny = static_cast<unsigned>(g.ny);
+  const unsigned jb = g.first + static_cast<unsigned>(chunk) * static_cast<unsigned>(g.block);
+  const unsigned row0 = udivm(jb, g.mrow), x0 = udivm(row0, g.mplane);
+  const unsigned z0 = jb - row0 * rowi, y0 = row0 - x0 * ny, left = ny - y0;
+  // (x, y, z) is cell x sx + y sy + z with sx = (ny + 2) sy: row r of the interior (r = (x - 1) ny + y - 1)
+  // starts at (r + 2 (x - 1) + ny + 3) sy
+  const unsigned base = (row0 + 2u * x0 + ny + 3u) * static_cast<unsigned>(g.sy);
+  Item it;
+  it.act = jb + threadIdx.x < g.first + g.count;
+  const unsigned n = z0 + (it.act ? threadIdx.x : 0u);
+  const unsigned dr = lane_div(n, g.inv_row);
+  const bool next = dr >= left;  // past the plane of the first item
+  const unsigned over = next ? dr - left : 0u, more = lane_div(over, g.inv_ny);
+  const unsigned dx = next ? more + 1u : 0u;
+  it.z = static_cast<int>(n - __umul24(dr, rowi)) + 1;
+  it.y = static_cast<int>(next ? over - __umul24(more, ny) : y0 + dr) + 1;
+  it.x = static_cast<int>(x0 + dx) + 1;
+  it.row = base + __umul24(dr + 2u * dx, static_cast<unsigned>(g.sy));
+  return it;
 }
 
-// One cell of one step: chunk L of the lattice described by a.
+// Bit f: the cell lies on face f (X0 XE Y0 YE Z0 ZE).
+__device__ __forceinline__ unsigned face_bits(const StepHot &g, int x, int y, int z) {
+  return (x == 1 ? 1u : 0u) | (x == g.nx ? 2u : 0u) | (y == 1 ? 4u : 0u) | (y == g.ny ? 8u : 0u) |
+         (z == 1 ? 16u : 0u) | (z == g.nz ? 32u : 0u);
+}
+
+// ~0 if the cell lies on the face of entry j of the face rule, else 0.
+__device__ __forceinline__ unsigned on_entry(const StepHot &g, unsigned fb, int j) {
+  return static_cast<unsigned>(__builtin_amdgcn_sbfe(static_cast<int>(fb), (g.fpos >> (4 * j)) & 15u, 1u));
+}
+
+// Bounce-back and constant links of a cell on the faces fb: entry by entry,
+// later ones over earlier ones.  Four vector instructions per entry, in place
+// of a search over three faces per link that was about 800 instructions in
+// every wavefront with a face cell, that is in nearly every wavefront where a
+// row is not much longer than one.  us per step of a closed box before and
+// after (256 x 128 x 128): D3Q19 FP32 126.2 -> 120.3, FP16 67.6 -> 62.4, FP64
+// 230 -> 211, D3Q27 FP16 111 -> 91.5, FP64 382 -> 328; 64^3: D3Q19 FP32 12.1
+// -> 9.6, FP16 10.8 -> 7.7.
+__device__ __forceinline__ void face_masks(const StepHot &g, unsigned fb, unsigned &bounce, unsigned &cnst) {
+  bounce = cnst = 0u;
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    const unsigned m = on_entry(g, fb, j) & g.flinks[j];
+    const bool b = (g.fbounce >> j) & 1u;
+    bounce = (bounce & ~m) | (b ? m : 0u);
+    cnst = (cnst & ~m) | (b ? 0u : m);
+  }
+}
+
+// Links that enter through face f.
+template <int Q>
+constexpr unsigned face_links(int f) {
+  unsigned m = 0;
+  for (int k = 1; k < Q; ++k)
+    if (Lat<Q>::c[k][f / 2] == (f % 2 == 0 ? 1 : -1)) m |= 1u << k;
+  return m;
+}
+
+// Adds (bounce-back) or sets (constant) the values of the faces that have
+// some, each on the links it won.  Only wavefronts with a cell on such a face
+// (an inlet, an outlet, a lid) get past the tests.  Faces and links are fixed
+// at compile time: with the entries' order the links would be tested one by
+// one, and the compiler threads those uniform branches into thousands of
+// scalar instructions.
+template <int Q, class C>
+__device__ __forceinline__ void face_values(const StepHot &g, const StepArgs &a, unsigned fb, C (&v)[Q]) {
+  if (g.fvalued == 0u) return;
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    if (!((g.fvalued >> f) & 1u)) continue;
+    unsigned own = ((fb >> f) & 1u) ? face_links<Q>(f) : 0u;
+    if (!__any(own != 0u)) continue;
+    const unsigned beats = a.fbeats[f];
+#pragma unroll
+    for (int h = 0; h < 6; ++h)
+      if (h / 2 != f / 2) own &= ((fb & beats) >> h) & 1u ? ~face_links<Q>(h) : ~0u;
+    const bool bounce = (a.fbounces >> f) & 1u;
+#pragma unroll
+    for (int k = 1; k < Q; ++k) {
+      if (!((face_links<Q>(f) >> k) & 1u)) continue;
+      const C val = sizeof(C) == 4 ? C(a.fval32[f][k]) : C(a.fval64[f][k]);
+      const C nv = (bounce ? v[k] : C(0)) + val;
+      v[k] = ((own >> k) & 1u) ? nv : v[k];
+    }
+  }
+}
+
+// One cell per lane of one step, chunk `chunk` of the launch g of the lattice
+// described by a.  Every direction array is addressed by a base in scalar
+// registers (array, shifted by the direction's offset on odd steps) plus the
+// lane's 32-bit byte offset, so that a load or store of an interior wavefront
+// takes no vector address arithmetic; an array stays below 4 GiB.
+// WIDE: the arrays together exceed 4 GiB (only the links that choose between
+// two slots are affected).
 // PEEK: instead of colliding and storing, write the populations the cell
 // receives (after every BC link is resolved) to peek[k * len + cell].
 template <int Q, class S, bool ODD, bool PER, bool WIDE, int CL = 0, bool PEEK = false>
-__device__ __forceinline__ void step_body(const StepArgs &a, const int L, void *peek = nullptr) {
+__device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, const int chunk, void *peek = nullptr) {
   using CD = Codec<S>;
   using C = typename CD::C;
   using M = typename CD::M;
   constexpr unsigned ES = sizeof(S);
-  const int plane = L / a.bpp;
-  const int chunk = L - plane * a.bpp;
-  unsigned off = static_cast<unsigned>(chunk * a.block) + threadIdx.x;
-  // The closure variant keeps every lane to the end (its network may run on
-  // matrix instructions across the wavefront): a lane without a cell of its
-  // own works on a stand-in interior cell of its plane and stores nothing.
-  bool act = off < static_cast<unsigned>(a.ny * a.sy);
+  const Item it = item_of(g, chunk);
+  // The closure variant keeps every lane to the end (its network runs on
+  // matrix instructions across the wavefront): a lane past the end works on a
+  // stand-in cell and stores nothing.
   if constexpr (!CL) {
-    if (!act) return;
-  } else {
-    if (!act) off = 1u;
+    if (!it.act) return;
   }
-  // Row and column inside the plane (exact: off * sy < 2^40, see StepArgs::zmagic).
-  const unsigned row = static_cast<unsigned>((static_cast<unsigned long long>(off) * a.zmagic) >> 40);
-  unsigned z = off - row * static_cast<unsigned>(a.sy);
-  if (z == 0 || z == static_cast<unsigned>(a.sy - 1)) {  // ghost columns
-    if constexpr (!CL) return;
-    act = false;
-    off = row * static_cast<unsigned>(a.sy) + 1u;
-    z = 1u;
-  }
-  const unsigned idx = static_cast<unsigned>((plane + 1) * a.sx + a.sy) + off;
-  const int x = plane + 1, y = static_cast<int>(row) + 1, zi = static_cast<int>(z);
-  const unsigned ib = idx * ES;
+  const unsigned idx = it.row + static_cast<unsigned>(it.z), ib = idx * ES;
+  char *const f = g.f;
 
-  // Byte offsets of x - c_k (rd) and x + c_k (wr).
-  auto nb = [&](int k, int sgn) -> unsigned {
-    if constexpr (PER) {
-      return ES * static_cast<unsigned>(wrap1(x + sgn * Lat<Q>::c[k][0], a.nx) * a.sx +
-                                        wrap1(y + sgn * Lat<Q>::c[k][1], a.ny) * a.sy +
-                                        wrap1(zi + sgn * Lat<Q>::c[k][2], a.nz));
+  // The slot of link k that a cell shares with its neighbour x - c_k: array
+  // inv k at x - c_k on odd steps, array k at x on even ones; outgoing k goes
+  // to array k at x + c_k (odd) or array inv k at x (even).
+  // Periodic lattices, odd steps: byte steps to the neighbours along each axis, wrapped.
+  unsigned nx_[3], ny_[3], nz_[3];  // for c = -1, 0, 1
+  if constexpr (PER && ODD) {
+    const unsigned sxb = ES * static_cast<unsigned>(g.sx), syb = ES * static_cast<unsigned>(g.sy);
+    nx_[0] = it.x == 1 ? (static_cast<unsigned>(g.nx) - 1u) * sxb : 0u - sxb;
+    nx_[2] = it.x == g.nx ? (1u - static_cast<unsigned>(g.nx)) * sxb : sxb;
+    ny_[0] = it.y == 1 ? (static_cast<unsigned>(g.ny) - 1u) * syb : 0u - syb;
+    ny_[2] = it.y == g.ny ? (1u - static_cast<unsigned>(g.ny)) * syb : syb;
+    nz_[0] = it.z == 1 ? (static_cast<unsigned>(g.nz) - 1u) * ES : 0u - ES;
+    nz_[2] = it.z == g.nz ? (1u - static_cast<unsigned>(g.nz)) * ES : ES;
+    nx_[1] = ny_[1] = nz_[1] = 0u;
+  }
+  // lane offset of x + sgn c_k (periodic odd steps); the base carries the shift otherwise
+  auto lane = [&](int k, int sgn) -> unsigned {
+    if constexpr (PER && ODD)
+      return ib + nx_[1 + sgn * Lat<Q>::c[k][0]] + ny_[1 + sgn * Lat<Q>::c[k][1]] + nz_[1 + sgn * Lat<Q>::c[k][2]];
+    else
+      return ib;
+  };
+  // base of array j, shifted by sgn c_k on non-periodic lattices (sh: shifted at all)
+  auto base = [&](int j, int k, int sgn, bool sh) -> char * {
+    char *b = f + static_cast<unsigned long long>(j) * g.qs;
+    if (!PER && sh) b += static_cast<long long>(sgn) * static_cast<long long>(ES) * offc<Q>(k, g.sx, g.sy);
+    return scalar_base(b);
+  };
+  auto in_base = [&](int k) -> char * { return base(ODD ? inv_dir<Q>(k) : k, k, -1, ODD); };
+  auto other_base = [&](int k) -> char * { return base(ODD ? k : inv_dir<Q>(k), k, -1, !ODD); };
+  auto out_base = [&](int k) -> char * { return base(ODD ? k : inv_dir<Q>(k), k, 1, ODD); };
+  // slot of link k, or the other slot of its pair where mask is ~0 (non-periodic)
+  auto load_sel = [&](int k, unsigned mask) -> C {
+    if constexpr (WIDE) {
+      return CD::ld(mask ? other_base(k) : in_base(k), ib);
     } else {
-      const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, a.sx, a.sy));
-      return sgn > 0 ? ib + o : ib - o;
+      const unsigned on = static_cast<unsigned>(in_base(k) - f), op = static_cast<unsigned>(other_base(k) - f);
+      return CD::ld(f, (ib + on) + (mask & (op - on)));
     }
   };
 
-  // Face rule (see StepArgs): bit f of fb is set if the cell lies on face f.
-  const bool raw = (a.flags & STEP_F_RAW) != 0;
-  unsigned fb = 0;
-  if (!PER && !raw)
-    fb = (x == 1 ? 1u : 0u) | (x == a.nx ? 2u : 0u) | (y == 1 ? 4u : 0u) | (y == a.ny ? 8u : 0u) |
-         (zi == 1 ? 16u : 0u) | (zi == a.nz ? 32u : 0u);
-  // Winning face BC of link k: slot * 4 + mode, and its value.
-  auto winner = [&](int k, C &val) -> int {
-    int wn = 0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const int cd = Lat<Q>::c[k][d];
-      if (cd == 0) continue;
-      const int fc = 2 * d + (cd > 0 ? 0 : 1);  // the face this link enters through
-      const int cand = ((fb >> fc) & 1u) ? a.fface[fc] : 0;
-      if (cand > wn) {
-        wn = cand;
-        val = face_val<C>(a, fc, k);
-      }
-    }
-    return wn;
-  };
-  // The face rule only touches wavefronts with a face cell: a wavefront-
-  // uniform branch, so interior wavefronts skip it and load plainly.
-  const bool faces = !PER && __any(fb != 0);
-  unsigned bmask = 0, cmask = 0;  // bounce-back / constant links
-  if (faces) {
-#pragma unroll
-    for (int k = 1; k < Q; ++k) {
-      C unused;
-      const int md = winner(k, unused) & 3;
-      if (md == MODE_BOUNCE) bmask |= 1u << k;
-      if (md == MODE_CONST) cmask |= 1u << k;
+  // Faces of the lattice (face rule, see StepHot): a wavefront-uniform branch,
+  // so interior wavefronts load plainly, and wavefronts whose face cells lie
+  // on z faces only (all wavefronts, where rows are short) choose a slot for
+  // the links through those only.
+  const bool raw = (g.flags & STEP_F_RAW) != 0;
+  unsigned fb = 0, bmask = 0, cmask = 0;
+  bool faces = false, xyfaces = false;
+  if constexpr (!PER) {
+    const bool bxy = (it.x == 1) | (it.x == g.nx) | (it.y == 1) | (it.y == g.ny);
+    const bool bz = (it.z == 1) | (it.z == g.nz);
+    xyfaces = __any(bxy & !raw);
+    faces = __any((bxy | bz) & !raw);
+    if (faces) {
+      fb = face_bits(g, it.x, it.y, it.z);
+      face_masks(g, fb, bmask, cmask);
     }
   }
 
   // One round of loads: the cell type and every population (bounce-back
-  // links read the other slot of their link pair, constant links nothing).
-  // All addresses lie inside the lattice for interior cells.
-  // Loads take no branch (divergent branches around loads into the same
-  // register force the compiler to wait for memory inside the branch).
-  const unsigned char code = *gload<unsigned char>(reinterpret_cast<const char *>(a.code) + idx);
+  // links read the other slot of their link pair; the value read for a
+  // constant link is replaced below).  All addresses lie inside the lattice
+  // for interior cells.  Loads take no divergent branch (branches around
+  // loads into the same register force the compiler to wait for memory inside
+  // the branch).
+  const unsigned char code = *gload<unsigned char>(reinterpret_cast<const char *>(g.code) + idx);
   C v[Q];
-  auto load_all = [&](unsigned bm) {
+  if (!faces) {
+#pragma unroll
+    for (int k = 0; k < Q; ++k) v[k] = CD::ld(in_base(k), lane(k, -1));
+  } else if (!xyfaces) {
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-      const int kb = inv_dir<Q>(k);
-      const bool bb = (bm >> k) & 1u;
-      if constexpr (WIDE) {
-        const char *pn = a.fd[ODD ? kb : k] + (ODD ? nb(k, -1) : ib);  // normal slot
-        const char *pp = a.fd[ODD ? k : kb] + (ODD ? ib : nb(k, -1));  // the other slot of the pair
-        v[k] = CD::ld(bb ? pp : pn, 0u);
-      } else {
-        // byte offsets from the first direction array
-        const unsigned on = static_cast<unsigned>(ODD ? kb : k) * a.qs32 + (ODD ? nb(k, -1) : ib);
-        if (bm == 0u) {
-          v[k] = CD::ld(a.fd[0], on);
-        } else {
-          const unsigned op = static_cast<unsigned>(ODD ? k : kb) * a.qs32 + (ODD ? ib : nb(k, -1));
-          v[k] = CD::ld(a.fd[0], bb ? op : on);
-        }
-      }
+      if (Lat<Q>::c[k][2] != 0)
+        v[k] = load_sel(k, static_cast<unsigned>(__builtin_amdgcn_sbfe(static_cast<int>(bmask), k, 1)));
+      else
+        v[k] = CD::ld(in_base(k), ib);
     }
-  };
-  if (faces)
-    load_all(bmask);
-  else
-    load_all(0u);
+  } else {
+    v[0] = CD::ld(in_base(0), ib);
+#pragma unroll
+    for (int k = 1; k < Q; ++k)
+      v[k] = load_sel(k, static_cast<unsigned>(__builtin_amdgcn_sbfe(static_cast<int>(bmask), k, 1)));
+  }
   // Keep the scheduler from hoisting the wait on the cell type above the
   // population loads.
   __builtin_amdgcn_sched_barrier(0);
-  if (faces) {
-#pragma unroll
-    for (int k = 1; k < Q; ++k) {
-      if (!(((bmask | cmask) >> k) & 1u)) continue;
-      C val = C(0);
-      (void)winner(k, val);
-      v[k] = ((bmask >> k) & 1u) ? v[k] + val : val;
-    }
-  }
+  if (faces) face_values<Q, C>(g, a, fb, v);
 
   // Cells that are not computed run the collision on whatever they read and
   // store nothing; cells with a link pattern re-read their links from it.
@@ -427,19 +537,9 @@ __device__ __forceinline__ void step_body(const StepArgs &a, const int L, void *
     const C *val = static_cast<const C *>(a.val);
 #pragma unroll
     for (int k = 1; k < Q; ++k) {
-      const int kb = inv_dir<Q>(k);
       const int slot = raw ? 0 : rec.slot[k];
       const unsigned char md = slot ? a.mode[slot] : static_cast<unsigned char>(MODE_NONE);
-      C x;
-      if constexpr (WIDE) {
-        const char *pn = a.fd[ODD ? kb : k] + (ODD ? nb(k, -1) : ib);
-        const char *pp = a.fd[ODD ? k : kb] + (ODD ? ib : nb(k, -1));
-        x = CD::ld(md == MODE_BOUNCE ? pp : pn, 0u);
-      } else {
-        const unsigned on = static_cast<unsigned>(ODD ? kb : k) * a.qs32 + (ODD ? nb(k, -1) : ib);
-        const unsigned op = static_cast<unsigned>(ODD ? k : kb) * a.qs32 + (ODD ? ib : nb(k, -1));
-        x = CD::ld(a.fd[0], md == MODE_BOUNCE ? op : on);
-      }
+      const C x = load_sel(k, md == MODE_BOUNCE ? ~0u : 0u);
       const C sv = val[slot * Q + k];
       v[k] = md == MODE_BOUNCE ? x + sv : (md == MODE_CONST ? sv : x);
     }
@@ -454,37 +554,31 @@ __device__ __forceinline__ void step_body(const StepArgs &a, const int L, void *
   }
 
   C r, m[3];
-  const bool omega = (a.flags & STEP_F_OMEGA) != 0;
+  const bool omega = (g.flags & STEP_F_OMEGA) != 0;
   C om[3] = {C(0), C(0), C(0)};
   if (omega) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) om[d] = sizeof(C) == 4 ? C(a.om32[d]) : C(a.om64[d]);
   }
-  collide<Q, C, CL>(v, C(a.w), (a.flags & STEP_F_COMPRESSIBLE) != 0, omega, om, r, m, a.cl, a.cl_tau0,
-                    (a.flags & STEP_F_TURB) != 0, sizeof(C) == 4 ? C(a.nu32) : C(a.nu64));
+  collide<Q, C, CL>(v, C(a.w), (g.flags & STEP_F_COMPRESSIBLE) != 0, omega, om, r, m, a.cl, a.cl_tau0,
+                    (g.flags & STEP_F_TURB) != 0, sizeof(C) == 4 ? C(a.nu32) : C(a.nu64));
 
-  if (!live || !act) return;
-  // Stores address every direction from fd[0] too (one scalar base pair
-  // instead of Q live pointers) unless the lattice is too large for it.
-  auto st = [&](int k) {
-    const int dir = ODD ? k : inv_dir<Q>(k);
-    const unsigned o = ODD ? nb(k, 1) : ib;
-    if constexpr (WIDE)
-      CD::st(a.fd[dir], o, v[k]);
-    else
-      CD::st(a.fd[0], static_cast<unsigned>(dir) * a.qs32 + o, v[k]);
-  };
+  if (!live || !it.act) return;
+  if constexpr (PER && ODD) {  // offsets formed again for the stores: 18 of them live across the collision cost waves
+#pragma unroll
+    for (int d = 0; d < 3; d += 2) asm("" : "+v"(nx_[d]), "+v"(ny_[d]), "+v"(nz_[d]));
+  }
   if (general) {
 #pragma unroll
     for (int k = 0; k < Q; ++k)
-      if (!((skipm >> k) & 1u)) st(k);
+      if (!((skipm >> k) & 1u)) CD::st(out_base(k), lane(k, 1), v[k]);
   } else {
 #pragma unroll
-    for (int k = 0; k < Q; ++k) st(k);
+    for (int k = 0; k < Q; ++k) CD::st(out_base(k), lane(k, 1), v[k]);
   }
-  if (a.flags & STEP_F_RHO) *gstore<M>(static_cast<char *>(a.rho) + sizeof(M) * idx) = M(r);
-  if (a.flags & STEP_F_VEL) {
-    const bool comp = (a.flags & STEP_F_COMPRESSIBLE) != 0;
+  if (g.flags & STEP_F_RHO) *gstore<M>(static_cast<char *>(a.rho) + sizeof(M) * idx) = M(r);
+  if (g.flags & STEP_F_VEL) {
+    const bool comp = (g.flags & STEP_F_COMPRESSIBLE) != 0;
     char *u = static_cast<char *>(a.u);
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -509,72 +603,42 @@ struct RunVec {
 // vector loads (wavefront-uniform branches), and a run with a cell that is
 // not computed, or that must not write some links, stores cell by cell.
 template <int Q, class S, bool ODD, int CPL>
-__device__ __forceinline__ void step_body_run(const StepArgs &a, const int L) {
+__device__ __forceinline__ void step_body_run(const StepHot &g, const StepArgs &a, const int chunk) {
   using CD = Codec<S>;
   using C = typename CD::C;
   using M = typename CD::M;
   using V = typename RunVec<S, CPL>::type;
   constexpr unsigned ES = sizeof(S);
-  const int plane = L / a.bpp;
-  const int chunk = L - plane * a.bpp;
-  const unsigned j = static_cast<unsigned>(chunk * a.block) + threadIdx.x;
-  if (j >= static_cast<unsigned>(a.ny * a.nzv)) return;
-  // row and run inside the plane (exact: j * nzv < 2^40, see StepArgs::vmagic)
-  const unsigned row = static_cast<unsigned>((static_cast<unsigned long long>(j) * a.vmagic) >> 40);
-  const int z0 = 1 + CPL * static_cast<int>(j - row * static_cast<unsigned>(a.nzv));
-  const int x = plane + 1, y = static_cast<int>(row) + 1;
-  const unsigned idx = static_cast<unsigned>(x * a.sx + y * a.sy + z0);
+  const Item it = item_of(g, chunk);
+  if (!it.act) return;
+  const int z0 = 1 + CPL * (it.z - 1);
+  const int x = it.x, y = it.y;
+  const unsigned idx = it.row + static_cast<unsigned>(z0);
   const unsigned ib = idx * ES;
-  const char *f0 = a.fd[0];
+  const char *f0 = g.f;
 
   // Face rule (as step_body), in one round of loads.  A run lies on an x or y
   // face with all its cells, so a bounce-back link there is a vector load of
   // the other slot of the link pair; only the first (z = 1) and the last
-  // (z = nz) cell of a row lie on a z face, and their links through it come
-  // from side loads of one element, issued with the vector loads.
-  const bool raw_links = (a.flags & STEP_F_RAW) != 0;
-  const unsigned fxy = raw_links ? 0u
-                                 : (x == 1 ? 1u : 0u) | (x == a.nx ? 2u : 0u) | (y == 1 ? 4u : 0u) |
-                                       (y == a.ny ? 8u : 0u);
-  const bool zlo = !raw_links && z0 == 1, zhi = !raw_links && z0 + CPL - 1 == a.nz;
+  // (z = nz) cell of a row lie on a z face, and their links with a z share
+  // come from side loads of one element, issued with the vector loads.
+  const bool raw_links = (g.flags & STEP_F_RAW) != 0;
+  const unsigned fxy = raw_links ? 0u : face_bits(g, x, y, 0);
+  const bool zlo = !raw_links && z0 == 1, zhi = !raw_links && z0 + CPL - 1 == g.nz;
   const bool xyf = __any(fxy != 0u), zf = __any(zlo || zhi);  // wavefront-uniform
-  // winning face BC of link k among the faces in fb: slot * 4 + mode, and its value
-  auto winner = [&](int k, unsigned fb, C &val) -> int {
-    int wn = 0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const int cd = Lat<Q>::c[k][d];
-      if (cd == 0) continue;
-      const int fc = 2 * d + (cd > 0 ? 0 : 1);  // the face this link enters through
-      const int cand = ((fb >> fc) & 1u) ? a.fface[fc] : 0;
-      if (cand > wn) {
-        wn = cand;
-        val = face_val<C>(a, fc, k);
-      }
-    }
-    return wn;
-  };
-  unsigned bxy = 0, cxy = 0;  // bounce-back / constant links of the x and y faces
-  if (xyf) {
-#pragma unroll
-    for (int k = 1; k < Q; ++k) {
-      C unused;
-      const int md = winner(k, fxy, unused) & 3;
-      if (md == MODE_BOUNCE) bxy |= 1u << k;
-      if (md == MODE_CONST) cxy |= 1u << k;
-    }
-  }
+  unsigned bxy = 0, cxy = 0;  // bounce-back links of the x and y faces
+  if (xyf) face_masks(g, fxy, bxy, cxy);
   // the other slot of link k's pair for the cell at byte offset ibc
   auto other = [&](int k, unsigned ibc) -> unsigned {
-    const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, a.sx, a.sy));
+    const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, g.sx, g.sy));
     return static_cast<unsigned>(ODD ? k : inv_dir<Q>(k)) * a.qs32 + (ODD ? ibc : ibc - o);
   };
   V raw[Q];
-  C side[Q];  // links through z = 1 (first cell) or z = nz (last cell): the other slot
+  C side[Q];  // links of the first (c_z > 0) or last (c_z < 0) cell: the other slot
 #pragma unroll
   for (int k = 0; k < Q; ++k) {
     // normal slot: (x, k) (even) or (x - c_k, inv k) (odd)
-    const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, a.sx, a.sy));
+    const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, g.sx, g.sy));
     const unsigned on = static_cast<unsigned>(ODD ? inv_dir<Q>(k) : k) * a.qs32 + (ODD ? ib - o : ib);
     if (xyf) {
       const unsigned op = other(k, ib);
@@ -585,7 +649,7 @@ __device__ __forceinline__ void step_body_run(const StepArgs &a, const int L) {
     if (zf && Lat<Q>::c[k][2] != 0) side[k] = CD::ld(f0, other(k, Lat<Q>::c[k][2] > 0 ? ib : ib + ES * (CPL - 1)));
   }
   unsigned codes = 0;  // CPL cell-type bytes
-  const char *cb = reinterpret_cast<const char *>(a.code) + idx;
+  const char *cb = reinterpret_cast<const char *>(g.code) + idx;
 #pragma unroll
   for (int c = 0; c < CPL; ++c) codes |= static_cast<unsigned>(*gload<unsigned char>(cb + c)) << (8 * c);
   __builtin_amdgcn_sched_barrier(0);
@@ -594,32 +658,23 @@ __device__ __forceinline__ void step_body_run(const StepArgs &a, const int L) {
   for (int c = 0; c < CPL; ++c)
 #pragma unroll
     for (int k = 0; k < Q; ++k) v[c][k] = CD::dec(raw[k][c]);
-  if (xyf) {
-#pragma unroll
-    for (int k = 1; k < Q; ++k) {
-      if (!(((bxy | cxy) >> k) & 1u)) continue;
-      C val = C(0);
-      (void)winner(k, fxy, val);
-#pragma unroll
-      for (int c = 0; c < CPL; ++c) v[c][k] = ((bxy >> k) & 1u) ? v[c][k] + val : val;
-    }
-  }
   if (zf) {
-    // a link through the z face of an end cell: the z face's BC where it wins
+    // bounce-back links with a z share of the end cells, whichever face they bounce at
+    unsigned blo, bhi, unused;
+    face_masks(g, fxy | (zlo ? 16u : 0u), blo, unused);
+    face_masks(g, fxy | (zhi ? 32u : 0u), bhi, unused);
 #pragma unroll
     for (int k = 1; k < Q; ++k) {
       const int cz = Lat<Q>::c[k][2];
       if (cz == 0) continue;
       const int c = cz > 0 ? 0 : CPL - 1;
-      const bool on_z = cz > 0 ? zlo : zhi;
-      const unsigned zbit = cz > 0 ? 16u : 32u;
-      C vz = C(0), vxy = C(0);
-      const int wz = winner(k, fxy | zbit, vz);
-      const int wxy = winner(k, fxy, vxy);
-      if (on_z && wz != wxy) {  // the z face wins the link
-        v[c][k] = (wz & 3) == MODE_BOUNCE ? side[k] + vz : vz;
-      }
+      if (cz > 0 ? zlo && ((blo >> k) & 1u) : zhi && ((bhi >> k) & 1u)) v[c][k] = side[k];
     }
+  }
+  if (xyf || zf) {
+#pragma unroll
+    for (int c = 0; c < CPL; ++c)
+      face_values<Q, C>(g, a, fxy | (c == 0 && zlo ? 16u : 0u) | (c == CPL - 1 && zhi ? 32u : 0u), v[c]);
   }
 
   // Cells with a link pattern re-read their links from it.
@@ -648,7 +703,7 @@ __device__ __forceinline__ void step_body_run(const StepArgs &a, const int L) {
       for (int k = 1; k < Q; ++k) {
         const int slot = raw_links ? 0 : rec.slot[k];
         const unsigned char md = slot ? a.mode[slot] : static_cast<unsigned char>(MODE_NONE);
-        const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, a.sx, a.sy));
+        const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, g.sx, g.sy));
         const unsigned on = static_cast<unsigned>(ODD ? inv_dir<Q>(k) : k) * a.qs32 + (ODD ? ibc - o : ibc);
         const unsigned op = static_cast<unsigned>(ODD ? k : inv_dir<Q>(k)) * a.qs32 + (ODD ? ibc : ibc - o);
         const C xk = CD::ld(f0, md == MODE_BOUNCE ? op : on);
@@ -658,8 +713,8 @@ __device__ __forceinline__ void step_body_run(const StepArgs &a, const int L) {
     }
   }
 
-  const bool omega = (a.flags & STEP_F_OMEGA) != 0;
-  const bool comp = (a.flags & STEP_F_COMPRESSIBLE) != 0;
+  const bool omega = (g.flags & STEP_F_OMEGA) != 0;
+  const bool comp = (g.flags & STEP_F_COMPRESSIBLE) != 0;
   C om[3] = {C(0), C(0), C(0)};
   if (omega) {
 #pragma unroll
@@ -672,11 +727,11 @@ __device__ __forceinline__ void step_body_run(const StepArgs &a, const int L) {
   bool plain = true;
 #pragma unroll
   for (int c = 0; c < CPL; ++c) plain = plain && live[c] && skipm[c] == 0u;
-  char *fw = a.fd[0];
+  char *fw = g.f;
 #pragma unroll
   for (int k = 0; k < Q; ++k) {
     // even: slot (x, inv k); odd: slot (x + c_k, k)
-    const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, a.sx, a.sy));
+    const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, g.sx, g.sy));
     const unsigned ow = static_cast<unsigned>(ODD ? k : inv_dir<Q>(k)) * a.qs32 + (ODD ? ib + o : ib);
     if (plain) {
       V out;
@@ -689,12 +744,12 @@ __device__ __forceinline__ void step_body_run(const StepArgs &a, const int L) {
         if (live[c] && !((skipm[c] >> k) & 1u)) CD::st(fw, ow + ES * c, v[c][k]);
     }
   }
-  if (a.flags & (STEP_F_RHO | STEP_F_VEL)) {
+  if (g.flags & (STEP_F_RHO | STEP_F_VEL)) {
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
       if (!live[c]) continue;
-      if (a.flags & STEP_F_RHO) static_cast<M *>(a.rho)[idx + c] = M(r[c]);
-      if (a.flags & STEP_F_VEL) {
+      if (g.flags & STEP_F_RHO) static_cast<M *>(a.rho)[idx + c] = M(r[c]);
+      if (g.flags & STEP_F_VEL) {
         M *u = static_cast<M *>(a.u);
 #pragma unroll
         for (int d = 0; d < 3; ++d) u[d * a.len + idx + c] = M(comp ? m[c][d] / r[c] : m[c][d]);
@@ -774,7 +829,7 @@ __device__ __forceinline__ int offc_rt(int j, int sx, int sy) {
 // for face cells, after it for link-pattern cells; the slot belongs to a
 // cell that is not computed, so its value does not change during the step).
 template <int Q, class S, bool ODD>
-__device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
+__device__ __forceinline__ void step_body_tile(const StepHot &g, const StepArgs &a, const int L) {
   using CD = Codec<S>;
   using C = typename CD::C;
   using M = typename CD::M;
@@ -795,12 +850,12 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
   const int plane = L / a.bpp;
   const int chunk = L - plane * a.bpp;
   const int c0 = chunk * TB;                // first cell of the tile in the plane's rows
-  const int n = min(TB, a.ny * a.sy - c0);  // cells in the tile
-  const long long idx0 = static_cast<long long>(plane + 1) * a.sx + a.sy + c0;
+  const int n = min(TB, g.ny * g.sy - c0);  // cells in the tile
+  const long long idx0 = static_cast<long long>(plane + 1) * g.sx + g.sy + c0;
   const long long len = a.len;
-  const char *f0 = a.fd[0];
+  const char *f0 = g.f;
   // first cell of row j's range (j at run time: scalar arithmetic)
-  auto row_base = [&](int j) -> long long { return ODD ? idx0 + offc_rt<Q>(j, a.sx, a.sy) : idx0; };
+  auto row_base = [&](int j) -> long long { return ODD ? idx0 + offc_rt<Q>(j, g.sx, g.sy) : idx0; };
   auto in_row = [](int k) -> int { return ODD ? inv_dir<Q>(k) : k; };   // incoming k, column t
   auto out_row = [](int k) -> int { return ODD ? k : inv_dir<Q>(k); };  // outgoing k, column t
 
@@ -808,11 +863,11 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
   const bool in_tile = t < n;
   const unsigned off = static_cast<unsigned>(c0 + (in_tile ? t : 0));
   const unsigned rw = static_cast<unsigned>((static_cast<unsigned long long>(off) * a.zmagic) >> 40);
-  const int zi = static_cast<int>(off - rw * static_cast<unsigned>(a.sy));
+  const int zi = static_cast<int>(off - rw * static_cast<unsigned>(g.sy));
   const int x = plane + 1, y = static_cast<int>(rw) + 1;
   const unsigned idx = static_cast<unsigned>(idx0 + (in_tile ? t : 0));
-  const bool column = in_tile && zi != 0 && zi != a.sy - 1;  // not a ghost column
-  const unsigned char code = column ? *gload<unsigned char>(reinterpret_cast<const char *>(a.code) + idx) : CODE_SKIP;
+  const bool column = in_tile && zi != 0 && zi != g.sy - 1;  // not a ghost column
+  const unsigned char code = column ? *gload<unsigned char>(reinterpret_cast<const char *>(g.code) + idx) : CODE_SKIP;
 
   // 1. rows into LDS: wavefront w moves rows w, w + NW, w + 2 NW, ..., lane
   // t elements e .. e + EPL - 1 (e = EPL (t % 64)) of each; every load is issued
@@ -828,9 +883,9 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
 #pragma unroll
     for (int i = 0; i < RPW; ++i) {
       const int j = w + i * NW;
-      const long long g = j < Q ? row_base(j) + e : 0;
-      vok[i] = g >= 0 && g + EPL <= len;
-      const unsigned gi = vok[i] ? static_cast<unsigned>(g) : 0u;
+      const long long gp = j < Q ? row_base(j) + e : 0;
+      vok[i] = gp >= 0 && gp + EPL <= len;
+      const unsigned gi = vok[i] ? static_cast<unsigned>(gp) : 0u;
       if (j < Q) xr[i] = *gload<V4>(f0 + static_cast<unsigned>(j) * a.qs32 + gi * ES);
     }
     bool fix = false;
@@ -841,11 +896,11 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
       for (int i = 0; i < RPW; ++i) {
         const int j = w + i * NW;
         if (j >= Q || vok[i]) continue;
-        const long long g = row_base(j) + e;
+        const long long gp = row_base(j) + e;
 #pragma unroll
         for (int q = 0; q < EPL; ++q)
-          if (g + q >= 0 && g + q < len)
-            xr[i][q] = *gload<S>(f0 + static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(g + q) * ES);
+          if (gp + q >= 0 && gp + q < len)
+            xr[i][q] = *gload<S>(f0 + static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(gp + q) * ES);
       }
     }
 #pragma unroll
@@ -861,46 +916,21 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
   }
 
   // face rule (as step_body)
-  const bool raw = (a.flags & STEP_F_RAW) != 0;
-  const unsigned fb = (!column || raw) ? 0u
-                                       : (x == 1 ? 1u : 0u) | (x == a.nx ? 2u : 0u) | (y == 1 ? 4u : 0u) |
-                                             (y == a.ny ? 8u : 0u) | (zi == 1 ? 16u : 0u) | (zi == a.nz ? 32u : 0u);
-  auto winner = [&](int k, C &val) -> int {
-    int wn = 0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const int cd = Lat<Q>::c[k][d];
-      if (cd == 0) continue;
-      const int fc = 2 * d + (cd > 0 ? 0 : 1);
-      const int cand = ((fb >> fc) & 1u) ? a.fface[fc] : 0;
-      if (cand > wn) {
-        wn = cand;
-        val = face_val<C>(a, fc, k);
-      }
-    }
-    return wn;
-  };
+  const bool raw = (g.flags & STEP_F_RAW) != 0;
+  const unsigned fb = (!column || raw) ? 0u : face_bits(g, x, y, zi);
   const bool faces = __any(fb != 0u);
   unsigned bmask = 0, cmask = 0;
-  if (faces) {
-#pragma unroll
-    for (int k = 1; k < Q; ++k) {
-      C unused;
-      const int md = winner(k, unused) & 3;
-      if (md == MODE_BOUNCE) bmask |= 1u << k;
-      if (md == MODE_CONST) cmask |= 1u << k;
-    }
-  }
+  if (faces) face_masks(g, fb, bmask, cmask);
   // the other slot of link k's pair: the outgoing row of k at column t - (offset of c_k)
-  auto other_col = [&](int k) -> int { return t - offc<Q>(k, a.sx, a.sy); };
+  auto other_col = [&](int k) -> int { return t - offc<Q>(k, g.sx, g.sy); };
   auto other_in_tile = [&](int k) -> bool {
     const int oc = other_col(k);
     return oc >= 0 && oc < n;
   };
   auto other_global = [&](int k) -> C {
     const int j = out_row(k);
-    const long long g = (ODD ? idx0 + offc<Q>(j, a.sx, a.sy) : idx0) + other_col(k);
-    return CD::ld(f0, static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(g) * ES);
+    const long long gp = (ODD ? idx0 + offc<Q>(j, g.sx, g.sy) : idx0) + other_col(k);
+    return CD::ld(f0, static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(gp) * ES);
   };
   C side[Q];  // bounce-back values of face cells from outside the tile
   if (faces) {
@@ -917,17 +947,9 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
   for (int k = 0; k < Q; ++k) v[k] = rd(in_row(k), tc);
   if (faces) {
 #pragma unroll
-    for (int k = 1; k < Q; ++k) {
-      if (!(((bmask | cmask) >> k) & 1u)) continue;
-      C val = C(0);
-      (void)winner(k, val);
-      if ((bmask >> k) & 1u) {
-        const C o = other_in_tile(k) ? rd(out_row(k), other_col(k)) : side[k];
-        v[k] = o + val;
-      } else {
-        v[k] = val;
-      }
-    }
+    for (int k = 1; k < Q; ++k)
+      if ((bmask >> k) & 1u) v[k] = other_in_tile(k) ? rd(out_row(k), other_col(k)) : side[k];
+    face_values<Q, C>(g, a, fb, v);
   }
   const bool live = code != CODE_SKIP;
   const bool bnd = live && code != CODE_FLUID;
@@ -951,8 +973,8 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
   // every lane has read what it needs from the rows before any lane writes them
   __syncthreads();
   C r, m[3];
-  const bool omega = (a.flags & STEP_F_OMEGA) != 0;
-  const bool comp = (a.flags & STEP_F_COMPRESSIBLE) != 0;
+  const bool omega = (g.flags & STEP_F_OMEGA) != 0;
+  const bool comp = (g.flags & STEP_F_COMPRESSIBLE) != 0;
   C om[3] = {C(0), C(0), C(0)};
   if (omega) {
 #pragma unroll
@@ -963,8 +985,8 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
 #pragma unroll
     for (int k = 0; k < Q; ++k)
       if (!((skipm >> k) & 1u)) row[out_row(k)][t] = LdsSlot<S>::put(CD::enc(v[k]));
-    if (a.flags & STEP_F_RHO) *gstore<M>(static_cast<char *>(a.rho) + sizeof(M) * idx) = M(r);
-    if (a.flags & STEP_F_VEL) {
+    if (g.flags & STEP_F_RHO) *gstore<M>(static_cast<char *>(a.rho) + sizeof(M) * idx) = M(r);
+    if (g.flags & STEP_F_VEL) {
       char *u = static_cast<char *>(a.u);
 #pragma unroll
       for (int d = 0; d < 3; ++d)
@@ -975,23 +997,23 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
 
   // 3. rows back to their ranges
   {
-    char *fw = a.fd[0];
+    char *fw = g.f;
 #pragma unroll
     for (int i = 0; i < RPW; ++i) {
       const int j = w + i * NW;
       if (j >= Q || e >= n) continue;
-      const long long g = row_base(j) + e;
-      if (e + EPL <= n && g >= 0 && g + EPL <= len) {
+      const long long gp = row_base(j) + e;
+      if (e + EPL <= n && gp >= 0 && gp + EPL <= len) {
         const L4 l4 = *reinterpret_cast<const L4 *>(&row[j][e]);
         V4 x4;
 #pragma unroll
         for (int q = 0; q < EPL; ++q) x4[q] = LdsSlot<S>::get(l4[q]);
-        *gstore<V4>(fw + static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(g) * ES) = x4;
+        *gstore<V4>(fw + static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(gp) * ES) = x4;
       } else {
 #pragma unroll
         for (int q = 0; q < EPL; ++q)
-          if (e + q < n && g + q >= 0 && g + q < len)
-            *gstore<S>(fw + static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(g + q) * ES) =
+          if (e + q < n && gp + q >= 0 && gp + q < len)
+            *gstore<S>(fw + static_cast<unsigned>(j) * a.qs32 + static_cast<unsigned>(gp + q) * ES) =
                 LdsSlot<S>::get(row[j][e + q]);
       }
     }
@@ -999,17 +1021,15 @@ __device__ __forceinline__ void step_body_tile(const StepArgs &a, const int L) {
 }
 
 template <int Q, class S, bool ODD>
-__global__ __launch_bounds__(STEP_TILE) void k_step_tile(const StepArgs *args) {
-  const StepArgs &a = *args;
-  const int b = ODD ? xcd_reverse(static_cast<int>(blockIdx.x), a.nblocks) : static_cast<int>(blockIdx.x);
-  step_body_tile<Q, S, ODD>(a, a.remap > 1 ? xcd_remap(b, a.nblocks, a.remap) : b);
+__global__ __launch_bounds__(STEP_TILE) void k_step_tile(const StepHot g, const StepArgs *args) {
+  step_body_tile<Q, S, ODD>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
 
-// The arguments live in device memory, not in the kernel-argument segment:
-// loads from the argument segment are invariant, and the compiler hoists all
-// of them (27 direction pointers, face tables) into scalar registers, runs
-// out of them and spills into vector registers (D3Q19 FP32: 103 VGPRs
-// instead of 70).  Loads through a plain pointer stay where they are used.
+// What a wavefront needs before its first load comes by value (StepHot); the
+// rest lives in device memory, not in the kernel-argument segment: loads from
+// that segment are invariant, the compiler hoists all of them (face values,
+// link tables) into scalar registers, runs out of them and spills into vector
+// registers.  Loads through a plain pointer stay where they are used.
 //
 // Odd steps take the chunks in reverse order (zig-zag over steps), each XCD
 // over its own share (xcd_reverse): a step then starts where the previous
@@ -1017,35 +1037,29 @@ __global__ __launch_bounds__(STEP_TILE) void k_step_tile(const StepArgs *args) {
 // holds.  Every cell's reads and writes in one step are its own (AA
 // pattern), so the order of the chunks does not change results.
 template <int Q, class S, bool ODD, bool PER, bool WIDE, int CL>
-__global__ __launch_bounds__(STEP_BLOCK) void k_step(const StepArgs *args) {
-  const StepArgs &a = *args;
-  const int b = ODD ? xcd_reverse(static_cast<int>(blockIdx.x), a.nblocks) : static_cast<int>(blockIdx.x);
-  step_body<Q, S, ODD, PER, WIDE, CL>(a, a.remap > 1 ? xcd_remap(b, a.nblocks, a.remap) : b);
+__global__ __launch_bounds__(STEP_BLOCK) void k_step(const StepHot g, const StepArgs *args) {
+  step_body<Q, S, ODD, PER, WIDE, CL>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
 
 // The matrix-core closure variant, held to 5 waves per SIMD (96 VGPRs).
 template <int Q, class S, bool ODD, bool PER, bool WIDE>
 __global__ __launch_bounds__(STEP_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_step_mfma(
-    const StepArgs *args) {
-  const StepArgs &a = *args;
-  const int b = ODD ? xcd_reverse(static_cast<int>(blockIdx.x), a.nblocks) : static_cast<int>(blockIdx.x);
-  step_body<Q, S, ODD, PER, WIDE, 2>(a, a.remap > 1 ? xcd_remap(b, a.nblocks, a.remap) : b);
+    const StepHot g, const StepArgs *args) {
+  step_body<Q, S, ODD, PER, WIDE, 2>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
 
 // The step with CPL cells per lane (step_body_run); same chunk order.  At
 // most STEP_RUN_BLOCK lanes per workgroup: four cells per lane hold about
 // 130 VGPRs, more than a 1024-lane workgroup allows without spilling.
 template <int Q, class S, bool ODD, int CPL>
-__global__ __launch_bounds__(STEP_RUN_BLOCK) void k_step_run(const StepArgs *args) {
-  const StepArgs &a = *args;
-  const int b = ODD ? xcd_reverse(static_cast<int>(blockIdx.x), a.nblocks) : static_cast<int>(blockIdx.x);
-  step_body_run<Q, S, ODD, CPL>(a, a.remap > 1 ? xcd_remap(b, a.nblocks, a.remap) : b);
+__global__ __launch_bounds__(STEP_RUN_BLOCK) void k_step_run(const StepHot g, const StepArgs *args) {
+  step_body_run<Q, S, ODD, CPL>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
 
 // The incoming populations of every computed cell for the next step.
 template <int Q, class S, bool ODD, bool PER>
-__global__ __launch_bounds__(STEP_BLOCK) void k_peek(const StepArgs *args, void *out) {
-  step_body<Q, S, ODD, PER, false, 0, true>(*args, static_cast<int>(blockIdx.x), out);
+__global__ __launch_bounds__(STEP_BLOCK) void k_peek(const StepHot g, const StepArgs *args, void *out) {
+  step_body<Q, S, ODD, PER, false, 0, true>(g, *args, static_cast<int>(blockIdx.x), out);
 }
 
 // asl::ComputeSurfaceForceMap / ComputeSurfaceFluxMap (src/num/aslLBGKBC.cxx:
@@ -1228,7 +1242,7 @@ template <int Q, class S, bool ODD, bool PER, bool WIDE>
 __global__ __launch_bounds__(STEP_BLOCK) void k_step_batch(const StepArgs *desc, const uint2 *ent) {
   const int b = static_cast<int>(blockIdx.x);
   const uint2 e = ent[ODD ? xcd_reverse(b, static_cast<int>(gridDim.x)) : b];
-  step_body<Q, S, ODD, PER, WIDE>(desc[e.x], static_cast<int>(e.y));
+  step_body<Q, S, ODD, PER, WIDE>(desc[e.x].g, desc[e.x], static_cast<int>(e.y));
 }
 
 // The same with LDS-staged tiles (entries are tiles of STEP_TILE cells).
@@ -1236,7 +1250,7 @@ template <int Q, class S, bool ODD>
 __global__ __launch_bounds__(STEP_TILE) void k_step_batch_tile(const StepArgs *desc, const uint2 *ent) {
   const int b = static_cast<int>(blockIdx.x);
   const uint2 e = ent[ODD ? xcd_reverse(b, static_cast<int>(gridDim.x)) : b];
-  step_body_tile<Q, S, ODD>(desc[e.x], static_cast<int>(e.y));
+  step_body_tile<Q, S, ODD>(desc[e.x].g, desc[e.x], static_cast<int>(e.y));
 }
 
 // Closure features of every interior cell of a periodic D3Q19 lattice: the
@@ -1249,7 +1263,7 @@ __global__ __launch_bounds__(256) void k_closure_features(const StepArgs *args, 
   using CD = Codec<S>;
   constexpr int Q = 19;
   constexpr unsigned ES = sizeof(S);
-  const StepArgs &a = *args;
+  const StepHot &a = args->g;
   const long long c = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
   if (c >= static_cast<long long>(a.nx) * a.ny * a.nz) return;
   const int z = static_cast<int>(c % a.nz) + 1;
@@ -1259,14 +1273,13 @@ __global__ __launch_bounds__(256) void k_closure_features(const StepArgs *args, 
   float v[Q];
 #pragma unroll
   for (int k = 0; k < Q; ++k) {
-    // each direction from its own base (a.qs32 is 0 on lattices over 4 GiB)
-    if (ODD) {
+        if (ODD) {
       const unsigned src = static_cast<unsigned>(wrap1(x - Lat<Q>::c[k][0], a.nx) * a.sx +
                                                  wrap1(y - Lat<Q>::c[k][1], a.ny) * a.sy +
                                                  wrap1(z - Lat<Q>::c[k][2], a.nz));
-      v[k] = CD::ld(a.fd[inv_dir<Q>(k)], ES * src);
+      v[k] = CD::ld(a.f + inv_dir<Q>(k) * a.qs, ES * src);
     } else {
-      v[k] = CD::ld(a.fd[k], ES * idx);
+      v[k] = CD::ld(a.f + k * a.qs, ES * idx);
     }
   }
   float r, m[3], f7[7];
@@ -1414,8 +1427,6 @@ __global__ __launch_bounds__(BLOCK) void k_unpermute(const UnpermuteArgs a) {
   }
 }
 
-constexpr int RED_MAX_BLOCKS = 1024;
-
 // FP64 mass / momentum / kinetic energy over computation nodes.
 template <int Q, class S>
 __global__ __launch_bounds__(BLOCK) void k_reduce(const ReduceArgs a) {
@@ -1478,45 +1489,46 @@ __global__ __launch_bounds__(BLOCK) void k_reduce_final(const double *partial, i
 
 template <int Q, class S, bool ODD, bool PER>
 hipError_t step_w(bool wide, const StepLaunch &a, hipStream_t s) {
-  const dim3 grid(a.nblocks), block(a.block);
+  const dim3 grid(a.hot.nchunks), block(a.hot.block);
   if (a.tile) {
     // the host sends only these: non-periodic, under 4 GiB, no per-cell relaxation, one cell per lane
-    if (PER || wide || a.variant || a.cpl != 1 || a.block != STEP_TILE) return hipErrorInvalidValue;
-    if constexpr (!PER) hipLaunchKernelGGL((k_step_tile<Q, S, ODD>), grid, block, 0, s, a.args);
+    if (PER || wide || a.variant || a.cpl != 1 || a.hot.block != STEP_TILE) return hipErrorInvalidValue;
+    if constexpr (!PER) hipLaunchKernelGGL((k_step_tile<Q, S, ODD>), grid, block, 0, s, a.hot, a.args);
     return hipGetLastError();
   }
   if (a.cpl > 1) {
     if (PER || wide || a.variant) return hipErrorInvalidValue;  // the host sends these one cell per lane
     if (a.cpl == 2)
-      hipLaunchKernelGGL((k_step_run<Q, S, ODD, 2>), grid, block, 0, s, a.args);
+      hipLaunchKernelGGL((k_step_run<Q, S, ODD, 2>), grid, block, 0, s, a.hot, a.args);
     else if (a.cpl == 4)
-      hipLaunchKernelGGL((k_step_run<Q, S, ODD, 4>), grid, block, 0, s, a.args);
+      hipLaunchKernelGGL((k_step_run<Q, S, ODD, 4>), grid, block, 0, s, a.hot, a.args);
     else
       return hipErrorInvalidValue;
     return hipGetLastError();
   }
+  // (periodic lattices never choose between two slots: one addressing variant)
   if (a.variant == 2) {  // the closure on the matrix cores: D3Q19 with FP32 collision (checked by the host)
     if constexpr (Q == 19 && sizeof(typename Codec<S>::C) == 4) {
-      if (wide)
-        hipLaunchKernelGGL((k_step_mfma<Q, S, ODD, PER, true>), grid, block, 0, s, a.args);
+      if (wide && !PER)
+        hipLaunchKernelGGL((k_step_mfma<Q, S, ODD, PER, !PER>), grid, block, 0, s, a.hot, a.args);
       else
-        hipLaunchKernelGGL((k_step_mfma<Q, S, ODD, PER, false>), grid, block, 0, s, a.args);
+        hipLaunchKernelGGL((k_step_mfma<Q, S, ODD, PER, false>), grid, block, 0, s, a.hot, a.args);
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;
     }
   }
   if (a.variant == 1) {  // LBGKTurbulence or the FP32 closure
-    if (wide)
-      hipLaunchKernelGGL((k_step<Q, S, ODD, PER, true, 1>), grid, block, 0, s, a.args);
+    if (wide && !PER)
+      hipLaunchKernelGGL((k_step<Q, S, ODD, PER, !PER, 1>), grid, block, 0, s, a.hot, a.args);
     else
-      hipLaunchKernelGGL((k_step<Q, S, ODD, PER, false, 1>), grid, block, 0, s, a.args);
+      hipLaunchKernelGGL((k_step<Q, S, ODD, PER, false, 1>), grid, block, 0, s, a.hot, a.args);
     return hipGetLastError();
   }
-  if (wide)
-    hipLaunchKernelGGL((k_step<Q, S, ODD, PER, true, 0>), grid, block, 0, s, a.args);
+  if (wide && !PER)
+    hipLaunchKernelGGL((k_step<Q, S, ODD, PER, !PER, 0>), grid, block, 0, s, a.hot, a.args);
   else
-    hipLaunchKernelGGL((k_step<Q, S, ODD, PER, false, 0>), grid, block, 0, s, a.args);
+    hipLaunchKernelGGL((k_step<Q, S, ODD, PER, false, 0>), grid, block, 0, s, a.hot, a.args);
   return hipGetLastError();
 }
 
@@ -1528,8 +1540,8 @@ hipError_t batch_w(bool wide, const BatchLaunch &b, hipStream_t s) {
     if constexpr (!PER) hipLaunchKernelGGL((k_step_batch_tile<Q, S, ODD>), grid, block, 0, s, b.desc, b.ent);
     return hipGetLastError();
   }
-  if (wide)
-    hipLaunchKernelGGL((k_step_batch<Q, S, ODD, PER, true>), grid, block, 0, s, b.desc, b.ent);
+  if (wide && !PER)
+    hipLaunchKernelGGL((k_step_batch<Q, S, ODD, PER, !PER>), grid, block, 0, s, b.desc, b.ent);
   else
     hipLaunchKernelGGL((k_step_batch<Q, S, ODD, PER, false>), grid, block, 0, s, b.desc, b.ent);
   return hipGetLastError();
@@ -1541,23 +1553,16 @@ hipError_t step_q_s(bool odd, bool per, bool wide, const StepLaunch &a, hipStrea
   return odd ? step_w<Q, S, true, false>(wide, a, s) : step_w<Q, S, false, false>(wide, a, s);
 }
 
+// This object's template (the library holds one object per template).
 template <template <int, class> class F, class... Args>
-hipError_t dispatch(int q, int dtype, Args &&...args) {
-#define ASLHIP_DT(QQ)                                                   \
-  switch (dtype) {                                                      \
-    case ASLHIP_F32: return F<QQ, float>::run(args...);                 \
-    case ASLHIP_F64: return F<QQ, double>::run(args...);                \
-    case ASLHIP_BF16: return F<QQ, unsigned short>::run(args...);       \
-    case ASLHIP_F16: return F<QQ, _Float16>::run(args...);              \
-    default: return hipErrorInvalidValue;                               \
-  }
-  switch (q) {
-    case 15: ASLHIP_DT(15)
-    case 19: ASLHIP_DT(19)
-    case 27: ASLHIP_DT(27)
+hipError_t dispatch(int dtype, Args &&...args) {
+  switch (dtype) {
+    case ASLHIP_F32: return F<ASLHIP_Q, float>::run(args...);
+    case ASLHIP_F64: return F<ASLHIP_Q, double>::run(args...);
+    case ASLHIP_BF16: return F<ASLHIP_Q, unsigned short>::run(args...);
+    case ASLHIP_F16: return F<ASLHIP_Q, _Float16>::run(args...);
     default: return hipErrorInvalidValue;
   }
-#undef ASLHIP_DT
 }
 
 template <int Q, class S>
@@ -1591,17 +1596,17 @@ struct InitF {
 template <int Q, class S>
 struct PeekF {
   static hipError_t run(bool odd, bool per, const StepLaunch &a, void *out, hipStream_t s) {
-    const dim3 grid(a.nblocks), block(a.block);
+    const dim3 grid(a.hot.nchunks), block(a.hot.block);
     if (per) {
       if (odd)
-        hipLaunchKernelGGL((k_peek<Q, S, true, true>), grid, block, 0, s, a.args, out);
+        hipLaunchKernelGGL((k_peek<Q, S, true, true>), grid, block, 0, s, a.hot, a.args, out);
       else
-        hipLaunchKernelGGL((k_peek<Q, S, false, true>), grid, block, 0, s, a.args, out);
+        hipLaunchKernelGGL((k_peek<Q, S, false, true>), grid, block, 0, s, a.hot, a.args, out);
     } else {
       if (odd)
-        hipLaunchKernelGGL((k_peek<Q, S, true, false>), grid, block, 0, s, a.args, out);
+        hipLaunchKernelGGL((k_peek<Q, S, true, false>), grid, block, 0, s, a.hot, a.args, out);
       else
-        hipLaunchKernelGGL((k_peek<Q, S, false, false>), grid, block, 0, s, a.args, out);
+        hipLaunchKernelGGL((k_peek<Q, S, false, false>), grid, block, 0, s, a.hot, a.args, out);
     }
     return hipGetLastError();
   }
@@ -1646,64 +1651,7 @@ struct ReduceF {
   }
 };
 
-}  // namespace
-
-// Staging memory of aslhip_read_f_noalloc: a file-scope device array, so the
-// entry point needs no allocation.  In host code `scratch` only names the
-// symbol; its device address on each GPU comes from hipGetSymbolAddress (the
-// array's name is never passed to a kernel or a copy).
-static __device__ __align__(256) unsigned char scratch[ASLHIP_NOALLOC_SCRATCH_BYTES];
-namespace {
-constexpr int SCRATCH_MAX_DEVICES = 64;
-std::mutex scratch_mu;
-void *scratch_ptr[SCRATCH_MAX_DEVICES] = {};  // its address on each device (null: not looked up yet)
-}  // namespace
-
-hipError_t noalloc_scratch(void **ptr) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= SCRATCH_MAX_DEVICES) return hipErrorInvalidDevice;
-  std::lock_guard<std::mutex> lock(scratch_mu);
-  if (!scratch_ptr[dev]) {
-    void *p = nullptr;
-    e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess) return e;
-    scratch_ptr[dev] = p;
-  }
-  *ptr = scratch_ptr[dev];
-  return hipSuccess;
-}
-
-int reduce_blocks(int len) {
-  const int nb = (len + BLOCK - 1) / BLOCK;
-  return nb < RED_MAX_BLOCKS ? (nb < 1 ? 1 : nb) : RED_MAX_BLOCKS;
-}
-
-hipError_t launch_step(int q, int dtype, bool odd, bool periodic, bool wide, const StepLaunch &a, hipStream_t s) {
-  return dispatch<StepF>(q, dtype, odd, periodic, wide, a, s);
-}
-hipError_t launch_step_batch(int q, int dtype, bool odd, bool periodic, bool wide, const BatchLaunch &b,
-                             hipStream_t s) {
-  return dispatch<BatchF>(q, dtype, odd, periodic, wide, b, s);
-}
-hipError_t launch_vlinks(int q, int dtype, const VLinkArgs &a, hipStream_t s) {
-  return dispatch<VLinkF>(q, dtype, a, s);
-}
-hipError_t launch_init(int q, int dtype, const InitArgs &a, hipStream_t s) { return dispatch<InitF>(q, dtype, a, s); }
-hipError_t launch_peek(int q, int dtype, bool odd, bool periodic, const StepLaunch &a, void *out, hipStream_t s) {
-  return dispatch<PeekF>(q, dtype, odd, periodic, a, out, s);
-}
-hipError_t launch_surface(int q, int dtype, const SurfaceArgs &a, hipStream_t s) {
-  return dispatch<SurfaceF>(q, dtype, a, s);
-}
-hipError_t launch_vis(int q, int dtype, const VisArgs &a, hipStream_t s) { return dispatch<VisF>(q, dtype, a, s); }
-hipError_t launch_write_f(int q, int dtype, const WriteFArgs &a, hipStream_t s) {
-  return dispatch<WriteFF>(q, dtype, a, s);
-}
-hipError_t launch_unpermute(int q, int dtype, const UnpermuteArgs &a, hipStream_t s) {
-  return dispatch<UnpermuteF>(q, dtype, a, s);
-}
+#if ASLHIP_Q == 19
 template <class T>
 void closure_features_w(bool odd, dim3 grid, const StepArgs *args, float *out, hipStream_t s) {
   if (odd)
@@ -1711,7 +1659,35 @@ void closure_features_w(bool odd, dim3 grid, const StepArgs *args, float *out, h
   else
     hipLaunchKernelGGL((k_closure_features<T, false>), grid, dim3(256), 0, s, args, out);
 }
+#endif
 
+}  // namespace
+
+#define ASLHIP_PASTE_(a, b) a##b
+#define ASLHIP_PASTE(a, b) ASLHIP_PASTE_(a, b)
+const KernelTable &ASLHIP_PASTE(kernels_q, ASLHIP_Q)() {
+  static const KernelTable t = {
+      [](int dt, bool odd, bool per, bool wide, const StepLaunch &a, hipStream_t s) {
+        return dispatch<StepF>(dt, odd, per, wide, a, s);
+      },
+      [](int dt, bool odd, bool per, bool wide, const BatchLaunch &b, hipStream_t s) {
+        return dispatch<BatchF>(dt, odd, per, wide, b, s);
+      },
+      [](int dt, const VLinkArgs &a, hipStream_t s) { return dispatch<VLinkF>(dt, a, s); },
+      [](int dt, const InitArgs &a, hipStream_t s) { return dispatch<InitF>(dt, a, s); },
+      [](int dt, const WriteFArgs &a, hipStream_t s) { return dispatch<WriteFF>(dt, a, s); },
+      [](int dt, bool odd, bool per, const StepLaunch &a, void *out, hipStream_t s) {
+        return dispatch<PeekF>(dt, odd, per, a, out, s);
+      },
+      [](int dt, const SurfaceArgs &a, hipStream_t s) { return dispatch<SurfaceF>(dt, a, s); },
+      [](int dt, const VisArgs &a, hipStream_t s) { return dispatch<VisF>(dt, a, s); },
+      [](int dt, const UnpermuteArgs &a, hipStream_t s) { return dispatch<UnpermuteF>(dt, a, s); },
+      [](int dt, const ReduceArgs &a, double *out, hipStream_t s) { return dispatch<ReduceF>(dt, a, out, s); },
+  };
+  return t;
+}
+
+#if ASLHIP_Q == 19
 hipError_t launch_closure_features(int dtype, bool odd, const StepArgs *args, long long ncell, float *out,
                                   hipStream_t s) {
   const dim3 grid(static_cast<unsigned>((ncell + 255) / 256));
@@ -1723,8 +1699,6 @@ hipError_t launch_closure_features(int dtype, bool odd, const StepArgs *args, lo
   }
   return hipGetLastError();
 }
-hipError_t launch_reduce(int q, int dtype, const ReduceArgs &a, double *out, hipStream_t s) {
-  return dispatch<ReduceF>(q, dtype, a, out, s);
-}
+#endif
 
 }  // namespace aslhip

@@ -24,55 +24,75 @@ enum : unsigned {
   STEP_F_CLOSURE = 32u,      // per-cell relaxation time from the closure network
   STEP_F_CLOSURE_MFMA = 64u, // ... evaluated with BF16 matrix instructions
   STEP_F_TURB = 128u,        // LBGKTurbulence's relaxation limiter
-  STEP_F_COUNT = 256u,       // number of flag combinations
+};
+
+// The part of a step's description that every wavefront reads before its
+// first load: passed by value to the single-lattice kernels (scalar loads
+// from the argument segment instead of a chain through device memory; with
+// the face rule below 5.9 -> 4.6 us per step of a 16^3 box, D3Q19 FP32),
+// read from StepArgs by the batch kernels.
+//
+// Work items are the interior cells j = (x ny + y) nz + z (0-based interior
+// coordinates) in ASL's order, or runs of cpl of them; a chunk is `block`
+// consecutive ones, so only the last chunk of a launch is partly empty,
+// whatever the plane size.  A launch covers the interior planes that hold
+// items first .. first + count - 1.  The LDS-staged tiles keep to the rows of
+// one plane (chunks of STEP_TILE cells, ghost columns included).
+//
+// Face rule.  A link k into a cell is claimed by the faces the cell lies on
+// whose inward direction e_f has c_k . e_f > 0; the BC executed last wins.
+// Entry j (ascending execution slots; entries past the last one claim no
+// links) names a face: fpos its bit, 4 bits per entry (0..5: X0 XE Y0 YE Z0
+// ZE), flinks the links it claims, bit j of fbounce whether it bounces (else
+// a constant); bit f of fvalued: face f has values to add or set.  Cells
+// whose links this rule does not describe (next to map obstacles, computed
+// ghost cells) carry CODE_FLUID_BC / CODE_GHOST and a link pattern instead.
+struct StepHot {
+  char *f;                    // first direction array
+  const unsigned char *code;  // packed cell types
+  unsigned long long qs;      // bytes between direction arrays
+  unsigned long long mrow;    // floor(2^64 / row items) + 1 (0: one item per row): item -> row, see udivm
+  unsigned long long mplane;  // floor(2^64 / ny) + 1 (0: one row): row -> plane
+  unsigned long long mspan;   // floor(2^64 / (8 remap)) + 1: chunk -> group of 8 runs
+  float inv_row, inv_ny;      // 1 / row items, 1 / ny (lane offsets, see lane_div)
+  int sx, sy;                 // strides of the layout: Sy*Sz and Sz
+  int nx, ny, nz;             // interior size
+  int rowi;                   // items per row: nz (one cell per lane) or nz / cpl
+  int block;                  // workgroup size (a multiple of 64, at most STEP_BLOCK)
+  unsigned first, count;      // items of this launch
+  int nchunks;                // workgroups of this launch
+  int remap;                  // runs of that many chunks per XCD (see xcd_remap; 1: the hardware order)
+  unsigned flags;             // STEP_F_*
+  unsigned fpos;              // face of each entry of the face rule
+  unsigned flinks[6];         // links each entry claims
+  unsigned fbounce, fvalued;  // bit j: entry j bounces; bit f: face f has values
 };
 
 // One fused collide+stream pass (AA pattern) over the ghost-inclusive block.
-// The launch is a 1-D grid of chunks of `block` lanes of the interior planes
-// x = 1..nx: with cpl = 1 a lane is one cell of rows y = 1..ny, every z
-// including the two ghost columns; with cpl = 2 or 4 a lane is a run of cpl
-// interior cells z0 .. z0 + cpl - 1 (nz a multiple of cpl).
-//
-// Links into cells of the six face layers are resolved from the cell's
-// coordinates: for each face, fface[f] = slot * 4 + mode of the last
-// executed slice BC on that face (0: none) and fval*[f][k] its value for
-// direction k.  A link k into a cell is claimed by the faces the cell lies on
-// whose inward direction e_f has c_k . e_f > 0; the highest slot wins (the
-// BC executed last).  Cells whose links this rule does not describe (next to
-// map obstacles, computed ghost cells) carry CODE_FLUID_BC / CODE_GHOST and a
-// link pattern instead.
 struct StepArgs {
-  char *fd[27];               // base of each direction array
+  StepHot g;                  // one cell per lane over the whole lattice (runs of cells: cpl > 1)
   unsigned qs32;              // bytes between direction arrays (if all fit in 4 GiB)
-  int sx, sy;                 // strides of the layout: Sy*Sz and Sz
-  int nx, ny, nz;             // interior size
   int len;                    // ghost-inclusive cell count
-  int block;                  // workgroup size (a multiple of 64, at most STEP_BLOCK)
-  int bpp;                    // block-cell chunks per plane
-  int nblocks;                // bpp * nx
-  unsigned long long zmagic;  // ceil(2^40 / sy): row = (off * zmagic) >> 40
-  int remap;                  // > 1: runs of that many chunks per XCD (see xcd_remap)
-  int cpl;                    // cells per lane along z (1: one cell per lane, ghost columns included)
-  int nzv;                    // runs per row, nz / cpl (cpl > 1)
-  unsigned long long vmagic;  // ceil(2^40 / nzv): row = (lane * vmagic) >> 40
+  int bpp;                    // LDS-staged tiles: chunks per plane
+  unsigned long long zmagic;  // ceil(2^40 / sy): row = (off * zmagic) >> 40 (tiles)
+  int cpl;                    // cells per lane along z
   int tile;                   // 1: LDS-staged tiles (block = STEP_TILE, cpl = 1)
-  int fface[6];               // per face: slot * 4 + mode of its winning slice BC
-  float fval32[6][27];        // per face and direction: addend / constant (FP32 lattices)
-  double fval64[6][27];       // the same for FP64 lattices
+  unsigned fbounces;          // bit f: face f bounces
+  unsigned fbeats[6];         // per face: the faces whose BC is executed later
+  float fval32[6][28];        // per face and direction: addend / constant (FP32 lattices)
+  double fval64[6][28];       // the same for FP64 lattices
   float om32[3];              // angular velocity of the frame (STEP_F_OMEGA)
   double om64[3];
   const ClosureParams *cl;    // closure network (STEP_F_CLOSURE)
   float cl_tau0;              // 3 nu + 1/2 in float
   float nu32;                 // viscosity (STEP_F_TURB)
   double nu64;
-  const unsigned char *code;  // packed cell types
   const unsigned short *pat;  // link pattern of CODE_FLUID_BC / CODE_GHOST cells
   const LinkRec *rec;         // link patterns
   const unsigned char *mode;  // resolution mode of each BC slot
   const void *val;            // [slot][Q] addend or constant, compute type
   void *rho, *u;              // macroscopic outputs (ASL layout)
   double w;                   // relaxation rate (exact in the compute type)
-  unsigned flags;
 };
 
 // Several lattices advanced by one launch of the step kernel: desc[l] is
@@ -179,15 +199,33 @@ struct ReduceArgs {
   double *partial;  // 5 per block
 };
 
-// One step of one lattice: args points to a StepArgs in device memory.
+// One step of one lattice: hot describes this launch, args points to the
+// lattice's StepArgs in device memory.
 struct StepLaunch {
+  StepHot hot;
   const StepArgs *args;
-  int nblocks;
-  int block;
   int variant;   // per-cell relaxation: 0 none, 1 LBGKTurbulence or the FP32 closure, 2 the matrix-core closure
   int cpl;       // cells per lane (2 or 4: the run variant; non-periodic, under 4 GiB, no closure)
   int tile;      // 1: LDS-staged tiles of STEP_TILE cells (same restrictions, cpl 1, block STEP_TILE)
 };
+
+// The launchers of one template's object (kernels.hip compiled with ASLHIP_Q
+// 15, 19 or 27); first argument: population type.
+struct KernelTable {
+  hipError_t (*step)(int, bool odd, bool periodic, bool wide, const StepLaunch &, hipStream_t);
+  hipError_t (*batch)(int, bool odd, bool periodic, bool wide, const BatchLaunch &, hipStream_t);
+  hipError_t (*vlinks)(int, const VLinkArgs &, hipStream_t);
+  hipError_t (*init)(int, const InitArgs &, hipStream_t);
+  hipError_t (*write_f)(int, const WriteFArgs &, hipStream_t);
+  hipError_t (*peek)(int, bool odd, bool periodic, const StepLaunch &, void *out, hipStream_t);
+  hipError_t (*surface)(int, const SurfaceArgs &, hipStream_t);
+  hipError_t (*vis)(int, const VisArgs &, hipStream_t);
+  hipError_t (*unpermute)(int, const UnpermuteArgs &, hipStream_t);
+  hipError_t (*reduce)(int, const ReduceArgs &, double *out, hipStream_t);
+};
+const KernelTable &kernels_q15();
+const KernelTable &kernels_q19();
+const KernelTable &kernels_q27();
 
 // wide: the populations span more than 4 GiB (64-bit per-lane addresses).
 hipError_t launch_step(int q, int dtype, bool odd, bool periodic, bool wide, const StepLaunch &a, hipStream_t s);

@@ -130,8 +130,7 @@ struct aslhip_lattice {
   VLink *vl = nullptr;
   VLinkBC *vlbc = nullptr;
   double *red_partial = nullptr, *red_out = nullptr;
-  // [2][STEP_F_COUNT]: step arguments of even and odd steps for each value of
-  // StepArgs::flags (the two parities differ when only even steps run tiles)
+  // step arguments of even and odd steps (they differ when only even steps run tiles)
   StepArgs *d_args = nullptr;
   std::vector<StepArgs> h_args;  // host copy of d_args (empty: not uploaded yet)
   // Captured runs of plain steps (the velocity-map link fills included):
@@ -646,43 +645,73 @@ int step_workgroup(const aslhip_lattice *h) {
   return effective_cpl(h) > 1 && h->tune_block > STEP_RUN_BLOCK ? STEP_RUN_BLOCK : h->tune_block;
 }
 
-// Kernel arguments of one step of h (flags filled in by the caller).  With
-// block and cpl 0 the lattice's own tuning for a step of that parity (LDS-
-// staged tiles included), else one cell per lane in workgroups of that size.
-StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd = false) {
-  StepArgs a;
-  std::memset(&a, 0, sizeof a);  // compared bytewise by upload_args
-  for (int k = 0; k < 27; ++k) a.fd[k] = k < h->Q ? h->f + k * h->qs_bytes : nullptr;
-  a.qs32 = is_wide(h) ? 0u : static_cast<unsigned>(h->qs_bytes);
-  for (int fc = 0; fc < 6; ++fc) {
-    a.fface[fc] = h->fface[fc];
-    for (int k = 0; k < 27; ++k) {
-      a.fval32[fc][k] = h->fval32[fc][k];
-      a.fval64[fc][k] = h->fval64[fc][k];
+// The divisor d of udivm (kernels.hip); 0 stands for d = 1.
+unsigned long long udiv_magic(unsigned d) { return d <= 1 ? 0ULL : ~0ULL / d + 1ULL; }
+
+// The face rule's entries (StepHot): the faces that have a slice BC, by the
+// execution slot of the last one on them.
+void face_entries(const aslhip_lattice *h, StepArgs &a) {
+  std::vector<int> fc;
+  for (int f = 0; f < 6; ++f)
+    if (h->fface[f]) fc.push_back(f);
+  std::stable_sort(fc.begin(), fc.end(), [h](int p, int q) { return h->fface[p] < h->fface[q]; });
+  for (size_t j = 0; j < fc.size(); ++j) {
+    const int f = fc[j], axis = f / 2, in = f % 2 == 0 ? 1 : -1;
+    const bool bounce = (h->fface[f] & 3) == MODE_BOUNCE;
+    bool valued = !bounce;
+    for (int k = 0; k < h->Q; ++k) {
+      a.fval32[f][k] = h->fval32[f][k];
+      a.fval64[f][k] = h->fval64[f][k];
+      valued = valued || (h->celem == 8 ? h->fval64[f][k] != 0. : h->fval32[f][k] != 0.f);
+      if (h->t.c[k][axis] == in) a.g.flinks[j] |= 1u << k;
     }
+    a.g.fpos |= static_cast<unsigned>(f) << (4 * j);
+    if (bounce) a.g.fbounce |= 1u << j;
+    if (bounce) a.fbounces |= 1u << f;
+    if (valued) a.g.fvalued |= 1u << f;
+    for (int p : fc)  // the same BC on two faces gives a shared link one value: neither beats the other
+      if (h->fface[p] / 4 > h->fface[f] / 4) a.fbeats[f] |= 1u << p;
   }
-  a.sx = h->sx;
-  a.sy = h->sy;
-  a.nx = h->n[0];
-  a.ny = h->n[1];
-  a.nz = h->n[2];
+}
+
+// Kernel arguments of one step of h over the whole lattice (STEP_F_* of the
+// lattice's parameters).  With block and cpl 0 the lattice's own tuning for a
+// step of that parity (LDS-staged tiles included), else one cell per lane in
+// workgroups of that size, or tiles if asked for.
+StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd = false, bool tiles = false) {
+  StepArgs a;
+  std::memset(static_cast<void *>(&a), 0, sizeof a);  // compared bytewise by upload_args
+  StepHot &g = a.g;
+  g.f = h->f;
+  g.code = h->code;
+  g.qs = static_cast<unsigned long long>(h->qs_bytes);
+  a.qs32 = is_wide(h) ? 0u : static_cast<unsigned>(h->qs_bytes);
+  face_entries(h, a);
+  g.sx = h->sx;
+  g.sy = h->sy;
+  g.nx = h->n[0];
+  g.ny = h->n[1];
+  g.nz = h->n[2];
   a.len = h->len;
   a.cpl = cpl > 0 ? cpl : effective_cpl(h);
-  a.block = block > 0 ? block : h->tune_block;
-  if (a.cpl > 1 && a.block > STEP_RUN_BLOCK) a.block = STEP_RUN_BLOCK;
+  g.block = block > 0 ? block : h->tune_block;
+  if (a.cpl > 1 && g.block > STEP_RUN_BLOCK) g.block = STEP_RUN_BLOCK;
   const int lds = effective_lds(h);
-  a.tile = block <= 0 && cpl <= 0 && (lds == 1 || (lds == 2 && !odd)) ? 1 : 0;
-  if (a.tile) a.block = STEP_TILE;
+  a.tile = tiles || (block <= 0 && cpl <= 0 && (lds == 1 || (lds == 2 && !odd))) ? 1 : 0;
+  if (a.tile) g.block = STEP_TILE;
 
-  a.nzv = h->n[2] / a.cpl;
-  // lanes per plane: every cell of the rows (ghost columns included), or the runs of the interior
-  const int lanes = a.cpl > 1 ? h->n[1] * a.nzv : h->n[1] * h->sy;
-  a.bpp = (lanes + a.block - 1) / a.block;
-  a.nblocks = a.bpp * h->n[0];
+  g.rowi = h->n[2] / a.cpl;
+  g.mrow = udiv_magic(static_cast<unsigned>(g.rowi));
+  g.mplane = udiv_magic(static_cast<unsigned>(g.ny));
+  g.inv_row = 1.f / static_cast<float>(g.rowi);
+  g.inv_ny = 1.f / static_cast<float>(g.ny);
+  g.first = 0;
+  g.count = static_cast<unsigned>(g.nx) * static_cast<unsigned>(g.ny) * static_cast<unsigned>(g.rowi);
+  a.bpp = (g.ny * g.sy + STEP_TILE - 1) / STEP_TILE;
+  g.nchunks = a.tile ? a.bpp * g.nx : static_cast<int>((static_cast<long long>(g.count) + g.block - 1) / g.block);
   a.zmagic = ((1ULL << 40) + (unsigned long long)h->sy - 1) / (unsigned long long)h->sy;
-  a.vmagic = ((1ULL << 40) + (unsigned long long)a.nzv - 1) / (unsigned long long)a.nzv;
-  a.remap = h->tune_remap;
-  a.code = h->code;
+  g.remap = std::max(1, h->tune_remap);
+  g.mspan = udiv_magic(8u * static_cast<unsigned>(g.remap));
   a.pat = h->pat;
   a.rec = h->rec;
   a.mode = h->mode;
@@ -698,7 +727,7 @@ StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd
   a.cl_tau0 = 3.f * static_cast<float>(h->nu) + .5f;
   a.nu32 = static_cast<float>(h->nu);
   a.nu64 = h->nu;
-  a.flags = base_flags(h);
+  g.flags = base_flags(h);
   return a;
 }
 
@@ -717,36 +746,31 @@ int prepare(aslhip_lattice *h, bool allow_open) {
   return h->dirty ? finalize_impl(h, allow_open) : 0;
 }
 
-// Brings the device copies of the step arguments (one per flags value) up to
-// date; they change with the BC tables, viscosity, compressibility and tuning.
+// Brings the device copies of the step arguments up to date; they change with
+// the BC tables, viscosity, compressibility and tuning.  Captured runs carry
+// the by-value part (StepHot) and are dropped when it changes.
 int upload_args(aslhip_lattice *h) {
   const StepArgs base[2] = {step_args(h, 0, 0, false), step_args(h, 0, 0, true)};
   if (!h->h_args.empty()) {
-    if (std::memcmp(&base[0], &h->h_args[base[0].flags], sizeof(StepArgs)) == 0 &&
-        std::memcmp(&base[1], &h->h_args[STEP_F_COUNT + base[1].flags], sizeof(StepArgs)) == 0)
-      return 0;
+    if (std::memcmp(base, h->h_args.data(), sizeof base) == 0) return 0;
+    for (int p = 0; p < 2; ++p)
+      if (std::memcmp(&base[p].g, &h->h_args[p].g, sizeof(StepHot)) != 0) drop_graphs(h);
     // the previous upload reads h_args: let it finish before overwriting
     HIPCHK(hipStreamSynchronize(h->stream));
   }
-  h->h_args.resize(2 * STEP_F_COUNT);
-  for (int p = 0; p < 2; ++p)
-    for (unsigned fl = 0; fl < STEP_F_COUNT; ++fl) {
-      h->h_args[p * STEP_F_COUNT + fl] = base[p];
-      h->h_args[p * STEP_F_COUNT + fl].flags = fl;
-    }
+  h->h_args.assign(base, base + 2);
   // stream-ordered: steps queued before still see the previous arguments
-  HIPCHK(hipMemcpyAsync(h->d_args, h->h_args.data(), 2 * STEP_F_COUNT * sizeof(StepArgs), hipMemcpyHostToDevice,
-                        h->stream));
+  HIPCHK(hipMemcpyAsync(h->d_args, h->h_args.data(), sizeof base, hipMemcpyHostToDevice, h->stream));
   return 0;
 }
 
 int launch_one(aslhip_lattice *h, unsigned fl, std::vector<hipEvent_t> *ev, int s) {
   StepLaunch a;
-  const int p0 = h->next_odd ? STEP_F_COUNT : 0;  // this parity's argument table
-  const StepArgs &A = h->h_args[p0];
-  a.nblocks = A.nblocks;
-  a.block = A.block;
-  a.args = h->d_args + p0 + fl;
+  const int p = h->next_odd ? 1 : 0;
+  const StepArgs &A = h->h_args[p];
+  a.hot = A.g;
+  a.hot.flags = fl;
+  a.args = h->d_args + p;
   // LBGKTurbulence takes precedence over a closure in the collision
   a.variant = h->turbulence ? 1 : (h->has_closure ? (h->closure_mfma ? 2 : 1) : 0);
   a.cpl = A.cpl;
@@ -1010,7 +1034,7 @@ int aslhip_lattice_create(aslhip_lattice **out, int nx, int ny, int nz, int q, i
   if (e == hipSuccess) e = hipMalloc(&h->mode, 256);
   if (e == hipSuccess) e = hipMalloc(&h->val, 256 * (size_t)q * h->celem);
   if (e == hipSuccess) e = hipMalloc(&h->vlbc, 256 * sizeof(VLinkBC));
-  if (e == hipSuccess) e = hipMalloc(&h->d_args, 2 * STEP_F_COUNT * sizeof(StepArgs));
+  if (e == hipSuccess) e = hipMalloc(&h->d_args, 2 * sizeof(StepArgs));
   if (e == hipSuccess) e = hipMalloc(&h->red_partial, (size_t)reduce_blocks((int)len) * 5 * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&h->red_out, 5 * sizeof(double));
   if (e != hipSuccess) {
@@ -1459,7 +1483,6 @@ int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   float *dmap = nullptr;
   StepArgs *dpk = nullptr;  // the step arguments with one cell per lane, for the peek
   StepArgs pk = step_args(h, 0, 1);
-  pk.flags = base_flags(h) & ~(STEP_F_CLOSURE | STEP_F_CLOSURE_MFMA);
   hipError_t e = hipMalloc(&post, view);
   if (e == hipSuccess) e = hipMalloc(&in, view);
   if (e == hipSuccess) e = hipMalloc(&dout, outb);
@@ -1488,8 +1511,7 @@ int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   }
   if (e == hipSuccess) {
     StepLaunch a;
-    a.nblocks = pk.nblocks;
-    a.block = pk.block;
+    a.hot = pk.g;
     a.args = dpk;
     a.variant = 0;
     a.cpl = 1;
@@ -1768,9 +1790,7 @@ bool batch_tile(const aslhip_batch *b) {
 // One lattice's step arguments in the batch's launch shape.
 StepArgs batch_args(const aslhip_batch *b, const aslhip_lattice *h) {
   const bool tile = batch_tile(b);
-  StepArgs a = step_args(h, tile ? STEP_TILE : b->block, 1);
-  a.tile = tile ? 1 : 0;
-  return a;
+  return step_args(h, b->block, 1, false, tile);
 }
 
 void batch_free(aslhip_batch *b) {
@@ -1812,7 +1832,7 @@ int batch_tables(aslhip_batch *b) {
     }
     gbytes += bytes;
     const StepArgs a = batch_args(b, b->lat[l]);
-    for (int c = 0; c < a.nblocks; ++c) ent.push_back(make_uint2(static_cast<unsigned>(l), static_cast<unsigned>(c)));
+    for (int c = 0; c < a.g.nchunks; ++c) ent.push_back(make_uint2(static_cast<unsigned>(l), static_cast<unsigned>(c)));
   }
   b->groups.emplace_back(static_cast<int>(gfirst), static_cast<int>(ent.size()));
   // replays in flight read the old tables and graphs: finish them first
@@ -1886,8 +1906,8 @@ int batch_step_impl(aslhip_batch *b, int nsteps, unsigned flags) {
     if (int r = order_after_consumer(h)) return r;
     desc[l] = batch_args(b, h);
     desc[n + l] = desc[l];
-    if (h->comp_rho) desc[n + l].flags |= STEP_F_RHO;
-    if (h->comp_vel) desc[n + l].flags |= STEP_F_VEL;
+    if (h->comp_rho) desc[n + l].g.flags |= STEP_F_RHO;
+    if (h->comp_vel) desc[n + l].g.flags |= STEP_F_VEL;
     // work queued on the lattice's own stream comes first
     HIPCHK(hipEventRecord(b->done, h->stream));
     HIPCHK(hipStreamWaitEvent(b->stream, b->done, 0));

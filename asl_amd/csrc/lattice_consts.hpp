@@ -64,14 +64,28 @@ struct Lat<27> {
   }
 };
 
-// Index of the opposite direction (ASL's invertVectors, aslTemplates.cxx:72-83).
+// Index of the opposite direction (ASL's invertVectors, aslTemplates.cxx:72-83),
+// as a table: in an unrolled loop a look-up folds at once, a search has to be
+// unrolled and folded for every use, and the compiler gives up on loops of 26
+// links that hold several (they then run with directions looked up at run time).
+template <int Q>
+struct InvDir {
+  int v[Q];
+  constexpr InvDir() : v() {
+    for (int i = 0; i < Q; ++i)
+      for (int j = 0; j < Q; ++j)
+        if (Lat<Q>::c[j][0] == -Lat<Q>::c[i][0] && Lat<Q>::c[j][1] == -Lat<Q>::c[i][1] &&
+            Lat<Q>::c[j][2] == -Lat<Q>::c[i][2])
+          v[i] = j;
+  }
+};
+template <int Q>
+struct InvTable {
+  static constexpr InvDir<Q> t{};
+};
 template <int Q>
 constexpr ASLHIP_HD int inv_dir(int i) {
-  for (int j = 0; j < Q; ++j)
-    if (Lat<Q>::c[j][0] == -Lat<Q>::c[i][0] && Lat<Q>::c[j][1] == -Lat<Q>::c[i][1] &&
-        Lat<Q>::c[j][2] == -Lat<Q>::c[i][2])
-      return j;
-  return -1;
+  return InvTable<Q>::t.v[i];
 }
 
 // Packed cell types (one byte per ghost-inclusive cell).

@@ -1,0 +1,60 @@
+"""The direct step kernel's items and face rule, against the CPU oracle.
+
+Workgroups take consecutive interior cells whatever the rows and planes they
+belong to, so the sizes here put row and plane ends inside wavefronts and
+chunks: rows of one cell, planes of one row, chunks over many planes, a last
+chunk of one cell.  Every face has a boundary condition of its own, with and
+without values, in two execution orders (which decides the edge links).
+Same operations in the same order on both sides: bit for bit.
+"""
+import numpy as np
+import pytest
+
+from asl_amd import _lib
+from gpu_common import add_bc, compare, pair, run
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1, 1), (2, 1, 67), (70, 3, 1), (1, 300, 2), (5, 3, 129), (13, 9, 7), (4, 33, 64)]
+
+
+def six_faces(G, O, rng):
+    kinds = [(_lib.BC_CONSTANT_VELOCITY, dict(u=(0.02, 0.01, -0.01))), (_lib.BC_CONSTANT_PRESSURE, dict(p=1.01)),
+             (_lib.BC_NOSLIP, {}), (_lib.BC_CONSTANT_PRESSURE_VELOCITY, dict(p=0.99, u=(0.01, -0.02, 0.0))),
+             (_lib.BC_NOSLIP, {}), (_lib.BC_CONSTANT_VELOCITY, dict(u=(-0.01, 0.02, 0.0)))]
+    faces = [_lib.X0, _lib.XE, _lib.Y0, _lib.YE, _lib.Z0, _lib.ZE]
+    kinds = [kinds[i] for i in rng.permutation(6)]
+    bcs = [add_bc(G, O, k, f, **p) for (k, p), f in zip(kinds, faces)]
+    return [bcs[i] for i in rng.permutation(6)]
+
+
+@pytest.mark.parametrize("q", [15, 19, 27])
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("wide", [0, 1])
+def test_rows_planes_and_faces(size, q, wide):
+    rng = np.random.default_rng(q + sum(size))
+    for dtype, block in (("f32", 512), ("f64", 64)):
+        G, O = pair(size, q, nu=0.08, dtype=dtype)
+        G.set_tuning(_lib.TUNE_WIDE, wide)
+        G.set_tuning(_lib.TUNE_BLOCK, block)
+        u = 0.02 * rng.standard_normal((3,) + G.S)
+        u = u.astype(G.host_dtype)
+        G.init_equilibrium(1.0, u)
+        O.init_f(1.0, u.astype(np.float64))
+        run(G, O, 7, six_faces(G, O, rng))
+        d = compare(G, O)
+        assert d["rho"] == 0.0 and d["u"] == 0.0 and d["f"] == 0.0, (dtype, d)
+
+
+@pytest.mark.parametrize("size", [(3, 3, 3), (2, 5, 66), (40, 3, 4)])
+@pytest.mark.parametrize("q", [19, 27])
+def test_periodic_wrap(size, q):
+    rng = np.random.default_rng(sum(size))
+    for dtype in ("f32", "f64"):
+        G, O = pair(size, q, nu=0.05, dtype=dtype, periodic=True)
+        u = (0.02 * rng.standard_normal((3,) + G.S)).astype(G.host_dtype)
+        G.init_equilibrium(1.0, u)
+        O.init_f(1.0, u.astype(np.float64))
+        run(G, O, 6, [])
+        d = compare(G, O)
+        assert d["rho"] == 0.0 and d["u"] == 0.0 and d["f"] == 0.0, (dtype, d)
