@@ -162,6 +162,96 @@ __device__ __forceinline__ void moments(const C (&v)[Q], C &r, C (&m)[3]) {
   for (int j = 1; j < Q; ++j) r = fmaT(v[j], C(LT::w(j)), r);
 }
 
+// x / r for many x and one r, the same bits as the IEEE division.
+//
+// y is the correctly rounded 1 / r and yl what it lacks, so that
+// q = x y + x yl (one rounding) lies within one unit in the last place of
+// x / r; for such a q the remainder x - r q is exact and fma(remainder, y, q)
+// is the correctly rounded quotient (P. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34,
+// 1990).  Four full-rate instructions instead of the eleven of a division
+// (one of them a quarter-rate reciprocal); a D3Q19 cell divides ten times by
+// its density, with LBGKTurbulence twenty times.  us per step with divisions
+// and with this, D3Q19: LBGKTurbulence 128^3 60.6 -> 53.8; FP16 box of
+// 256 x 128 x 128 65.0 -> 62.3; FP32 boxes 64^3 9.9 -> 9.7, 16^3 4.6 -> 4.3.
+// Nothing may overflow or underflow on the way: recip_safe.
+template <class C>
+struct Quotient {
+  C r, y, yl;
+  __device__ __forceinline__ explicit Quotient(C d) : r(d) {
+    y = C(1.) / d;
+    yl = fmaT(-d, y, C(1.)) * y;
+  }
+  __device__ __forceinline__ C operator()(C x) const {
+    const C q = fmaT(x, y, x * yl);
+    return fmaT(fmaT(-r, q, x), y, q);
+  }
+};
+
+// The division itself, for cells outside recip_safe.
+template <class C>
+struct Division {
+  C r;
+  __device__ __forceinline__ explicit Division(C d) : r(d) {}
+  __device__ __forceinline__ C operator()(C x) const { return x / r; }
+};
+
+// Whether Quotient(r) gives the terms of an equilibrium (4.5 a^2 / r and
+// 1.5 m^2 / r = mm / r) as a division would.  r lies in [2^-16, 2^16] and
+// x <= 2^42: no overflow, and no underflow for x >= 2^-100 (q >= 2^-116, its
+// remainder a multiple of 2^-146).  A smaller x may be off in its last bits,
+// but then it is below 2^-84 and is added to or subtracted from a value of at
+// least r / 2 >= 2^-17 (a < 2^-50 there), whose rounding it cannot reach.
+// NaN and infinities fail the comparisons.
+template <class C>
+__device__ __forceinline__ bool recip_safe(C r, C mm) {
+  return r >= C(0x1p-16) && r <= C(0x1p16) && mm <= C(0x1p40);
+}
+
+// 1.5 m . m
+template <class C>
+__device__ __forceinline__ C square15(const C (&m)[3]) {
+  C mm = (C(1.5) * m[0]) * m[0];
+  mm = fmaT(C(1.5) * m[1], m[1], mm);
+  return fmaT(C(1.5) * m[2], m[2], mm);
+}
+
+// The equilibria of all directions of a cell, compressible or not
+// (src/num/aslLBGK.cxx:220-231), handed to f0(feq_0) and f(i, j, feq_i,
+// feq_j) for each pair of opposite directions.  Opposite directions share
+// (4.5 a^2)/rho: a_inv(i) = -a_i exactly in IEEE arithmetic, so this is the
+// same value ASL computes twice.
+template <int Q, class C, class D, class F0, class F>
+__device__ __forceinline__ void equilibria(bool compressible, C r, const C (&m)[3], C mm, const D &over_r, F0 f0,
+                                           F f) {
+  const C mmr = compressible ? over_r(mm) : mm;
+  f0(r - mmr);
+#pragma unroll
+  for (int i = 1; i < Q; ++i) {
+    const int j = inv_dir<Q>(i);
+    if (j < i) continue;
+    const C a = dot_c<Q>(m, i);
+    if (compressible) {
+      const C t = over_r(C(4.5) * (a * a));
+      f(i, j, (fmaT(C(3.), a, r) + t) - mmr, (fmaT(C(3.), -a, r) + t) - mmr);
+    } else {
+      const C aa = a * a;
+      f(i, j, fmaT(C(4.5), aa, fmaT(C(3.), a, r)) - mmr, fmaT(C(4.5), aa, fmaT(C(3.), -a, r)) - mmr);
+    }
+  }
+}
+
+// FP64 divides: its steps are bound by memory either way (D3Q19 128^3: 111 us
+// per step with divisions and with quotients).
+template <int Q, class C, class F0, class F>
+__device__ __forceinline__ void equilibria_of(bool compressible, C r, const C (&m)[3], F0 f0, F f) {
+  const C mm = square15<C>(m);
+  if (sizeof(C) == 4 && compressible && __all(recip_safe(r, mm)))
+    equilibria<Q, C>(true, r, m, mm, Quotient<C>(r), f0, f);
+  else
+    equilibria<Q, C>(compressible, r, m, mm, Division<C>(r), f0, f);
+}
+
 // LBGKTurbulence::init0 (src/num/aslLBGK.cxx:298-355): the relaxation of a
 // cell from how far its populations are from equilibrium,
 //   r = 4 |f - feq|^2 / |f|^2,   w = r > 1 ? 1 / (3 min(nu r, 1/2) + 1/2) : 1 / (3 nu + 1/2).
@@ -170,21 +260,19 @@ __device__ __forceinline__ void moments(const C (&v)[Q], C &r, C (&m)[3]) {
 // rotating-frame term), the value that statement is evidently meant to use.
 template <int Q, class C>
 __device__ __forceinline__ C turbulence_w(const C (&v)[Q], C r, const C (&m)[3], bool compressible, C nu, C w0) {
-  C mm = (C(1.5) * m[0]) * m[0];
-  mm = fmaT(C(1.5) * m[1], m[1], mm);
-  mm = fmaT(C(1.5) * m[2], m[2], mm);
-  const C mmr = compressible ? mm / r : mm;
+  C d[Q];  // f - feq, summed in direction order
+  equilibria_of<Q, C>(
+      compressible, r, m, [&](C e) { d[0] = v[0] - e; },
+      [&](int i, int j, C ei, C ej) {
+        d[i] = v[i] - ei;
+        d[j] = v[j] - ej;
+      });
   C fl2 = v[0] * v[0];
-  C d = v[0] - (r - mmr);
-  C dl2 = d * d;
+  C dl2 = d[0] * d[0];
 #pragma unroll
   for (int i = 1; i < Q; ++i) {
-    const C a = dot_c<Q>(m, i);
-    const C fe = compressible ? (fmaT(C(3.), a, r) + (C(4.5) * (a * a)) / r) - mmr
-                              : fmaT(C(4.5), a * a, fmaT(C(3.), a, r)) - mmr;
     fl2 = fmaT(v[i], v[i], fl2);
-    const C di = v[i] - fe;
-    dl2 = fmaT(di, di, dl2);
+    dl2 = fmaT(d[i], d[i], dl2);
   }
   const C rt = C(4.) * (dl2 / fl2);
   const C nr = nu * rt;
@@ -195,14 +283,13 @@ __device__ __forceinline__ C turbulence_w(const C (&v)[Q], C r, const C (&m)[3],
 // The BGK collision of one cell: ASL's LBGK::init0 (src/num/aslLBGK.cxx:
 // 187-235) with computeRho / computeMomentum / a_i_dot_v (:46-72).  Each
 // x*y + z of ASL's expression tree is one fma (OpenCL's default FP_CONTRACT
-// ON); the CPU oracle contracts the same sites.  Opposite directions share
-// (4.5 a^2)/rho: a_inv(i) = -a_i exactly in IEEE arithmetic, so this is the
-// same value ASL computes twice.  On return v holds the post-collision
-// populations, r the density and m the momentum.  CL: a per-cell relaxation
-// replaces w: 1 LBGKTurbulence's (turb) or the closure network's in FP32 on
-// the vector ALUs, 2 the closure network's on the matrix cores (closure:
-// D3Q19, FP32 collision).  Each is its own kernel, so that the plain and the
-// matrix-core variants do not hold the registers of the FP32 network.
+// ON); the CPU oracle contracts the same sites.  On return v holds the
+// post-collision populations, r the density and m the momentum.  CL: a
+// per-cell relaxation replaces w: 1 LBGKTurbulence's (turb) or the closure
+// network's in FP32 on the vector ALUs, 2 the closure network's on the matrix
+// cores (closure: D3Q19, FP32 collision).  Each is its own kernel, so that the
+// plain and the matrix-core variants do not hold the registers of the FP32
+// network.
 template <int Q, class C, int CL = 0>
 __device__ __forceinline__ void collide(C (&v)[Q], C w, bool compressible, bool omega, const C (&om)[3], C &r_o,
                                         C (&m_o)[3], const ClosureParams *cl = nullptr, float tau0 = 0.f,
@@ -231,30 +318,13 @@ __device__ __forceinline__ void collide(C (&v)[Q], C w, bool compressible, bool 
     m[1] = fmaT(t, fmaT(om[2], m[0], -(om[0] * m[2])), m[1]);
     m[2] = fmaT(t, fmaT(om[0], m[1], -(om[1] * m[0])), m[2]);
   }
-  C mm = (C(1.5) * m[0]) * m[0];
-  mm = fmaT(C(1.5) * m[1], m[1], mm);
-  mm = fmaT(C(1.5) * m[2], m[2], mm);
-  const C mmr = compressible ? mm / r : mm;
   const C one_w = C(1.) - w;
-  v[0] = fmaT(v[0], one_w, w * (r - mmr));
-#pragma unroll
-  for (int i = 1; i < Q; ++i) {
-    const int j = inv_dir<Q>(i);
-    if (j < i) continue;
-    const C a = dot_c<Q>(m, i);
-    C fi, fj;
-    if (compressible) {
-      const C t = (C(4.5) * (a * a)) / r;
-      fi = (fmaT(C(3.), a, r) + t) - mmr;
-      fj = (fmaT(C(3.), -a, r) + t) - mmr;
-    } else {
-      const C aa = a * a;
-      fi = fmaT(C(4.5), aa, fmaT(C(3.), a, r)) - mmr;
-      fj = fmaT(C(4.5), aa, fmaT(C(3.), -a, r)) - mmr;
-    }
-    v[i] = fmaT(v[i], one_w, w * fi);
-    v[j] = fmaT(v[j], one_w, w * fj);
-  }
+  equilibria_of<Q, C>(
+      compressible, r, m, [&](C e) { v[0] = fmaT(v[0], one_w, w * e); },
+      [&](int i, int j, C ei, C ej) {
+        v[i] = fmaT(v[i], one_w, w * ei);
+        v[j] = fmaT(v[j], one_w, w * ej);
+      });
   r_o = r;
 #pragma unroll
   for (int d = 0; d < 3; ++d) m_o[d] = m[d];
@@ -1037,13 +1107,15 @@ __global__ __launch_bounds__(STEP_TILE) void k_step_tile(const StepHot g, const 
 // holds.  Every cell's reads and writes in one step are its own (AA
 // pattern), so the order of the chunks does not change results.
 template <int Q, class S, bool ODD, bool PER, bool WIDE, int CL>
-__global__ __launch_bounds__(STEP_BLOCK) void k_step(const StepHot g, const StepArgs *args) {
+__global__ __launch_bounds__(step_block(Q, sizeof(S))) void k_step(const StepHot g, const StepArgs *args) {
   step_body<Q, S, ODD, PER, WIDE, CL>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
 
-// The matrix-core closure variant, held to 5 waves per SIMD (96 VGPRs).
+// The matrix-core closure variant, held to 5 waves per SIMD (96 VGPRs) on
+// periodic lattices; with the boundary links those spill about 30 (128^3 box:
+// 177 us per step, 69 with 100 VGPRs and 4 waves).
 template <int Q, class S, bool ODD, bool PER, bool WIDE>
-__global__ __launch_bounds__(STEP_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_step_mfma(
+__global__ __launch_bounds__(STEP_BLOCK) __attribute__((amdgpu_waves_per_eu(PER ? 5 : 4))) void k_step_mfma(
     const StepHot g, const StepArgs *args) {
   step_body<Q, S, ODD, PER, WIDE, 2>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
@@ -1058,7 +1130,7 @@ __global__ __launch_bounds__(STEP_RUN_BLOCK) void k_step_run(const StepHot g, co
 
 // The incoming populations of every computed cell for the next step.
 template <int Q, class S, bool ODD, bool PER>
-__global__ __launch_bounds__(STEP_BLOCK) void k_peek(const StepHot g, const StepArgs *args, void *out) {
+__global__ __launch_bounds__(step_block(Q, sizeof(S))) void k_peek(const StepHot g, const StepArgs *args, void *out) {
   step_body<Q, S, ODD, PER, false, 0, true>(g, *args, static_cast<int>(blockIdx.x), out);
 }
 
@@ -1239,7 +1311,7 @@ __global__ __launch_bounds__(BLOCK) void k_vis(const VisArgs a) {
 // which cut the waves per SIMD from 7 to 4 at 256-lane workgroups.
 // Odd steps take the entries in reverse order, as k_step does.
 template <int Q, class S, bool ODD, bool PER, bool WIDE>
-__global__ __launch_bounds__(STEP_BLOCK) void k_step_batch(const StepArgs *desc, const uint2 *ent) {
+__global__ __launch_bounds__(step_block(Q, sizeof(S))) void k_step_batch(const StepArgs *desc, const uint2 *ent) {
   const int b = static_cast<int>(blockIdx.x);
   const uint2 e = ent[ODD ? xcd_reverse(b, static_cast<int>(gridDim.x)) : b];
   step_body<Q, S, ODD, PER, WIDE>(desc[e.x].g, desc[e.x], static_cast<int>(e.y));

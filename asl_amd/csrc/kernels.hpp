@@ -13,6 +13,10 @@ namespace aslhip {
 constexpr int STEP_BLOCK = 1024;
 constexpr int STEP_RUN_BLOCK = 512;
 constexpr int STEP_TILE = 256;
+// D3Q27 in FP64 holds 54 registers of populations alone: 1024 lanes per
+// workgroup leave 128 registers and spill (periodic 128^3: 159 us per step),
+// 512 leave it the 132 to 140 it takes (151 us).
+constexpr int step_block(int q, int elem_bytes) { return q == 27 && elem_bytes == 8 ? 512 : STEP_BLOCK; }
 
 // Step-kernel flags.
 enum : unsigned {

@@ -642,7 +642,8 @@ int effective_cpl(const aslhip_lattice *h) {
 // steps only: the odd steps' workgroup).
 int step_workgroup(const aslhip_lattice *h) {
   if (effective_lds(h) == 1) return STEP_TILE;
-  return effective_cpl(h) > 1 && h->tune_block > STEP_RUN_BLOCK ? STEP_RUN_BLOCK : h->tune_block;
+  const int most = step_block(h->Q, static_cast<int>(h->selem));
+  return std::min(h->tune_block, effective_cpl(h) > 1 ? std::min(most, STEP_RUN_BLOCK) : most);
 }
 
 // The divisor d of udivm (kernels.hip); 0 stands for d = 1.
@@ -696,6 +697,7 @@ StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd
   a.cpl = cpl > 0 ? cpl : effective_cpl(h);
   g.block = block > 0 ? block : h->tune_block;
   if (a.cpl > 1 && g.block > STEP_RUN_BLOCK) g.block = STEP_RUN_BLOCK;
+  g.block = std::min(g.block, step_block(h->Q, static_cast<int>(h->selem)));
   const int lds = effective_lds(h);
   a.tile = tiles || (block <= 0 && cpl <= 0 && (lds == 1 || (lds == 2 && !odd))) ? 1 : 0;
   if (a.tile) g.block = STEP_TILE;
@@ -1810,7 +1812,7 @@ int batch_launch(aslhip_batch *b, bool odd, bool macro, int e0, int e1) {
   L.ent = b->ent + e0;
   L.nblocks = e1 - e0;
   L.tile = batch_tile(b) ? 1 : 0;
-  L.block = L.tile ? STEP_TILE : b->block;
+  L.block = L.tile ? STEP_TILE : std::min(b->block, step_block(b->Q, static_cast<int>(b->lat[0]->selem)));
   HIPCHK(launch_step_batch(b->Q, b->dtype, odd, b->periodic, b->wide, L, b->stream));
   return 0;
 }
@@ -2017,7 +2019,7 @@ int aslhip_batch_autotune(aslhip_batch *b, int nsteps, int *best_block) {
     if (int r = trial(0, blk)) return r;
   if (int r = aslhip_batch_set_tuning(b, ASLHIP_TUNE_LDS, bl)) return r;
   if (int r = aslhip_batch_set_tuning(b, ASLHIP_TUNE_BLOCK, bb)) return r;
-  if (best_block) *best_block = bl ? STEP_TILE : bb;
+  if (best_block) *best_block = bl ? STEP_TILE : std::min(bb, step_block(b->Q, static_cast<int>(b->lat[0]->selem)));
   return 0;
 }
 

@@ -370,7 +370,8 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  *   consecutive chunks (neighbouring chunks share one L2; default 4, 64 for
  *   FP16 / BF16 storage); 0 or 1 = the hardware round-robin order.
  *   ASLHIP_TUNE_BLOCK: workgroup size, a multiple of 64 up to 1024 (default
- *   512); a workgroup takes that many consecutive cells of a plane. */
+ *   512); a workgroup takes that many consecutive interior cells.  D3Q27 in FP64
+ *   runs with at most 512. */
 #define ASLHIP_TUNE_XCD_REMAP 1
 #define ASLHIP_TUNE_BLOCK 2
 /* Batches only: graph chunks step groups of consecutive lattices of at most
