@@ -133,6 +133,7 @@ struct aslhip_lattice {
   // step arguments of even and odd steps (they differ when only even steps run tiles)
   StepArgs *d_args = nullptr;
   std::vector<StepArgs> h_args;  // host copy of d_args (empty: not uploaded yet)
+  StepHot h_direct;              // one cell per lane over the whole lattice (plane ranges are cut from it)
   // Captured runs of plain steps (the velocity-map link fills included):
   // full chunks of ASLHIP_GRAPH_CHUNK steps and the shorter remainders of
   // step counts that are not a multiple of it, each for a starting parity
@@ -188,6 +189,7 @@ struct aslhip_lattice {
   int tune_remap = 4;  // chunk runs per XCD (measured best for graph chunks; 64 for 16-bit storage; the autotuner may choose others)
   int tune_cpl = 0;    // cells per lane along z: 0 automatic, else 1, 2 or 4 (ASLHIP_TUNE_CPL)
   int tune_lds = -1;   // LDS-staged tiles: 0 off, 1 every step, 2 even steps, -1 automatic (ASLHIP_TUNE_LDS)
+  int tune_sweep = -1; // sweeps: window in KiB, 0 off, -1 automatic (ASLHIP_TUNE_SWEEP_KB)
   bool vmap_skip_outer = false;  // velocity-map averages skip outer-layer neighbours (opt-in)
   // face rule: per face slot * 4 + mode of the winning slice BC, and values
   int fface[6] = {0, 0, 0, 0, 0, 0};
@@ -617,15 +619,16 @@ bool is_wide(const aslhip_lattice *h) { return h->force_wide || h->qs_bytes * h-
 // LDS-staged tiles apply to non-periodic lattices under 4 GiB without a
 // per-cell relaxation unless runs of 2 or 4 cells per lane are asked for:
 // 0 none, 1 every step, 2 even steps only (odd steps one cell per lane).
-// Automatic: every step for FP32 storage whose populations outgrow the
-// 256 MiB Infinity Cache (the sphere channel, 331 MB: 0.1225 against 0.128
-// ms per step); none for lattices the cache holds (64^3 cavity, 22 MB: 15 us
-// against 11 us) and for FP16 / BF16 / FP64 storage (the direct kernel is
-// faster there).
-constexpr long long TILE_MIN_BYTES = 256LL << 20;
+// Automatic: every step for D3Q19 FP32 lattices whose populations outgrow the
+// 256 MiB Infinity Cache (box of 256 x 128 x 128, 331 MB: 116 us per step, 128
+// direct); none for lattices the cache holds (64^3 box, 22 MB: 12.7 against
+// 9.7 us), for the other templates (D3Q27 300 x 130 x 140: 226 against 224 us,
+// and sweeps gain beside other lattices; D3Q15: 282 against 123 us) and for
+// FP16 / BF16 / FP64 storage (the direct kernel is faster there).
+constexpr long long CACHE_BYTES = 256LL << 20;  // the Infinity Cache
 int effective_lds(const aslhip_lattice *h) {
-  const bool big = h->qs_bytes * h->Q > TILE_MIN_BYTES;
-  const int mode = h->tune_lds < 0 ? (h->dtype == ASLHIP_F32 && big ? 1 : 0) : h->tune_lds;
+  const bool big = h->qs_bytes * h->Q > CACHE_BYTES;
+  const int mode = h->tune_lds < 0 ? (h->Q == 19 && h->dtype == ASLHIP_F32 && big ? 1 : 0) : h->tune_lds;
   return h->tune_cpl <= 1 && !(h->periodic || is_wide(h) || h->has_closure || h->turbulence) ? mode : 0;
 }
 
@@ -761,28 +764,123 @@ int upload_args(aslhip_lattice *h) {
     HIPCHK(hipStreamSynchronize(h->stream));
   }
   h->h_args.assign(base, base + 2);
+  h->h_direct = step_args(h, h->tune_block, 1).g;
   // stream-ordered: steps queued before still see the previous arguments
   HIPCHK(hipMemcpyAsync(h->d_args, h->h_args.data(), sizeof base, hipMemcpyHostToDevice, h->stream));
   return 0;
 }
 
-int launch_one(aslhip_lattice *h, unsigned fl, std::vector<hipEvent_t> *ev, int s) {
+// One launch of the step kernel: step args for parity odd, flags fl, the
+// interior planes p0 .. p0 + np - 1 one cell per lane (np < 0: the whole
+// lattice with its tuning).
+int launch_planes(aslhip_lattice *h, bool odd, unsigned fl, int p0, int np) {
   StepLaunch a;
-  const int p = h->next_odd ? 1 : 0;
+  const int p = odd ? 1 : 0;
   const StepArgs &A = h->h_args[p];
-  a.hot = A.g;
+  a.hot = np < 0 ? A.g : h->h_direct;
   a.hot.flags = fl;
   a.args = h->d_args + p;
   // LBGKTurbulence takes precedence over a closure in the collision
   a.variant = h->turbulence ? 1 : (h->has_closure ? (h->closure_mfma ? 2 : 1) : 0);
-  a.cpl = A.cpl;
-  a.tile = A.tile;
+  a.cpl = np < 0 ? A.cpl : 1;
+  a.tile = np < 0 ? A.tile : 0;
+  if (np >= 0) {
+    const unsigned plane = static_cast<unsigned>(a.hot.ny) * static_cast<unsigned>(a.hot.nz);
+    a.hot.first = static_cast<unsigned>(p0) * plane;
+    a.hot.count = static_cast<unsigned>(np) * plane;
+    a.hot.nchunks = static_cast<int>((static_cast<long long>(a.hot.count) + a.hot.block - 1) / a.hot.block);
+  }
+  HIPCHK(launch_step(h->Q, h->dtype, odd, h->periodic, is_wide(h), a, h->stream));
+  return 0;
+}
+
+// The shape of the sweeps (sweep_plan) of a run of steps: g planes per launch,
+// t steps per sweep; t = 0: one launch per step over the whole lattice.
+// Automatic: for lattices that the 256 MiB Infinity Cache cannot hold and that
+// do not run LDS-staged tiles, a window of 192 MiB (g + t planes) that takes up
+// to 16 steps, so that most reads and writes of a step find their lines there.
+// us per step, alone / with two more lattices stepped beside it, before and
+// after: D3Q27 FP32 224^3 periodic 462 / 522 -> 438 / 469, D3Q27 FP64
+// 200 x 160 x 160 422 / 482 -> 422 / 391, D3Q19 FP64 256 x 128 x 128 225 / 271
+// -> 217 / 217, FP16 384 x 160 x 144 150 / 151 -> 141 / 151.  Tiles and sweeps
+// of D3Q19 FP32: 116 / 135 and 109 / 123 on 256 x 128 x 128, 149 / 158 and 152
+// / 165 on 300 x 130 x 140, 111 / 111 and 108 / 118 on 160 x 203 x 121: tiles
+// stay.  Windows of 64 MiB gain only beside other lattices, 240 MiB less than
+// 192 there.  Velocity-map links are filled after every step of the whole
+// lattice: no sweeps.
+constexpr long long SWEEP_WINDOW = 192LL << 20;
+constexpr int SWEEP_STEPS = 16;
+void sweep_shape(const aslhip_lattice *h, int &g, int &t) {
+  g = t = 0;
+  if (h->nvl || h->tune_sweep == 0) return;
+  if (h->tune_sweep < 0 && (h->qs_bytes * h->Q <= CACHE_BYTES || effective_lds(h) == 1)) return;
+  const long long window = h->tune_sweep > 0 ? static_cast<long long>(h->tune_sweep) << 10 : SWEEP_WINDOW;
+  const long long plane = static_cast<long long>(h->Q) * h->selem * h->sx;
+  const int wp = static_cast<int>(std::min<long long>(window / plane, h->n[0]));
+  const int m = std::min(SWEEP_STEPS, wp / 2);
+  if (m < 2 || wp >= h->n[0]) return;
+  t = m;
+  g = wp - m;
+}
+
+// Launches of a run of n steps, see sweep_plan.
+struct SweepLaunch {
+  int step;    // step of the run
+  int p0, np;  // interior planes (x - 1) of this launch
+};
+
+// Orders n steps of a lattice of nx planes so that a window of planes takes
+// several steps while it stays in the Infinity Cache.  A step of plane x
+// needs planes x - 1, x, x + 1 one step earlier and nothing else (each slot of
+// the AA pattern belongs to one cell in every step, and to a cell at most one
+// plane away in the next), so blocks of g planes, shifted one plane back per
+// step, can take t steps one block after the other: block b does planes
+// [b g - s, (b + 1) g - s) in step s.  Periodic lattices: step s covers planes
+// s .. nx + s - 1 (modulo nx), so that the first block starts from planes
+// nobody needs yet and the last one closes the ring.
+void sweep_plan(int nx, bool periodic, int g, int t, int n, std::vector<SweepLaunch> &out) {
+  for (int s0 = 0; s0 < n; s0 += t) {
+    const int m = std::min(t, n - s0);
+    const int end = periodic ? nx + m - 1 : nx;  // planes of the last step end here
+    for (int b = 0; b * g - (m - 1) < end; ++b)
+      for (int s = 0; s < m; ++s) {
+        const int lo = std::max(b * g - s, periodic ? s : 0), hi = std::min((b + 1) * g - s, periodic ? nx + s : nx);
+        if (lo >= hi) continue;
+        if (lo < nx) out.push_back({s0 + s, lo, std::min(hi, nx) - lo});
+        if (hi > nx) out.push_back({s0 + s, std::max(lo, nx) - nx, hi - std::max(lo, nx)});
+      }
+  }
+}
+
+int launch_one(aslhip_lattice *h, unsigned fl, std::vector<hipEvent_t> *ev, int s) {
   if (ev) HIPCHK(hipEventRecord((*ev)[2 * s], h->stream));
-  HIPCHK(launch_step(h->Q, h->dtype, h->next_odd, h->periodic, is_wide(h), a, h->stream));
+  if (int r = launch_planes(h, h->next_odd, fl, 0, -1)) return r;
   if (ev) HIPCHK(hipEventRecord((*ev)[2 * s + 1], h->stream));
   const bool was_odd = h->next_odd;
   h->next_odd = !h->next_odd;
   return run_vlinks(h, was_odd);
+}
+
+// n steps with the flags fl, the last one with last_fl.
+int launch_run(aslhip_lattice *h, unsigned fl, unsigned last_fl, int n) {
+  int g = 0, t = 0;
+  if (n > 1) sweep_shape(h, g, t);
+  if (!t) {
+    for (int s = 0; s < n; ++s)
+      if (int r = launch_one(h, s == n - 1 ? last_fl : fl, nullptr, s)) return r;
+    return 0;
+  }
+  std::vector<SweepLaunch> plan;
+  for (int s = 0; s < n; s += t) {
+    const int m = std::min(t, n - s);
+    plan.clear();
+    sweep_plan(h->n[0], h->periodic, g, t, m, plan);
+    for (const auto &l : plan)
+      if (int r = launch_planes(h, h->next_odd != ((l.step & 1) != 0), s + l.step == n - 1 ? last_fl : fl, l.p0, l.np))
+        return r;
+    if (m & 1) h->next_odd = !h->next_odd;
+  }
+  return 0;
 }
 
 // At most this many captured remainders (runs shorter than a chunk) are kept.
@@ -827,7 +925,7 @@ int get_graph(aslhip_lattice *h, int n, bool odd, hipGraphExec_t *out) {
   hipGraph_t graph = nullptr;
   HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
   int r = 0;
-  for (int s = 0; s < n && !r; ++s) r = launch_one(h, fl, nullptr, s);
+  r = launch_run(h, fl, fl, n);
   hipError_t e = hipStreamEndCapture(h->stream, &graph);
   h->next_odd = keep;
   if (r) {
@@ -845,7 +943,9 @@ int get_graph(aslhip_lattice *h, int n, bool odd, hipGraphExec_t *out) {
 }
 
 // graph: run whole chunks of plain steps (not the raw first one, not the
-// one writing rho/u) as hipGraph replays.  consume: the BC executions
+// one writing rho/u) as hipGraph replays, unless the lattice sweeps: its
+// launches are long enough to hide the next one's submission, and a graph of
+// several launches per step would have to be captured first.  consume: the BC executions
 // recorded since the last step become the active order first (a deferred
 // step runs with the order folded in when it was requested instead: the
 // executions recorded since then belong to the step after it).
@@ -864,7 +964,9 @@ int run_steps(aslhip_lattice *h, int nsteps, bool first_after_init, bool raw_fir
   for (int s = 0; s < nsteps;) {
     const bool raw = s == 0 && raw_first;
     const int plain = nsteps - s - (macro_last ? 1 : 0);  // plain steps left
-    if (graph && !ev && !raw && plain >= 1) {
+    int sg = 0, st = 0;
+    if (!raw && !ev && nsteps - s > 1) sweep_shape(h, sg, st);
+    if (graph && !ev && !raw && plain >= 1 && !st) {
       const int n = plain < ASLHIP_GRAPH_CHUNK ? plain : ASLHIP_GRAPH_CHUNK;
       hipGraphExec_t g = nullptr;
       if (int r = get_graph(h, n, h->next_odd, &g)) return r;
@@ -873,14 +975,20 @@ int run_steps(aslhip_lattice *h, int nsteps, bool first_after_init, bool raw_fir
       if (n & 1) h->next_odd = !h->next_odd;
       continue;
     }
-    unsigned fl = base_flags(h);
-    if (raw) fl |= STEP_F_RAW;
-    if (s == nsteps - 1 && macro_last) {
-      if (h->comp_rho) fl |= STEP_F_RHO;
-      if (h->comp_vel) fl |= STEP_F_VEL;
+    unsigned fl = base_flags(h), last = fl;
+    if (macro_last) {
+      if (h->comp_rho) last |= STEP_F_RHO;
+      if (h->comp_vel) last |= STEP_F_VEL;
     }
-    if (int r = launch_one(h, fl, ev, s)) return r;
-    ++s;
+    if (raw || ev || (graph && !st)) {  // one step
+      if (s == nsteps - 1) fl = last;
+      if (raw) fl |= STEP_F_RAW;
+      if (int r = launch_one(h, fl, ev, s)) return r;
+      ++s;
+    } else {
+      if (int r = launch_run(h, fl, last, nsteps - s)) return r;
+      s = nsteps;
+    }
   }
   return 0;
 }
@@ -1632,6 +1740,12 @@ int aslhip_set_tuning(aslhip_lattice *h, int knob, int value) {
     h->tune_block = value;
     return 0;
   }
+  if (knob == ASLHIP_TUNE_SWEEP_KB) {
+    if (value < -1) return fail(ASLHIP_EINVAL, "ASL ERROR: ASLHIP_TUNE_SWEEP_KB takes a window in KiB, 0 or -1");
+    if (int r = flush_deferred(h)) return r;
+    h->tune_sweep = value;
+    return 0;
+  }
   if (knob == ASLHIP_TUNE_LDS) {
     if (value < 0 || value > 2) return fail(ASLHIP_EINVAL, "ASL ERROR: ASLHIP_TUNE_LDS takes 0, 1 or 2");
     if (int r = flush_deferred(h)) return r;
@@ -1640,6 +1754,19 @@ int aslhip_set_tuning(aslhip_lattice *h, int knob, int value) {
     return 0;
   }
   return fail(ASLHIP_EINVAL, "ASL ERROR: unknown tuning knob %d", knob);
+}
+
+int aslhip_sweep_plan(int nx, int periodic, int planes, int steps, int nsteps, int *out, int cap) {
+  if (nx < 1 || planes < 1 || steps < 1 || nsteps < 0 || cap < 0 || (cap > 0 && !out))
+    return fail(ASLHIP_EINVAL, "ASL ERROR: sweep_plan: bad arguments");
+  std::vector<SweepLaunch> plan;
+  sweep_plan(nx, periodic != 0, planes, steps, nsteps, plan);
+  for (size_t i = 0; i < plan.size() && i < static_cast<size_t>(cap); ++i) {
+    out[3 * i] = plan[i].step;
+    out[3 * i + 1] = plan[i].p0;
+    out[3 * i + 2] = plan[i].np;
+  }
+  return static_cast<int>(plan.size());
 }
 
 int aslhip_tuning_value(aslhip_lattice *h, int knob, int *value) {
@@ -1651,6 +1778,7 @@ int aslhip_tuning_value(aslhip_lattice *h, int knob, int *value) {
     case ASLHIP_TUNE_WIDE: *value = is_wide(h) ? 1 : 0; return 0;
     case ASLHIP_TUNE_CPL: *value = effective_cpl(h); return 0;
     case ASLHIP_TUNE_LDS: *value = effective_lds(h); return 0;
+    case ASLHIP_TUNE_SWEEP_KB: *value = h->tune_sweep; return 0;
     default: return fail(ASLHIP_EINVAL, "ASL ERROR: unknown tuning knob %d", knob);
   }
 }
@@ -1780,12 +1908,12 @@ struct aslhip_batch {
 namespace {
 
 // Tiles for the batch's steps: non-periodic batches under 4 GiB per lattice;
-// automatic as for single lattices (FP32 storage, the batch's populations
+// automatic as for single lattices (D3Q19 FP32, the batch's populations
 // beyond the 256 MiB Infinity Cache).
 bool batch_tile(const aslhip_batch *b) {
   long long bytes = 0;
   for (const aslhip_lattice *h : b->lat) bytes += h->qs_bytes * h->Q;
-  const bool on = b->tune_lds < 0 ? b->dtype == ASLHIP_F32 && bytes > TILE_MIN_BYTES : b->tune_lds != 0;
+  const bool on = b->tune_lds < 0 ? b->Q == 19 && b->dtype == ASLHIP_F32 && bytes > CACHE_BYTES : b->tune_lds != 0;
   return on && !b->periodic && !b->wide;
 }
 

@@ -393,12 +393,25 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  * consecutive cells through LDS (16-byte loads and stores of each
  * direction's slots for FP32, workgroup 256); 2 = tiles on even steps only,
  * odd steps direct; 0 = direct, one cell per lane (or the runs
- * ASLHIP_TUNE_CPL asks for).  Default: 1 for FP32 storage over 256 MiB of
- * populations (lattices the 256 MiB Infinity Cache cannot hold), else 0.  Tiles apply to the same lattices as runs of cells
- * when ASLHIP_TUNE_CPL is 0 or 1; results are bit for bit the same for
+ * ASLHIP_TUNE_CPL asks for).  Default: 1 for D3Q19 FP32 lattices over
+ * 256 MiB of populations (that the Infinity Cache cannot hold), else 0.
+ * Tiles apply to the same lattices as runs of cells when ASLHIP_TUNE_CPL is 0
+ * or 1; results are bit for bit the same for
  * every value. */
 #define ASLHIP_TUNE_LDS 6
+/* Lattices: window in KiB of the sweeps of a run of several steps: blocks of
+ * planes take several steps one block after the other while their
+ * populations stay in the Infinity Cache (in eager launches also under
+ * ASLHIP_STEP_GRAPH; one cell per lane).  0: off, -1: automatic (default:
+ * lattices over 256 MiB of populations that do not run tiles).  Lattices with
+ * velocity-map BCs do
+ * not sweep.  Results are bit for bit the same for every value. */
+#define ASLHIP_TUNE_SWEEP_KB 7
 int aslhip_set_tuning(aslhip_lattice *h, int knob, int value);
+/* The launches of a sweep of nsteps steps over nx planes, blocks of `planes`
+ * planes and `steps` steps per sweep: triples (step, first plane, planes) in
+ * launch order, the first cap of them to out.  Returns their number. */
+int aslhip_sweep_plan(int nx, int periodic, int planes, int steps, int nsteps, int *out, int cap);
 /* The value a tuning knob has now (ASLHIP_TUNE_CPL: the cells per lane the
  * step kernel runs with; ASLHIP_TUNE_LDS: 0, 1 or 2 as it runs LDS-staged
  * tiles on no step, every step or even steps). */
@@ -487,7 +500,7 @@ int aslhip_batch_step(aslhip_batch *b, int nsteps, unsigned flags);
 /* As aslhip_batch_step, timed with HIP events on the batch's stream. */
 int aslhip_batch_time_steps(aslhip_batch *b, int nsteps, unsigned flags, double *ms_total);
 /* Workgroup size (ASLHIP_TUNE_BLOCK), LDS-staged tiles (ASLHIP_TUNE_LDS 1
- * or 0; default: tiles for non-periodic FP32 batches over 256 MiB of
+ * or 0; default: tiles for non-periodic D3Q19 FP32 batches over 256 MiB of
  * populations) or group
  * size (ASLHIP_TUNE_GROUP_MB) of the batch's launches; the autotuners choose
  * between tiles and the direct kernel's workgroup size (256/512/1024,
