@@ -1,8 +1,8 @@
 // C ABI of the closure-network trainer (include/aslhip.h, "learned closure").
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
-#include <vector>
 
 #include "../../include/aslhip.h"
 #include "closure.hpp"
@@ -18,7 +18,8 @@ struct aslhip_mlp {
   long long n = 0;
   float *partial = nullptr;
   int partial_blocks = 0;
-  double *loss = nullptr;
+  double *loss = nullptr;       // of the last gradient, or of the last steps of a training run
+  int loss_cap = 1;             // doubles at loss
   long long adam_t = 0;  // Adam steps taken
 };
 
@@ -41,15 +42,28 @@ int ensure_partial(aslhip_mlp *m, int nblocks) {
   return 0;
 }
 
+int ensure_losses(aslhip_mlp *m, int n) {
+  if (n <= m->loss_cap) return 0;
+  HIPCHK(hipStreamSynchronize(m->stream));
+  double *d = nullptr;
+  HIPCHK(hipMalloc(&d, (size_t)n * sizeof(double)));
+  (void)hipFree(m->loss);
+  m->loss = d;
+  m->loss_cap = n;
+  return 0;
+}
+
 unsigned long long mix64(unsigned long long z) {
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
   z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
   return z ^ (z >> 31);
 }
 
-// Gradient of the batch into m->g and its loss into m->loss (device).
-int batch_gradient(aslhip_mlp *m, long long first, int count, unsigned long long seed) {
-  const int nb = (count + MLP_GRAD_BLOCK - 1) / MLP_GRAD_BLOCK;
+// Gradient of the batch into m->g and its loss into *loss (device); with adam
+// the parameters take that step.
+int batch_gradient(aslhip_mlp *m, long long first, int count, unsigned long long seed, double *loss,
+                   const AdamArgs *adam) {
+  const int nb = mlp_grad_blocks(count);
   if (int r = ensure_partial(m, nb)) return r;
   MlpGradArgs a;
   a.x = m->x;
@@ -61,8 +75,11 @@ int batch_gradient(aslhip_mlp *m, long long first, int count, unsigned long long
   a.inv_batch = 1.f / static_cast<float>(count);
   a.p = m->p;
   a.partial = m->partial;
-  HIPCHK(launch_mlp_grad(a, nb, m->stream));
-  HIPCHK(launch_mlp_reduce(m->partial, nb, 1.0 / count, m->g, m->loss, m->stream));
+  HIPCHK(launch_mlp_grad(a, m->stream));
+  if (adam)
+    HIPCHK(launch_mlp_reduce_adam(m->partial, nb, 1.0 / count, m->g, loss, m->p, m->m, m->v, *adam, m->stream));
+  else
+    HIPCHK(launch_mlp_reduce(m->partial, nb, 1.0 / count, m->g, loss, m->stream));
   return 0;
 }
 
@@ -123,7 +140,7 @@ int aslhip_mlp_gradient(aslhip_mlp *m, long long first, int count, float *grad, 
   if (first < 0 || count < 1 || first + count > m->n)
     return fail(ASLHIP_EINVAL, "ASL ERROR: mlp_gradient: samples %lld..%lld outside the data set of %lld", first,
                 first + count - 1, m->n);
-  if (int r = batch_gradient(m, first, count, 0ull)) return r;
+  if (int r = batch_gradient(m, first, count, 0ull, m->loss, nullptr)) return r;
   if (grad) HIPCHK(hipMemcpyAsync(grad, m->g, CL_NPARAM * sizeof(float), hipMemcpyDeviceToHost, m->stream));
   if (loss) HIPCHK(hipMemcpyAsync(loss, m->loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   HIPCHK(hipStreamSynchronize(m->stream));
@@ -133,25 +150,30 @@ int aslhip_mlp_gradient(aslhip_mlp *m, long long first, int count, float *grad, 
 int aslhip_mlp_train(aslhip_mlp *m, int steps, int batch, double lr, unsigned long long seed, double *losses) {
   if (!m || !m->n) return fail(ASLHIP_ESTATE, "ASL ERROR: mlp_train before mlp_set_data");
   if (steps < 0 || batch < 1 || !(lr > 0.)) return fail(ASLHIP_EINVAL, "ASL ERROR: mlp_train: bad arguments");
-  std::vector<double> lv(losses ? steps : 0);
   const double b1 = 0.9, b2 = 0.999;
+  // The losses stay on the device and come over in one copy per run of
+  // LOSS_RUN steps: a copy per step held the host up until the step had ended.
+  constexpr int LOSS_RUN = 4096;
+  if (int r = ensure_losses(m, losses ? std::min(steps, LOSS_RUN) : 1)) return r;
   for (int s = 0; s < steps; ++s) {
     unsigned long long sd = mix64(seed + 0x9E3779B97F4A7C15ull * (static_cast<unsigned long long>(m->adam_t) + 1ull));
     if (sd == 0) sd = 1;
-    if (int r = batch_gradient(m, 0, batch, sd)) return r;
-    ++m->adam_t;
     AdamArgs a;
     a.lr = static_cast<float>(lr);
     a.beta1 = static_cast<float>(b1);
     a.beta2 = static_cast<float>(b2);
     a.eps = 1e-8f;
-    a.bc1 = static_cast<float>(1. - std::pow(b1, static_cast<double>(m->adam_t)));
-    a.bc2 = static_cast<float>(1. - std::pow(b2, static_cast<double>(m->adam_t)));
-    HIPCHK(launch_adam(m->p, m->g, m->m, m->v, a, m->stream));
-    if (losses) HIPCHK(hipMemcpyAsync(&lv[s], m->loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
+    a.bc1 = static_cast<float>(1. - std::pow(b1, static_cast<double>(m->adam_t + 1)));
+    a.bc2 = static_cast<float>(1. - std::pow(b2, static_cast<double>(m->adam_t + 1)));
+    const int at = losses ? s % LOSS_RUN : 0;
+    if (int r = batch_gradient(m, 0, batch, sd, m->loss + at, &a)) return r;
+    ++m->adam_t;
+    if (losses && (at == LOSS_RUN - 1 || s == steps - 1)) {
+      HIPCHK(hipStreamSynchronize(m->stream));
+      HIPCHK(hipMemcpy(losses + s - at, m->loss, (size_t)(at + 1) * sizeof(double), hipMemcpyDeviceToHost));
+    }
   }
   HIPCHK(hipStreamSynchronize(m->stream));
-  for (int s = 0; s < (losses ? steps : 0); ++s) losses[s] = lv[s];
   return 0;
 }
 

@@ -1,10 +1,11 @@
 // Training kernels of the closure network (7-32-32-1, ReLU; parameter
 // layout and model in closure.hpp): forward + backward of a batch with
-// deterministic per-block gradient sums, the reduction over blocks, and Adam.
+// deterministic per-workgroup gradient sums, and the reduction over
+// workgroups with the Adam update.
 //
 // Loss: half the mean squared error over the batch.  Adam: Kingma & Ba,
 // "Adam: A Method for Stochastic Optimization" (ICLR 2015), Algorithm 1.
-// All FP32 except the cross-block gradient and loss sums (FP64).
+// All FP32 except the cross-wavefront gradient and loss sums (FP64).
 #include <hip/hip_runtime.h>
 
 #include "closure.hpp"
@@ -13,9 +14,7 @@
 namespace aslhip {
 namespace {
 
-constexpr int GB = MLP_GRAD_BLOCK;  // samples per workgroup
-constexpr int ROW = 7 + 4 * CL_H + 2;  // per sample in LDS: xn, h1, dh1, h2, dh2, dy, r^2 / 2
-constexpr int RDY = ROW - 2, RLOSS = ROW - 1;
+typedef float f4 __attribute__((ext_vector_type(4)));
 
 // splitmix64 finaliser (S. Vigna, public domain): sample indices of a batch.
 __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
@@ -24,140 +23,269 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
   return z ^ (z >> 31);
 }
 
-__global__ __launch_bounds__(GB) void k_mlp_grad(const MlpGradArgs a) {
-  __shared__ float sh[ROW][GB];
-  const int k = blockIdx.x * GB + threadIdx.x;  // sample within the batch
-  const bool live = k < a.count;
-  long long s = 0;
-  if (live)
-    s = a.seed ? static_cast<long long>(mix64(a.seed + (static_cast<unsigned long long>(k) + 1ull) *
-                                                          0x9E3779B97F4A7C15ull) %
-                                        static_cast<unsigned long long>(a.n))
-               : a.first + k;
+__device__ __forceinline__ f32x16_t mfma(float a, float b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+// Rows of a tile in LDS: 32 values and 4 of padding (16-byte rows, other banks).
+constexpr int LROW = 36;
+constexpr int NWAVE = MLP_GRAD_BLOCK / 64;
+
+// The row of D[row][lane % 32] that register r of v_mfma_f32_32x32x2f32's
+// result holds in half h of the wavefront.
+__device__ __forceinline__ constexpr int drow(int r, int h) { return 8 * (r / 4) + 4 * h + r % 4; }
+
+// Forward and backward on the FP32 matrix instructions: every wavefront takes
+// 32 samples at a time, one per column, as five products
+//   H1 = relu(W1' x')   (x' = (x, 1), W1' = (W1, b1)),   H2 = relu(W2 H1 + b2),
+//   dH1 = W2^T dH2 [H1 > 0],   gW2 += dH2 H1^T,   gW1' += dH1 x'^T.
+// v_mfma_f32_32x32x2f32 takes A[l % 32][l / 32] and B[l / 32][l % 32] from lane
+// l; the order of the products within a sum is free, so k-step r uses rows
+// drow(r, 0) and drow(r, 1), which is how the previous product left its result:
+// layers chain without moving data.  The two gradients contract over samples;
+// their operands go through LDS once, transposed.  g_b2, g_w3, g_b3 and the
+// loss are sums per lane, added up at the end.  Sums of at most 64 samples
+// (SPW blocks of 32) are kept in FP32, as few roundings as 64-sample blocks
+// on the vector ALUs had; everything beyond is FP64.
+//
+// Bound by latency: 16384 samples are 118 MFLOP (1 us of the matrix cores) in
+// one block per wavefront, 60 dependent instructions of 64 cycles; 91 us
+// before, on the vector ALUs with the weight products summed from LDS one
+// sample after the other.  A training step of 16384 samples: 163 -> 10.7 us
+// with the reduction below; error of the gradient against FP64 2.8e-8 both.
+template <int SPW>
+__global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a) {
+  __shared__ __attribute__((aligned(16))) float tile[NWAVE][3][CL_H * LROW];  // dH2, H1, dH1: [unit][sample]
+  __shared__ __attribute__((aligned(16))) float xt[NWAVE][8 * LROW];          // x': [input][sample]
+  const int w = static_cast<int>(threadIdx.x) >> 6, l = static_cast<int>(threadIdx.x) & 63;
+  const int col = l & 31, half = l >> 5;
+  float *dh2t = tile[w][0], *h1t = tile[w][1], *dh1t = tile[w][2], *x8 = xt[w];
   const float *p = a.p;
-  float xn[7], h1[CL_H], a1m[CL_H], h2[CL_H], dh2[CL_H];
+
+  // weights in operand order
+  float w1[4], w2[16], w2t[16], b2[16], w3[16];
 #pragma unroll
-  for (int j = 0; j < 7; ++j) xn[j] = live ? a.x[s * 7 + j] : 0.f;
-#pragma unroll
-  for (int o = 0; o < CL_H; ++o) {
-    float v = p[CL_B1 + o];
-#pragma unroll
-    for (int j = 0; j < 7; ++j) v = __builtin_fmaf(p[CL_W1 + o * 7 + j], xn[j], v);
-    a1m[o] = v > 0.f ? 1.f : 0.f;
-    h1[o] = v > 0.f ? v : 0.f;
+  for (int k = 0; k < 4; ++k) {
+    const int in = 2 * k + half;
+    w1[k] = in < CL_NIN ? p[CL_W1 + col * CL_NIN + in] : p[CL_B1 + col];
   }
-  float y = p[CL_B3];
 #pragma unroll
-  for (int o = 0; o < CL_H; ++o) {
-    float v = p[CL_B2 + o];
-#pragma unroll
-    for (int j = 0; j < CL_H; ++j) v = __builtin_fmaf(p[CL_W2 + o * CL_H + j], h1[j], v);
-    h2[o] = v > 0.f ? v : 0.f;
-    dh2[o] = v > 0.f ? 1.f : 0.f;  // mask for now
-    y = __builtin_fmaf(p[CL_W3 + o], h2[o], y);
+  for (int r = 0; r < 16; ++r) {
+    w2[r] = p[CL_W2 + col * CL_H + drow(r, half)];
+    w2t[r] = p[CL_W2 + drow(r, half) * CL_H + col];
+    b2[r] = p[CL_B2 + drow(r, half)];
+    w3[r] = p[CL_W3 + drow(r, half)];
   }
-  const float r = live ? y - a.t[s] : 0.f;
-  const float dy = r * a.inv_batch;
+  const float b3 = p[CL_B3];
+
+  f32x16_t gw2 = {}, gw1 = {};
+  float gb2[16], gw3[16], gb3 = 0.f, loss = 0.f;
 #pragma unroll
-  for (int o = 0; o < CL_H; ++o) dh2[o] *= dy * p[CL_W3 + o];
-  float dh1[CL_H];
+  for (int r = 0; r < 16; ++r) gb2[r] = gw3[r] = 0.f;
+
+#pragma unroll 1
+  for (int it = 0; it < SPW; ++it) {
+    // this column's sample within the batch
+    const int k = ((static_cast<int>(blockIdx.x) * SPW + it) * NWAVE + w) * 32 + col;
+    const bool live = k < a.count;
+    long long s = 0;
+    if (live)
+      s = a.seed ? static_cast<long long>(mix64(a.seed + (static_cast<unsigned long long>(k) + 1ull) *
+                                                            0x9E3779B97F4A7C15ull) %
+                                          static_cast<unsigned long long>(a.n))
+                 : a.first + k;
+    float x[4];  // inputs half, 2 + half, 4 + half, 6 + half (the eighth: 1)
 #pragma unroll
-  for (int j = 0; j < CL_H; ++j) {
-    float v = 0.f;
-#pragma unroll
-    for (int o = 0; o < CL_H; ++o) v = __builtin_fmaf(p[CL_W2 + o * CL_H + j], dh2[o], v);
-    dh1[j] = v * a1m[j];
-  }
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int j = 0; j < 7; ++j) sh[j][t] = xn[j];
-#pragma unroll
-  for (int o = 0; o < CL_H; ++o) {
-    sh[7 + o][t] = h1[o];
-    sh[7 + CL_H + o][t] = dh1[o];
-    sh[7 + 2 * CL_H + o][t] = h2[o];
-    sh[7 + 3 * CL_H + o][t] = dh2[o];
-  }
-  sh[RDY][t] = dy;
-  sh[RLOSS][t] = 0.5f * r * r;
-  __syncthreads();
-  // parameter q of this block: sum over the block's samples of u * v
-  float *out = a.partial + static_cast<long long>(blockIdx.x) * MLP_PSTRIDE;
-  for (int q = t; q < CL_NPARAM; q += GB) {
-    int ru, rv;  // LDS rows of the two factors (rv < 0: factor 1)
-    if (q < CL_B1) {
-      ru = 7 + CL_H + q / 7;  // dh1[o]
-      rv = q % 7;             // xn[j]
-    } else if (q < CL_W2) {
-      ru = 7 + CL_H + (q - CL_B1);
-      rv = -1;
-    } else if (q < CL_B2) {
-      ru = 7 + 3 * CL_H + (q - CL_W2) / CL_H;  // dh2[o]
-      rv = 7 + (q - CL_W2) % CL_H;             // h1[j]
-    } else if (q < CL_W3) {
-      ru = 7 + 3 * CL_H + (q - CL_B2);
-      rv = -1;
-    } else if (q < CL_B3) {
-      ru = RDY;
-      rv = 7 + 2 * CL_H + (q - CL_W3);  // h2[j]
-    } else {
-      ru = RDY;
-      rv = -1;
+    for (int j = 0; j < 4; ++j) {
+      const int in = 2 * j + half;
+      x[j] = in == CL_NIN ? 1.f : (live ? a.x[s * CL_NIN + in] : 0.f);
     }
-    float acc = 0.f;
-    for (int i = 0; i < GB; ++i) acc = __builtin_fmaf(sh[ru][i], rv >= 0 ? sh[rv][i] : 1.f, acc);
-    out[q] = acc;
+    const float t = live ? a.t[s] : 0.f;
+
+    f32x16_t h1 = {};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h1 = mfma(w1[j], x[j], h1);
+    float m1[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      m1[r] = h1[r] > 0.f ? 1.f : 0.f;
+      h1[r] = h1[r] > 0.f ? h1[r] : 0.f;
+    }
+    f32x16_t h2;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) h2[r] = b2[r];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) h2 = mfma(w2[r], h1[r], h2);
+    float part = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part = __builtin_fmaf(w3[r], h2[r] > 0.f ? h2[r] : 0.f, part);
+    const float y = part + __shfl_xor(part, 32) + b3;
+    const float res = live ? y - t : 0.f;
+    const float dy = res * a.inv_batch;
+    f32x16_t d1 = {};
+    float d2[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float v = h2[r] > 0.f ? h2[r] : 0.f;
+      d2[r] = (h2[r] > 0.f ? 1.f : 0.f) * (dy * w3[r]);
+      gw3[r] = __builtin_fmaf(dy, v, gw3[r]);
+      gb2[r] += d2[r];
+    }
+    gb3 += dy;
+    loss += 0.5f * res * res;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) d1 = mfma(w2t[r], d2[r], d1);
+
+    if (SPW > 1 && it) __syncthreads();  // the last block's operands have been read
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int o = drow(r, half) * LROW + col;
+      dh2t[o] = d2[r];
+      h1t[o] = h1[r];
+      dh1t[o] = d1[r] * m1[r];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x8[(2 * j + half) * LROW + col] = live ? x[j] : 0.f;
+    __syncthreads();
+    // samples 16 half .. 16 half + 15 of unit (input) col; k-step i pairs samples i and 16 + i
+    const f4 *ra = reinterpret_cast<const f4 *>(dh2t + col * LROW + 16 * half);
+    const f4 *rb = reinterpret_cast<const f4 *>(h1t + col * LROW + 16 * half);
+    const f4 *rc = reinterpret_cast<const f4 *>(dh1t + col * LROW + 16 * half);
+    const f4 *rx = reinterpret_cast<const f4 *>(x8 + (col & 7) * LROW + 16 * half);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f4 va = ra[i], vb = rb[i], vc = rc[i];
+      f4 vx = rx[i];
+      if (col >= 8) vx = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        gw2 = mfma(va[j], vb[j], gw2);
+        gw1 = mfma(vc[j], vx[j], gw1);
+      }
+    }
   }
-  if (t == 0) {
-    float l = 0.f;
-    for (int i = 0; i < GB; ++i) l += sh[RLOSS][i];
-    out[CL_NPARAM] = l;
+
+  // sums over the lanes of a column block: transposed through LDS, each lane adds 16, then the two halves
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int o = drow(r, half) * LROW + col;
+    dh2t[o] = gb2[r];
+    h1t[o] = gw3[r];
+  }
+  x8[col] = gb3;  // both halves hold the same sample's dy and loss
+  x8[LROW + col] = loss;
+  __syncthreads();
+  float sb2 = 0.f, sw3 = 0.f, sl = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    sb2 += dh2t[col * LROW + 16 * half + i];
+    sw3 += h1t[col * LROW + 16 * half + i];
+    sl += x8[(col & 1) * LROW + 16 * half + i];
+  }
+  sb2 += __shfl_xor(sb2, 32);
+  sw3 += __shfl_xor(sw3, 32);
+  sl += __shfl_xor(sl, 32);
+  __syncthreads();
+  // this wavefront's sums in parameter order
+  static_assert(3 * CL_H * LROW >= CL_NPARAM + 1, "the tiles hold one set of parameters");
+  float *out = tile[w][0];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int o = drow(r, half);
+    out[CL_W2 + o * CL_H + col] = gw2[r];
+    if (col < CL_NIN) out[CL_W1 + o * CL_NIN + col] = gw1[r];
+    if (col == CL_NIN) out[CL_B1 + o] = gw1[r];
+  }
+  if (half == 0) {
+    out[CL_B2 + col] = sb2;
+    out[CL_W3 + col] = sw3;
+    if (col < 2) out[CL_B3 + col] = sl;  // g_b3, then the loss
+  }
+  __syncthreads();
+  float *dst = a.partial + static_cast<long long>(blockIdx.x) * MLP_PSTRIDE;
+  for (int q = static_cast<int>(threadIdx.x); q <= CL_NPARAM; q += MLP_GRAD_BLOCK) {
+    double acc = 0.;
+#pragma unroll
+    for (int v = 0; v < NWAVE; ++v) acc += static_cast<double>(tile[v][0][q]);
+    dst[q] = static_cast<float>(acc);
   }
 }
 
-// grad[q] = sum over blocks of partial[b][q] (FP64, in block order); the last
-// entry is the loss (0.5 * sum r^2 / count).
+// Parameters per workgroup of the reduction, and the slices that share the
+// partial sums of one.
+constexpr int RP = 32, RS = 256 / RP;
+
+// grad[q] = sum over workgroups of partial[b][q] (FP64; slice s takes b = s,
+// s + RS, ..., then the slices in order); the last entry is the loss
+// (0.5 * sum r^2 / count).  ADAM: the parameter's update follows at once,
+// which saves a launch per step.  Eight slices of 32 parameters per workgroup
+// read whole 128-byte lines; with one thread per parameter, 16384 samples'
+// partials took 61 us.
+template <bool ADAM>
 __global__ __launch_bounds__(256) void k_mlp_reduce(const float *partial, int nblocks, double inv_count, float *grad,
-                                                    double *loss) {
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q > CL_NPARAM) return;
+                                                    double *loss, float *p, float *m, float *v, AdamArgs a) {
+  __shared__ double sh[RS][RP];
+  const int i = static_cast<int>(threadIdx.x) % RP, s = static_cast<int>(threadIdx.x) / RP;
+  const int q = static_cast<int>(blockIdx.x) * RP + i;
   double acc = 0.;
-  for (int b = 0; b < nblocks; ++b) acc += static_cast<double>(partial[static_cast<long long>(b) * MLP_PSTRIDE + q]);
-  if (q < CL_NPARAM)
-    grad[q] = static_cast<float>(acc);
-  else
+  if (q <= CL_NPARAM) {
+#pragma unroll 8
+    for (int b = s; b < nblocks; b += RS)
+      acc += static_cast<double>(partial[static_cast<long long>(b) * MLP_PSTRIDE + q]);
+  }
+  sh[s][i] = acc;
+  __syncthreads();
+  if (s != 0 || q > CL_NPARAM) return;
+#pragma unroll
+  for (int k = 1; k < RS; ++k) acc += sh[k][i];
+  if (q == CL_NPARAM) {
     *loss = acc * inv_count;
-}
-
-__global__ __launch_bounds__(256) void k_adam(float *p, const float *g, float *m, float *v, AdamArgs a) {
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= CL_NPARAM) return;
-  const float gq = g[q];
-  const float mq = __builtin_fmaf(a.beta1, m[q], (1.f - a.beta1) * gq);
-  const float vq = __builtin_fmaf(a.beta2, v[q], (1.f - a.beta2) * gq * gq);
-  m[q] = mq;
-  v[q] = vq;
-  const float mhat = mq / a.bc1;
-  const float vhat = vq / a.bc2;
-  p[q] = p[q] - a.lr * mhat / (__builtin_sqrtf(vhat) + a.eps);
+    return;
+  }
+  const float gq = static_cast<float>(acc);
+  grad[q] = gq;
+  if constexpr (ADAM) {
+    const float mq = __builtin_fmaf(a.beta1, m[q], (1.f - a.beta1) * gq);
+    const float vq = __builtin_fmaf(a.beta2, v[q], (1.f - a.beta2) * gq * gq);
+    m[q] = mq;
+    v[q] = vq;
+    const float mhat = mq / a.bc1;
+    const float vhat = vq / a.bc2;
+    p[q] = p[q] - a.lr * mhat / (__builtin_sqrtf(vhat) + a.eps);
+  }
 }
 
 }  // namespace
 
-hipError_t launch_mlp_grad(const MlpGradArgs &a, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_grad, dim3(nblocks), dim3(GB), 0, s, a);
+// One block of 32 samples per wavefront while that leaves CUs without work
+// (256 workgroups of 128 samples), else two: half the partial sums.
+int mlp_grad_blocks(int count) {
+  const int per = count <= 256 * 32 * NWAVE ? 32 * NWAVE : 64 * NWAVE;
+  return static_cast<int>((static_cast<long long>(count) + per - 1) / per);
+}
+
+hipError_t launch_mlp_grad(const MlpGradArgs &a, hipStream_t s) {
+  const dim3 grid(mlp_grad_blocks(a.count)), block(MLP_GRAD_BLOCK);
+  if (a.count <= 256 * 32 * NWAVE)
+    hipLaunchKernelGGL(k_mlp_grad<1>, grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL(k_mlp_grad<2>, grid, block, 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_mlp_reduce(const float *partial, int nblocks, double inv_count, float *grad, double *loss,
                              hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((CL_NPARAM + 1 + 255) / 256), dim3(256), 0, s, partial, nblocks, inv_count,
-                     grad, loss);
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((CL_NPARAM + RP) / RP), dim3(256), 0, s, partial, nblocks, inv_count,
+                     grad, loss, static_cast<float *>(nullptr), static_cast<float *>(nullptr),
+                     static_cast<float *>(nullptr), AdamArgs{});
   return hipGetLastError();
 }
 
-hipError_t launch_adam(float *p, const float *g, float *m, float *v, const AdamArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(k_adam, dim3((CL_NPARAM + 255) / 256), dim3(256), 0, s, p, g, m, v, a);
+hipError_t launch_mlp_reduce_adam(const float *partial, int nblocks, double inv_count, float *grad, double *loss,
+                                  float *p, float *m, float *v, const AdamArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((CL_NPARAM + RP) / RP), dim3(256), 0, s, partial, nblocks, inv_count,
+                     grad, loss, p, m, v, a);
   return hipGetLastError();
 }
 

@@ -5,8 +5,8 @@
 
 namespace aslhip {
 
-constexpr int MLP_GRAD_BLOCK = 64;    // samples per gradient workgroup
-constexpr int MLP_PSTRIDE = 1346;     // floats per block partial: 1345 gradients + loss
+constexpr int MLP_GRAD_BLOCK = 256;   // lanes of a gradient workgroup (4 wavefronts of 32 samples at a time)
+constexpr int MLP_PSTRIDE = 1376;     // floats per workgroup partial: 1345 gradients + loss, whole 128-byte lines
 
 struct MlpGradArgs {
   const float *x;        // n x 7 normalised inputs
@@ -25,9 +25,13 @@ struct AdamArgs {
   float bc1, bc2;  // 1 - beta1^t, 1 - beta2^t
 };
 
-hipError_t launch_mlp_grad(const MlpGradArgs &a, int nblocks, hipStream_t s);
+// Workgroups (partial sums) of a batch of count samples.
+int mlp_grad_blocks(int count);
+hipError_t launch_mlp_grad(const MlpGradArgs &a, hipStream_t s);
 hipError_t launch_mlp_reduce(const float *partial, int nblocks, double inv_count, float *grad, double *loss,
                              hipStream_t s);
-hipError_t launch_adam(float *p, const float *g, float *m, float *v, const AdamArgs &a, hipStream_t s);
+// The reduction followed by an Adam step of the parameters p (moments m, v).
+hipError_t launch_mlp_reduce_adam(const float *partial, int nblocks, double inv_count, float *grad, double *loss,
+                                  float *p, float *m, float *v, const AdamArgs &a, hipStream_t s);
 
 }  // namespace aslhip
