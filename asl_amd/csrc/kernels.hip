@@ -488,10 +488,8 @@ __device__ __forceinline__ void face_values(const StepHot &g, const StepArgs &a,
 // takes no vector address arithmetic; an array stays below 4 GiB.
 // WIDE: the arrays together exceed 4 GiB (only the links that choose between
 // two slots are affected).
-// PEEK: instead of colliding and storing, write the populations the cell
-// receives (after every BC link is resolved) to peek[k * len + cell].
-template <int Q, class S, bool ODD, bool PER, bool WIDE, int CL = 0, bool PEEK = false>
-__device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, const int chunk, void *peek = nullptr) {
+template <int Q, class S, bool ODD, bool PER, bool WIDE, int CL = 0>
+__device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, const int chunk) {
   using CD = Codec<S>;
   using C = typename CD::C;
   using M = typename CD::M;
@@ -613,14 +611,6 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
       const C sv = val[slot * Q + k];
       v[k] = md == MODE_BOUNCE ? x + sv : (md == MODE_CONST ? sv : x);
     }
-  }
-
-  if constexpr (PEEK) {
-    if (!live) return;
-    M *o = static_cast<M *>(peek);
-#pragma unroll
-    for (int k = 0; k < Q; ++k) o[static_cast<long long>(k) * a.len + idx] = M(v[k]);
-    return;
   }
 
   C r, m[3];
@@ -1128,60 +1118,124 @@ __global__ __launch_bounds__(STEP_RUN_BLOCK) void k_step_run(const StepHot g, co
   step_body_run<Q, S, ODD, CPL>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
 
-// The incoming populations of every computed cell for the next step.
-template <int Q, class S, bool ODD, bool PER>
-__global__ __launch_bounds__(step_block(Q, sizeof(S))) void k_peek(const StepHot g, const StepArgs *args, void *out) {
-  step_body<Q, S, ODD, PER, false, 0, true>(g, *args, static_cast<int>(blockIdx.x), out);
+// Cell idx + sgn c_i, wrapped into the interior for interior cells of periodic
+// lattices.  sgn 1: the cell whose slot i holds population i of cell idx after
+// an odd step.
+template <int Q>
+__device__ __forceinline__ int shifted(int idx, int i, int sgn, int sx, int sy, int per, int nx, int ny, int nz) {
+  if (!per) return idx + sgn * offc<Q>(i, sx, sy);
+  const int x = idx / sx, rem = idx - x * sx, y = rem / sy, z = rem - y * sy;
+  if (x < 1 || x > nx || y < 1 || y > ny || z < 1 || z > nz) return idx + sgn * offc<Q>(i, sx, sy);
+  return wrap1(x + sgn * Lat<Q>::c[i][0], nx) * sx + wrap1(y + sgn * Lat<Q>::c[i][1], ny) * sy +
+         wrap1(z + sgn * Lat<Q>::c[i][2], nz);
+}
+
+// Population i of cell idx after the last step (ASL's view).  Slots outside
+// the array (outer ghost layer) read as NaN.
+template <int Q, class S>
+__device__ __forceinline__ typename Codec<S>::C outgoing(const StepHot &g, int per, int len, int after_odd, int idx,
+                                                         int i) {
+  using CD = Codec<S>;
+  if (!after_odd) return CD::ld(g.f + inv_dir<Q>(i) * g.qs, static_cast<unsigned>(idx) * sizeof(S));
+  const int src = shifted<Q>(idx, i, 1, g.sx, g.sy, per, g.nx, g.ny, g.nz);
+  if (src < 0 || src >= len) return typename CD::C(__builtin_nan(""));
+  return CD::ld(g.f + i * g.qs, static_cast<unsigned>(src) * sizeof(S));
+}
+
+// Population k that cell idx receives in the next step, every BC resolved as
+// step_body does (face rule, link patterns); 0 for cells that are not computed.
+template <int Q, class S>
+__device__ __forceinline__ typename Codec<S>::C incoming(const StepHot &g, const StepArgs &a, int per, int after_odd,
+                                                         int idx, int k) {
+  using CD = Codec<S>;
+  using C = typename CD::C;
+  const int x = idx / g.sx, rem = idx - x * g.sx, y = rem / g.sy, z = rem - y * g.sy;
+  if (x < 1 || x > g.nx || y < 1 || y > g.ny || z < 1 || z > g.nz) return C(0);
+  const unsigned char code = g.code[idx];
+  if (code == CODE_SKIP) return C(0);
+  bool bounce = false, cnst = false;
+  C val = C(0);
+  if (!per && code == CODE_FLUID) {
+    const unsigned fb = face_bits(g, x, y, z) & a.fset;
+    int f = -1;  // the face that claims the link, the one executed last
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int cd = Lat<Q>::c[k][d], c = 2 * d + (cd > 0 ? 0 : 1);
+      if (cd != 0 && ((fb >> c) & 1u) && (f < 0 || ((a.fbeats[f] >> c) & 1u))) f = c;
+    }
+    if (f >= 0) {
+      bounce = (a.fbounces >> f) & 1u;
+      cnst = !bounce;
+      val = sizeof(C) == 4 ? C(a.fval32[f][k]) : C(a.fval64[f][k]);
+    }
+  } else if (!per) {
+    const int slot = a.rec[a.pat[idx]].slot[k];
+    const unsigned char md = slot ? a.mode[slot] : static_cast<unsigned char>(MODE_NONE);
+    bounce = md == MODE_BOUNCE;
+    cnst = md == MODE_CONST;
+    val = static_cast<const C *>(a.val)[slot * Q + k];
+  }
+  if (cnst) return val;
+  // array inv k at idx - c_k before an odd step, array k at idx before an even one; bounce-back: the other of the two
+  const bool near = bounce == !after_odd;
+  const int src = near ? idx : shifted<Q>(idx, k, -1, g.sx, g.sy, per, g.nx, g.ny, g.nz);
+  const C v = CD::ld(g.f + (near ? k : inv_dir<Q>(k)) * g.qs, static_cast<unsigned>(src) * sizeof(S));
+  return bounce ? v + val : v;
 }
 
 // asl::ComputeSurfaceForceMap / ComputeSurfaceFluxMap (src/num/aslLBGKBC.cxx:
-// 623-736) from two host-layout views: post[i * len + x] = f_i of cell x after
-// the last collision, in_[i * len + x] = f_i that cell x receives next (the
-// value ASL's BCs leave at ghost x - c_i).  For a ghost cell x (map <= 0) next
-// to a computation node y = x + c_i (map > 0), ASL's f_i(x) is in_[i][y];
-// for a computation node x next to a ghost y, ASL's f_inv(i)(y) is
-// in_[inv(i)][x].  Cells with |map| >= 0.9999 get 0 (ASL leaves them as they
-// were); map reads outside the block are -0.9 (a ghost node), as in ASL.
+// 623-736).  For a ghost cell x (map <= 0) next to a computation node y =
+// x + c_i (map > 0), ASL's f_i(x) is the population i that y receives next
+// (the value ASL's BCs leave at the ghost); for a computation node x next to a
+// ghost y, ASL's f_inv(i)(y) is the population inv(i) that x receives.  Cells
+// with |map| >= 0.9999 get 0 (ASL leaves them as they were); map reads outside
+// the block are -0.9 (a ghost node), as in ASL.
+//
+// The populations are taken from the step kernel's slots, and only next to
+// the surface: a read of the map and a write of the result for the other
+// cells.  Full views of outgoing and incoming populations, as before, cost
+// two copies of the lattice: 25 + 24 + 16 us and a clear of 11 on
+// 160 x 72 x 60, D3Q19 FP32; 20 steps of LBGKTurbulence there with a force and
+// a read of u 2461 -> 1696 us, allocations included.
 template <int Q, class S>
-__global__ __launch_bounds__(BLOCK) void k_surface(const SurfaceArgs a) {
+__global__ __launch_bounds__(BLOCK) void k_surface(const SurfaceArgs s, const StepHot g, const StepArgs *args) {
   using C = typename Codec<S>::C;
   using M = typename Codec<S>::M;
   const int x = blockIdx.x * BLOCK + threadIdx.x;
-  if (x >= a.len) return;
-  const M *post = static_cast<const M *>(a.post), *in = static_cast<const M *>(a.in);
-  M *out = static_cast<M *>(a.out);
-  const float m0 = a.map[x];
+  if (x >= s.len) return;
+  M *out = static_cast<M *>(s.out);
+  const float m0 = s.map[x];
   C acc[3] = {C(0), C(0), C(0)};
   if (__builtin_fabsf(m0) < .9999f) {
 #pragma unroll
     for (int i = 1; i < Q; ++i) {
       const int kb = inv_dir<Q>(i);
-      const long long y = static_cast<long long>(x) + offc<Q>(i, a.sx, a.sy);
-      const float my = (y < 0 || y > a.len - 1) ? -.9f : a.map[y];
+      const long long y = static_cast<long long>(x) + offc<Q>(i, g.sx, g.sy);
+      const float my = (y < 0 || y > s.len - 1) ? -.9f : s.map[y];
       const bool b0 = m0 <= 0.f && my > 0.f;  // isGhostNode(0) && isComputationNode(i)
       const bool bi = m0 > 0.f && my <= 0.f;  // isGhostNode(i) && isComputationNode(0)
-      const long long yy = b0 ? y : x;        // the computation node of the link
-      const C f0 = b0 ? C(in[static_cast<long long>(i) * a.len + yy]) : C(post[static_cast<long long>(i) * a.len + x]);
-      const C fI = b0 ? C(post[static_cast<long long>(kb) * a.len + yy]) : C(in[static_cast<long long>(kb) * a.len + x]);
-      if (a.flux) {
+      if (!b0 && !bi) continue;  // adds 0
+      const int c = b0 ? static_cast<int>(y) : x;  // the computation node of the link
+      const C in = incoming<Q, S>(g, *args, s.per, s.after_odd, c, b0 ? i : kb);
+      const C post = outgoing<Q, S>(g, s.per, s.len, s.after_odd, c, b0 ? kb : i);
+      const C f0 = b0 ? in : post, fI = b0 ? post : in;
+      if (s.flux) {
         const C wi = C(Lat<Q>::w(i));
-        acc[0] = acc[0] + (b0 ? (f0 - fI) * wi : C(0));
-        acc[0] = acc[0] + (bi ? (fI - f0) * wi : C(0));
+        acc[0] = acc[0] + (b0 ? (f0 - fI) * wi : (fI - f0) * wi);
       } else {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
           const C wc = C(Lat<Q>::w(i) * double(Lat<Q>::c[i][d]));
-          acc[d] = acc[d] + (b0 ? ((f0 + fI) - C(2.)) * wc : C(0));
-          acc[d] = acc[d] + (bi ? ((-f0 - fI) + C(2.)) * wc : C(0));
+          acc[d] = acc[d] + (b0 ? ((f0 + fI) - C(2.)) * wc : ((-f0 - fI) + C(2.)) * wc);
         }
       }
     }
   }
-  if (a.flux) {
+  if (s.flux) {
     out[x] = M(acc[0]);
   } else {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) out[static_cast<long long>(d) * a.len + x] = M(acc[d]);
+    for (int d = 0; d < 3; ++d) out[static_cast<long long>(d) * s.len + x] = M(acc[d]);
   }
 }
 
@@ -1464,16 +1518,6 @@ __global__ __launch_bounds__(BLOCK) void k_write_f(const WriteFArgs a) {
   for (int d = 0; d < 3; ++d) static_cast<M *>(a.u)[d * a.len + idx] = M(a.compressible ? m[d] / r : m[d]);
 }
 
-// Cell whose slot i holds population i of cell idx after an odd step: idx + c_i,
-// wrapped into the interior on periodic lattices.
-template <int Q>
-__device__ __forceinline__ int odd_slot(int idx, int i, int sx, int sy, int per, int nx, int ny, int nz) {
-  if (!per) return idx + offc<Q>(i, sx, sy);
-  const int x = idx / sx, rem = idx - x * sx, y = rem / sy, z = rem - y * sy;
-  if (x < 1 || x > nx || y < 1 || y > ny || z < 1 || z > nz) return idx + offc<Q>(i, sx, sy);
-  return wrap1(x + Lat<Q>::c[i][0], nx) * sx + wrap1(y + Lat<Q>::c[i][1], ny) * sy + wrap1(z + Lat<Q>::c[i][2], nz);
-}
-
 // The post-collision populations in ASL's view (f_i of cell x), from the AA
 // state.  Slots outside the array (outer ghost layer) read as NaN.
 template <int Q, class S>
@@ -1488,7 +1532,7 @@ __global__ __launch_bounds__(BLOCK) void k_unpermute(const UnpermuteArgs a) {
   for (int i = 0; i < Q; ++i) {
     M v;
     if (a.after_odd) {
-      const int src = odd_slot<Q>(idx, i, a.sx, a.sy, a.per, a.nx, a.ny, a.nz);
+      const int src = shifted<Q>(idx, i, 1, a.sx, a.sy, a.per, a.nx, a.ny, a.nz);
       v = (src >= 0 && src < a.len)
               ? M(CD::ld(a.f + i * a.qs_bytes, static_cast<unsigned>(src) * sizeof(S)))
               : M(__builtin_nan(""));
@@ -1514,7 +1558,7 @@ __global__ __launch_bounds__(BLOCK) void k_reduce(const ReduceArgs a) {
       double fi;
       if (a.after_odd)
         fi = double(CD::ld(a.f + i * a.qs_bytes,
-                           static_cast<unsigned>(odd_slot<Q>(idx, i, a.sx, a.sy, a.per, a.nx, a.ny, a.nz)) * sizeof(S)));
+                           static_cast<unsigned>(shifted<Q>(idx, i, 1, a.sx, a.sy, a.per, a.nx, a.ny, a.nz)) * sizeof(S)));
       else
         fi = double(CD::ld(a.f + inv_dir<Q>(i) * a.qs_bytes, static_cast<unsigned>(idx) * sizeof(S)));
       fi *= Lat<Q>::w(i);
@@ -1666,27 +1710,9 @@ struct InitF {
   }
 };
 template <int Q, class S>
-struct PeekF {
-  static hipError_t run(bool odd, bool per, const StepLaunch &a, void *out, hipStream_t s) {
-    const dim3 grid(a.hot.nchunks), block(a.hot.block);
-    if (per) {
-      if (odd)
-        hipLaunchKernelGGL((k_peek<Q, S, true, true>), grid, block, 0, s, a.hot, a.args, out);
-      else
-        hipLaunchKernelGGL((k_peek<Q, S, false, true>), grid, block, 0, s, a.hot, a.args, out);
-    } else {
-      if (odd)
-        hipLaunchKernelGGL((k_peek<Q, S, true, false>), grid, block, 0, s, a.hot, a.args, out);
-      else
-        hipLaunchKernelGGL((k_peek<Q, S, false, false>), grid, block, 0, s, a.hot, a.args, out);
-    }
-    return hipGetLastError();
-  }
-};
-template <int Q, class S>
 struct SurfaceF {
-  static hipError_t run(const SurfaceArgs &a, hipStream_t s) {
-    hipLaunchKernelGGL((k_surface<Q, S>), dim3((a.len + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, s, a);
+  static hipError_t run(const SurfaceArgs &a, const StepHot &g, const StepArgs *args, hipStream_t s) {
+    hipLaunchKernelGGL((k_surface<Q, S>), dim3((a.len + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, s, a, g, args);
     return hipGetLastError();
   }
 };
@@ -1748,10 +1774,9 @@ const KernelTable &ASLHIP_PASTE(kernels_q, ASLHIP_Q)() {
       [](int dt, const VLinkArgs &a, hipStream_t s) { return dispatch<VLinkF>(dt, a, s); },
       [](int dt, const InitArgs &a, hipStream_t s) { return dispatch<InitF>(dt, a, s); },
       [](int dt, const WriteFArgs &a, hipStream_t s) { return dispatch<WriteFF>(dt, a, s); },
-      [](int dt, bool odd, bool per, const StepLaunch &a, void *out, hipStream_t s) {
-        return dispatch<PeekF>(dt, odd, per, a, out, s);
+      [](int dt, const SurfaceArgs &a, const StepHot &g, const StepArgs *args, hipStream_t s) {
+        return dispatch<SurfaceF>(dt, a, g, args, s);
       },
-      [](int dt, const SurfaceArgs &a, hipStream_t s) { return dispatch<SurfaceF>(dt, a, s); },
       [](int dt, const VisArgs &a, hipStream_t s) { return dispatch<VisF>(dt, a, s); },
       [](int dt, const UnpermuteArgs &a, hipStream_t s) { return dispatch<UnpermuteF>(dt, a, s); },
       [](int dt, const ReduceArgs &a, double *out, hipStream_t s) { return dispatch<ReduceF>(dt, a, out, s); },

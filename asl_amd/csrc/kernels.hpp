@@ -81,7 +81,7 @@ struct StepArgs {
   unsigned long long zmagic;  // ceil(2^40 / sy): row = (off * zmagic) >> 40 (tiles)
   int cpl;                    // cells per lane along z
   int tile;                   // 1: LDS-staged tiles (block = STEP_TILE, cpl = 1)
-  unsigned fbounces;          // bit f: face f bounces
+  unsigned fset, fbounces;    // bit f: face f has a BC / it bounces
   unsigned fbeats[6];         // per face: the faces whose BC is executed later
   float fval32[6][28];        // per face and direction: addend / constant (FP32 lattices)
   double fval64[6][28];       // the same for FP64 lattices
@@ -144,15 +144,14 @@ struct InitArgs {
   void *rho, *u;
 };
 
-// per: periodic lattice of interior size nx x ny x nz (after an odd step the
-// populations of a face cell sit in the wrapped neighbour's slots).
-// Surface force (3 x len) or flux (len) of a level-set map, in the
-// macroscopic type, from post-collision and incoming population views.
+// Surface force (3 x len) or flux (len) of a level-set map, in the macroscopic
+// type, from the populations after the last step.
 struct SurfaceArgs {
   const float *map;
-  const void *post, *in;  // Q * len each
   void *out;
-  int sx, sy, len;
+  int len;
+  int per;                // periodic lattice
+  int after_odd;          // state after an odd step (else after an even one / init)
   int flux;               // 1: ComputeSurfaceFluxMap, 0: ComputeSurfaceForceMap
 };
 
@@ -182,7 +181,9 @@ struct WriteFArgs {
 };
 
 // The cells first .. first + count - 1 (count = len: all of them) go to
-// out[i * count + cell - first].
+// out[i * count + cell - first].  per: periodic lattice of interior size
+// nx x ny x nz (after an odd step the populations of a face cell sit in the
+// wrapped neighbour's slots).
 struct UnpermuteArgs {
   const char *f;
   long long qs_bytes;
@@ -221,8 +222,7 @@ struct KernelTable {
   hipError_t (*vlinks)(int, const VLinkArgs &, hipStream_t);
   hipError_t (*init)(int, const InitArgs &, hipStream_t);
   hipError_t (*write_f)(int, const WriteFArgs &, hipStream_t);
-  hipError_t (*peek)(int, bool odd, bool periodic, const StepLaunch &, void *out, hipStream_t);
-  hipError_t (*surface)(int, const SurfaceArgs &, hipStream_t);
+  hipError_t (*surface)(int, const SurfaceArgs &, const StepHot &, const StepArgs *, hipStream_t);
   hipError_t (*vis)(int, const VisArgs &, hipStream_t);
   hipError_t (*unpermute)(int, const UnpermuteArgs &, hipStream_t);
   hipError_t (*reduce)(int, const ReduceArgs &, double *out, hipStream_t);
@@ -242,10 +242,9 @@ hipError_t launch_closure_features(int dtype, bool odd, const StepArgs *args, lo
                                   hipStream_t s);
 hipError_t launch_init(int q, int dtype, const InitArgs &a, hipStream_t s);
 hipError_t launch_write_f(int q, int dtype, const WriteFArgs &a, hipStream_t s);
-// The populations every computed cell receives in the next step (Q * len,
-// macroscopic type, other cells untouched); lattices under 4 GiB.
-hipError_t launch_peek(int q, int dtype, bool odd, bool periodic, const StepLaunch &a, void *out, hipStream_t s);
-hipError_t launch_surface(int q, int dtype, const SurfaceArgs &a, hipStream_t s);
+// g, args: the lattice's step description (args in device memory).
+hipError_t launch_surface(int q, int dtype, const SurfaceArgs &a, const StepHot &g, const StepArgs *args,
+                          hipStream_t s);
 hipError_t launch_vis(int q, int dtype, const VisArgs &a, hipStream_t s);
 hipError_t launch_unpermute(int q, int dtype, const UnpermuteArgs &a, hipStream_t s);
 // The allocation-free staging array (ASLHIP_NOALLOC_SCRATCH_BYTES bytes of

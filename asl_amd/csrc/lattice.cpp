@@ -157,6 +157,7 @@ struct aslhip_lattice {
   bool closure_mfma = true;  // evaluate the network with BF16 matrix instructions
   ClosureParams *d_cl = nullptr;
   float *d_feat = nullptr;  // closure features scratch (7 per interior cell)
+  void *d_surface = nullptr;  // surface force / flux: result (3 len macroscopic values), then the map (len floats)
   double dx = 1., pos0[3] = {0., 0., 0.};
   // a stream reading rho / u through aslhip_macro_device: the next work that
   // writes them waits for what it has queued by then
@@ -219,7 +220,7 @@ void drop_graphs(aslhip_lattice *h) {
 void free_all(aslhip_lattice *h) {
   drop_graphs(h);
   void *ptrs[] = {h->f,  h->rho,  h->u,           h->code,         h->pat, h->rec, h->mode,
-                  h->val, h->vl, h->vlbc, h->red_partial, h->red_out, h->d_args, h->d_cl, h->d_feat};
+                  h->val, h->vl, h->vlbc, h->red_partial, h->red_out, h->d_args, h->d_cl, h->d_feat, h->d_surface};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (auto &v : h->vis)
@@ -671,6 +672,7 @@ void face_entries(const aslhip_lattice *h, StepArgs &a) {
     }
     a.g.fpos |= static_cast<unsigned>(f) << (4 * j);
     if (bounce) a.g.fbounce |= 1u << j;
+    a.fset |= 1u << f;
     if (bounce) a.fbounces |= 1u << f;
     if (valued) a.g.fvalued |= 1u << f;
     for (int p : fc)  // the same BC on two faces gives a shared link one value: neither beats the other
@@ -1577,8 +1579,9 @@ int aslhip_read_f(aslhip_lattice *h, void *out) {
 
 namespace {
 
-// ComputeSurfaceForceMap / ComputeSurfaceFluxMap on the device: post-collision
-// view, incoming view (peek), then the surface kernel.
+// ComputeSurfaceForceMap / ComputeSurfaceFluxMap on the device.  The map and
+// the result go through a buffer that the lattice keeps (allocating and freeing
+// on each call took longer than the kernel).
 int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   if (int r = check(h)) return r;
   if (!map || !out) return fail(ASLHIP_EINVAL, "ASL ERROR: surface force/flux needs a map and an output field");
@@ -1587,66 +1590,24 @@ int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   if (int r = flush_deferred(h)) return r;
   if (int r = prepare(h, false)) return r;
   if (int r = upload_args(h)) return r;
-  const size_t view = (size_t)h->len * h->Q * h->melem;
-  const size_t outb = (size_t)h->len * (flux ? 1 : 3) * h->melem;
-  void *post = nullptr, *in = nullptr, *dout = nullptr;
-  float *dmap = nullptr;
-  StepArgs *dpk = nullptr;  // the step arguments with one cell per lane, for the peek
-  StepArgs pk = step_args(h, 0, 1);
-  hipError_t e = hipMalloc(&post, view);
-  if (e == hipSuccess) e = hipMalloc(&in, view);
-  if (e == hipSuccess) e = hipMalloc(&dout, outb);
-  if (e == hipSuccess) e = hipMalloc(&dmap, (size_t)h->len * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&dpk, sizeof(StepArgs));
-  int r = 0;
-  if (e == hipSuccess) e = hipMemcpyAsync(dpk, &pk, sizeof(StepArgs), hipMemcpyHostToDevice, h->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(dmap, map, (size_t)h->len * sizeof(float), hipMemcpyHostToDevice, h->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(in, 0, view, h->stream);
-  if (e == hipSuccess) {
-    UnpermuteArgs u;
-    u.f = h->f;
-    u.qs_bytes = h->qs_bytes;
-    u.sx = h->sx;
-    u.sy = h->sy;
-    u.len = h->len;
-    u.per = h->periodic ? 1 : 0;
-    u.nx = h->n[0];
-    u.ny = h->n[1];
-    u.nz = h->n[2];
-    u.after_odd = h->next_odd ? 0 : 1;
-    u.first = 0;
-    u.count = h->len;
-    u.out = post;
-    e = launch_unpermute(h->Q, h->dtype, u, h->stream);
+  const size_t len = (size_t)h->len, outb = len * 3 * h->melem, mapb = len * sizeof(float);
+  if (!h->d_surface) {
+    if (hipMalloc(&h->d_surface, outb + mapb) != hipSuccess) {
+      h->d_surface = nullptr;
+      return fail(ASLHIP_EHIP, "ASL ERROR: surface force/flux: out of memory");
+    }
   }
-  if (e == hipSuccess) {
-    StepLaunch a;
-    a.hot = pk.g;
-    a.args = dpk;
-    a.variant = 0;
-    a.cpl = 1;
-    a.tile = 0;
-    e = launch_peek(h->Q, h->dtype, h->next_odd, h->periodic, a, in, h->stream);
-  }
-  if (e == hipSuccess) {
-    SurfaceArgs s;
-    s.map = dmap;
-    s.post = post;
-    s.in = in;
-    s.out = dout;
-    s.sx = h->sx;
-    s.sy = h->sy;
-    s.len = h->len;
-    s.flux = flux ? 1 : 0;
-    e = launch_surface(h->Q, h->dtype, s, h->stream);
-  }
-  if (e == hipSuccess) r = copy_out(h, dout, out, outb);
-  else r = fail(ASLHIP_EHIP, "ASL ERROR: surface force/flux: %s", hipGetErrorString(e));
-  (void)hipStreamSynchronize(h->stream);
-  void *ptrs[] = {post, in, dout, dmap, dpk};
-  for (void *p : ptrs)
-    if (p) (void)hipFree(p);
-  return r;
+  SurfaceArgs s;
+  s.out = h->d_surface;
+  float *dmap = reinterpret_cast<float *>(static_cast<char *>(h->d_surface) + outb);
+  s.map = dmap;
+  s.len = h->len;
+  s.per = h->periodic ? 1 : 0;
+  s.after_odd = h->next_odd ? 0 : 1;
+  s.flux = flux ? 1 : 0;
+  HIPCHK(hipMemcpyAsync(dmap, map, mapb, hipMemcpyHostToDevice, h->stream));
+  HIPCHK(launch_surface(h->Q, h->dtype, s, h->h_direct, h->d_args, h->stream));
+  return copy_out(h, h->d_surface, out, flux ? len * h->melem : outb);
 }
 
 }  // namespace

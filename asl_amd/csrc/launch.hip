@@ -75,13 +75,10 @@ hipError_t launch_write_f(int q, int dtype, const WriteFArgs &a, hipStream_t s) 
   const KernelTable *t = table(q);
   return t ? t->write_f(dtype, a, s) : hipErrorInvalidValue;
 }
-hipError_t launch_peek(int q, int dtype, bool odd, bool periodic, const StepLaunch &a, void *out, hipStream_t s) {
+hipError_t launch_surface(int q, int dtype, const SurfaceArgs &a, const StepHot &g, const StepArgs *args,
+                          hipStream_t s) {
   const KernelTable *t = table(q);
-  return t ? t->peek(dtype, odd, periodic, a, out, s) : hipErrorInvalidValue;
-}
-hipError_t launch_surface(int q, int dtype, const SurfaceArgs &a, hipStream_t s) {
-  const KernelTable *t = table(q);
-  return t ? t->surface(dtype, a, s) : hipErrorInvalidValue;
+  return t ? t->surface(dtype, a, g, args, s) : hipErrorInvalidValue;
 }
 hipError_t launch_vis(int q, int dtype, const VisArgs &a, hipStream_t s) {
   const KernelTable *t = table(q);
