@@ -44,6 +44,6 @@ def test_force_and_flux_links(q, steps, body, dtype):
     inner = ((slice(2, -2) if body == "corner" else slice(1, -1)),) * 3
     fg, fo = G.surface_force(mapv), O.surface_force(mapv)
     qg, qo = G.surface_flux(mapv), O.surface_flux(mapv)
-    assert np.abs(fo).max() > 0
+    assert np.abs(np.asarray(fo)[(slice(None),) + inner]).max() > 0
     assert np.array_equal(fg[(slice(None),) + inner], np.asarray(fo)[(slice(None),) + inner].astype(G.host_dtype))
     assert np.array_equal(qg[inner], np.asarray(qo)[inner].astype(G.host_dtype))
