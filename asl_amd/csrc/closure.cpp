@@ -8,6 +8,7 @@
 #include "closure.hpp"
 #include "mlp.hpp"
 #include "status.hpp"
+#include "transfer.hpp"
 
 using namespace aslhip;
 
@@ -30,6 +31,7 @@ void mlp_free(aslhip_mlp *m) {
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (m->stream) (void)hipStreamDestroy(m->stream);
+  transfer_drop();
 }
 
 int ensure_partial(aslhip_mlp *m, int nblocks) {
@@ -93,6 +95,7 @@ int aslhip_mlp_create(aslhip_mlp **out, const float *params) {
   for (int i = 0; i < CL_NPARAM; ++i)
     if (!std::isfinite(params[i])) return fail(ASLHIP_EINVAL, "ASL ERROR: mlp_create: non-finite parameter %d", i);
   aslhip_mlp *m = new aslhip_mlp();
+  transfer_hold();
   const size_t pb = CL_NPARAM * sizeof(float);
   hipError_t e = hipStreamCreate(&m->stream);
   if (e == hipSuccess) e = hipMalloc(&m->p, pb);
@@ -129,8 +132,8 @@ int aslhip_mlp_set_data(aslhip_mlp *m, const float *x, const float *t, long long
   m->n = 0;
   HIPCHK(hipMalloc(&m->x, (size_t)n * CL_NIN * sizeof(float)));
   HIPCHK(hipMalloc(&m->t, (size_t)n * sizeof(float)));
-  HIPCHK(hipMemcpy(m->x, x, (size_t)n * CL_NIN * sizeof(float), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(m->t, t, (size_t)n * sizeof(float), hipMemcpyHostToDevice));
+  HIPCHK(to_device(m->x, x, (size_t)n * CL_NIN * sizeof(float), m->stream));
+  HIPCHK(to_device(m->t, t, (size_t)n * sizeof(float), m->stream));
   m->n = n;
   return 0;
 }
@@ -169,8 +172,7 @@ int aslhip_mlp_train(aslhip_mlp *m, int steps, int batch, double lr, unsigned lo
     if (int r = batch_gradient(m, 0, batch, sd, m->loss + at, &a)) return r;
     ++m->adam_t;
     if (losses && (at == LOSS_RUN - 1 || s == steps - 1)) {
-      HIPCHK(hipStreamSynchronize(m->stream));
-      HIPCHK(hipMemcpy(losses + s - at, m->loss, (size_t)(at + 1) * sizeof(double), hipMemcpyDeviceToHost));
+      HIPCHK(to_host(losses + s - at, m->loss, (size_t)(at + 1) * sizeof(double), m->stream));
     }
   }
   HIPCHK(hipStreamSynchronize(m->stream));
@@ -179,8 +181,7 @@ int aslhip_mlp_train(aslhip_mlp *m, int steps, int batch, double lr, unsigned lo
 
 int aslhip_mlp_get_params(aslhip_mlp *m, float *out) {
   if (!m || !out) return fail(ASLHIP_EINVAL, "ASL ERROR: mlp_get_params needs a handle and a buffer");
-  HIPCHK(hipStreamSynchronize(m->stream));
-  HIPCHK(hipMemcpy(out, m->p, CL_NPARAM * sizeof(float), hipMemcpyDeviceToHost));
+  HIPCHK(to_host(out, m->p, CL_NPARAM * sizeof(float), m->stream));
   return 0;
 }
 

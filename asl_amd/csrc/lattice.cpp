@@ -27,6 +27,7 @@
 #include "kernels.hpp"
 #include "lattice_consts.hpp"
 #include "status.hpp"
+#include "transfer.hpp"
 
 using namespace aslhip;
 
@@ -157,6 +158,7 @@ struct aslhip_lattice {
   bool closure_mfma = true;  // evaluate the network with BF16 matrix instructions
   ClosureParams *d_cl = nullptr;
   float *d_feat = nullptr;  // closure features scratch (7 per interior cell)
+  void *d_view = nullptr;     // one view of the populations (read_f, write_f), kept up to VIEW_KEEP bytes
   void *d_surface = nullptr;  // surface force / flux: result (3 len macroscopic values), then the map (len floats)
   double dx = 1., pos0[3] = {0., 0., 0.};
   // a stream reading rho / u through aslhip_macro_device: the next work that
@@ -220,7 +222,7 @@ void drop_graphs(aslhip_lattice *h) {
 void free_all(aslhip_lattice *h) {
   drop_graphs(h);
   void *ptrs[] = {h->f,  h->rho,  h->u,           h->code,         h->pat, h->rec, h->mode,
-                  h->val, h->vl, h->vlbc, h->red_partial, h->red_out, h->d_args, h->d_cl, h->d_feat, h->d_surface};
+                  h->val, h->vl, h->vlbc, h->red_partial, h->red_out, h->d_args, h->d_cl, h->d_feat, h->d_view, h->d_surface};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (auto &v : h->vis)
@@ -228,6 +230,7 @@ void free_all(aslhip_lattice *h) {
   if (h->ev_macro) (void)hipEventDestroy(h->ev_macro);
   if (h->ev_consumer) (void)hipEventDestroy(h->ev_consumer);
   if (h->stream) (void)hipStreamDestroy(h->stream);
+  transfer_drop();
 }
 
 // Work about to be queued on the lattice's stream may overwrite rho / u (and
@@ -1030,15 +1033,33 @@ int step_impl(aslhip_lattice *h, int nsteps, unsigned flags, std::vector<hipEven
   return run_steps(h, nsteps, first, raw, (flags & ASLHIP_STEP_WRITE_MACRO) != 0, ev, graph);
 }
 
+// A device buffer for one view of the populations (Q len macroscopic values).
+// Views of up to VIEW_KEEP bytes keep it: allocating and freeing 45 MB took 0.4
+// ms of a read or write of 1.6.
+constexpr size_t VIEW_KEEP = 256u << 20;
+int view_buffer(aslhip_lattice *h, void **buf, size_t *bytes) {
+  *bytes = (size_t)h->len * h->Q * h->melem;
+  if (h->d_view) {
+    *buf = h->d_view;
+    return 0;
+  }
+  HIPCHK(hipMalloc(buf, *bytes));
+  if (*bytes <= VIEW_KEEP) h->d_view = *buf;
+  return 0;
+}
+int view_done(aslhip_lattice *h, void *buf) {
+  if (buf != h->d_view) HIPCHK(hipFree(buf));
+  return 0;
+}
+
 int copy_out(aslhip_lattice *h, const void *dev, void *host, size_t bytes) {
-  HIPCHK(hipStreamSynchronize(h->stream));
-  HIPCHK(hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost));
+  HIPCHK(to_host(host, dev, bytes, h->stream));
   return 0;
 }
 
 }  // namespace
 
-int aslhip::read_f_through(aslhip_lattice *h, void *out, void *buf, size_t buf_bytes) {
+int aslhip::read_f_through(aslhip_lattice *h, void *out, void *buf, size_t buf_bytes, bool staged) {
   if (int r = flush_deferred(h)) return r;
   const size_t cell_bytes = (size_t)h->Q * h->melem;  // one cell's Q values
   const size_t per = std::min(buf_bytes / cell_bytes, (size_t)h->len);
@@ -1061,6 +1082,7 @@ int aslhip::read_f_through(aslhip_lattice *h, void *out, void *buf, size_t buf_b
     a.first = static_cast<int>(first);
     a.count = static_cast<int>(count);
     HIPCHK(launch_unpermute(h->Q, h->dtype, a, h->stream));
+    if (staged && count == (size_t)h->len) return copy_out(h, buf, out, cell_bytes * count);  // one contiguous view
     HIPCHK(hipStreamSynchronize(h->stream));
     // piece i of the view: cells first .. first + count - 1 of direction i
     HIPCHK(hipMemcpy2D(o + first * h->melem, (size_t)h->len * h->melem, buf, count * h->melem, count * h->melem,
@@ -1109,6 +1131,7 @@ int aslhip_lattice_create(aslhip_lattice **out, int nx, int ny, int nz, int q, i
   const long long len = S0 * S1 * S2;
   if (len > 0x7fffffffLL - 4096) return fail(ASLHIP_EINVAL, "ASL ERROR: block too large for one lattice");
   aslhip_lattice *h = new aslhip_lattice();
+  transfer_hold();
   h->n[0] = nx;
   h->n[1] = ny;
   h->n[2] = nz;
@@ -1313,10 +1336,15 @@ int aslhip_init_equilibrium_field(aslhip_lattice *h, const void *rho, const void
   void *drho = nullptr, *du = nullptr;
   const size_t n = (size_t)h->len * h->melem;
   HIPCHK(hipMalloc(&du, 3 * n));
-  HIPCHK(hipMemcpyAsync(du, u, 3 * n, hipMemcpyHostToDevice, h->stream));
+  // small fields need no wait here: the stream is waited for below, before the caller may change them
+  auto up = [h](void *dst, const void *src, size_t bytes) {
+    return bytes <= (128u << 10) ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream)
+                                 : to_device(dst, src, bytes, h->stream);
+  };
+  HIPCHK(up(du, u, 3 * n));
   if (rho) {
     HIPCHK(hipMalloc(&drho, n));
-    HIPCHK(hipMemcpyAsync(drho, rho, n, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(up(drho, rho, n));
   }
   InitArgs a;
   a.f = h->f;
@@ -1358,9 +1386,9 @@ int aslhip_write_f(aslhip_lattice *h, const void *f) {
   if (int r = flush_deferred(h)) return r;
   if (int r = order_after_consumer(h)) return r;
   void *d = nullptr;
-  const size_t bytes = (size_t)h->len * h->Q * h->melem;
-  HIPCHK(hipMalloc(&d, bytes));
-  HIPCHK(hipMemcpyAsync(d, f, bytes, hipMemcpyHostToDevice, h->stream));
+  size_t bytes = 0;
+  if (int r = view_buffer(h, &d, &bytes)) return r;
+  HIPCHK(to_device(d, f, bytes, h->stream));
   WriteFArgs a;
   a.f = h->f;
   a.qs_bytes = h->qs_bytes;
@@ -1370,8 +1398,8 @@ int aslhip_write_f(aslhip_lattice *h, const void *f) {
   a.rho = h->rho;
   a.u = h->u;
   HIPCHK(launch_write_f(h->Q, h->dtype, a, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  HIPCHK(hipFree(d));
+  if (d != h->d_view) HIPCHK(hipStreamSynchronize(h->stream));  // before it is freed
+  if (int r = view_done(h, d)) return r;
   h->initialized = true;
   h->fresh = true;
   h->bc_since_init = false;
@@ -1557,7 +1585,7 @@ int aslhip_read_f_noalloc(aslhip_lattice *h, void *out) {
                                "(an allocation); call aslhip_finalize first");
   void *buf = nullptr;
   HIPCHK(noalloc_scratch(&buf));
-  int r = aslhip::read_f_through(h, out, buf, ASLHIP_NOALLOC_SCRATCH_BYTES);
+  int r = aslhip::read_f_through(h, out, buf, ASLHIP_NOALLOC_SCRATCH_BYTES, false);
   (void)hipStreamSynchronize(h->stream);
   return r;
 }
@@ -1567,11 +1595,11 @@ int aslhip_read_f(aslhip_lattice *h, void *out) {
   if (!out) return fail(ASLHIP_EINVAL, "ASL ERROR: read_f needs an output buffer");
   if (int r = flush_deferred(h)) return r;
   void *d = nullptr;
-  const size_t bytes = (size_t)h->len * h->Q * h->melem;
-  HIPCHK(hipMalloc(&d, bytes));
-  int r = aslhip::read_f_through(h, out, d, bytes);
+  size_t bytes = 0;
+  if (int r = view_buffer(h, &d, &bytes)) return r;
+  int r = aslhip::read_f_through(h, out, d, bytes, true);
   (void)hipStreamSynchronize(h->stream);
-  HIPCHK(hipFree(d));
+  if (int r2 = view_done(h, d)) return r2;
   return r;
 }
 
@@ -1605,7 +1633,7 @@ int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   s.per = h->periodic ? 1 : 0;
   s.after_odd = h->next_odd ? 0 : 1;
   s.flux = flux ? 1 : 0;
-  HIPCHK(hipMemcpyAsync(dmap, map, mapb, hipMemcpyHostToDevice, h->stream));
+  HIPCHK(to_device(dmap, map, mapb, h->stream));
   HIPCHK(launch_surface(h->Q, h->dtype, s, h->h_direct, h->d_args, h->stream));
   return copy_out(h, h->d_surface, out, flux ? len * h->melem : outb);
 }

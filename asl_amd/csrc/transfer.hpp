@@ -1,0 +1,19 @@
+// Copies between device memory and ordinary (pageable) host memory.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace aslhip {
+
+// Every object that transfers (lattice, trainer) holds one reference; the
+// staging buffers go back with the last one.
+void transfer_hold();
+void transfer_drop();
+
+// Copies n bytes after the work queued on s; returns when dst holds them.
+hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s);
+// Copies n bytes; returns when src may change, work queued on s afterwards sees dst.
+hipError_t to_device(void *dst, const void *src, size_t n, hipStream_t s);
+
+}  // namespace aslhip
