@@ -1883,12 +1883,17 @@ struct aslhip_batch {
   uint2 *ent = nullptr;      // per workgroup: lattice, chunk
   int nblocks = 0;
   int block = STEP_BLOCK;    // workgroup size of all lattices of the batch (direct kernel)
-  int tune_lds = -1;         // LDS-staged tiles: 1 on, 0 off, -1 automatic (FP32 storage)
-  // Graph chunks go group by group: each group of consecutive lattices (at
-  // most group_mb MiB of populations; 0: one group) takes all the chunk's
-  // steps before the next starts, so a group that fits the 256 MiB Infinity
-  // Cache is stepped from cache.  Entry ranges [first, second) of each group.
-  int group_mb = 0;
+  int tune_lds = 0;          // LDS-staged tiles: 1 on, 0 off
+  // Runs of several steps go group by group: each group of consecutive
+  // lattices (at most group_mb MiB of populations; 0: one group; -1: automatic)
+  // takes all the run's steps (a graph chunk, or the steps of an eager call)
+  // before the next starts, so a group that fits the 256 MiB Infinity Cache is
+  // stepped from cache.  Entry ranges [first, second) of each group.
+  int group_mb = -1;
+  // Measured on D3Q19 FP32 cavities, one group -> groups of 192 MiB: 16 of
+  // 32^3..96^3 (330 MiB) 135 -> 122 us per step, 64 of 32^3..160^3 (4.1 GiB)
+  // 1675 -> 1562; 128 MiB: 128.5 and 1633 (512 lanes; 192 MiB 127.5 and 1621,
+  // 224 MiB 127.0 and 1588).
   std::vector<std::pair<int, int>> groups;
   hipGraphExec_t graph[2] = {nullptr, nullptr};  // chunks starting with an even / odd step
   std::vector<StepArgs> hdesc;                    // host copy of desc (source of the async upload)
@@ -1896,14 +1901,57 @@ struct aslhip_batch {
 
 namespace {
 
-// Tiles for the batch's steps: non-periodic batches under 4 GiB per lattice;
-// automatic as for single lattices (D3Q19 FP32, the batch's populations
-// beyond the 256 MiB Infinity Cache).
-bool batch_tile(const aslhip_batch *b) {
+// Tiles for the batch's steps: non-periodic batches under 4 GiB per lattice.
+// Not automatic: groups step from the cache, where the direct kernel is the
+// faster one (the cavities above: 127 against 136 us, 1621 against 1708).
+bool batch_tile(const aslhip_batch *b) { return b->tune_lds != 0 && !b->periodic && !b->wide; }
+
+// Steps from which an eager run goes group by group: a group's first step reads
+// HBM in any case, and every group adds launches.  16 cavities of 32^3..96^3,
+// one group -> groups, us per step: 2 steps 242 -> 285, 10 steps 178 -> 173,
+// 100 steps 152 -> 145; 20 FP16 cavities of 96^3: 438 -> 496, 358 -> 336, 327 -> 294.
+constexpr int BATCH_GROUP_STEPS = 8;
+
+// Populations a group may hold, in bytes (0: all lattices form one group).
+// Automatic: 192 MiB where the batch is larger than the Infinity Cache, except
+// for D3Q27 in FP64, whose arithmetic hides HBM already (10 periodic lattices of
+// 40^3..70^3: 161 us per step in one group, 165 in groups).
+long long batch_group_bytes(const aslhip_batch *b) {
+  if (b->group_mb >= 0) return static_cast<long long>(b->group_mb) << 20;
+  if (step_block(b->Q, static_cast<int>(b->lat[0]->selem)) < STEP_BLOCK) return 0;
   long long bytes = 0;
   for (const aslhip_lattice *h : b->lat) bytes += h->qs_bytes * h->Q;
-  const bool on = b->tune_lds < 0 ? b->Q == 19 && b->dtype == ASLHIP_F32 && bytes > CACHE_BYTES : b->tune_lds != 0;
-  return on && !b->periodic && !b->wide;
+  return bytes > CACHE_BYTES ? SWEEP_WINDOW : 0;
+}
+
+// The group of each lattice, ascending from 0.  Lattices larger than the
+// Infinity Cache stream from HBM in any case and share a group of their own (a
+// launch per step for all of them); the others fill groups in order, split
+// evenly so that no group is a small rest.
+std::vector<int> batch_group_of(const aslhip_batch *b) {
+  const long long budget = batch_group_bytes(b);
+  std::vector<int> of(b->lat.size(), 0);
+  if (!budget) return of;
+  auto bytes = [&](size_t l) { return b->lat[l]->qs_bytes * b->lat[l]->Q; };
+  long long rest = 0;
+  int g = 0;
+  for (size_t l = 0; l < of.size(); ++l)
+    if (bytes(l) <= CACHE_BYTES)
+      rest += bytes(l);
+    else
+      g = 1;
+  const long long n = (rest + budget - 1) / budget, target = n ? (rest + n - 1) / n : 0;
+  long long in = 0;
+  for (size_t l = 0; l < of.size(); ++l) {
+    if (bytes(l) > CACHE_BYTES) continue;
+    if (in && (in >= target || in + bytes(l) > budget)) {
+      ++g;
+      in = 0;
+    }
+    in += bytes(l);
+    of[l] = g;
+  }
+  return of;
 }
 
 // One lattice's step arguments in the batch's launch shape.
@@ -1938,22 +1986,18 @@ int batch_launch(aslhip_batch *b, bool odd, bool macro, int e0, int e1) {
 int batch_tables(aslhip_batch *b) {
   std::vector<uint2> ent;
   b->groups.clear();
-  const double budget = 1048576.0 * b->group_mb;
-  size_t gfirst = 0;
-  double gbytes = 0.;
-  for (size_t l = 0; l < b->lat.size(); ++l) {
-    const aslhip_lattice *h = b->lat[l];
-    const double bytes = static_cast<double>(h->Q) * h->selem * h->len;
-    if (b->group_mb > 0 && ent.size() > gfirst && gbytes + bytes > budget) {
-      b->groups.emplace_back(static_cast<int>(gfirst), static_cast<int>(ent.size()));
-      gfirst = ent.size();
-      gbytes = 0.;
+  const std::vector<int> of = batch_group_of(b);
+  const int last = *std::max_element(of.begin(), of.end());
+  for (int g = 0; g <= last; ++g) {
+    const size_t first = ent.size();
+    for (size_t l = 0; l < b->lat.size(); ++l) {
+      if (of[l] != g) continue;
+      const StepArgs a = batch_args(b, b->lat[l]);
+      for (int c = 0; c < a.g.nchunks; ++c)
+        ent.push_back(make_uint2(static_cast<unsigned>(l), static_cast<unsigned>(c)));
     }
-    gbytes += bytes;
-    const StepArgs a = batch_args(b, b->lat[l]);
-    for (int c = 0; c < a.g.nchunks; ++c) ent.push_back(make_uint2(static_cast<unsigned>(l), static_cast<unsigned>(c)));
+    b->groups.emplace_back(static_cast<int>(first), static_cast<int>(ent.size()));
   }
-  b->groups.emplace_back(static_cast<int>(gfirst), static_cast<int>(ent.size()));
   // replays in flight read the old tables and graphs: finish them first
   HIPCHK(hipStreamSynchronize(b->stream));
   for (auto &g : b->graph)
@@ -2042,8 +2086,12 @@ int batch_step_impl(aslhip_batch *b, int nsteps, unsigned flags) {
       left -= ASLHIP_GRAPH_CHUNK;  // an even count: the parity is unchanged
     }
   }
-  for (; left > 0; --left, o = !o)
-    if (int r = batch_launch(b, o, macro && left == 1, 0, b->nblocks)) return r;
+  // The steps left, group by group; fewer than BATCH_GROUP_STEPS in one launch
+  // each for all lattices.
+  const std::vector<std::pair<int, int>> all = {{0, b->nblocks}};
+  for (const auto &g : left < BATCH_GROUP_STEPS ? all : b->groups)
+    for (int s = 0; s < left; ++s)
+      if (int r = batch_launch(b, o != ((s & 1) != 0), macro && s == left - 1, g.first, g.second)) return r;
   for (auto *h : b->lat) h->next_odd = (nsteps % 2) ? !odd : odd;
   // the lattices' own streams see the result in order
   HIPCHK(hipEventRecord(b->done, b->stream));
@@ -2144,7 +2192,7 @@ int aslhip_batch_autotune_groups(aslhip_batch *b, int chunks, int *best_mb) {
   if (!b) return fail(ASLHIP_EINVAL, "ASL ERROR: null batch handle");
   if (chunks < 1) return fail(ASLHIP_EINVAL, "ASL ERROR: autotune needs at least one chunk per candidate");
   double best = 1e300;
-  int bm = b->group_mb;
+  int bm = static_cast<int>(batch_group_bytes(b) >> 20);
   for (int mb : {0, 64, 128, 160, 192, 224, 256, 384}) {
     if (int r = aslhip_batch_set_tuning(b, ASLHIP_TUNE_GROUP_MB, mb)) return r;
     // the first chunk captures the graphs; the timed ones replay them

@@ -374,9 +374,11 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  *   runs with at most 512. */
 #define ASLHIP_TUNE_XCD_REMAP 1
 #define ASLHIP_TUNE_BLOCK 2
-/* Batches only: graph chunks step groups of consecutive lattices of at most
- * this many MiB of populations one group at a time (0: all lattices each
- * step), so that a group can stay in the 256 MiB Infinity Cache. */
+/* Batches only: the steps of a graph chunk, or 8 eager steps and more, go
+ * group by group, groups of consecutive lattices of at most this many MiB of
+ * populations (0: all lattices each step; lattices over 256 MiB form one
+ * group), so that a group can stay in the 256 MiB Infinity Cache.  Default:
+ * 192 for batches over 256 MiB (not D3Q27 in FP64), else 0. */
 #define ASLHIP_TUNE_GROUP_MB 3
 /* Lattices: 1 = address the populations with 64-bit offsets (the variant
  * that lattices over 4 GiB of populations use) whatever the size; 0 = by
@@ -499,9 +501,8 @@ int aslhip_batch_destroy(aslhip_batch *b);
 int aslhip_batch_step(aslhip_batch *b, int nsteps, unsigned flags);
 /* As aslhip_batch_step, timed with HIP events on the batch's stream. */
 int aslhip_batch_time_steps(aslhip_batch *b, int nsteps, unsigned flags, double *ms_total);
-/* Workgroup size (ASLHIP_TUNE_BLOCK), LDS-staged tiles (ASLHIP_TUNE_LDS 1
- * or 0; default: tiles for non-periodic D3Q19 FP32 batches over 256 MiB of
- * populations) or group
+/* Workgroup size (ASLHIP_TUNE_BLOCK, default 1024), LDS-staged tiles
+ * (ASLHIP_TUNE_LDS 1 or 0; default 0) or group
  * size (ASLHIP_TUNE_GROUP_MB) of the batch's launches; the autotuners choose
  * between tiles and the direct kernel's workgroup size (256/512/1024,
  * timing nsteps real eager steps each; returns 256 for tiles) and the group
