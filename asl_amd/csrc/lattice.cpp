@@ -188,6 +188,7 @@ struct aslhip_lattice {
   bool deferred_first = false;
   // launch tuning
   int tune_block = 512;   // workgroup size (measured best with runs of 4 chunks per XCD)
+  bool block_set = false; // tune_block was chosen by the user or the autotuner
   bool force_wide = false;  // 64-bit addressing on any size (ASLHIP_TUNE_WIDE)
   int tune_remap = 4;  // chunk runs per XCD (measured best for graph chunks; 64 for 16-bit storage; the autotuner may choose others)
   int tune_cpl = 0;    // cells per lane along z: 0 automatic, else 1, 2 or 4 (ASLHIP_TUNE_CPL)
@@ -653,6 +654,21 @@ int step_workgroup(const aslhip_lattice *h) {
   return std::min(h->tune_block, effective_cpl(h) > 1 ? std::min(most, STEP_RUN_BLOCK) : most);
 }
 
+// Lanes per workgroup of the direct kernel: tune_block, unless nobody chose it
+// and the lattice is small.  A step of one workgroup per CU or less takes as
+// long as one workgroup, and smaller ones start and end sooner: 16^3 D3Q19
+// FP32 in a graph 4.29 us (512 lanes), 3.71 (256), 3.55 (128); 16^3 D3Q27 FP64
+// 6.79, 5.62, 5.09; 32^3 4.61, 4.14, 4.26; 40^3 5.33, 5.08, 5.70; from 48^3 up
+// 512 is level or better.  So the smallest of 128, 256 lanes that gives every
+// CU at most one workgroup.  The matrix-core closure kernel shares one copy of
+// the weights per workgroup and keeps the large ones.
+int step_lanes(const aslhip_lattice *h) {
+  if (!h->block_set && !h->has_closure)
+    for (int lanes : {128, 256})
+      if (1LL * h->n[0] * h->n[1] * h->n[2] <= 256LL * lanes) return std::min(lanes, h->tune_block);
+  return h->tune_block;
+}
+
 // The divisor d of udivm (kernels.hip); 0 stands for d = 1.
 unsigned long long udiv_magic(unsigned d) { return d <= 1 ? 0ULL : ~0ULL / d + 1ULL; }
 
@@ -703,7 +719,7 @@ StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd
   g.nz = h->n[2];
   a.len = h->len;
   a.cpl = cpl > 0 ? cpl : effective_cpl(h);
-  g.block = block > 0 ? block : h->tune_block;
+  g.block = block > 0 ? block : step_lanes(h);
   if (a.cpl > 1 && g.block > STEP_RUN_BLOCK) g.block = STEP_RUN_BLOCK;
   g.block = std::min(g.block, step_block(h->Q, static_cast<int>(h->selem)));
   const int lds = effective_lds(h);
@@ -769,7 +785,7 @@ int upload_args(aslhip_lattice *h) {
     HIPCHK(hipStreamSynchronize(h->stream));
   }
   h->h_args.assign(base, base + 2);
-  h->h_direct = step_args(h, h->tune_block, 1).g;
+  h->h_direct = step_args(h, step_lanes(h), 1).g;
   // stream-ordered: steps queued before still see the previous arguments
   HIPCHK(hipMemcpyAsync(h->d_args, h->h_args.data(), sizeof base, hipMemcpyHostToDevice, h->stream));
   return 0;
@@ -1725,8 +1741,9 @@ int aslhip_set_tuning(aslhip_lattice *h, int knob, int value) {
     if (value < 64 || value > STEP_BLOCK || value % 64)
       return fail(ASLHIP_EINVAL, "ASL ERROR: workgroup size %d is not a multiple of 64 in 64..%d", value, STEP_BLOCK);
     if (int r = flush_deferred(h)) return r;
-    if (value != h->tune_block) drop_graphs(h);  // captured launches carry the old grid
+    if (value != h->tune_block || !h->block_set) drop_graphs(h);  // captured launches carry the old grid
     h->tune_block = value;
+    h->block_set = true;
     return 0;
   }
   if (knob == ASLHIP_TUNE_SWEEP_KB) {

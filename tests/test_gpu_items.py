@@ -82,3 +82,24 @@ def test_conservation_wraps_after_odd_steps(size, q):
             O.run(1, [o for _, o in bcs])
             tol = 4 * q * n * 2.0**-53 * n * 2  # |w c f| summed: at most 2 per cell
             assert np.abs(np.subtract(G.conservation(), O.conservation(mask))).max() <= tol
+
+
+@pytest.mark.parametrize("size", [(1, 1, 5), (32, 32, 32), (33, 32, 32), (64, 32, 32), (65, 32, 32)])
+def test_small_lattices_pick_their_workgroup(size):
+    """Without a choice of the caller's, lattices around the limits of 32768
+    and 65536 cells end bit for bit where 512-lane workgroups take them."""
+    for q, dtype, periodic in ((19, "f32", False), (27, "f64", True), (15, "f32", False)):
+        ends = []
+        for block in (None, 512):
+            rng = np.random.default_rng(q)
+            G, O = pair(size, q, nu=0.08, dtype=dtype, periodic=periodic)
+            if block:
+                G.set_tuning(_lib.TUNE_BLOCK, block)
+            G.init_equilibrium(1.0, (0.02 * rng.standard_normal((3,) + G.S)).astype(np.float32))
+            run(G, O, 0, [] if periodic else six_faces(G, O, rng))
+            G.step(3)
+            G.step(205, graph=True)
+            assert G.tuning()[0] == 512
+            ends.append((G.f(), G.rho(), G.velocity()))
+        inner = (Ellipsis,) + (slice(1, -1),) * 3
+        assert all(np.array_equal(a[inner], b[inner], equal_nan=True) for a, b in zip(*ends))
