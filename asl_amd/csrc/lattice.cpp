@@ -624,8 +624,8 @@ bool is_wide(const aslhip_lattice *h) { return h->force_wide || h->qs_bytes * h-
 // LDS-staged tiles apply to non-periodic lattices under 4 GiB without a
 // per-cell relaxation unless runs of 2 or 4 cells per lane are asked for:
 // 0 none, 1 every step, 2 even steps only (odd steps one cell per lane).
-// Automatic: every step for D3Q19 FP32 lattices whose populations outgrow the
-// 256 MiB Infinity Cache (box of 256 x 128 x 128, 331 MB: 116 us per step, 128
+// Automatic: every step that is not part of a sweep (sweep_shape) for D3Q19
+// FP32 lattices whose populations outgrow the 256 MiB Infinity Cache (box of 256 x 128 x 128, 331 MB: 116 us per step, 128
 // direct); none for lattices the cache holds (64^3 box, 22 MB: 12.7 against
 // 9.7 us), for the other templates (D3Q27 300 x 130 x 140: 226 against 224 us,
 // and sweeps gain beside other lattices; D3Q15: 282 against 123 us) and for
@@ -815,26 +815,37 @@ int launch_planes(aslhip_lattice *h, bool odd, unsigned fl, int p0, int np) {
   return 0;
 }
 
-// The shape of the sweeps (sweep_plan) of a run of steps: g planes per launch,
+// The shape of the sweeps (sweep_plan) of a run of n steps: g planes per launch,
 // t steps per sweep; t = 0: one launch per step over the whole lattice.
-// Automatic: for lattices that the 256 MiB Infinity Cache cannot hold and that
-// do not run LDS-staged tiles, a window of 192 MiB (g + t planes) that takes up
-// to 16 steps, so that most reads and writes of a step find their lines there.
-// us per step, alone / with two more lattices stepped beside it, before and
-// after: D3Q27 FP32 224^3 periodic 462 / 522 -> 438 / 469, D3Q27 FP64
-// 200 x 160 x 160 422 / 482 -> 422 / 391, D3Q19 FP64 256 x 128 x 128 225 / 271
-// -> 217 / 217, FP16 384 x 160 x 144 150 / 151 -> 141 / 151.  Tiles and sweeps
-// of D3Q19 FP32: 116 / 135 and 109 / 123 on 256 x 128 x 128, 149 / 158 and 152
-// / 165 on 300 x 130 x 140, 111 / 111 and 108 / 118 on 160 x 203 x 121: tiles
-// stay.  Windows of 64 MiB gain only beside other lattices, 240 MiB less than
-// 192 there.  Velocity-map links are filled after every step of the whole
-// lattice: no sweeps.
-constexpr long long SWEEP_WINDOW = 192LL << 20;
-constexpr int SWEEP_STEPS = 16;
-void sweep_shape(const aslhip_lattice *h, int &g, int &t) {
+// Automatic: for lattices that the 256 MiB Infinity Cache cannot hold, a window
+// of 224 MiB (g + t planes) that takes up to 16 steps, so that most reads and
+// writes of a step find their lines there.  us per step, alone / with two more
+// lattices stepped beside it, before and after: D3Q27 FP32 224^3 periodic 463 /
+// 518 -> 438 / 466, D3Q27 FP64 160^3 periodic 326 / 386 -> 317 / 309, D3Q19
+// FP64 256 x 128 x 128 226 / 281 -> 215 / 222, D3Q15 BF16 300 x 200 x 200 161 /
+// 161 -> 151 / 161.  192 MiB is 1 to 3 % slower, 64 MiB gains only beside other
+// lattices.
+// Runs of less than 4 steps read too much twice: 2 steps of the last two, 161
+// -> 161 and 226 -> 244 us per step, 4 steps 159 -> 157 and 226 -> 224.
+// D3Q19 FP32 lattices that run tiles sweep from 560 MiB and 6 steps on; tiles
+// -> sweeps of 20 steps: 256 x 128 x 128 (346 MB) 113 / 119 -> 109 / 124, 300 x
+// 128 x 128 137 / 141 -> 131 / 145, 192^3 194 / 203 -> 192 / 208; 320 x 160 x
+// 160 (642 MB) 231 / 256 -> 223 / 256, 256 x 256 x 128 226 / 271 -> 219 / 242,
+// 256^3 462 / 583 -> 447 / 482, 512 x 256 x 256 942 / 1211 -> 896 / 985; of 4
+// steps 256 x 256 x 128 225 -> 227, of 6 steps 223 -> 223.
+// Velocity-map links are filled after every step of the whole lattice: no
+// sweeps.
+constexpr long long SWEEP_WINDOW = 224LL << 20;
+constexpr long long SWEEP_TILED_BYTES = 560LL << 20;
+constexpr int SWEEP_STEPS = 16, SWEEP_MIN_STEPS = 4, SWEEP_TILED_MIN_STEPS = 6;
+void sweep_shape(const aslhip_lattice *h, int n, int &g, int &t) {
   g = t = 0;
-  if (h->nvl || h->tune_sweep == 0) return;
-  if (h->tune_sweep < 0 && (h->qs_bytes * h->Q <= CACHE_BYTES || effective_lds(h) == 1)) return;
+  if (n < 2 || h->nvl || h->tune_sweep == 0) return;
+  if (h->tune_sweep < 0) {
+    const long long bytes = h->qs_bytes * h->Q;
+    if (bytes <= CACHE_BYTES || n < SWEEP_MIN_STEPS) return;
+    if (effective_lds(h) == 1 && (h->tune_lds == 1 || bytes <= SWEEP_TILED_BYTES || n < SWEEP_TILED_MIN_STEPS)) return;
+  }
   const long long window = h->tune_sweep > 0 ? static_cast<long long>(h->tune_sweep) << 10 : SWEEP_WINDOW;
   const long long plane = static_cast<long long>(h->Q) * h->selem * h->sx;
   const int wp = static_cast<int>(std::min<long long>(window / plane, h->n[0]));
@@ -885,7 +896,7 @@ int launch_one(aslhip_lattice *h, unsigned fl, std::vector<hipEvent_t> *ev, int 
 // n steps with the flags fl, the last one with last_fl.
 int launch_run(aslhip_lattice *h, unsigned fl, unsigned last_fl, int n) {
   int g = 0, t = 0;
-  if (n > 1) sweep_shape(h, g, t);
+  sweep_shape(h, n, g, t);
   if (!t) {
     for (int s = 0; s < n; ++s)
       if (int r = launch_one(h, s == n - 1 ? last_fl : fl, nullptr, s)) return r;
@@ -986,7 +997,7 @@ int run_steps(aslhip_lattice *h, int nsteps, bool first_after_init, bool raw_fir
     const bool raw = s == 0 && raw_first;
     const int plain = nsteps - s - (macro_last ? 1 : 0);  // plain steps left
     int sg = 0, st = 0;
-    if (!raw && !ev && nsteps - s > 1) sweep_shape(h, sg, st);
+    if (!raw && !ev) sweep_shape(h, nsteps - s, sg, st);
     if (graph && !ev && !raw && plain >= 1 && !st) {
       const int n = plain < ASLHIP_GRAPH_CHUNK ? plain : ASLHIP_GRAPH_CHUNK;
       hipGraphExec_t g = nullptr;
@@ -1907,10 +1918,10 @@ struct aslhip_batch {
   // before the next starts, so a group that fits the 256 MiB Infinity Cache is
   // stepped from cache.  Entry ranges [first, second) of each group.
   int group_mb = -1;
-  // Measured on D3Q19 FP32 cavities, one group -> groups of 192 MiB: 16 of
-  // 32^3..96^3 (330 MiB) 135 -> 122 us per step, 64 of 32^3..160^3 (4.1 GiB)
-  // 1675 -> 1562; 128 MiB: 128.5 and 1633 (512 lanes; 192 MiB 127.5 and 1621,
-  // 224 MiB 127.0 and 1588).
+  // Measured on D3Q19 FP32 cavities, one group -> groups of 224 MiB: 16 of
+  // 32^3..96^3 (330 MiB) 135 -> 123 us per step, 64 of 32^3..160^3 (4.1 GiB)
+  // 1675 -> 1535; with 512 lanes 128 MiB 128.5 and 1633, 192 MiB 127.5 and 1621,
+  // 224 MiB 127.0 and 1588.
   std::vector<std::pair<int, int>> groups;
   hipGraphExec_t graph[2] = {nullptr, nullptr};  // chunks starting with an even / odd step
   std::vector<StepArgs> hdesc;                    // host copy of desc (source of the async upload)
@@ -1930,7 +1941,7 @@ bool batch_tile(const aslhip_batch *b) { return b->tune_lds != 0 && !b->periodic
 constexpr int BATCH_GROUP_STEPS = 8;
 
 // Populations a group may hold, in bytes (0: all lattices form one group).
-// Automatic: 192 MiB where the batch is larger than the Infinity Cache, except
+// Automatic: 224 MiB where the batch is larger than the Infinity Cache, except
 // for D3Q27 in FP64, whose arithmetic hides HBM already (10 periodic lattices of
 // 40^3..70^3: 161 us per step in one group, 165 in groups).
 long long batch_group_bytes(const aslhip_batch *b) {

@@ -379,7 +379,7 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  * group by group, groups of consecutive lattices of at most this many MiB of
  * populations (0: all lattices each step; lattices over 256 MiB form one
  * group), so that a group can stay in the 256 MiB Infinity Cache.  Default:
- * 192 for batches over 256 MiB (not D3Q27 in FP64), else 0. */
+ * 224 for batches over 256 MiB (not D3Q27 in FP64), else 0. */
 #define ASLHIP_TUNE_GROUP_MB 3
 /* Lattices: 1 = address the populations with 64-bit offsets (the variant
  * that lattices over 4 GiB of populations use) whatever the size; 0 = by
@@ -397,18 +397,18 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  * direction's slots for FP32, workgroup 256); 2 = tiles on even steps only,
  * odd steps direct; 0 = direct, one cell per lane (or the runs
  * ASLHIP_TUNE_CPL asks for).  Default: 1 for D3Q19 FP32 lattices over
- * 256 MiB of populations (that the Infinity Cache cannot hold), else 0.
- * Tiles apply to the same lattices as runs of cells when ASLHIP_TUNE_CPL is 0
- * or 1; results are bit for bit the same for
- * every value. */
+ * 256 MiB of populations (that the Infinity Cache cannot hold), for steps that
+ * do not sweep (ASLHIP_TUNE_SWEEP_KB), else 0.  Tiles apply to the same lattices
+ * as runs of cells when ASLHIP_TUNE_CPL is 0 or 1; results are bit for bit the
+ * same for every value. */
 #define ASLHIP_TUNE_LDS 6
 /* Lattices: window in KiB of the sweeps of a run of several steps: blocks of
  * planes take several steps one block after the other while their
  * populations stay in the Infinity Cache (in eager launches also under
  * ASLHIP_STEP_GRAPH; one cell per lane).  0: off, -1: automatic (default:
- * lattices over 256 MiB of populations that do not run tiles).  Lattices with
- * velocity-map BCs do
- * not sweep.  Results are bit for bit the same for every value. */
+ * lattices over 256 MiB of populations in runs of at least 4 steps; those that
+ * run tiles by default over 560 MiB and 6 steps).  Lattices with velocity-map
+ * BCs do not sweep.  Results are bit for bit the same for every value. */
 #define ASLHIP_TUNE_SWEEP_KB 7
 int aslhip_set_tuning(aslhip_lattice *h, int knob, int value);
 /* The launches of a sweep of nsteps steps over nx planes, blocks of `planes`

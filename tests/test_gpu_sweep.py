@@ -58,3 +58,17 @@ def test_sweep_knob():
     assert L.tuning_value(_lib.TUNE_SWEEP_KB) == 64
     with pytest.raises(asl_amd.ASLError):
         L.set_tuning(_lib.TUNE_SWEEP_KB, -2)
+
+
+@pytest.mark.parametrize("size,q,periodic", [((230, 200, 172), 19, False), ((230, 120, 130), 27, True)])
+def test_automatic_sweeps_keep_results(size, q, periodic):
+    """Large lattices: run lengths around the shortest ones that sweep (4; 6
+    where single steps run tiles)."""
+    G, E = (build(q, "f32", periodic, None, kb, size) for kb in (-1, 0))
+    assert G.tuning_value(_lib.TUNE_LDS) == (0 if periodic else 1)
+    for n, graph in ((3, False), (4, False), (6, False), (5, True), (19, True)):
+        G.step(n, graph=graph)
+        E.step(n, graph=graph)
+    inner = (Ellipsis,) + (slice(1, -1),) * 3
+    assert np.array_equal(G.rho()[inner], E.rho()[inner])
+    assert np.array_equal(G.f()[inner], E.f()[inner])
