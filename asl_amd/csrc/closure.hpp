@@ -12,6 +12,8 @@
 // chain, so results agree bit for bit).
 #pragma once
 
+#include <cstddef>
+
 #include "lattice_consts.hpp"
 
 namespace aslhip {
@@ -33,6 +35,17 @@ struct ClosureParams {
   alignas(16) float b2[2][16];            // half h, register r: b2[8 (r / 4) + 4 h + r % 4]
   alignas(16) float w3[2][16];            // half h, register r: w3[8 (r / 4) + 4 h + r % 4]
 };
+
+// The part of ClosureParams from p[CL_B3] on: what the matrix-core path reads,
+// copied to LDS once per workgroup.
+struct alignas(16) ClosureLds {
+  float b3, mu[CL_NIN], sc[CL_NIN], out;
+  unsigned long long a1[64], a2[4][64];
+  float b2[2][16], w3[2][16];
+};
+static_assert(offsetof(ClosureParams, w3) + sizeof(ClosureParams::w3) == CL_B3 * sizeof(float) + sizeof(ClosureLds) &&
+                  offsetof(ClosureParams, a1) == CL_B3 * sizeof(float) + offsetof(ClosureLds, a1),
+              "ClosureLds mirrors the end of ClosureParams");
 
 // BF16 bits of an already BF16-rounded float (the top half of its bits).
 inline unsigned long long bf16x4_pack(const float *v) {
@@ -92,19 +105,37 @@ __device__ __forceinline__ void closure_features(const float (&f)[Q], float r, c
   x[6] = r - 1.f;
 }
 
-__device__ __forceinline__ float closure_relax(float y, const ClosureParams &c, float tau0) {
-  const float tau = tau0 + y * c.out;
+__device__ __forceinline__ float closure_relax(float y, float out, float tau0) {
+  const float tau = tau0 + y * out;
   const float lo = 0.5f + 0.5f * (tau0 - 0.5f);
   return 1.f / (tau < lo ? lo : tau);
 }
 
-// Round to the nearest BF16 (ties to even); the bits of the result.  gfx950
-// converts in hardware (v_cvt_pk_bf16_f32, two values per instruction).
-__device__ __forceinline__ unsigned short bf16_bits(float x) {
-  const __bf16 b = static_cast<__bf16>(x);
-  unsigned short u;
-  __builtin_memcpy(&u, &b, 2);
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+
+// Two values rounded to the nearest BF16 (ties to even), lo in the low half:
+// one v_cvt_pk_bf16_f32.
+__device__ __forceinline__ unsigned bf16_pair(float lo, float hi) {
+  const f32x2_t f = {lo, hi};
+  const bf16x2_t b = __builtin_convertvector(f, bf16x2_t);
+  unsigned u;
+  __builtin_memcpy(&u, &b, 4);
   return u;
+}
+
+// x > 0 ? x : 0 in one instruction: the median of x, 0 and inf (infinity, from
+// a register: the compiler turns a known one into a maximum, which needs a
+// second instruction to quiet signalling NaNs).  NaN gives the smaller of the
+// others, 0, as the comparison does.
+__device__ __forceinline__ float relu(float x, float inf) { return __builtin_amdgcn_fmed3f(x, 0.f, inf); }
+
+// Exchanges the upper half-wavefront of a with the lower one of b.
+__device__ __forceinline__ void swap_halves(unsigned &a, unsigned &b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
 }
 
 typedef short bf16x4_t __attribute__((ext_vector_type(4)));
@@ -121,45 +152,50 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // B[4 (l / 32) + j][l % 32], j < 4; result register r holds
 // D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32] — the layout the next layer's B
 // operand needs for k-block r / 4, so layers chain without shuffles.
-__device__ __forceinline__ float closure_y_mfma(const float (&x)[7], const ClosureParams &c) {
+//
+// Beside the 10 MFMAs this is vector work (a wavefront instruction takes 4
+// cycles) that has to stay in the shadow of the step's memory traffic: paired
+// conversions, one instruction per relu, v_permlane32_swap for the exchange of
+// halves.  The parameters come from LDS; loads of them from memory were waited
+// for one layer after the other.  Even periodic step: 1003 -> 856 instructions
+// with the rare paths, 66 -> 61 us for 128^3 FP32, and 52.5 (6.1 TB/s; the plain
+// step 50) with the registers it asks for (97 to 103, 4 waves per SIMD):
+// held to 96, it spilled 8.
+__device__ __forceinline__ float closure_y_mfma(const float (&x)[7], const ClosureLds &c) {
   const int l = static_cast<int>(threadIdx.x) & 63;
   const int half = l >> 5;
   // own inputs as BF16 pairs: (x0, x1), (x2, x3), (x4, x5), (x6, 1.0 = the bias column of W1')
-  unsigned own[4];
+  float xn[8];
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const unsigned lo = bf16_bits((x[2 * p] - c.mu[2 * p]) * c.sc[2 * p]);
-    const unsigned hi = p < 3 ? bf16_bits((x[2 * p + 1] - c.mu[2 * p + 1]) * c.sc[2 * p + 1]) : 0x3f80u;
-    own[p] = lo | (hi << 16);
-  }
-  // inputs 4 half .. 4 half + 3 of the partner lane's cell (lane l ^ 32)
-  const unsigned send0 = half ? own[0] : own[2], send1 = half ? own[1] : own[3];
-  const unsigned par0 = static_cast<unsigned>(__shfl_xor(static_cast<int>(send0), 32));
-  const unsigned par1 = static_cast<unsigned>(__shfl_xor(static_cast<int>(send1), 32));
+  for (int j = 0; j < 7; ++j) xn[j] = (x[j] - c.mu[j]) * c.sc[j];
+  xn[7] = 1.f;
+  // Column block cb holds cells 32 cb + col; a lane supplies inputs 4 half ..
+  // 4 half + 3 of its column.  Inputs 0 .. 3 (in[cb = 0] before the exchange)
+  // of the upper cells trade places with inputs 4 .. 7 of the lower ones.
+  unsigned in[2][2];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) in[p / 2][p % 2] = bf16_pair(xn[2 * p], xn[2 * p + 1]);
+  swap_halves(in[0][0], in[1][0]);
+  swap_halves(in[0][1], in[1][1]);
   bf16x4_t a1;
   __builtin_memcpy(&a1, &c.a1[l], 8);  // weights in lane order (pack_closure)
-  float y[2];
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  float part[2];
 #pragma unroll
   for (int cb = 0; cb < 2; ++cb) {
-    // column block cb holds cells 32 cb + col; this lane supplies inputs 4 half .. 4 half + 3
-    const bool mine = (half == cb);  // the cell 32 cb + col is this lane's own
-    const unsigned b0 = mine ? own[2 * half] : par0, b1w = mine ? own[2 * half + 1] : par1;
     bf16x4_t b1;
-    b1[0] = static_cast<short>(b0 & 0xffffu);
-    b1[1] = static_cast<short>(b0 >> 16);
-    b1[2] = static_cast<short>(b1w & 0xffffu);
-    b1[3] = static_cast<short>(b1w >> 16);
+    __builtin_memcpy(&b1, in[cb], 8);
     f32x16_t d1 = {};
     d1 = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a1, b1, d1, 0, 0, 0);
     // relu and BF16 rounding of the hidden layer first: d1 is dead before the second layer starts
     bf16x4_t hb[4];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float h = d1[4 * kb + j];
-        hb[kb][j] = static_cast<short>(bf16_bits(h > 0.f ? h : 0.f));
-      }
+    for (int kb = 0; kb < 4; ++kb) {
+      const unsigned h[2] = {bf16_pair(relu(d1[4 * kb], inf), relu(d1[4 * kb + 1], inf)),
+                             bf16_pair(relu(d1[4 * kb + 2], inf), relu(d1[4 * kb + 3], inf))};
+      __builtin_memcpy(&hb[kb], h, 8);
+    }
     f32x16_t d2;
     __builtin_memcpy(&d2, c.b2[half], 64);
 #pragma unroll
@@ -168,16 +204,14 @@ __device__ __forceinline__ float closure_y_mfma(const float (&x)[7], const Closu
       __builtin_memcpy(&a2, &c.a2[kb][l], 8);
       d2 = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a2, hb[kb], d2, 0, 0, 0);
     }
-    float part = 0.f;
+    part[cb] = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float h = d2[r] > 0.f ? d2[r] : 0.f;
-      part = __builtin_fmaf(c.w3[half][r], h, part);
-    }
-    const float other = __shfl_xor(part, 32);
-    y[cb] = (half == 0 ? part + other : other + part) + c.p[CL_B3];
+    for (int r = 0; r < 16; ++r) part[cb] = __builtin_fmaf(c.w3[half][r], relu(d2[r], inf), part[cb]);
   }
-  return y[half];
+  // the lane's own cell: units of the lower half-wavefront + those of the upper one
+  unsigned lo = __float_as_uint(part[0]), hi = __float_as_uint(part[1]);
+  swap_halves(lo, hi);
+  return (__uint_as_float(lo) + __uint_as_float(hi)) + c.b3;
 }
 
 // tau0: the plain relaxation time 3 nu + 1/2 (float).
@@ -201,7 +235,7 @@ __device__ __forceinline__ float closure_w(const float (&x)[7], const ClosurePar
     const float h2 = a > 0.f ? a : 0.f;
     y = __builtin_fmaf(c.p[CL_W3 + o], h2, y);
   }
-  return closure_relax(y, c, tau0);
+  return closure_relax(y, c.out, tau0);
 }
 
 }  // namespace aslhip

@@ -293,7 +293,7 @@ __device__ __forceinline__ C turbulence_w(const C (&v)[Q], C r, const C (&m)[3],
 template <int Q, class C, int CL = 0>
 __device__ __forceinline__ void collide(C (&v)[Q], C w, bool compressible, bool omega, const C (&om)[3], C &r_o,
                                         C (&m_o)[3], const ClosureParams *cl = nullptr, float tau0 = 0.f,
-                                        bool turb = false, C nu = C(0)) {
+                                        bool turb = false, C nu = C(0), const ClosureLds *lds = nullptr) {
   C m[3], r;
   moments<Q, C>(v, r, m);
   if constexpr (CL == 1) {  // LBGKTurbulence or the FP32 closure
@@ -307,7 +307,7 @@ __device__ __forceinline__ void collide(C (&v)[Q], C w, bool compressible, bool 
   } else if constexpr (CL == 2 && Q == 19 && sizeof(C) == 4) {  // the closure on the matrix cores
     float x[7];
     closure_features<Q>(v, r, m, x);
-    w = closure_relax(closure_y_mfma(x, *cl), *cl, tau0);
+    w = closure_relax(closure_y_mfma(x, *lds), lds->out, tau0);
   }
   // LBGK::setOmega (src/num/aslLBGK.cxx:207-208): momentum += (2/w) omega x
   // momentum, one component after the other, each seeing the ones before it
@@ -597,6 +597,15 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
   // Keep the scheduler from hoisting the wait on the cell type above the
   // population loads.
   __builtin_amdgcn_sched_barrier(0);
+  const ClosureLds *lds = nullptr;
+  if constexpr (CL == 2) {  // the network's parameters: 2.9 KB from L2, waited for with the populations
+    __shared__ ClosureLds sh;
+    const char *src = reinterpret_cast<const char *>(a.cl) + CL_B3 * sizeof(float);
+    for (unsigned i = threadIdx.x * 16u; i < sizeof(ClosureLds); i += static_cast<unsigned>(g.block) * 16u)
+      *reinterpret_cast<u32x4_t *>(reinterpret_cast<char *>(&sh) + i) = *gload<u32x4_t>(src + i);
+    __syncthreads();
+    lds = &sh;
+  }
   if (faces) face_values<Q, C>(g, a, fb, v);
 
   // Cells that are not computed run the collision on whatever they read and
@@ -627,7 +636,7 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
     for (int d = 0; d < 3; ++d) om[d] = sizeof(C) == 4 ? C(a.om32[d]) : C(a.om64[d]);
   }
   collide<Q, C, CL>(v, C(a.w), (g.flags & STEP_F_COMPRESSIBLE) != 0, omega, om, r, m, a.cl, a.cl_tau0,
-                    (g.flags & STEP_F_TURB) != 0, sizeof(C) == 4 ? C(a.nu32) : C(a.nu64));
+                    (g.flags & STEP_F_TURB) != 0, sizeof(C) == 4 ? C(a.nu32) : C(a.nu64), lds);
 
   if (!live || !it.act) return;
   if constexpr (PER && ODD) {  // offsets formed again for the stores: 18 of them live across the collision cost waves
@@ -1105,15 +1114,6 @@ __global__ __launch_bounds__(STEP_TILE) void k_step_tile(const StepHot g, const 
 template <int Q, class S, bool ODD, bool PER, bool WIDE, int CL>
 __global__ __launch_bounds__(step_block(Q, sizeof(S))) void k_step(const StepHot g, const StepArgs *args) {
   step_body<Q, S, ODD, PER, WIDE, CL>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
-}
-
-// The matrix-core closure variant, held to 5 waves per SIMD (96 VGPRs) on
-// periodic lattices; with the boundary links those spill about 30 (128^3 box:
-// 177 us per step, 69 with 100 VGPRs and 4 waves).
-template <int Q, class S, bool ODD, bool PER, bool WIDE>
-__global__ __launch_bounds__(STEP_BLOCK) __attribute__((amdgpu_waves_per_eu(PER ? 5 : 4))) void k_step_mfma(
-    const StepHot g, const StepArgs *args) {
-  step_body<Q, S, ODD, PER, WIDE, 2>(g, *args, chunk_of<ODD>(g, static_cast<int>(blockIdx.x), g.nchunks));
 }
 
 // The step with CPL cells per lane (step_body_run); same chunk order.  At
@@ -1648,9 +1648,9 @@ hipError_t step_w(bool wide, const StepLaunch &a, hipStream_t s) {
   if (a.variant == 2) {  // the closure on the matrix cores: D3Q19 with FP32 collision (checked by the host)
     if constexpr (Q == 19 && sizeof(typename Codec<S>::C) == 4) {
       if (wide && !PER)
-        hipLaunchKernelGGL((k_step_mfma<Q, S, ODD, PER, !PER>), grid, block, 0, s, a.hot, a.args);
+        hipLaunchKernelGGL((k_step<Q, S, ODD, PER, !PER, 2>), grid, block, 0, s, a.hot, a.args);
       else
-        hipLaunchKernelGGL((k_step_mfma<Q, S, ODD, PER, false>), grid, block, 0, s, a.hot, a.args);
+        hipLaunchKernelGGL((k_step<Q, S, ODD, PER, false, 2>), grid, block, 0, s, a.hot, a.args);
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;
