@@ -259,14 +259,10 @@ __device__ __forceinline__ void equilibria_of(bool compressible, C r, const C (&
 // here feq is the equilibrium of the cell's own rho and momentum (before the
 // rotating-frame term), the value that statement is evidently meant to use.
 template <int Q, class C>
-__device__ __forceinline__ C turbulence_w(const C (&v)[Q], C r, const C (&m)[3], bool compressible, C nu, C w0) {
+__device__ __forceinline__ C turbulence_w(const C (&v)[Q], const C (&e)[Q], C nu, C w0) {
   C d[Q];  // f - feq, summed in direction order
-  equilibria_of<Q, C>(
-      compressible, r, m, [&](C e) { d[0] = v[0] - e; },
-      [&](int i, int j, C ei, C ej) {
-        d[i] = v[i] - ei;
-        d[j] = v[j] - ej;
-      });
+#pragma unroll
+  for (int i = 0; i < Q; ++i) d[i] = v[i] - e[i];
   C fl2 = v[0] * v[0];
   C dl2 = d[0] * d[0];
 #pragma unroll
@@ -285,29 +281,35 @@ __device__ __forceinline__ C turbulence_w(const C (&v)[Q], C r, const C (&m)[3],
 // x*y + z of ASL's expression tree is one fma (OpenCL's default FP_CONTRACT
 // ON); the CPU oracle contracts the same sites.  On return v holds the
 // post-collision populations, r the density and m the momentum.  CL: a
-// per-cell relaxation replaces w: 1 LBGKTurbulence's (turb) or the closure
-// network's in FP32 on the vector ALUs, 2 the closure network's on the matrix
-// cores (closure: D3Q19, FP32 collision).  Each is its own kernel, so that the
-// plain and the matrix-core variants do not hold the registers of the FP32
-// network.
+// per-cell relaxation replaces w: 1 LBGKTurbulence's, 2 the closure network's on
+// the matrix cores, 3 the closure network's in FP32 on the vector ALUs
+// (closures: D3Q19, FP32 collision).  Each is its own kernel, so that none holds
+// the registers of another.  LBGKTurbulence apart from the FP32 network and with
+// its equilibria formed once: 100 -> 64 VGPRs, FP16 box of 128^3 43.5 -> 34.6 us
+// per step, FP32 box of 160 x 72 x 60 22.9 -> 21.1.
 template <int Q, class C, int CL = 0>
 __device__ __forceinline__ void collide(C (&v)[Q], C w, bool compressible, bool omega, const C (&om)[3], C &r_o,
                                         C (&m_o)[3], const ClosureParams *cl = nullptr, float tau0 = 0.f,
-                                        bool turb = false, C nu = C(0), const ClosureLds *lds = nullptr) {
+                                        C nu = C(0), const ClosureLds *lds = nullptr) {
   C m[3], r;
   moments<Q, C>(v, r, m);
-  if constexpr (CL == 1) {  // LBGKTurbulence or the FP32 closure
-    if (turb) {
-      w = turbulence_w<Q, C>(v, r, m, compressible, nu, w);
-    } else if constexpr (Q == 19 && sizeof(C) == 4) {
-      float x[7];
-      closure_features<Q>(v, r, m, x);
-      w = closure_w(x, *cl, tau0);
-    }
-  } else if constexpr (CL == 2 && Q == 19 && sizeof(C) == 4) {  // the closure on the matrix cores
+  // LBGKTurbulence: the equilibria, in FP32 kept for the collision (a rotating
+  // frame needs others); FP64 has no registers for them.
+  constexpr bool KEEP = CL == 1 && sizeof(C) == 4;
+  [[maybe_unused]] C e[Q];
+  auto keep0 = [&](C x) { e[0] = x; };
+  auto keep = [&](int i, int j, C xi, C xj) {
+    e[i] = xi;
+    e[j] = xj;
+  };
+  if constexpr (CL == 1) {
+    equilibria_of<Q, C>(compressible, r, m, keep0, keep);
+    w = turbulence_w<Q, C>(v, e, nu, w);
+  }
+  if constexpr (CL >= 2) {
     float x[7];
     closure_features<Q>(v, r, m, x);
-    w = closure_relax(closure_y_mfma(x, *lds), lds->out, tau0);
+    w = CL == 2 ? closure_relax(closure_y_mfma(x, *lds), lds->out, tau0) : closure_w(x, *cl, tau0);
   }
   // LBGK::setOmega (src/num/aslLBGK.cxx:207-208): momentum += (2/w) omega x
   // momentum, one component after the other, each seeing the ones before it
@@ -317,14 +319,20 @@ __device__ __forceinline__ void collide(C (&v)[Q], C w, bool compressible, bool 
     m[0] = fmaT(t, fmaT(om[1], m[2], -(om[2] * m[1])), m[0]);
     m[1] = fmaT(t, fmaT(om[2], m[0], -(om[0] * m[2])), m[1]);
     m[2] = fmaT(t, fmaT(om[0], m[1], -(om[1] * m[0])), m[2]);
+    if constexpr (KEEP) equilibria_of<Q, C>(compressible, r, m, keep0, keep);
   }
   const C one_w = C(1.) - w;
-  equilibria_of<Q, C>(
-      compressible, r, m, [&](C e) { v[0] = fmaT(v[0], one_w, w * e); },
-      [&](int i, int j, C ei, C ej) {
-        v[i] = fmaT(v[i], one_w, w * ei);
-        v[j] = fmaT(v[j], one_w, w * ej);
-      });
+  if constexpr (KEEP) {
+#pragma unroll
+    for (int i = 0; i < Q; ++i) v[i] = fmaT(v[i], one_w, w * e[i]);
+  } else {
+    equilibria_of<Q, C>(
+        compressible, r, m, [&](C x) { v[0] = fmaT(v[0], one_w, w * x); },
+        [&](int i, int j, C xi, C xj) {
+          v[i] = fmaT(v[i], one_w, w * xi);
+          v[j] = fmaT(v[j], one_w, w * xj);
+        });
+  }
   r_o = r;
 #pragma unroll
   for (int d = 0; d < 3; ++d) m_o[d] = m[d];
@@ -495,10 +503,10 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
   using M = typename CD::M;
   constexpr unsigned ES = sizeof(S);
   const Item it = item_of(g, chunk);
-  // The closure variant keeps every lane to the end (its network runs on
+  // The matrix-core closure keeps every lane to the end (its network runs on
   // matrix instructions across the wavefront): a lane past the end works on a
   // stand-in cell and stores nothing.
-  if constexpr (!CL) {
+  if constexpr (CL != 2) {
     if (!it.act) return;
   }
   const unsigned idx = it.row + static_cast<unsigned>(it.z), ib = idx * ES;
@@ -636,7 +644,7 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
     for (int d = 0; d < 3; ++d) om[d] = sizeof(C) == 4 ? C(a.om32[d]) : C(a.om64[d]);
   }
   collide<Q, C, CL>(v, C(a.w), (g.flags & STEP_F_COMPRESSIBLE) != 0, omega, om, r, m, a.cl, a.cl_tau0,
-                    (g.flags & STEP_F_TURB) != 0, sizeof(C) == 4 ? C(a.nu32) : C(a.nu64), lds);
+                    sizeof(C) == 4 ? C(a.nu32) : C(a.nu64), lds);
 
   if (!live || !it.act) return;
   if constexpr (PER && ODD) {  // offsets formed again for the stores: 18 of them live across the collision cost waves
@@ -1645,18 +1653,22 @@ hipError_t step_w(bool wide, const StepLaunch &a, hipStream_t s) {
     return hipGetLastError();
   }
   // (periodic lattices never choose between two slots: one addressing variant)
-  if (a.variant == 2) {  // the closure on the matrix cores: D3Q19 with FP32 collision (checked by the host)
+  if (a.variant >= 2) {  // the closure: D3Q19 with FP32 collision (checked by the host)
     if constexpr (Q == 19 && sizeof(typename Codec<S>::C) == 4) {
-      if (wide && !PER)
+      if (wide && !PER && a.variant == 2)
         hipLaunchKernelGGL((k_step<Q, S, ODD, PER, !PER, 2>), grid, block, 0, s, a.hot, a.args);
-      else
+      else if (a.variant == 2)
         hipLaunchKernelGGL((k_step<Q, S, ODD, PER, false, 2>), grid, block, 0, s, a.hot, a.args);
+      else if (wide && !PER)
+        hipLaunchKernelGGL((k_step<Q, S, ODD, PER, !PER, 3>), grid, block, 0, s, a.hot, a.args);
+      else
+        hipLaunchKernelGGL((k_step<Q, S, ODD, PER, false, 3>), grid, block, 0, s, a.hot, a.args);
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;
     }
   }
-  if (a.variant == 1) {  // LBGKTurbulence or the FP32 closure
+  if (a.variant == 1) {  // LBGKTurbulence
     if (wide && !PER)
       hipLaunchKernelGGL((k_step<Q, S, ODD, PER, !PER, 1>), grid, block, 0, s, a.hot, a.args);
     else

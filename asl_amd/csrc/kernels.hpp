@@ -211,7 +211,7 @@ struct ReduceArgs {
 struct StepLaunch {
   StepHot hot;
   const StepArgs *args;
-  int variant;   // per-cell relaxation: 0 none, 1 LBGKTurbulence or the FP32 closure, 2 the matrix-core closure
+  int variant;   // per-cell relaxation: 0 none, 1 LBGKTurbulence, 2 / 3 the closure on the matrix cores / in FP32
   int cpl;       // cells per lane (2 or 4: the run variant; non-periodic, under 4 GiB, no closure)
   int tile;      // 1: LDS-staged tiles of STEP_TILE cells (same restrictions, cpl 1, block STEP_TILE)
 };

@@ -802,7 +802,7 @@ int launch_planes(aslhip_lattice *h, bool odd, unsigned fl, int p0, int np) {
   a.hot.flags = fl;
   a.args = h->d_args + p;
   // LBGKTurbulence takes precedence over a closure in the collision
-  a.variant = h->turbulence ? 1 : (h->has_closure ? (h->closure_mfma ? 2 : 1) : 0);
+  a.variant = h->turbulence ? 1 : (h->has_closure ? (h->closure_mfma ? 2 : 3) : 0);
   a.cpl = np < 0 ? A.cpl : 1;
   a.tile = np < 0 ? A.tile : 0;
   if (np >= 0) {
