@@ -190,7 +190,8 @@ struct aslhip_lattice {
   int tune_block = 512;   // workgroup size (measured best with runs of 4 chunks per XCD)
   bool block_set = false; // tune_block was chosen by the user or the autotuner
   bool force_wide = false;  // 64-bit addressing on any size (ASLHIP_TUNE_WIDE)
-  int tune_remap = 4;  // chunk runs per XCD (measured best for graph chunks; 64 for 16-bit storage; the autotuner may choose others)
+  int tune_remap = 4;  // chunks per XCD run, where xcd_run does not choose
+  bool remap_set = false;  // tune_remap was chosen by the user or the autotuner
   int tune_cpl = 0;    // cells per lane along z: 0 automatic, else 1, 2 or 4 (ASLHIP_TUNE_CPL)
   int tune_lds = -1;   // LDS-staged tiles: 0 off, 1 every step, 2 even steps, -1 automatic (ASLHIP_TUNE_LDS)
   int tune_sweep = -1; // sweeps: window in KiB, 0 off, -1 automatic (ASLHIP_TUNE_SWEEP_KB)
@@ -669,6 +670,28 @@ int step_lanes(const aslhip_lattice *h) {
   return h->tune_block;
 }
 
+// Consecutive chunks per XCD run of a launch of n chunks; at most an XCD's share.
+// Unless somebody chose it, each XCD takes one slab of a lattice that the
+// Infinity Cache holds, so that chunks whose cells exchange populations along x
+// and y meet in one L2, within a step and from one step to the next.  us per
+// step alone, runs of 4 -> slabs: D3Q19 FP32 48^3 6.5 -> 5.5, 64^3 9.5 -> 8.4,
+// 96^3 24.9 -> 22.3, 112^3 38.7 -> 35.5, 128^3 52.0 -> 51.4; D3Q15 300 x 50 x 50
+// 19.5 -> 16.2; D3Q19 FP64 64^3 14.8 -> 13.7; 97 x 61 x 83 14.9 -> 12.6; FP16 64^3
+// 8.5 -> 7.5.  Four slabs per XCD over 150 MiB, which are level alone and better
+// beside others; alone / beside two more, runs of 4, one slab, four: D3Q19 FP32
+// 132^3 (175 MB) 59.5 / 69.0, 57.4 / 72.3, 57.9 / 68.6, 144^3 73.0 / 88.0, 70.5 /
+// 89.4, 70.7 / 88.0; with 16-bit storage runs of 64 there, FP16 256 x 128 x 128 60.9
+// / 69.3, one slab 59.6 / 75.7, four 62.1 / 72.4.  Larger lattices and tiles keep short runs: D3Q27 224^3 in sweeps 435
+// (runs of 4), 447 (four slabs), 517 (one); tiles on 256 x 128 x 128 114, 121, 122.
+constexpr long long SLAB_BYTES = 150LL << 20;
+int xcd_run(const aslhip_lattice *h, int n, bool tile) {
+  const int share = std::max(1, n / 8);
+  const long long bytes = h->qs_bytes * h->Q;
+  if (h->remap_set || tile || bytes > CACHE_BYTES) return std::min(std::max(1, h->tune_remap), share);
+  if (bytes <= SLAB_BYTES) return share;
+  return h->selem == 2 ? std::min(h->tune_remap, share) : std::max(1, share / 4);
+}
+
 // The divisor d of udivm (kernels.hip); 0 stands for d = 1.
 unsigned long long udiv_magic(unsigned d) { return d <= 1 ? 0ULL : ~0ULL / d + 1ULL; }
 
@@ -736,7 +759,7 @@ StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd
   a.bpp = (g.ny * g.sy + STEP_TILE - 1) / STEP_TILE;
   g.nchunks = a.tile ? a.bpp * g.nx : static_cast<int>((static_cast<long long>(g.count) + g.block - 1) / g.block);
   a.zmagic = ((1ULL << 40) + (unsigned long long)h->sy - 1) / (unsigned long long)h->sy;
-  g.remap = std::max(1, h->tune_remap);
+  g.remap = xcd_run(h, g.nchunks, a.tile != 0);
   g.mspan = udiv_magic(8u * static_cast<unsigned>(g.remap));
   a.pat = h->pat;
   a.rec = h->rec;
@@ -810,6 +833,8 @@ int launch_planes(aslhip_lattice *h, bool odd, unsigned fl, int p0, int np) {
     a.hot.first = static_cast<unsigned>(p0) * plane;
     a.hot.count = static_cast<unsigned>(np) * plane;
     a.hot.nchunks = static_cast<int>((static_cast<long long>(a.hot.count) + a.hot.block - 1) / a.hot.block);
+    a.hot.remap = xcd_run(h, a.hot.nchunks, false);
+    a.hot.mspan = udiv_magic(8u * static_cast<unsigned>(a.hot.remap));
   }
   HIPCHK(launch_step(h->Q, h->dtype, odd, h->periodic, is_wide(h), a, h->stream));
   return 0;
@@ -1173,8 +1198,7 @@ int aslhip_lattice_create(aslhip_lattice **out, int nx, int ny, int nz, int q, i
   h->periodic = per == 7;
   h->t = make_templ(q);
   h->selem = dtype == ASLHIP_F64 ? 8 : (dtype == ASLHIP_F32 ? 4 : 2);
-  // 16-bit storage: runs of 64 chunks per XCD measured fastest on the sphere
-  // channel (0.068 against 0.076 ms per step with runs of 4)
+  // 16-bit storage: the run length reported until somebody chooses one
   if (h->selem == 2) h->tune_remap = 64;
   h->melem = h->celem = dtype == ASLHIP_F64 ? 8 : 4;
   // direction arrays 256-byte aligned
@@ -1737,7 +1761,10 @@ int aslhip_set_tuning(aslhip_lattice *h, int knob, int value) {
   }
   if (knob == ASLHIP_TUNE_XCD_REMAP) {
     if (value < 0 || value > 4096) return fail(ASLHIP_EINVAL, "ASL ERROR: XCD run length %d outside 0..4096", value);
+    if (int r = flush_deferred(h)) return r;
+    if (value != h->tune_remap || !h->remap_set) drop_graphs(h);  // captured launches carry the old order
     h->tune_remap = value;
+    h->remap_set = true;
     return 0;
   }
   if (knob == ASLHIP_TUNE_CPL) {
@@ -1805,12 +1832,14 @@ int aslhip_autotune(aslhip_lattice *h, int nsteps, int *best_block, int *best_re
   if (nsteps < 1) return fail(ASLHIP_EINVAL, "ASL ERROR: autotune needs at least one step per candidate");
   nsteps += nsteps & 1;
   const int remaps[6] = {0, 2, 4, 8, 16, 64};
+  const int preset = h->selem == 2 ? 64 : 4;  // direct kernel: stands for the automatic order (xcd_run)
   double best = 1e300;
   int bb = h->tune_block, br = h->tune_remap, bc = h->tune_cpl, bl = effective_lds(h);
   auto trial = [&](int lds, int cpl, int remap, int blk) -> int {
     if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_LDS, lds)) return r;
     if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_CPL, cpl)) return r;
     if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_XCD_REMAP, remap)) return r;
+    h->remap_set = remap != preset;
     if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_BLOCK, blk)) return r;
     double tot = 0., ker = 0.;
     if (int r = aslhip_time_steps(h, nsteps, 0u, &tot, &ker, nullptr)) return r;
@@ -1848,6 +1877,7 @@ int aslhip_autotune(aslhip_lattice *h, int nsteps, int *best_block, int *best_re
   if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_LDS, bl)) return r;
   if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_CPL, bc)) return r;
   if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_XCD_REMAP, br)) return r;
+  h->remap_set = br != preset;
   if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_BLOCK, bb)) return r;
   if (best_block) *best_block = step_workgroup(h);
   if (best_remap) *best_remap = br;
@@ -1908,7 +1938,7 @@ struct aslhip_batch {
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
   StepArgs *desc = nullptr;  // [2][n]: plain steps, then steps writing rho/u
-  uint2 *ent = nullptr;      // per workgroup: lattice, chunk
+  uint2 *ent = nullptr;      // [2][nblocks], per workgroup: lattice, chunk; group by group, then for launches of all groups
   int nblocks = 0;
   int block = STEP_BLOCK;    // workgroup size of all lattices of the batch (direct kernel)
   int tune_lds = 0;          // LDS-staged tiles: 1 on, 0 off
@@ -2026,6 +2056,23 @@ int batch_tables(aslhip_batch *b) {
     }
     b->groups.emplace_back(static_cast<int>(first), static_cast<int>(ent.size()));
   }
+  // Each XCD (workgroup id modulo 8) takes one run of the chunks of a group that
+  // the Infinity Cache holds (see xcd_run), others the hardware order: the
+  // cavities of batch_group_bytes's figures 123 -> 115 and 1535 -> 1437, 20 FP16
+  // ones of 96^3 293 -> 272; streamed from HBM, 200^3 and three small D3Q27
+  // lattices would take 362 instead of 344.
+  const std::vector<uint2> plain = ent;
+  const size_t nb = plain.size();
+  ent.insert(ent.end(), plain.begin(), plain.end());
+  for (size_t g = 0; g < b->groups.size(); ++g) {
+    long long bytes = 0;
+    for (size_t l = 0; l < b->lat.size(); ++l)
+      if (of[l] == static_cast<int>(g)) bytes += b->lat[l]->qs_bytes * b->lat[l]->Q;
+    const size_t first = static_cast<size_t>(b->groups[g].first);
+    const size_t share = (static_cast<size_t>(b->groups[g].second) - first) / 8;
+    if (bytes > CACHE_BYTES) continue;
+    for (size_t i = 0; i < 8 * share; ++i) ent[first + i] = plain[first + (i % 8) * share + i / 8];
+  }
   // replays in flight read the old tables and graphs: finish them first
   HIPCHK(hipStreamSynchronize(b->stream));
   for (auto &g : b->graph)
@@ -2037,7 +2084,7 @@ int batch_tables(aslhip_batch *b) {
   b->ent = nullptr;
   HIPCHK(hipMalloc(&b->ent, ent.size() * sizeof(uint2)));
   HIPCHK(hipMemcpy(b->ent, ent.data(), ent.size() * sizeof(uint2), hipMemcpyHostToDevice));
-  b->nblocks = static_cast<int>(ent.size());
+  b->nblocks = static_cast<int>(nb);
   return 0;
 }
 
@@ -2116,8 +2163,8 @@ int batch_step_impl(aslhip_batch *b, int nsteps, unsigned flags) {
   }
   // The steps left, group by group; fewer than BATCH_GROUP_STEPS in one launch
   // each for all lattices.
-  const std::vector<std::pair<int, int>> all = {{0, b->nblocks}};
-  for (const auto &g : left < BATCH_GROUP_STEPS ? all : b->groups)
+  const std::vector<std::pair<int, int>> all = {{b->nblocks, 2 * b->nblocks}};
+  for (const auto &g : left < BATCH_GROUP_STEPS && b->groups.size() > 1 ? all : b->groups)
     for (int s = 0; s < left; ++s)
       if (int r = batch_launch(b, o != ((s & 1) != 0), macro && s == left - 1, g.first, g.second)) return r;
   for (auto *h : b->lat) h->next_odd = (nsteps % 2) ? !odd : odd;
