@@ -35,24 +35,33 @@ constexpr int NWAVE = MLP_GRAD_BLOCK / 64;
 // result holds in half h of the wavefront.
 __device__ __forceinline__ constexpr int drow(int r, int h) { return 8 * (r / 4) + 4 * h + r % 4; }
 
+// The hidden unit at row q of a layer's products: the rows are arranged so that
+// register r in half h holds unit 2 r + h.
+__device__ __forceinline__ int unit_at(int q) { return 2 * (4 * (q >> 3) + (q & 3)) + ((q >> 2) & 1); }
+
 // Forward and backward on the FP32 matrix instructions: every wavefront takes
 // 32 samples at a time, one per column, as five products
-//   H1 = relu(W1' x')   (x' = (x, 1), W1' = (W1, b1)),   H2 = relu(W2 H1 + b2),
-//   dH1 = W2^T dH2 [H1 > 0],   gW2 += dH2 H1^T,   gW1' += dH1 x'^T.
+//   H1 = relu(W1 x + b1),   H2 = relu(W2 H1 + b2),
+//   dH1 = W2^T dH2 [H1 > 0],   gW2 += dH2 H1^T,   (gW1, gb1) += dH1 (x, 1)^T.
 // v_mfma_f32_32x32x2f32 takes A[l % 32][l / 32] and B[l / 32][l % 32] from lane
-// l; the order of the products within a sum is free, so k-step r uses rows
-// drow(r, 0) and drow(r, 1), which is how the previous product left its result:
-// layers chain without moving data.  The two gradients contract over samples;
-// their operands go through LDS once, transposed.  g_b2, g_w3, g_b3 and the
-// loss are sums per lane, added up at the end.  Sums of at most 64 samples
-// (SPW blocks of 32) are kept in FP32, as few roundings as 64-sample blocks
-// on the vector ALUs had; everything beyond is FP64.
+// l; with the units in unit_at's order k-step r uses units 2 r and 2 r + 1, which
+// is how the previous product left its result: layers chain without moving data.
+// It also adds every sum over units up in index order, biases first, which are
+// the bits of a chain of fma on the vector ALUs (1.6 million values of gradients
+// of single samples: all equal).  In another order a unit whose input lies within
+// a rounding of zero may switch sides (a third of the H2 differed in their last
+// bit, and one training run in three by 2e-6).
+// The two gradients contract over samples; their operands go through LDS once,
+// transposed.  g_b2, g_w3, g_b3 and the loss are sums per lane, added up at the
+// end.  Sums of at most 64 samples (SPW blocks of 32) are kept in FP32, as few
+// roundings as 64-sample blocks on the vector ALUs had; everything beyond is
+// FP64.
 //
 // Bound by latency: 16384 samples are 118 MFLOP (1 us of the matrix cores) in
-// one block per wavefront, 60 dependent instructions of 64 cycles; 91 us
-// before, on the vector ALUs with the weight products summed from LDS one
-// sample after the other.  A training step of 16384 samples: 163 -> 10.7 us
-// with the reduction below; error of the gradient against FP64 2.8e-8 both.
+// one block per wavefront, 76 dependent instructions of 64 cycles; before, on
+// the vector ALUs with the weight products summed from LDS one sample after the
+// other, 91 us.  20 training steps of 16384 samples: 3370 -> 300 us with the
+// reduction below (270 without the order of the sums).
 template <int SPW>
 __global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a) {
   __shared__ __attribute__((aligned(16))) float tile[NWAVE][3][CL_H * LROW];  // dH2, H1, dH1: [unit][sample]
@@ -63,19 +72,28 @@ __global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a
   const float *p = a.p;
 
   // weights in operand order
-  float w1[4], w2[16], w2t[16], b2[16], w3[16];
+  float w1[4], w2[16], w2t[16], b1[16], b2[16], w3[16];
+  const int unit = unit_at(col);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int in = 2 * k + half;
-    w1[k] = in < CL_NIN ? p[CL_W1 + col * CL_NIN + in] : p[CL_B1 + col];
+    w1[k] = in < CL_NIN ? p[CL_W1 + unit * CL_NIN + in] : 0.f;
   }
+  auto every_other = [&](const float *q, float (&d)[16]) {  // q[2 r + half]
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    w2[r] = p[CL_W2 + col * CL_H + drow(r, half)];
-    w2t[r] = p[CL_W2 + drow(r, half) * CL_H + col];
-    b2[r] = p[CL_B2 + drow(r, half)];
-    w3[r] = p[CL_W3 + drow(r, half)];
-  }
+    for (int i = 0; i < 8; ++i) {
+      const f4 v = *reinterpret_cast<const f4 *>(q + 4 * i);
+      d[2 * i] = half ? v[1] : v[0];
+      d[2 * i + 1] = half ? v[3] : v[2];
+    }
+  };
+  static_assert(CL_W2 % 4 == 0 && CL_B1 % 4 == 0 && CL_B2 % 4 == 0 && CL_W3 % 4 == 0, "16-byte loads");
+  every_other(p + CL_W2 + unit * CL_H, w2);
+  every_other(p + CL_B1, b1);
+  every_other(p + CL_B2, b2);
+  every_other(p + CL_W3, w3);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) w2t[r] = p[CL_W2 + (2 * r + half) * CL_H + unit];
   const float b3 = p[CL_B3];
 
   f32x16_t gw2 = {}, gw1 = {};
@@ -102,7 +120,9 @@ __global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a
     }
     const float t = live ? a.t[s] : 0.f;
 
-    f32x16_t h1 = {};
+    f32x16_t h1;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) h1[r] = b1[r];
 #pragma unroll
     for (int j = 0; j < 4; ++j) h1 = mfma(w1[j], x[j], h1);
     float m1[16];
@@ -116,10 +136,13 @@ __global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a
     for (int r = 0; r < 16; ++r) h2[r] = b2[r];
 #pragma unroll
     for (int r = 0; r < 16; ++r) h2 = mfma(w2[r], h1[r], h2);
-    float part = 0.f;
+    // y as row 0 and, for the upper half, row 4 of one more product
+    f32x16_t yr;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) part = __builtin_fmaf(w3[r], h2[r] > 0.f ? h2[r] : 0.f, part);
-    const float y = part + __shfl_xor(part, 32) + b3;
+    for (int r = 0; r < 16; ++r) yr[r] = b3;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) yr = mfma((col & ~4) == 0 ? w3[r] : 0.f, h2[r] > 0.f ? h2[r] : 0.f, yr);
+    const float y = yr[0];
     const float res = live ? y - t : 0.f;
     const float dy = res * a.inv_batch;
     f32x16_t d1 = {};
@@ -139,7 +162,7 @@ __global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a
     if (SPW > 1 && it) __syncthreads();  // the last block's operands have been read
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int o = drow(r, half) * LROW + col;
+      const int o = (2 * r + half) * LROW + col;
       dh2t[o] = d2[r];
       h1t[o] = h1[r];
       dh1t[o] = d1[r] * m1[r];
@@ -169,7 +192,7 @@ __global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
-    const int o = drow(r, half) * LROW + col;
+    const int o = (2 * r + half) * LROW + col;
     dh2t[o] = gb2[r];
     h1t[o] = gw3[r];
   }
