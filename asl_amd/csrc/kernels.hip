@@ -18,8 +18,9 @@
 //   MODE_CONST   a constant population (pressure BCs);
 //   MODE_LINK    written between steps by the boundary-link kernel
 //                (velocity map BCs, whose value needs rho at the ghost node).
-// Wavefronts test the cell types with a ballot: a wavefront without
-// boundary cells runs the plain streaming path.
+// Cells on the lattice's faces follow a rule on their coordinates instead.
+// Both are wavefront-uniform branches: a wavefront without such cells runs the
+// plain streaming path.
 //
 // The collision is ASL's LBGK::init0 (src/num/aslLBGK.cxx:187-235) in ASL's
 // operation order; the library is compiled with -ffp-contract=off so each

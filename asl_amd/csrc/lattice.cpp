@@ -953,7 +953,7 @@ int get_graph(aslhip_lattice *h, int n, bool odd, hipGraphExec_t *out) {
       return 0;
     }
   // A run captured with other flags (frame, compressibility, relaxation
-  // model) names the old kernel variant and argument slot, and the oldest
+  // model) names the old kernel variant and flags, and the oldest
   // remainder makes room for a new one: destroyed once replays of them have
   // finished.
   auto drop = [h](size_t i) -> int {

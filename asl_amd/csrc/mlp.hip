@@ -50,7 +50,7 @@ __device__ __forceinline__ int unit_at(int q) { return 2 * (4 * (q >> 3) + (q & 
 // the bits of a chain of fma on the vector ALUs (1.6 million values of gradients
 // of single samples: all equal).  In another order a unit whose input lies within
 // a rounding of zero may switch sides (a third of the H2 differed in their last
-// bit, and one training run in three by 2e-6).
+// bit, and some training runs by 2e-6).
 // The two gradients contract over samples; their operands go through LDS once,
 // transposed.  g_b2, g_w3, g_b3 and the loss are sums per lane, added up at the
 // end.  Sums of at most 64 samples (SPW blocks of 32) are kept in FP32, as few
