@@ -661,12 +661,16 @@ int step_workgroup(const aslhip_lattice *h) {
 // FP32 in a graph 4.29 us (512 lanes), 3.71 (256), 3.55 (128); 16^3 D3Q27 FP64
 // 6.79, 5.62, 5.09; 32^3 4.61, 4.14, 4.26; 40^3 5.33, 5.08, 5.70; from 48^3 up
 // 512 is level or better.  So the smallest of 128, 256 lanes that gives every
-// CU at most one workgroup.  The matrix-core closure kernel shares one copy of
-// the weights per workgroup and keeps the large ones.
+// CU at most one workgroup.  D3Q27 in FP64, of which a CU holds 12 wavefronts,
+// takes 256 lanes throughout, so that all 12 find room: 64^3 periodic 18.6 (512)
+// -> 17.8, 97^3 63.4 -> 61.4, beside two more 75.5 -> 73.9.  The matrix-core closure
+// kernel shares one copy of the weights per workgroup and keeps the large ones.
 int step_lanes(const aslhip_lattice *h) {
+  const bool tall = step_block(h->Q, static_cast<int>(h->selem)) < STEP_BLOCK;
   if (!h->block_set && !h->has_closure)
     for (int lanes : {128, 256})
-      if (1LL * h->n[0] * h->n[1] * h->n[2] <= 256LL * lanes) return std::min(lanes, h->tune_block);
+      if ((tall && lanes == 256) || 1LL * h->n[0] * h->n[1] * h->n[2] <= 256LL * lanes)
+        return std::min(lanes, h->tune_block);
   return h->tune_block;
 }
 

@@ -373,8 +373,9 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  *   one to four runs per XCD.
  *   ASLHIP_TUNE_BLOCK: workgroup size, a multiple of 64 up to 1024 (default
  *   512); a workgroup takes that many consecutive interior cells.  D3Q27 in FP64
- *   runs with at most 512; lattices of at most 65536 cells run with 128 or 256
- *   as long as neither the caller nor the autotuner has set it. */
+ *   runs with at most 512; as long as neither the caller nor the autotuner has
+ *   set it, lattices of at most 65536 cells run with 128 or 256 and D3Q27 in FP64
+ *   with 256. */
 #define ASLHIP_TUNE_XCD_REMAP 1
 #define ASLHIP_TUNE_BLOCK 2
 /* Batches only: the steps of a graph chunk, or 8 eager steps and more, go
