@@ -1975,12 +1975,9 @@ bool batch_tile(const aslhip_batch *b) { return b->tune_lds != 0 && !b->periodic
 constexpr int BATCH_GROUP_STEPS = 8;
 
 // Populations a group may hold, in bytes (0: all lattices form one group).
-// Automatic: 224 MiB where the batch is larger than the Infinity Cache, except
-// for D3Q27 in FP64, whose arithmetic hides HBM already (10 periodic lattices of
-// 40^3..70^3: 161 us per step in one group, 165 in groups).
+// Automatic: 224 MiB where the batch is larger than the Infinity Cache.
 long long batch_group_bytes(const aslhip_batch *b) {
   if (b->group_mb >= 0) return static_cast<long long>(b->group_mb) << 20;
-  if (step_block(b->Q, static_cast<int>(b->lat[0]->selem)) < STEP_BLOCK) return 0;
   long long bytes = 0;
   for (const aslhip_lattice *h : b->lat) bytes += h->qs_bytes * h->Q;
   return bytes > CACHE_BYTES ? SWEEP_WINDOW : 0;
@@ -2192,6 +2189,9 @@ int aslhip_batch_create(aslhip_batch **out, aslhip_lattice *const *lattices, int
   b->dtype = lattices[0]->dtype;
   b->periodic = lattices[0]->periodic;
   b->wide = is_wide(lattices[0]);
+  // D3Q27 in FP64 (see step_lanes), 512 -> 256 lanes: 10 lattices of 40^3..70^3 in
+  // groups 160 -> 153 us per step, 12 of 24^3 18.1 -> 16.3
+  if (step_block(b->Q, static_cast<int>(lattices[0]->selem)) < STEP_BLOCK) b->block = 256;
   for (int l = 0; l < n; ++l) {
     aslhip_lattice *h = lattices[l];
     if (!h || h->Q != b->Q || h->dtype != b->dtype || h->periodic != b->periodic || is_wide(h) != b->wide) {

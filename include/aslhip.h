@@ -382,7 +382,7 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  * group by group, groups of consecutive lattices of at most this many MiB of
  * populations (0: all lattices each step; lattices over 256 MiB form one
  * group), so that a group can stay in the 256 MiB Infinity Cache.  Default:
- * 224 for batches over 256 MiB (not D3Q27 in FP64), else 0. */
+ * 224 for batches over 256 MiB, else 0. */
 #define ASLHIP_TUNE_GROUP_MB 3
 /* Lattices: 1 = address the populations with 64-bit offsets (the variant
  * that lattices over 4 GiB of populations use) whatever the size; 0 = by
@@ -505,7 +505,8 @@ int aslhip_batch_destroy(aslhip_batch *b);
 int aslhip_batch_step(aslhip_batch *b, int nsteps, unsigned flags);
 /* As aslhip_batch_step, timed with HIP events on the batch's stream. */
 int aslhip_batch_time_steps(aslhip_batch *b, int nsteps, unsigned flags, double *ms_total);
-/* Workgroup size (ASLHIP_TUNE_BLOCK, default 1024), LDS-staged tiles
+/* Workgroup size (ASLHIP_TUNE_BLOCK, default 1024; 256 for D3Q27
+ * in FP64), LDS-staged tiles
  * (ASLHIP_TUNE_LDS 1 or 0; default 0) or group
  * size (ASLHIP_TUNE_GROUP_MB) of the batch's launches; the autotuners choose
  * between tiles and the direct kernel's workgroup size (256/512/1024,

@@ -27,3 +27,25 @@ def test_automatic_groups_equal_one_group(sizes):
         assert np.array_equal(interior(L.f()), interior(R.f()))
         assert np.array_equal(interior(L.rho()), interior(R.rho()))
         assert np.array_equal(interior(L.velocity()), interior(R.velocity()))
+
+
+def test_automatic_groups_of_fp64_d3q27():
+    """D3Q27 FP64 periodic lattices of 300 MiB in groups, with 256 lanes."""
+    def lattices():
+        out = []
+        for i, n in enumerate((60, 64, 20, 70, 63, 64)):
+            L = asl_amd.Lattice((n, n, n + 1), 27, dtype="f64", periodic=True, nu=0.01 * (i + 1))
+            rng = np.random.default_rng(i)
+            L.init_equilibrium(1.0, 0.02 * rng.standard_normal((3,) + L.S))
+            out.append(L)
+        return out
+    auto, one = lattices(), lattices()
+    A, B = asl_amd.Batch(auto), asl_amd.Batch(one)
+    B.set_tuning(_lib.TUNE_GROUP_MB, 0)
+    B.set_tuning(_lib.TUNE_BLOCK, 512)
+    for steps, graph in ((9, False), (101, True)):
+        for batch in (A, B):
+            batch.step(steps, graph=graph)
+    for L, R in zip(auto, one):
+        assert np.array_equal(interior(L.f()), interior(R.f()))
+        assert np.array_equal(interior(L.velocity()), interior(R.velocity()))
