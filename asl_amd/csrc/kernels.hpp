@@ -84,7 +84,7 @@ struct StepArgs {
   int cpl;                    // cells per lane along z
   int tile;                   // 1: LDS-staged tiles (block = STEP_TILE, cpl = 1)
   unsigned fset;              // bit f: face f has a BC
-  unsigned fbeats[6];         // per face: the faces whose BC is executed later
+  unsigned fbeats[6];         // per face: the faces that own links they share with it (BC executed later, or the same BC)
   float fval32[6][28];        // per face and direction: addend / constant (FP32 lattices)
   double fval64[6][28];       // the same for FP64 lattices
   float om32[3];              // angular velocity of the frame (STEP_F_OMEGA)

@@ -721,8 +721,10 @@ void face_entries(const aslhip_lattice *h, StepArgs &a) {
     a.fset |= 1u << f;
     if (bounce) a.g.fbfaces |= 1u << f;
     if (valued) a.g.fvalued |= 1u << f;
-    for (int p : fc)  // the same BC on two faces gives a shared link one value: neither beats the other
-      if (h->fface[p] / 4 > h->fface[f] / 4) a.fbeats[f] |= 1u << p;
+    for (int p : fc) {  // of faces with one BC the last one owns their common links: each link has one owner
+      const int sp = h->fface[p] / 4, sf = h->fface[f] / 4;
+      if (sp > sf || (sp == sf && p > f)) a.fbeats[f] |= 1u << p;
+    }
   }
 }
 
