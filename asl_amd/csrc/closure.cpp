@@ -39,7 +39,7 @@ int ensure_partial(aslhip_mlp *m, int nblocks) {
   HIPCHK(hipStreamSynchronize(m->stream));
   if (m->partial) HIPCHK(hipFree(m->partial));
   m->partial = nullptr;
-  HIPCHK(hipMalloc(&m->partial, (size_t)nblocks * MLP_PSTRIDE * sizeof(float)));
+  HIPCHK(device_alloc(&m->partial, (size_t)nblocks * MLP_PSTRIDE * sizeof(float)));
   m->partial_blocks = nblocks;
   return 0;
 }
@@ -48,7 +48,7 @@ int ensure_losses(aslhip_mlp *m, int n) {
   if (n <= m->loss_cap) return 0;
   HIPCHK(hipStreamSynchronize(m->stream));
   double *d = nullptr;
-  HIPCHK(hipMalloc(&d, (size_t)n * sizeof(double)));
+  HIPCHK(device_alloc(&d, (size_t)n * sizeof(double)));
   (void)hipFree(m->loss);
   m->loss = d;
   m->loss_cap = n;
@@ -98,11 +98,11 @@ int aslhip_mlp_create(aslhip_mlp **out, const float *params) {
   transfer_hold();
   const size_t pb = CL_NPARAM * sizeof(float);
   hipError_t e = hipStreamCreate(&m->stream);
-  if (e == hipSuccess) e = hipMalloc(&m->p, pb);
-  if (e == hipSuccess) e = hipMalloc(&m->g, pb);
-  if (e == hipSuccess) e = hipMalloc(&m->m, pb);
-  if (e == hipSuccess) e = hipMalloc(&m->v, pb);
-  if (e == hipSuccess) e = hipMalloc(&m->loss, sizeof(double));
+  if (e == hipSuccess) e = device_alloc(&m->p, pb);
+  if (e == hipSuccess) e = device_alloc(&m->g, pb);
+  if (e == hipSuccess) e = device_alloc(&m->m, pb);
+  if (e == hipSuccess) e = device_alloc(&m->v, pb);
+  if (e == hipSuccess) e = device_alloc(&m->loss, sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(m->p, params, pb, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(m->m, 0, pb);
   if (e == hipSuccess) e = hipMemset(m->v, 0, pb);
@@ -130,8 +130,8 @@ int aslhip_mlp_set_data(aslhip_mlp *m, const float *x, const float *t, long long
   if (m->t) HIPCHK(hipFree(m->t));
   m->x = m->t = nullptr;
   m->n = 0;
-  HIPCHK(hipMalloc(&m->x, (size_t)n * CL_NIN * sizeof(float)));
-  HIPCHK(hipMalloc(&m->t, (size_t)n * sizeof(float)));
+  HIPCHK(device_alloc(&m->x, (size_t)n * CL_NIN * sizeof(float)));
+  HIPCHK(device_alloc(&m->t, (size_t)n * sizeof(float)));
   HIPCHK(to_device(m->x, x, (size_t)n * CL_NIN * sizeof(float), m->stream));
   HIPCHK(to_device(m->t, t, (size_t)n * sizeof(float), m->stream));
   m->n = n;

@@ -130,8 +130,8 @@ int df_run(const double *prog, int nwords, const int size[3], const double pos[3
   hipStream_t s = nullptr;
   HIPCHK(hipStreamCreate(&s));
   Buf dprog, dout;
-  hipError_t e = hipMalloc(&dprog.p, nwords * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&dout.p, n * sizeof(T));
+  hipError_t e = device_alloc(&dprog.p, nwords * sizeof(double));
+  if (e == hipSuccess) e = device_alloc(&dout.p, n * sizeof(T));
   if (e == hipSuccess) e = hipMemcpyAsync(dprog.p, prog, nwords * sizeof(double), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) {
     const unsigned nb = static_cast<unsigned>((n + DF_BLOCK - 1) / DF_BLOCK);

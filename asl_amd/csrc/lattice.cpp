@@ -581,7 +581,7 @@ int finalize_impl(aslhip_lattice *h, bool allow_open = false) {
   HIPCHK(hipMemcpyAsync(h->pat, pat.data(), (size_t)len * 2, hipMemcpyHostToDevice, h->stream));
   if (h->rec) HIPCHK(hipFree(h->rec));
   h->rec = nullptr;
-  HIPCHK(hipMalloc(&h->rec, recs.size() * sizeof(LinkRec)));
+  HIPCHK(device_alloc(&h->rec, recs.size() * sizeof(LinkRec)));
   HIPCHK(hipMemcpyAsync(h->rec, recs.data(), recs.size() * sizeof(LinkRec), hipMemcpyHostToDevice, h->stream));
   HIPCHK(hipMemcpyAsync(h->mode, mode.data(), 256, hipMemcpyHostToDevice, h->stream));
   HIPCHK(hipMemcpyAsync(h->val, val.data(), val.size(), hipMemcpyHostToDevice, h->stream));
@@ -589,7 +589,7 @@ int finalize_impl(aslhip_lattice *h, bool allow_open = false) {
   h->vl = nullptr;
   h->nvl = static_cast<int>(vlinks.size());
   if (h->nvl) {
-    HIPCHK(hipMalloc(&h->vl, vlinks.size() * sizeof(VLink)));
+    HIPCHK(device_alloc(&h->vl, vlinks.size() * sizeof(VLink)));
     HIPCHK(hipMemcpyAsync(h->vl, vlinks.data(), vlinks.size() * sizeof(VLink), hipMemcpyHostToDevice, h->stream));
   }
   HIPCHK(hipMemcpyAsync(h->vlbc, vlbc.data(), 256 * sizeof(VLinkBC), hipMemcpyHostToDevice, h->stream));
@@ -1101,7 +1101,7 @@ int view_buffer(aslhip_lattice *h, void **buf, size_t *bytes) {
     *buf = h->d_view;
     return 0;
   }
-  HIPCHK(hipMalloc(buf, *bytes));
+  HIPCHK(device_alloc(buf, *bytes));
   if (*bytes <= VIEW_KEEP) h->d_view = *buf;
   return 0;
 }
@@ -1218,17 +1218,17 @@ int aslhip_lattice_create(aslhip_lattice **out, int nx, int ny, int nz, int q, i
   h->qs_bytes = qs_elems * (long long)h->selem;
   hipError_t e = hipGetDevice(&h->device);
   if (e == hipSuccess) e = hipStreamCreate(&h->stream);
-  if (e == hipSuccess) e = hipMalloc(&h->f, (size_t)h->qs_bytes * q);
-  if (e == hipSuccess) e = hipMalloc(&h->rho, (size_t)len * h->melem);
-  if (e == hipSuccess) e = hipMalloc(&h->u, (size_t)len * 3 * h->melem);
-  if (e == hipSuccess) e = hipMalloc(&h->code, (size_t)len);
-  if (e == hipSuccess) e = hipMalloc(&h->pat, (size_t)len * 2);
-  if (e == hipSuccess) e = hipMalloc(&h->mode, 256);
-  if (e == hipSuccess) e = hipMalloc(&h->val, 256 * (size_t)q * h->celem);
-  if (e == hipSuccess) e = hipMalloc(&h->vlbc, 256 * sizeof(VLinkBC));
-  if (e == hipSuccess) e = hipMalloc(&h->d_args, 2 * sizeof(StepArgs));
-  if (e == hipSuccess) e = hipMalloc(&h->red_partial, (size_t)reduce_blocks((int)len) * 5 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&h->red_out, 5 * sizeof(double));
+  if (e == hipSuccess) e = device_alloc(&h->f, (size_t)h->qs_bytes * q);
+  if (e == hipSuccess) e = device_alloc(&h->rho, (size_t)len * h->melem);
+  if (e == hipSuccess) e = device_alloc(&h->u, (size_t)len * 3 * h->melem);
+  if (e == hipSuccess) e = device_alloc(&h->code, (size_t)len);
+  if (e == hipSuccess) e = device_alloc(&h->pat, (size_t)len * 2);
+  if (e == hipSuccess) e = device_alloc(&h->mode, 256);
+  if (e == hipSuccess) e = device_alloc(&h->val, 256 * (size_t)q * h->celem);
+  if (e == hipSuccess) e = device_alloc(&h->vlbc, 256 * sizeof(VLinkBC));
+  if (e == hipSuccess) e = device_alloc(&h->d_args, 2 * sizeof(StepArgs));
+  if (e == hipSuccess) e = device_alloc(&h->red_partial, (size_t)reduce_blocks((int)len) * 5 * sizeof(double));
+  if (e == hipSuccess) e = device_alloc(&h->red_out, 5 * sizeof(double));
   if (e != hipSuccess) {
     free_all(h);
     delete h;
@@ -1317,7 +1317,7 @@ int aslhip_closure_set(aslhip_lattice *h, const float *params, const float mu[7]
   }
   c.out = out_scale;
   pack_closure(c);
-  if (!h->d_cl) HIPCHK(hipMalloc(&h->d_cl, sizeof(ClosureParams)));
+  if (!h->d_cl) HIPCHK(device_alloc(&h->d_cl, sizeof(ClosureParams)));
   HIPCHK(hipStreamSynchronize(h->stream));  // steps queued earlier read the old parameters
   HIPCHK(hipMemcpy(h->d_cl, &c, sizeof c, hipMemcpyHostToDevice));
   h->has_closure = true;
@@ -1351,7 +1351,7 @@ int aslhip_closure_features(aslhip_lattice *h, float *out) {
   if (int r = prepare(h, false)) return r;
   if (int r = upload_args(h)) return r;
   const long long ncell = (long long)h->n[0] * h->n[1] * h->n[2];
-  if (!h->d_feat) HIPCHK(hipMalloc(&h->d_feat, (size_t)ncell * CL_NIN * sizeof(float)));
+  if (!h->d_feat) HIPCHK(device_alloc(&h->d_feat, (size_t)ncell * CL_NIN * sizeof(float)));
   HIPCHK(launch_closure_features(h->dtype, h->next_odd, h->d_args, ncell, h->d_feat, h->stream));
   return copy_out(h, h->d_feat, out, (size_t)ncell * CL_NIN * sizeof(float));
 }
@@ -1392,7 +1392,7 @@ int aslhip_init_equilibrium_field(aslhip_lattice *h, const void *rho, const void
   if (!u) return fail(ASLHIP_EINVAL, "ASL ERROR: initF needs a velocity field");
   void *drho = nullptr, *du = nullptr;
   const size_t n = (size_t)h->len * h->melem;
-  HIPCHK(hipMalloc(&du, 3 * n));
+  HIPCHK(device_alloc(&du, 3 * n));
   // small fields need no wait here: the stream is waited for below, before the caller may change them
   auto up = [h](void *dst, const void *src, size_t bytes) {
     return bytes <= (128u << 10) ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream)
@@ -1400,7 +1400,7 @@ int aslhip_init_equilibrium_field(aslhip_lattice *h, const void *rho, const void
   };
   HIPCHK(up(du, u, 3 * n));
   if (rho) {
-    HIPCHK(hipMalloc(&drho, n));
+    HIPCHK(device_alloc(&drho, n));
     HIPCHK(up(drho, rho, n));
   }
   InitArgs a;
@@ -1518,7 +1518,7 @@ int aslhip_vis_add(aslhip_lattice *h, int kind, const float *map, const double u
   if (rot)
     for (int d = 0; d < 6; ++d) v.rot[d] = rot[d];
   const size_t bytes = (size_t)h->len * sizeof(float);
-  if (hipMalloc(&v.map, bytes) != hipSuccess) return fail(ASLHIP_ENOMEM, "ASL ERROR: visualisation fill: out of memory");
+  if (device_alloc(&v.map, bytes) != hipSuccess) return fail(ASLHIP_ENOMEM, "ASL ERROR: visualisation fill: out of memory");
   if (hipMemcpy(v.map, map, bytes, hipMemcpyHostToDevice) != hipSuccess) {
     (void)hipFree(v.map);
     return fail(ASLHIP_EHIP, "ASL ERROR: visualisation fill: map upload failed");
@@ -1677,7 +1677,7 @@ int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   if (int r = upload_args(h)) return r;
   const size_t len = (size_t)h->len, outb = len * 3 * h->melem, mapb = len * sizeof(float);
   if (!h->d_surface) {
-    if (hipMalloc(&h->d_surface, outb + mapb) != hipSuccess) {
+    if (device_alloc(&h->d_surface, outb + mapb) != hipSuccess) {
       h->d_surface = nullptr;
       return fail(ASLHIP_EHIP, "ASL ERROR: surface force/flux: out of memory");
     }
@@ -2085,7 +2085,7 @@ int batch_tables(aslhip_batch *b) {
     }
   if (b->ent) HIPCHK(hipFree(b->ent));
   b->ent = nullptr;
-  HIPCHK(hipMalloc(&b->ent, ent.size() * sizeof(uint2)));
+  HIPCHK(device_alloc(&b->ent, ent.size() * sizeof(uint2)));
   HIPCHK(hipMemcpy(b->ent, ent.data(), ent.size() * sizeof(uint2), hipMemcpyHostToDevice));
   b->nblocks = static_cast<int>(nb);
   return 0;
@@ -2203,7 +2203,7 @@ int aslhip_batch_create(aslhip_batch **out, aslhip_lattice *const *lattices, int
   }
   hipError_t e = hipStreamCreate(&b->stream);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipMalloc(&b->desc, 2 * (size_t)n * sizeof(StepArgs));
+  if (e == hipSuccess) e = device_alloc(&b->desc, 2 * (size_t)n * sizeof(StepArgs));
   if (e != hipSuccess) {
     batch_free(b);
     delete b;

@@ -281,8 +281,8 @@ int aslhip_surface_distance_map(const double *tri, long long ntri, const int siz
   StreamHold st;
   HIPCHK(hipStreamCreate(&st.s));
   DevBuf d2, dmap, dbox, dpc;
-  HIPCHK(hipMalloc(&d2.p, n * sizeof(unsigned)));
-  HIPCHK(hipMalloc(&dmap.p, n * sizeof(float)));
+  HIPCHK(device_alloc(&d2.p, n * sizeof(unsigned)));
+  HIPCHK(device_alloc(&dmap.p, n * sizeof(float)));
   const float cap2 = static_cast<float>(cap * cap);
   unsigned cap2bits;
   std::memcpy(&cap2bits, &cap2, 4);
@@ -290,8 +290,8 @@ int aslhip_surface_distance_map(const double *tri, long long ntri, const int siz
   hipLaunchKernelGGL(k_dist_fill, dim3(nb), dim3(DIST_BLOCK), 0, st.s, static_cast<unsigned *>(d2.p), n, cap2bits);
   HIPCHK(hipGetLastError());
   if (!pieces.empty()) {
-    HIPCHK(hipMalloc(&dbox.p, boxes.size() * sizeof(TriBox)));
-    HIPCHK(hipMalloc(&dpc.p, pieces.size() * sizeof(Piece)));
+    HIPCHK(device_alloc(&dbox.p, boxes.size() * sizeof(TriBox)));
+    HIPCHK(device_alloc(&dpc.p, pieces.size() * sizeof(Piece)));
     HIPCHK(hipMemcpyAsync(dbox.p, boxes.data(), boxes.size() * sizeof(TriBox), hipMemcpyHostToDevice, st.s));
     HIPCHK(hipMemcpyAsync(dpc.p, pieces.data(), pieces.size() * sizeof(Piece), hipMemcpyHostToDevice, st.s));
     for (size_t first = 0; first < pieces.size(); first += 0x7fffffffu) {

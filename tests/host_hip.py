@@ -1,0 +1,51 @@
+"""The library's host side without a GPU: a program run in a process of its own
+in which tests/cpp/host_hip.cpp stands in for the HIP runtime (memory is host
+memory, kernels do nothing, launches are logged and take the time a test gives
+them)."""
+import os
+import subprocess
+import sys
+import tempfile
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes, sys
+sys.path.insert(0, %r)
+H = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)  # before the library: its HIP calls bind to these
+H.host_hip_used.restype = ctypes.c_size_t
+H.host_hip_limit.argtypes = [ctypes.c_size_t]
+H.host_hip_cost.argtypes = [ctypes.c_char_p, ctypes.c_uint, ctypes.c_double]
+H.host_hip_launches.restype = ctypes.c_char_p
+import numpy as np
+import asl_amd
+from asl_amd import _lib
+
+
+def launches(part="k_step"):
+    \"\"\"(grid, block) of the launches of kernels with `part` in their name since the last call.\"\"\"
+    out = [l.rsplit(" ", 2) for l in H.host_hip_launches().decode().splitlines()]
+    H.host_hip_forget()
+    return [(int(g), int(b)) for n, g, b in out if part in n]
+
+
+def cavity(size, q=19, **k):
+    L = asl_amd.Lattice(size, q, nu=0.05, **k)
+    L.init_equilibrium()
+    if not k.get("periodic"):
+        for b in (L.add_slice_bc(_lib.BC_NOSLIP, 63),):
+            L.execute_bc(b)
+    return L
+"""
+
+
+def run(program, timeout=300):
+    """Runs the program (Python source) over the stand-in; returns what it printed."""
+    with tempfile.TemporaryDirectory() as d:
+        so = os.path.join(d, "libhosthip.so")
+        subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", so,
+                        os.path.join(ROOT, "tests", "cpp", "host_hip.cpp")], check=True)
+        r = subprocess.run([sys.executable, "-c", PRELUDE % (ROOT, so) + program], capture_output=True, text=True,
+                           timeout=timeout, cwd=d)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
