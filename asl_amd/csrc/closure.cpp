@@ -39,6 +39,7 @@ int ensure_partial(aslhip_mlp *m, int nblocks) {
   HIPCHK(hipStreamSynchronize(m->stream));
   if (m->partial) HIPCHK(hipFree(m->partial));
   m->partial = nullptr;
+  m->partial_blocks = 0;  // as long as the new one is not there
   HIPCHK(device_alloc(&m->partial, (size_t)nblocks * MLP_PSTRIDE * sizeof(float)));
   m->partial_blocks = nblocks;
   return 0;

@@ -20,3 +20,26 @@ for call in (lambda: asl_amd.Lattice((64, 64, 64), 19, nu=0.1), L.f, lambda: L.s
     assert len(launches()) == 2
     H.host_hip_limit(0)
 """)
+
+
+def test_training_after_a_batch_that_did_not_fit():
+    """The sums of a smaller batch get a buffer again (the kernel would write through a null pointer)."""
+    host_hip.run("""
+M = asl_amd.Mlp(np.zeros(_lib.CLOSURE_NPARAM, np.float32))
+n = 1 << 20
+M.set_data(np.zeros((n, 7), np.float32), np.zeros(n, np.float32))
+M.gradient(0, 256)
+held = H.host_hip_used()
+for call in (lambda: M.gradient(0, n), lambda: M.train(1, n, 1e-3)):
+    H.host_hip_limit(held + 100000)
+    try:
+        call()
+        raise SystemExit("the large batch fitted")
+    except asl_amd.ASLError:
+        pass
+    M.gradient(0, 256)
+    assert H.host_hip_used() == held, (H.host_hip_used(), held)
+    H.host_hip_limit(0)
+M.gradient(0, n)
+assert H.host_hip_used() > held + 100000
+""")
