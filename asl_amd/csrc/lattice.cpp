@@ -2043,10 +2043,11 @@ int batch_launch(aslhip_batch *b, bool odd, bool macro, int e0, int e1) {
   return 0;
 }
 
-// The workgroup table for the batch's workgroup size (the lattices in order).
+// The workgroup table for the batch's settings (the lattices in order).  On
+// failure the batch keeps the table it has.
 int batch_tables(aslhip_batch *b) {
   std::vector<uint2> ent;
-  b->groups.clear();
+  std::vector<std::pair<int, int>> groups;
   const std::vector<int> of = batch_group_of(b);
   const int last = *std::max_element(of.begin(), of.end());
   for (int g = 0; g <= last; ++g) {
@@ -2057,7 +2058,7 @@ int batch_tables(aslhip_batch *b) {
       for (int c = 0; c < a.g.nchunks; ++c)
         ent.push_back(make_uint2(static_cast<unsigned>(l), static_cast<unsigned>(c)));
     }
-    b->groups.emplace_back(static_cast<int>(first), static_cast<int>(ent.size()));
+    groups.emplace_back(static_cast<int>(first), static_cast<int>(ent.size()));
   }
   // Each XCD (workgroup id modulo 8) takes one run of the chunks of a group that
   // the Infinity Cache holds (see xcd_run), others the hardware order: the
@@ -2067,26 +2068,31 @@ int batch_tables(aslhip_batch *b) {
   const std::vector<uint2> plain = ent;
   const size_t nb = plain.size();
   ent.insert(ent.end(), plain.begin(), plain.end());
-  for (size_t g = 0; g < b->groups.size(); ++g) {
+  for (size_t g = 0; g < groups.size(); ++g) {
     long long bytes = 0;
     for (size_t l = 0; l < b->lat.size(); ++l)
       if (of[l] == static_cast<int>(g)) bytes += b->lat[l]->qs_bytes * b->lat[l]->Q;
-    const size_t first = static_cast<size_t>(b->groups[g].first);
-    const size_t share = (static_cast<size_t>(b->groups[g].second) - first) / 8;
+    const size_t first = static_cast<size_t>(groups[g].first);
+    const size_t share = (static_cast<size_t>(groups[g].second) - first) / 8;
     if (bytes > CACHE_BYTES) continue;
     for (size_t i = 0; i < 8 * share; ++i) ent[first + i] = plain[first + (i % 8) * share + i / 8];
   }
   // replays in flight read the old tables and graphs: finish them first
   HIPCHK(hipStreamSynchronize(b->stream));
+  uint2 *d = nullptr;
+  HIPCHK(device_alloc(&d, ent.size() * sizeof(uint2)));
+  if (hipError_t e = hipMemcpy(d, ent.data(), ent.size() * sizeof(uint2), hipMemcpyHostToDevice); e != hipSuccess) {
+    (void)hipFree(d);
+    return fail(ASLHIP_EHIP, "ASL ERROR: batch tables: %s", hipGetErrorString(e));
+  }
   for (auto &g : b->graph)
     if (g) {
       (void)hipGraphExecDestroy(g);
       g = nullptr;
     }
-  if (b->ent) HIPCHK(hipFree(b->ent));
-  b->ent = nullptr;
-  HIPCHK(device_alloc(&b->ent, ent.size() * sizeof(uint2)));
-  HIPCHK(hipMemcpy(b->ent, ent.data(), ent.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  if (b->ent) (void)hipFree(b->ent);
+  b->ent = d;
+  b->groups = groups;
   b->nblocks = static_cast<int>(nb);
   return 0;
 }
@@ -2220,25 +2226,26 @@ int aslhip_batch_create(aslhip_batch **out, aslhip_lattice *const *lattices, int
 
 int aslhip_batch_set_tuning(aslhip_batch *b, int knob, int value) {
   if (!b) return fail(ASLHIP_EINVAL, "ASL ERROR: null batch handle");
+  int *setting = nullptr;
   if (knob == ASLHIP_TUNE_GROUP_MB) {
     if (value < 0 || value > (1 << 20)) return fail(ASLHIP_EINVAL, "ASL ERROR: group size %d MiB out of 0..2^20", value);
-    if (value == b->group_mb) return 0;
-    b->group_mb = value;
-    return batch_tables(b);
-  }
-  if (knob == ASLHIP_TUNE_LDS) {
+    setting = &b->group_mb;
+  } else if (knob == ASLHIP_TUNE_LDS) {
     if (value != 0 && value != 1) return fail(ASLHIP_EINVAL, "ASL ERROR: batches take ASLHIP_TUNE_LDS 0 or 1");
-    if (value == b->tune_lds) return 0;
-    b->tune_lds = value;
-    return batch_tables(b);
-  }
-  if (knob != ASLHIP_TUNE_BLOCK)
+    setting = &b->tune_lds;
+  } else if (knob == ASLHIP_TUNE_BLOCK) {
+    if (value < 64 || value > STEP_BLOCK || value % 64)
+      return fail(ASLHIP_EINVAL, "ASL ERROR: workgroup size %d is not a multiple of 64 in 64..%d", value, STEP_BLOCK);
+    setting = &b->block;
+  } else {
     return fail(ASLHIP_EINVAL, "ASL ERROR: batches tune the workgroup size, the tiles and the group size only");
-  if (value < 64 || value > STEP_BLOCK || value % 64)
-    return fail(ASLHIP_EINVAL, "ASL ERROR: workgroup size %d is not a multiple of 64 in 64..%d", value, STEP_BLOCK);
-  if (value == b->block) return 0;
-  b->block = value;
-  return batch_tables(b);
+  }
+  const int old = *setting;
+  if (value == old) return 0;
+  *setting = value;
+  const int r = batch_tables(b);
+  if (r) *setting = old;  // the table of the old setting is still there
+  return r;
 }
 
 int aslhip_batch_autotune(aslhip_batch *b, int nsteps, int *best_block) {

@@ -43,3 +43,26 @@ for call in (lambda: M.gradient(0, n), lambda: M.train(1, n, 1e-3)):
 M.gradient(0, n)
 assert H.host_hip_used() > held + 100000
 """)
+
+
+def test_a_batch_keeps_its_setting_when_the_new_table_does_not_fit():
+    """Launches of another workgroup size than the table's would read it past its end."""
+    host_hip.run("""
+Ls = [cavity((24, 24, 24)) for _ in range(3)]
+B = asl_amd.Batch(Ls)
+B.step(3)
+before = launches("k_step_batch")
+for knob, value in ((_lib.TUNE_BLOCK, 256), (_lib.TUNE_LDS, 1), (_lib.TUNE_GROUP_MB, 1)):
+    H.host_hip_limit(H.host_hip_used() + 1)
+    try:
+        B.set_tuning(knob, value)
+        raise SystemExit("it fitted")
+    except asl_amd.ASLError:
+        pass
+    B.step(2)
+    assert launches("k_step_batch") == before, value
+H.host_hip_limit(0)
+B.set_tuning(_lib.TUNE_BLOCK, 256)
+B.step(1)
+assert launches("k_step_batch")[0] == (3 * 24**3 // 256, 256)
+""")
