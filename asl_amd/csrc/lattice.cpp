@@ -1393,15 +1393,11 @@ int aslhip_init_equilibrium_field(aslhip_lattice *h, const void *rho, const void
   void *drho = nullptr, *du = nullptr;
   const size_t n = (size_t)h->len * h->melem;
   HIPCHK(device_alloc(&du, 3 * n));
-  // small fields need no wait here: the stream is waited for below, before the caller may change them
-  auto up = [h](void *dst, const void *src, size_t bytes) {
-    return bytes <= (128u << 10) ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream)
-                                 : to_device(dst, src, bytes, h->stream);
-  };
-  HIPCHK(up(du, u, 3 * n));
+  // the stream is waited for below, before the caller may change the fields
+  HIPCHK(to_device(du, u, 3 * n, h->stream, false));
   if (rho) {
     HIPCHK(device_alloc(&drho, n));
-    HIPCHK(up(drho, rho, n));
+    HIPCHK(to_device(drho, rho, n, h->stream, false));
   }
   InitArgs a;
   a.f = h->f;

@@ -1,15 +1,27 @@
 // Copies between device memory and ordinary (pageable) host memory through
 // pinned buffers: the runtime's own path for pageable memory copies to and
 // from its staging buffer in turn with the DMA (18 GB/s to the host, 32 GB/s
-// from it; 2.5 GB/s at 1 MB), while pinned memory moves at 56 GB/s and one core
-// copies 35 to 80 GB/s (5 GB/s into memory that was never touched: the first
-// write of a page faults, which only more cores make up for).  So chunks go
-// through a ring of pinned buffers, the DMA of one beside the host copy of
-// others, and larger transfers take a few threads.  Before and after: restart
-// of a 120 x 70 x 66 D3Q19 lattice (populations in, 10 steps, populations, rho
-// and u out, 100 MB) 7.4 -> 3.4 ms; 100 steps of a 300 x 50 x 50 D3Q15 duct with
-// rho and u read (13 MB) 2.74 -> 2.50 ms; 20 steps on 160 x 72 x 60 with a
-// surface force and u (17 MB) 1.70 -> 1.29 ms.
+// from it; 2.5 GB/s for a process's first 17 MB), while pinned memory moves at 56
+// GB/s and one core copies 35 to 80 GB/s (5 GB/s into memory that was never
+// touched: the first write of a page faults, which only more cores make up for).
+// So chunks go through a ring of pinned buffers, the DMA of one beside the host
+// copy of others, and larger transfers take a few threads.  Before and after:
+// restart of a 120 x 70 x 66 D3Q19 lattice (populations in, 10 steps,
+// populations, rho and u out, 100 MB) 7.4 -> 3.4 ms; 100 steps of a 300 x 50 x 50
+// D3Q15 duct with rho and u read (13 MB) 2.74 -> 2.50 ms; 20 steps on 160 x 72 x
+// 60 with a surface force and u (17 MB) 1.70 -> 1.29 ms.
+//
+// Which way a transfer goes, us, runtime / ring with events (memory touched
+// before, after the process's first ones):
+//   to the host     70 KB 11.1 / 17.9, 512 KB 29 / 35, 1 MB 59 / 66, 2 MB 118 /
+//                   115, 3 MB 178 / 153, 8 MB 465 / 315, 32 MB 1890 / 930
+//   to the device   70 KB 10.5 / 17.8, 1 MB 51 / 59, 4 MB 131 / 183, 8 MB 240 /
+//                   315, 24 MB 680 / 708, 32 MB 910 / 905, 48 MB 1757 / 1323
+// - memory that the runtime knows (pinned, on a device): its own path; 3.4 MB
+//   into pinned memory take 69 us there and 157 through the ring;
+// - to the host, one chunk or less: one buffer and a wait for the stream in
+//   place of an event (23 KB 9.5, 70 KB 12, 443 KB 26);
+// - to the device, less than RING_FROM: the runtime's path.
 //
 // One ring for the process (RING buffers of CHUNK bytes), held while some
 // lattice or trainer exists; a second thread that transfers meanwhile takes
@@ -30,6 +42,7 @@ constexpr size_t CHUNK = 2u << 20;
 constexpr int RING = 8;                      // buffers: chunks in flight and chunks being copied
 constexpr int COPIERS = 4;                   // copy threads
 constexpr size_t THREADS_FROM = 4u << 20;    // smaller transfers end before a thread would pay
+constexpr size_t RING_FROM = 30u << 20;      // to the device: smaller transfers take the runtime's path
 constexpr int MAX_DEVICES = 64;
 
 std::mutex ring_mu;   // held during a transfer
@@ -46,6 +59,14 @@ void release_ring() {
       }
   if (ring) (void)hipHostFree(ring);
   ring = nullptr;
+}
+
+// Ordinary host memory, nothing that the runtime allocated or registered.
+bool pageable(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
 }
 
 // The ring and the current device's events (null: use the runtime's path).
@@ -147,11 +168,18 @@ void transfer_drop() {
 
 hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s) {
   if (n == 0) return hipStreamSynchronize(s);
-  std::unique_lock<std::mutex> lock(ring_mu, std::try_to_lock);
-  hipEvent_t *ev = lock.owns_lock() ? ring_ready() : nullptr;
+  std::unique_lock<std::mutex> lock(ring_mu, std::defer_lock);
+  hipEvent_t *ev = pageable(dst) && lock.try_lock() ? ring_ready() : nullptr;
   if (!ev) {
     const hipError_t e = hipStreamSynchronize(s);
     return e != hipSuccess ? e : hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+  }
+  if (n <= CHUNK) {
+    hipError_t e = hipMemcpyAsync(ring, src, n, hipMemcpyDeviceToHost, s);
+    const hipError_t w = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = w;
+    if (e == hipSuccess) std::memcpy(dst, ring, n);
+    return e;
   }
   const long chunks = static_cast<long>((n + CHUNK - 1) / CHUNK);
   hipError_t e = hipSuccess;
@@ -181,13 +209,13 @@ hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s) {
   return hipSuccess;
 }
 
-hipError_t to_device(void *dst, const void *src, size_t n, hipStream_t s) {
+hipError_t to_device(void *dst, const void *src, size_t n, hipStream_t s, bool wait) {
   if (n == 0) return hipSuccess;
-  std::unique_lock<std::mutex> lock(ring_mu, std::try_to_lock);
-  hipEvent_t *ev = lock.owns_lock() ? ring_ready() : nullptr;
+  std::unique_lock<std::mutex> lock(ring_mu, std::defer_lock);
+  hipEvent_t *ev = n >= RING_FROM && pageable(src) && lock.try_lock() ? ring_ready() : nullptr;
   if (!ev) {
     const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, s);
-    return e != hipSuccess ? e : hipStreamSynchronize(s);
+    return e != hipSuccess || !wait ? e : hipStreamSynchronize(s);
   }
   const long chunks = static_cast<long>((n + CHUNK - 1) / CHUNK);
   hipError_t e = hipSuccess;

@@ -1,8 +1,8 @@
 // The HIP host calls that libaslhip.so makes, on host memory: loaded before the
 // library (tests/host_hip.py) they let its host side run without a GPU.
-// Kernels do nothing but are logged; copies are copies; every launch takes a
-// time that the test chooses, which events measure; a limit on the memory and
-// the current device can be set.  Errors are HIP's: 2 out of memory, 400
+// Kernels do nothing but are logged; copies are copies and logged too; every
+// launch takes a time that the test chooses, which events measure; a limit on
+// the memory and the current device can be set.  Errors are HIP's: 2 out of memory, 400
 // invalid handle (an event recorded on a stream of another device).
 #include <atomic>
 #include <cstdint>
@@ -46,6 +46,12 @@ size_t used = 0, limit = 0;
 int device = 0, last = 0;
 double now = 0.;
 std::vector<Launch> launches;
+struct Copy {
+  char to, from;  // d device, p pinned, h other host memory
+  size_t bytes;
+};
+std::vector<Copy> copies;
+std::map<const void *, size_t> pinned;
 std::vector<Cost> costs;
 std::string text;
 thread_local struct {
@@ -54,6 +60,18 @@ thread_local struct {
   void *stream;
 } config;
 int fail(int e) { return last = e; }
+template <class M>
+bool within(const M &m, const void *p) {
+  auto it = m.upper_bound(const_cast<void *>(p));
+  if (it == m.begin()) return false;
+  --it;
+  return static_cast<const char *>(p) < static_cast<const char *>(it->first) + it->second;
+}
+char kind(const void *p) { return within(allocated, p) ? 'd' : within(pinned, p) ? 'p' : 'h'; }
+void copied(void *d, const void *s, size_t n) {
+  copies.push_back({kind(d), kind(s), n});
+  std::memcpy(d, s, n);
+}
 }  // namespace
 
 #define LOCK std::lock_guard<std::recursive_mutex> lock(mu)
@@ -65,7 +83,15 @@ void host_hip_device(int d) { device = d; }
 void host_hip_limit(size_t n) { limit = n; }
 size_t host_hip_used() { return used; }
 void host_hip_cost(const char *part, unsigned block, double ms) { costs.push_back({part, block, ms}); }
-void host_hip_forget() { launches.clear(); }
+void host_hip_forget() {
+  launches.clear();
+  copies.clear();
+}
+const char *host_hip_copies() {  // "to from bytes" lines
+  text.clear();
+  for (const auto &c : copies) text += std::string(1, c.to) + " " + c.from + " " + std::to_string(c.bytes) + "\n";
+  return text.c_str();
+}
 const char *host_hip_launches() {  // "kernel grid block" lines
   text.clear();
   for (const auto &l : launches) text += l.name + " " + std::to_string(l.grid) + " " + std::to_string(l.block) + "\n";
@@ -132,17 +158,31 @@ int hipFree(void *p) {
   std::free(p);
   return 0;
 }
-int hipHostMalloc(void **p, size_t n, unsigned) { return (*p = std::malloc(n)) ? 0 : fail(2); }
+int hipHostMalloc(void **p, size_t n, unsigned) {
+  LOCK;
+  if (!(*p = std::malloc(n))) return fail(2);
+  pinned[*p] = n;
+  return 0;
+}
 int hipHostFree(void *p) {
+  LOCK;
+  pinned.erase(p);
   std::free(p);
   return 0;
 }
+int hipPointerGetAttributes(int *type, const void *p) {  // the first member of hipPointerAttribute_t
+  LOCK;
+  *type = kind(p) == 'd' ? 2 : kind(p) == 'p' ? 1 : 0;
+  return 0;
+}
 int hipMemcpy(void *d, const void *s, size_t n, int) {
-  std::memcpy(d, s, n);
+  LOCK;
+  copied(d, s, n);
   return 0;
 }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) {
-  std::memcpy(d, s, n);
+  LOCK;
+  copied(d, s, n);
   return 0;
 }
 int hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, int) {

@@ -16,17 +16,24 @@ H = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)  # before the library: its HIP call
 H.host_hip_used.restype = ctypes.c_size_t
 H.host_hip_limit.argtypes = [ctypes.c_size_t]
 H.host_hip_cost.argtypes = [ctypes.c_char_p, ctypes.c_uint, ctypes.c_double]
-H.host_hip_launches.restype = ctypes.c_char_p
+H.host_hip_launches.restype = H.host_hip_copies.restype = ctypes.c_char_p
 import numpy as np
 import asl_amd
 from asl_amd import _lib
 
 
 def launches(part="k_step"):
-    \"\"\"(grid, block) of the launches of kernels with `part` in their name since the last call.\"\"\"
+    # (grid, block) of the launches of kernels with `part` in their name since the last call
     out = [l.rsplit(" ", 2) for l in H.host_hip_launches().decode().splitlines()]
     H.host_hip_forget()
     return [(int(g), int(b)) for n, g, b in out if part in n]
+
+
+def copies():
+    # (to, from, bytes) of the copies since the last call: d device, p pinned, h other host memory
+    out = [l.split() for l in H.host_hip_copies().decode().splitlines()]
+    H.host_hip_forget()
+    return [(t, f, int(n)) for t, f, n in out]
 
 
 def cavity(size, q=19, **k):

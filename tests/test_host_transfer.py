@@ -1,0 +1,36 @@
+"""Which way host transfers go, over the stand-in for the HIP runtime (host_hip.py)."""
+import host_hip
+
+
+def test_memory_the_runtime_knows_is_copied_directly():
+    """Reads into pinned memory and writes from it take no detour through the ring's buffers."""
+    host_hip.run("""
+L = cavity((60, 60, 60))
+view = L.q * L.len * 4
+buf = ctypes.c_void_p()
+assert H.hipHostMalloc(ctypes.byref(buf), ctypes.c_size_t(view), 0) == 0
+H.host_hip_forget()
+_lib.call("aslhip_read_velocity", L.h, buf)
+assert copies() == [("p", "d", 12 * L.len)]
+_lib.call("aslhip_read_f", L.h, buf)
+assert copies() == [("p", "d", view)]
+_lib.call("aslhip_write_f", L.h, buf)
+assert copies() == [("d", "p", view)]
+""")
+
+
+def test_small_transfers():
+    """To the device without the ring up to 30 MiB, to the host through one buffer up to 2 MiB; all bytes arrive."""
+    host_hip.run("""
+MB = 1 << 20
+M = asl_amd.Mlp(np.arange(_lib.CLOSURE_NPARAM, dtype=np.float32))
+H.host_hip_forget()
+assert np.array_equal(M.params(), np.arange(_lib.CLOSURE_NPARAM))
+assert copies() == [("p", "d", 4 * _lib.CLOSURE_NPARAM)]
+for n, direct in ((3, True), (30 * MB // 28 - 1, True), (30 * MB // 28 + 1, False)):
+    x = np.zeros((n, 7), np.float32)
+    M.set_data(x, np.zeros(n, np.float32))
+    got = [c for c in copies() if c[0] == "d"]
+    assert sum(c[2] for c in got) == 32 * n
+    assert (got[0] == ("d", "h", 28 * n)) == direct, (n, got[:3])
+""")
