@@ -69,10 +69,13 @@ bool pageable(const void *p) {
   return true;
 }
 
-// The ring and the current device's events (null: use the runtime's path).
-hipEvent_t *ring_ready() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return nullptr;
+// The ring and the current device's events (null: use the runtime's path, also
+// for a stream of another device, on which they cannot be recorded).
+hipEvent_t *ring_ready(hipStream_t s) {
+  int dev = 0, of = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipStreamGetDevice(s, &of) != hipSuccess || of != dev || dev < 0 ||
+      dev >= MAX_DEVICES)
+    return nullptr;
   if (!ring && hipHostMalloc(&ring, RING * CHUNK, hipHostMallocPortable) != hipSuccess) {
     (void)hipGetLastError();
     ring = nullptr;
@@ -169,7 +172,7 @@ void transfer_drop() {
 hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s) {
   if (n == 0) return hipStreamSynchronize(s);
   std::unique_lock<std::mutex> lock(ring_mu, std::defer_lock);
-  hipEvent_t *ev = pageable(dst) && lock.try_lock() ? ring_ready() : nullptr;
+  hipEvent_t *ev = pageable(dst) && lock.try_lock() ? ring_ready(s) : nullptr;
   if (!ev) {
     const hipError_t e = hipStreamSynchronize(s);
     return e != hipSuccess ? e : hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
@@ -212,7 +215,7 @@ hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s) {
 hipError_t to_device(void *dst, const void *src, size_t n, hipStream_t s, bool wait) {
   if (n == 0) return hipSuccess;
   std::unique_lock<std::mutex> lock(ring_mu, std::defer_lock);
-  hipEvent_t *ev = n >= RING_FROM && pageable(src) && lock.try_lock() ? ring_ready() : nullptr;
+  hipEvent_t *ev = n >= RING_FROM && pageable(src) && lock.try_lock() ? ring_ready(s) : nullptr;
   if (!ev) {
     const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, s);
     return e != hipSuccess || !wait ? e : hipStreamSynchronize(s);

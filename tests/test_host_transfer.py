@@ -34,3 +34,20 @@ for n, direct in ((3, True), (30 * MB // 28 - 1, True), (30 * MB // 28 + 1, Fals
     assert sum(c[2] for c in got) == 32 * n
     assert (got[0] == ("d", "h", 28 * n)) == direct, (n, got[:3])
 """)
+
+
+def test_a_lattice_of_another_device_than_the_current_one():
+    """The ring's events belong to a device: transfers on another one's stream do without them."""
+    host_hip.run("""
+L = asl_amd.Lattice((80, 80, 80), 19, nu=0.05, periodic=True)
+L.init_equilibrium()
+M = asl_amd.Mlp(np.zeros(_lib.CLOSURE_NPARAM, np.float32))
+f = np.ones((19,) + L.S, np.float32)
+assert f.nbytes >= 30 << 20
+L.velocity()
+for device in (1, 0, 1):
+    H.host_hip_device(device)
+    L.write_f(f)
+    L.velocity()
+    L.rho()
+""")
