@@ -31,8 +31,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace aslhip {
@@ -111,7 +111,7 @@ struct Copiers {
     try {
       for (int w = 0; w < COPIERS; ++w) th[w] = std::thread([this, w] { work(w); });
       running = true;
-    } catch (const std::system_error &) {  // no thread to be had
+    } catch (const std::exception &) {  // no thread, or no memory for one, to be had
       finish();
     }
   }

@@ -45,6 +45,7 @@ std::map<void *, size_t> allocated;
 size_t used = 0, limit = 0;
 int device = 0, last = 0;
 double now = 0.;
+bool no_new = false;
 std::vector<Launch> launches;
 struct Copy {
   char to, from;  // d device, p pinned, h other host memory
@@ -69,10 +70,19 @@ bool within(const M &m, const void *p) {
 }
 char kind(const void *p) { return within(allocated, p) ? 'd' : within(pinned, p) ? 'p' : 'h'; }
 void copied(void *d, const void *s, size_t n) {
-  copies.push_back({kind(d), kind(s), n});
+  if (copies.size() < copies.capacity() || !no_new) copies.push_back({kind(d), kind(s), n});
   std::memcpy(d, s, n);
 }
 }  // namespace
+
+// the library's allocations on the host, which a test can make fail
+void *operator new(size_t n) {
+  void *p = no_new ? nullptr : std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 #define LOCK std::lock_guard<std::recursive_mutex> lock(mu)
 
@@ -82,6 +92,7 @@ extern "C" {
 void host_hip_device(int d) { device = d; }
 void host_hip_limit(size_t n) { limit = n; }
 size_t host_hip_used() { return used; }
+void host_hip_no_new(int on) { no_new = on != 0; }
 void host_hip_cost(const char *part, unsigned block, double ms) { costs.push_back({part, block, ms}); }
 void host_hip_forget() {
   launches.clear();

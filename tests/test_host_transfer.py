@@ -51,3 +51,21 @@ for device in (1, 0, 1):
     L.velocity()
     L.rho()
 """)
+
+
+def test_no_memory_for_the_copy_threads():
+    """The caller copies by itself, and no exception leaves the C entry."""
+    host_hip.run("""
+L = asl_amd.Lattice((80, 80, 80), 19, nu=0.05, periodic=True)
+L.init_equilibrium()
+out = np.zeros(3 * L.len, np.float32)
+lib = _lib.load_library()
+p = ctypes.c_void_p(out.ctypes.data)
+assert lib.aslhip_read_velocity(L.h, p) == 0  # the ring is there
+want = out.copy()
+out[:] = 7
+H.host_hip_no_new(1)
+r = lib.aslhip_read_velocity(L.h, p)
+H.host_hip_no_new(0)
+assert r == 0 and want.tobytes() == out.tobytes()
+""")
