@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -901,17 +902,25 @@ struct SweepLaunch {
 // [b g - s, (b + 1) g - s) in step s.  Periodic lattices: step s covers planes
 // s .. nx + s - 1 (modulo nx), so that the first block starts from planes
 // nobody needs yet and the last one closes the ring.
-void sweep_plan(int nx, bool periodic, int g, int t, int n, std::vector<SweepLaunch> &out) {
-  for (int s0 = 0; s0 < n; s0 += t) {
-    const int m = std::min(t, n - s0);
-    const int end = periodic ? nx + m - 1 : nx;  // planes of the last step end here
-    for (int b = 0; b * g - (m - 1) < end; ++b)
-      for (int s = 0; s < m; ++s) {
-        const int lo = std::max(b * g - s, periodic ? s : 0), hi = std::min((b + 1) * g - s, periodic ? nx + s : nx);
-        if (lo >= hi) continue;
-        if (lo < nx) out.push_back({s0 + s, lo, std::min(hi, nx) - lo});
-        if (hi > nx) out.push_back({s0 + s, std::max(lo, nx) - nx, hi - std::max(lo, nx)});
+// Hands the launches to emit in order until it returns false.
+template <class F>
+void sweep_plan(long long nx, bool periodic, long long g, long long t, long long n, F emit) {
+  for (long long s0 = 0; s0 < n; s0 += t) {
+    const long long m = std::min(t, n - s0);
+    const long long end = periodic ? nx + m - 1 : nx;  // planes of the last step end here
+    for (long long b = 0; b * g - (m - 1) < end; ++b) {
+      // the steps that have planes in this block
+      const long long over = std::max(0LL, b * g - nx + 1), below = (b + 1) * g;
+      const long long first = periodic ? (over + 1) / 2 : over, last = std::min(m, periodic ? (below + 1) / 2 : below);
+      for (long long s = first; s < last; ++s) {
+        const long long lo = std::max(b * g - s, periodic ? s : 0), hi = std::min((b + 1) * g - s, periodic ? nx + s : nx);
+        if (lo < nx && !emit(SweepLaunch{static_cast<int>(s0 + s), static_cast<int>(lo), static_cast<int>(std::min(hi, nx) - lo)}))
+          return;
+        if (hi > nx && !emit(SweepLaunch{static_cast<int>(s0 + s), static_cast<int>(std::max(lo, nx) - nx),
+                                         static_cast<int>(hi - std::max(lo, nx))}))
+          return;
       }
+    }
   }
 }
 
@@ -933,14 +942,14 @@ int launch_run(aslhip_lattice *h, unsigned fl, unsigned last_fl, int n) {
       if (int r = launch_one(h, s == n - 1 ? last_fl : fl, nullptr, s)) return r;
     return 0;
   }
-  std::vector<SweepLaunch> plan;
   for (int s = 0; s < n; s += t) {
     const int m = std::min(t, n - s);
-    plan.clear();
-    sweep_plan(h->n[0], h->periodic, g, t, m, plan);
-    for (const auto &l : plan)
-      if (int r = launch_planes(h, h->next_odd != ((l.step & 1) != 0), s + l.step == n - 1 ? last_fl : fl, l.p0, l.np))
-        return r;
+    int r = 0;
+    sweep_plan(h->n[0], h->periodic, g, t, m, [&](const SweepLaunch &l) {
+      r = launch_planes(h, h->next_odd != ((l.step & 1) != 0), s + l.step == n - 1 ? last_fl : fl, l.p0, l.np);
+      return r == 0;
+    });
+    if (r) return r;
     if (m & 1) h->next_odd = !h->next_odd;
   }
   return 0;
@@ -1803,16 +1812,22 @@ int aslhip_set_tuning(aslhip_lattice *h, int knob, int value) {
 }
 
 int aslhip_sweep_plan(int nx, int periodic, int planes, int steps, int nsteps, int *out, int cap) {
-  if (nx < 1 || planes < 1 || steps < 1 || nsteps < 0 || cap < 0 || (cap > 0 && !out))
+  if (nx < 1 || planes < 1 || steps < 1 || nsteps < 0 || cap < 0 || (cap > 0 && !out) || (periodic && steps > nx))
     return fail(ASLHIP_EINVAL, "ASL ERROR: sweep_plan: bad arguments");
-  std::vector<SweepLaunch> plan;
-  sweep_plan(nx, periodic != 0, planes, steps, nsteps, plan);
-  for (size_t i = 0; i < plan.size() && i < static_cast<size_t>(cap); ++i) {
-    out[3 * i] = plan[i].step;
-    out[3 * i + 1] = plan[i].p0;
-    out[3 * i + 2] = plan[i].np;
-  }
-  return static_cast<int>(plan.size());
+  // a step has at least one launch per block
+  long long count = nsteps * ((static_cast<long long>(nx) + planes - 1) / planes);
+  if (count > INT_MAX) return fail(ASLHIP_EINVAL, "ASL ERROR: sweep_plan: too many launches to count");
+  count = 0;
+  sweep_plan(nx, periodic != 0, planes, steps, nsteps, [&](const SweepLaunch &l) {
+    if (count < cap) {
+      out[3 * count] = l.step;
+      out[3 * count + 1] = l.p0;
+      out[3 * count + 2] = l.np;
+    }
+    return ++count <= INT_MAX;
+  });
+  if (count > INT_MAX) return fail(ASLHIP_EINVAL, "ASL ERROR: sweep_plan: too many launches to count");
+  return static_cast<int>(count);
 }
 
 int aslhip_tuning_value(aslhip_lattice *h, int knob, int *value) {

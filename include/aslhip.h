@@ -416,7 +416,9 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
 int aslhip_set_tuning(aslhip_lattice *h, int knob, int value);
 /* The launches of a sweep of nsteps steps over nx planes, blocks of `planes`
  * planes and `steps` steps per sweep: triples (step, first plane, planes) in
- * launch order, the first cap of them to out.  Returns their number. */
+ * launch order, the first cap of them to out.  Returns their number; refused:
+ * numbers below 1, more launches than an int counts, on a periodic lattice more
+ * steps than planes. */
 int aslhip_sweep_plan(int nx, int periodic, int planes, int steps, int nsteps, int *out, int cap);
 /* The value a tuning knob has now (ASLHIP_TUNE_CPL: the cells per lane the
  * step kernel runs with; ASLHIP_TUNE_LDS: 0, 1 or 2 as it runs LDS-staged
