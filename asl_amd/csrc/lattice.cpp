@@ -865,21 +865,42 @@ int launch_planes(aslhip_lattice *h, bool odd, unsigned fl, int p0, int np) {
 // 160 (642 MB) 231 / 256 -> 223 / 256, 256 x 256 x 128 226 / 271 -> 219 / 242,
 // 256^3 462 / 583 -> 447 / 482, 512 x 256 x 256 942 / 1211 -> 896 / 985; of 4
 // steps 256 x 256 x 128 225 -> 227, of 6 steps 223 -> 223.
+// FP64 lattices below 768 MiB, which lose 2 to 4 % alone and gain 4 to 19 % beside
+// others, sweep from 8 steps on (156 x 153 x 150 D3Q19, 539 MB, alone, 4 steps: 190
+// -> 197).
 // Velocity-map links are filled after every step of the whole lattice: no
 // sweeps.
 constexpr long long SWEEP_WINDOW = 224LL << 20;
-constexpr long long SWEEP_TILED_BYTES = 560LL << 20;
-constexpr int SWEEP_STEPS = 16, SWEEP_MIN_STEPS = 4, SWEEP_TILED_MIN_STEPS = 6;
+constexpr long long SWEEP_TILED_BYTES = 560LL << 20, SWEEP_F64_BYTES = 768LL << 20;
+constexpr int SWEEP_STEPS = 16, SWEEP_MIN_STEPS = 4, SWEEP_TILED_MIN_STEPS = 6, SWEEP_F64_MIN_STEPS = 8;
+
+// Whether a window of wp planes pays.  Every launch of a window costs some 5 us
+// of its own and a sweep takes wp / 2 steps, so thick planes lose, more so in
+// boxes (the direct kernel's own reuse, odd steps from the other end, is worth
+// 256 MiB a step).  us per step of 20 alone, launch per step -> sweeps: 16 planes
+// and more at least level but for FP64 (above); 12 planes, D3Q19 FP64 400 x 300:
+// 20 planes 121 -> 132, 60 403 -> 396, box 402 -> 408; 11, D3Q19 FP32 512 x 512: 24
+// 165 -> 179, 80 604 -> 587; 8, D3Q27 FP32 512 x 512: 40 439 -> 474, 200 2276 ->
+// 2243, box 2257 -> 2366; 10, FP16 750 x 750: 80 708 -> 720, box 711 -> 753; 4,
+// D3Q27 FP32 700 x 700: 300 6490 -> 6990; FP64 500 x 500: 20 408 -> 429, 200 4925 ->
+// 4309, box 4665 -> 4601; D3Q19 FP64 512 x 512 (5): 300 4937 -> 4528, box 4685 -> 4837.
+bool sweep_pays(const aslhip_lattice *h, long long wp, long long bytes) {
+  if (wp >= 16) return true;
+  if (wp >= 8) return h->periodic && h->selem >= 4 && bytes >= 1536LL << 20;
+  return h->selem == 8 && (h->periodic || h->Q == 27) && bytes >= 8LL << 30;
+}
+
 void sweep_shape(const aslhip_lattice *h, int n, int &g, int &t) {
   g = t = 0;
   if (n < 2 || h->nvl || h->tune_sweep == 0) return;
+  const long long plane = static_cast<long long>(h->Q) * h->selem * h->sx;
   if (h->tune_sweep < 0) {
     const long long bytes = h->qs_bytes * h->Q;
-    if (bytes <= CACHE_BYTES || n < SWEEP_MIN_STEPS) return;
+    if (bytes <= CACHE_BYTES || n < SWEEP_MIN_STEPS || !sweep_pays(h, SWEEP_WINDOW / plane, bytes)) return;
+    if (h->selem == 8 && bytes < SWEEP_F64_BYTES && n < SWEEP_F64_MIN_STEPS) return;
     if (effective_lds(h) == 1 && (h->tune_lds == 1 || bytes <= SWEEP_TILED_BYTES || n < SWEEP_TILED_MIN_STEPS)) return;
   }
   const long long window = h->tune_sweep > 0 ? static_cast<long long>(h->tune_sweep) << 10 : SWEEP_WINDOW;
-  const long long plane = static_cast<long long>(h->Q) * h->selem * h->sx;
   const int wp = static_cast<int>(std::min<long long>(window / plane, h->n[0]));
   const int m = std::min(SWEEP_STEPS, wp / 2);
   if (m < 2 || wp >= h->n[0]) return;

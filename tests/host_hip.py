@@ -46,13 +46,18 @@ def cavity(size, q=19, **k):
 """
 
 
+_built = []  # the directory that holds the stand-in, built once a process
+
+
 def run(program, timeout=300):
     """Runs the program (Python source) over the stand-in; returns what it printed."""
-    with tempfile.TemporaryDirectory() as d:
-        so = os.path.join(d, "libhosthip.so")
-        subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", so,
+    if not _built:
+        _built.append(tempfile.TemporaryDirectory())
+        subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o",
+                        os.path.join(_built[0].name, "libhosthip.so"),
                         os.path.join(ROOT, "tests", "cpp", "host_hip.cpp")], check=True)
-        r = subprocess.run([sys.executable, "-c", PRELUDE % (ROOT, so) + program], capture_output=True, text=True,
-                           timeout=timeout, cwd=d)
+    d = _built[0].name
+    r = subprocess.run([sys.executable, "-c", PRELUDE % (ROOT, os.path.join(d, "libhosthip.so")) + program],
+                       capture_output=True, text=True, timeout=timeout, cwd=d)
     assert r.returncode == 0, r.stdout + r.stderr
     return r.stdout
