@@ -20,6 +20,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -1975,32 +1976,42 @@ struct aslhip_batch {
   bool periodic = false, wide = false;
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
-  StepArgs *desc = nullptr;  // [2][n]: plain steps, then steps writing rho/u
-  uint2 *ent = nullptr;      // [2][nblocks], per workgroup: lattice, chunk; group by group, then for launches of all groups
-  int nblocks = 0;
+  StepArgs *desc = nullptr;  // [2][2][n]: launches of groups, of all; each plain steps, then steps writing rho/u
+  uint2 *ent = nullptr;      // [2][all workgroups]: lattice, chunk; group by group, then for launches of all groups
   int block = STEP_BLOCK;    // workgroup size of all lattices of the batch (direct kernel)
-  int tune_lds = 0;          // LDS-staged tiles: 1 on, 0 off
+  int tune_lds = -1;         // LDS-staged tiles: 1 on, 0 off, -1 by group (batch_tile)
   // Runs of several steps go group by group: each group of consecutive
   // lattices (at most group_mb MiB of populations; 0: one group; -1: automatic)
   // takes all the run's steps (a graph chunk, or the steps of an eager call)
   // before the next starts, so a group that fits the 256 MiB Infinity Cache is
-  // stepped from cache.  Entry ranges [first, second) of each group.
+  // stepped from cache.
   int group_mb = -1;
   // Measured on D3Q19 FP32 cavities, one group -> groups of 224 MiB: 16 of
   // 32^3..96^3 (330 MiB) 135 -> 123 us per step, 64 of 32^3..160^3 (4.1 GiB)
   // 1675 -> 1535; with 512 lanes 128 MiB 128.5 and 1633, 192 MiB 127.5 and 1621,
   // 224 MiB 127.0 and 1588.
-  std::vector<std::pair<int, int>> groups;
+  struct Range {  // workgroups of one launch: entries [first, end)
+    int first, end;
+    bool tile, all;
+  };
+  std::vector<Range> groups;  // one launch per step of each group
+  Range all;                  // one launch per step of all lattices
+  std::vector<char> tile;     // per lattice: its group's
   hipGraphExec_t graph[2] = {nullptr, nullptr};  // chunks starting with an even / odd step
   std::vector<StepArgs> hdesc;                    // host copy of desc (source of the async upload)
 };
 
 namespace {
 
-// Tiles for the batch's steps: non-periodic batches under 4 GiB per lattice.
-// Not automatic: groups step from the cache, where the direct kernel is the
-// faster one (the cavities above: 127 against 136 us, 1621 against 1708).
-bool batch_tile(const aslhip_batch *b) { return b->tune_lds != 0 && !b->periodic && !b->wide; }
+// Tiles for the steps of a group of that many bytes: non-periodic batches under
+// 4 GiB per lattice.  Automatic for D3Q19 FP32 groups that stream from HBM, as for
+// single lattices: three of 220^3 1056 (direct) -> 1010 us per step, six of 166^3
+// 969 -> 951; groups that step from the cache are faster with the direct kernel
+// (the cavities of batch_group_bytes's figures: 127 against 136, 1621 against 1708).
+bool batch_tile(const aslhip_batch *b, long long bytes) {
+  if (b->periodic || b->wide) return false;
+  return b->tune_lds < 0 ? b->Q == 19 && b->dtype == ASLHIP_F32 && bytes > CACHE_BYTES : b->tune_lds != 0;
+}
 
 // Steps from which an eager run goes group by group: a group's first step reads
 // HBM in any case, and every group adds launches.  16 cavities of 32^3..96^3,
@@ -2048,8 +2059,7 @@ std::vector<int> batch_group_of(const aslhip_batch *b) {
 }
 
 // One lattice's step arguments in the batch's launch shape.
-StepArgs batch_args(const aslhip_batch *b, const aslhip_lattice *h) {
-  const bool tile = batch_tile(b);
+StepArgs batch_args(const aslhip_batch *b, const aslhip_lattice *h, bool tile) {
   return step_args(h, b->block, 1, false, tile);
 }
 
@@ -2064,13 +2074,13 @@ void batch_free(aslhip_batch *b) {
 }
 
 // One step of the lattices whose workgroup entries are [e0, e1).
-int batch_launch(aslhip_batch *b, bool odd, bool macro, int e0, int e1) {
+int batch_launch(aslhip_batch *b, bool odd, bool macro, const aslhip_batch::Range &e) {
   BatchLaunch L;
-  L.desc = b->desc + (macro ? b->lat.size() : 0);
-  L.ent = b->ent + e0;
-  L.nblocks = e1 - e0;
-  L.tile = batch_tile(b) ? 1 : 0;
-  L.block = L.tile ? STEP_TILE : std::min(b->block, step_block(b->Q, static_cast<int>(b->lat[0]->selem)));
+  L.desc = b->desc + ((e.all ? 2 : 0) + (macro ? 1 : 0)) * b->lat.size();
+  L.ent = b->ent + e.first;
+  L.nblocks = e.end - e.first;
+  L.tile = e.tile ? 1 : 0;
+  L.block = e.tile ? STEP_TILE : std::min(b->block, step_block(b->Q, static_cast<int>(b->lat[0]->selem)));
   HIPCHK(launch_step_batch(b->Q, b->dtype, odd, b->periodic, b->wide, L, b->stream));
   return 0;
 }
@@ -2078,37 +2088,41 @@ int batch_launch(aslhip_batch *b, bool odd, bool macro, int e0, int e1) {
 // The workgroup table for the batch's settings (the lattices in order).  On
 // failure the batch keeps the table it has.
 int batch_tables(aslhip_batch *b) {
-  std::vector<uint2> ent;
-  std::vector<std::pair<int, int>> groups;
   const std::vector<int> of = batch_group_of(b);
-  const int last = *std::max_element(of.begin(), of.end());
-  for (int g = 0; g <= last; ++g) {
-    const size_t first = ent.size();
-    for (size_t l = 0; l < b->lat.size(); ++l) {
-      if (of[l] != g) continue;
-      const StepArgs a = batch_args(b, b->lat[l]);
-      for (int c = 0; c < a.g.nchunks; ++c)
-        ent.push_back(make_uint2(static_cast<unsigned>(l), static_cast<unsigned>(c)));
-    }
-    groups.emplace_back(static_cast<int>(first), static_cast<int>(ent.size()));
-  }
+  const int ng = *std::max_element(of.begin(), of.end()) + 1;
+  std::vector<long long> bytes(ng, 0);
+  for (size_t l = 0; l < of.size(); ++l) bytes[of[l]] += b->lat[l]->qs_bytes * b->lat[l]->Q;
+  std::vector<char> tile(of.size());
+  for (size_t l = 0; l < of.size(); ++l) tile[l] = batch_tile(b, bytes[of[l]]);
+  std::vector<uint2> ent;
+  auto add = [&](size_t l, bool t) {
+    const StepArgs a = batch_args(b, b->lat[l], t);
+    for (int c = 0; c < a.g.nchunks; ++c) ent.push_back(make_uint2(static_cast<unsigned>(l), static_cast<unsigned>(c)));
+  };
   // Each XCD (workgroup id modulo 8) takes one run of the chunks of a group that
   // the Infinity Cache holds (see xcd_run), others the hardware order: the
   // cavities of batch_group_bytes's figures 123 -> 115 and 1535 -> 1437, 20 FP16
   // ones of 96^3 293 -> 272; streamed from HBM, 200^3 and three small D3Q27
   // lattices would take 362 instead of 344.
-  const std::vector<uint2> plain = ent;
-  const size_t nb = plain.size();
-  ent.insert(ent.end(), plain.begin(), plain.end());
-  for (size_t g = 0; g < groups.size(); ++g) {
-    long long bytes = 0;
-    for (size_t l = 0; l < b->lat.size(); ++l)
-      if (of[l] == static_cast<int>(g)) bytes += b->lat[l]->qs_bytes * b->lat[l]->Q;
-    const size_t first = static_cast<size_t>(groups[g].first);
-    const size_t share = (static_cast<size_t>(groups[g].second) - first) / 8;
-    if (bytes > CACHE_BYTES) continue;
-    for (size_t i = 0; i < 8 * share; ++i) ent[first + i] = plain[first + (i % 8) * share + i / 8];
+  std::vector<aslhip_batch::Range> groups;
+  for (int g = 0; g < ng; ++g) {
+    const size_t first = ent.size();
+    for (size_t l = 0; l < of.size(); ++l)
+      if (of[l] == g) add(l, tile[l] != 0);
+    if (bytes[g] <= CACHE_BYTES) {
+      const std::vector<uint2> plain(ent.begin() + first, ent.end());
+      const size_t share = plain.size() / 8;
+      for (size_t i = 0; i < 8 * share; ++i) ent[first + i] = plain[(i % 8) * share + i / 8];
+    }
+    groups.push_back({static_cast<int>(first), static_cast<int>(ent.size()), batch_tile(b, bytes[g]), false});
   }
+  // all in one launch: streamed from HBM if there are several groups
+  const bool t = batch_tile(b, std::accumulate(bytes.begin(), bytes.end(), 0LL));
+  const size_t first = ent.size();
+  for (int g = 0; g < ng; ++g)
+    for (size_t l = 0; l < of.size(); ++l)
+      if (of[l] == g) add(l, t);
+  const aslhip_batch::Range all = {static_cast<int>(first), static_cast<int>(ent.size()), t, true};
   // replays in flight read the old tables and graphs: finish them first
   HIPCHK(hipStreamSynchronize(b->stream));
   uint2 *d = nullptr;
@@ -2124,9 +2138,19 @@ int batch_tables(aslhip_batch *b) {
     }
   if (b->ent) (void)hipFree(b->ent);
   b->ent = d;
-  b->groups = groups;
-  b->nblocks = static_cast<int>(nb);
+  b->groups = std::move(groups);
+  b->all = all;
+  b->tile = std::move(tile);
   return 0;
+}
+
+int batch_set(aslhip_batch *b, int *setting, int value) {
+  const int old = *setting;
+  if (value == old) return 0;
+  *setting = value;
+  const int r = batch_tables(b);
+  if (r) *setting = old;  // the table of the old setting is still there
+  return r;
 }
 
 int batch_graph(aslhip_batch *b, bool odd) {
@@ -2137,7 +2161,7 @@ int batch_graph(aslhip_batch *b, bool odd) {
   int r = 0;
   for (const auto &g : b->groups) {
     bool o = odd;
-    for (int s = 0; s < ASLHIP_GRAPH_CHUNK && !r; ++s, o = !o) r = batch_launch(b, o, false, g.first, g.second);
+    for (int s = 0; s < ASLHIP_GRAPH_CHUNK && !r; ++s, o = !o) r = batch_launch(b, o, false, g);
   }
   hipError_t e = hipStreamEndCapture(b->stream, &graph);
   if (r) {
@@ -2173,8 +2197,15 @@ int batch_step_impl(aslhip_batch *b, int nsteps, unsigned flags) {
   // the previous upload may still be in flight from this buffer
   HIPCHK(hipStreamSynchronize(b->stream));
   std::vector<StepArgs> &desc = b->hdesc;
-  desc.resize(2 * n);
+  desc.resize(4 * n);
   const bool odd = b->lat[0]->next_odd;
+  // Whole graph chunks go group by group, and so do the steps left; fewer than
+  // BATCH_GROUP_STEPS in one launch each for all lattices.
+  const bool macro = (flags & ASLHIP_STEP_WRITE_MACRO) != 0;
+  const int chunks = flags & ASLHIP_STEP_GRAPH ? (nsteps - (macro ? 1 : 0)) / ASLHIP_GRAPH_CHUNK : 0;
+  const int left = nsteps - chunks * ASLHIP_GRAPH_CHUNK;
+  const bool at_once = left < BATCH_GROUP_STEPS && b->groups.size() > 1;
+  const int k0 = chunks || !at_once ? 0 : 1, k1 = at_once ? 1 : 0;  // the descriptions needed
   for (size_t l = 0; l < n; ++l) {
     aslhip_lattice *h = b->lat[l];
     if (int r = prepare(h, false)) return r;
@@ -2183,31 +2214,27 @@ int batch_step_impl(aslhip_batch *b, int nsteps, unsigned flags) {
       return fail(ASLHIP_EINVAL, "ASL ERROR: per-cell relaxation (closure, turbulence) is not supported in batches");
     if (h->next_odd != odd) return fail(ASLHIP_ESTATE, "ASL ERROR: batch lattices are at different step parities");
     if (int r = order_after_consumer(h)) return r;
-    desc[l] = batch_args(b, h);
-    desc[n + l] = desc[l];
-    if (h->comp_rho) desc[n + l].g.flags |= STEP_F_RHO;
-    if (h->comp_vel) desc[n + l].g.flags |= STEP_F_VEL;
+    for (int k = k0; k <= k1; ++k) {
+      StepArgs &plain = desc[2 * k * n + l], &writing = desc[(2 * k + 1) * n + l];
+      plain = batch_args(b, h, k ? b->all.tile : b->tile[l] != 0);
+      writing = plain;
+      if (h->comp_rho) writing.g.flags |= STEP_F_RHO;
+      if (h->comp_vel) writing.g.flags |= STEP_F_VEL;
+    }
     // work queued on the lattice's own stream comes first
     HIPCHK(hipEventRecord(b->done, h->stream));
     HIPCHK(hipStreamWaitEvent(b->stream, b->done, 0));
   }
-  HIPCHK(hipMemcpyAsync(b->desc, desc.data(), desc.size() * sizeof(StepArgs), hipMemcpyHostToDevice, b->stream));
-  const bool macro = (flags & ASLHIP_STEP_WRITE_MACRO) != 0;
-  int left = nsteps;
-  bool o = odd;
-  if (flags & ASLHIP_STEP_GRAPH) {
-    while (left - (macro ? 1 : 0) >= ASLHIP_GRAPH_CHUNK) {
-      if (int r = batch_graph(b, o)) return r;
-      HIPCHK(hipGraphLaunch(b->graph[o ? 1 : 0], b->stream));
-      left -= ASLHIP_GRAPH_CHUNK;  // an even count: the parity is unchanged
-    }
+  HIPCHK(hipMemcpyAsync(b->desc + 2 * k0 * n, desc.data() + 2 * k0 * n, 2 * (k1 - k0 + 1) * n * sizeof(StepArgs),
+                        hipMemcpyHostToDevice, b->stream));
+  for (int c = 0; c < chunks; ++c) {  // an even number of steps each: the parity is unchanged
+    if (int r = batch_graph(b, odd)) return r;
+    HIPCHK(hipGraphLaunch(b->graph[odd ? 1 : 0], b->stream));
   }
-  // The steps left, group by group; fewer than BATCH_GROUP_STEPS in one launch
-  // each for all lattices.
-  const std::vector<std::pair<int, int>> all = {{b->nblocks, 2 * b->nblocks}};
-  for (const auto &g : left < BATCH_GROUP_STEPS && b->groups.size() > 1 ? all : b->groups)
+  const std::vector<aslhip_batch::Range> one = {b->all};
+  for (const auto &g : at_once ? one : b->groups)
     for (int s = 0; s < left; ++s)
-      if (int r = batch_launch(b, o != ((s & 1) != 0), macro && s == left - 1, g.first, g.second)) return r;
+      if (int r = batch_launch(b, odd != ((s & 1) != 0), macro && s == left - 1, g)) return r;
   for (auto *h : b->lat) h->next_odd = (nsteps % 2) ? !odd : odd;
   // the lattices' own streams see the result in order
   HIPCHK(hipEventRecord(b->done, b->stream));
@@ -2241,7 +2268,7 @@ int aslhip_batch_create(aslhip_batch **out, aslhip_lattice *const *lattices, int
   }
   hipError_t e = hipStreamCreate(&b->stream);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
-  if (e == hipSuccess) e = device_alloc(&b->desc, 2 * (size_t)n * sizeof(StepArgs));
+  if (e == hipSuccess) e = device_alloc(&b->desc, 4 * (size_t)n * sizeof(StepArgs));
   if (e != hipSuccess) {
     batch_free(b);
     delete b;
@@ -2272,12 +2299,7 @@ int aslhip_batch_set_tuning(aslhip_batch *b, int knob, int value) {
   } else {
     return fail(ASLHIP_EINVAL, "ASL ERROR: batches tune the workgroup size, the tiles and the group size only");
   }
-  const int old = *setting;
-  if (value == old) return 0;
-  *setting = value;
-  const int r = batch_tables(b);
-  if (r) *setting = old;  // the table of the old setting is still there
-  return r;
+  return batch_set(b, setting, value);
 }
 
 int aslhip_batch_autotune(aslhip_batch *b, int nsteps, int *best_block) {
@@ -2285,10 +2307,10 @@ int aslhip_batch_autotune(aslhip_batch *b, int nsteps, int *best_block) {
   if (nsteps < 1) return fail(ASLHIP_EINVAL, "ASL ERROR: autotune needs at least one step per candidate");
   nsteps += nsteps & 1;
   double best = 1e300;
-  int bb = b->block, bl = batch_tile(b) ? 1 : 0;
+  int bb = b->block, bl = b->tune_lds;
   auto trial = [&](int lds, int blk) -> int {
-    if (int r = aslhip_batch_set_tuning(b, ASLHIP_TUNE_LDS, lds)) return r;
-    if (int r = aslhip_batch_set_tuning(b, ASLHIP_TUNE_BLOCK, blk)) return r;
+    if (int r = batch_set(b, &b->tune_lds, lds)) return r;
+    if (int r = batch_set(b, &b->block, blk)) return r;
     double ms = 0.;
     if (int r = aslhip_batch_time_steps(b, nsteps, 0u, &ms)) return r;
     if (ms < best) {
@@ -2301,10 +2323,10 @@ int aslhip_batch_autotune(aslhip_batch *b, int nsteps, int *best_block) {
   if (!b->periodic && !b->wide)
     if (int r = trial(1, b->block)) return r;  // tiles: fixed workgroup
   for (int blk : {256, 512, 1024})
-    if (int r = trial(0, blk)) return r;
-  if (int r = aslhip_batch_set_tuning(b, ASLHIP_TUNE_LDS, bl)) return r;
-  if (int r = aslhip_batch_set_tuning(b, ASLHIP_TUNE_BLOCK, bb)) return r;
-  if (best_block) *best_block = bl ? STEP_TILE : std::min(bb, step_block(b->Q, static_cast<int>(b->lat[0]->selem)));
+    if (int r = trial(-1, blk)) return r;  // tiles for groups that stream from HBM only
+  if (int r = batch_set(b, &b->tune_lds, bl)) return r;
+  if (int r = batch_set(b, &b->block, bb)) return r;
+  if (best_block) *best_block = bl == 1 ? STEP_TILE : std::min(bb, step_block(b->Q, static_cast<int>(b->lat[0]->selem)));
   return 0;
 }
 
