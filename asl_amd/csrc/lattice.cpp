@@ -730,6 +730,11 @@ void face_entries(const aslhip_lattice *h, StepArgs &a) {
   }
 }
 
+// That many lanes per workgroup, at most what the direct kernel takes.
+int direct_block(const aslhip_lattice *h, int lanes) {
+  return std::min(lanes, step_block(h->Q, static_cast<int>(h->selem)));
+}
+
 // Kernel arguments of one step of h over the whole lattice (STEP_F_* of the
 // lattice's parameters).  With block and cpl 0 the lattice's own tuning for a
 // step of that parity (LDS-staged tiles included), else one cell per lane in
@@ -752,7 +757,7 @@ StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd
   a.cpl = cpl > 0 ? cpl : effective_cpl(h);
   g.block = block > 0 ? block : step_lanes(h);
   if (a.cpl > 1 && g.block > STEP_RUN_BLOCK) g.block = STEP_RUN_BLOCK;
-  g.block = std::min(g.block, step_block(h->Q, static_cast<int>(h->selem)));
+  g.block = direct_block(h, g.block);
   const int lds = effective_lds(h);
   a.tile = tiles || (block <= 0 && cpl <= 0 && (lds == 1 || (lds == 2 && !odd))) ? 1 : 0;
   if (a.tile) g.block = STEP_TILE;
@@ -809,7 +814,11 @@ int prepare(aslhip_lattice *h, bool allow_open) {
 int upload_args(aslhip_lattice *h) {
   const StepArgs base[2] = {step_args(h, 0, 0, false), step_args(h, 0, 0, true)};
   if (!h->h_args.empty()) {
-    if (std::memcmp(base, h->h_args.data(), sizeof base) == 0) return 0;
+    if (std::memcmp(base, h->h_args.data(), sizeof base) == 0) {
+      // tiles and runs of cells do not show every change of the workgroup size that the sweeps take
+      if (h->h_direct.block != direct_block(h, step_lanes(h))) h->h_direct = step_args(h, step_lanes(h), 1).g;
+      return 0;
+    }
     for (int p = 0; p < 2; ++p)
       if (std::memcmp(&base[p].g, &h->h_args[p].g, sizeof(StepHot)) != 0) drop_graphs(h);
     // the previous upload reads h_args: let it finish before overwriting
