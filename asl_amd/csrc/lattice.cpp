@@ -648,13 +648,13 @@ int effective_cpl(const aslhip_lattice *h) {
   return c;
 }
 
-// Workgroup size the step kernel runs with (runs of cells: at most
-// STEP_RUN_BLOCK; LDS-staged tiles on every step: STEP_TILE; tiles on even
-// steps only: the odd steps' workgroup).
-int step_workgroup(const aslhip_lattice *h) {
+// Workgroup size of single steps whose direct kernel takes that many lanes (runs
+// of cells: at most STEP_RUN_BLOCK; LDS-staged tiles on every step: STEP_TILE;
+// tiles on even steps only: the odd steps' workgroup).
+int step_workgroup(const aslhip_lattice *h, int lanes) {
   if (effective_lds(h) == 1) return STEP_TILE;
   const int most = step_block(h->Q, static_cast<int>(h->selem));
-  return std::min(h->tune_block, effective_cpl(h) > 1 ? std::min(most, STEP_RUN_BLOCK) : most);
+  return std::min(lanes, effective_cpl(h) > 1 ? std::min(most, STEP_RUN_BLOCK) : most);
 }
 
 // Lanes per workgroup of the direct kernel: tune_block, unless nobody chose it
@@ -1787,7 +1787,7 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]) {
 
 int aslhip_get_tuning(aslhip_lattice *h, int *block, int *remap) {
   if (int r = check(h)) return r;
-  if (block) *block = step_workgroup(h);
+  if (block) *block = step_workgroup(h, h->tune_block);
   if (remap) *remap = h->tune_remap;
   return 0;
 }
@@ -1865,8 +1865,8 @@ int aslhip_tuning_value(aslhip_lattice *h, int knob, int *value) {
   if (int r = check(h)) return r;
   if (!value) return fail(ASLHIP_EINVAL, "ASL ERROR: tuning_value needs an output");
   switch (knob) {
-    case ASLHIP_TUNE_XCD_REMAP: *value = h->tune_remap; return 0;
-    case ASLHIP_TUNE_BLOCK: *value = step_workgroup(h); return 0;
+    case ASLHIP_TUNE_XCD_REMAP: *value = h->remap_set ? h->tune_remap : step_args(h).g.remap; return 0;
+    case ASLHIP_TUNE_BLOCK: *value = step_workgroup(h, step_lanes(h)); return 0;
     case ASLHIP_TUNE_WIDE: *value = is_wide(h) ? 1 : 0; return 0;
     case ASLHIP_TUNE_CPL: *value = effective_cpl(h); return 0;
     case ASLHIP_TUNE_LDS: *value = effective_lds(h); return 0;
@@ -1927,7 +1927,7 @@ int aslhip_autotune(aslhip_lattice *h, int nsteps, int *best_block, int *best_re
   if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_XCD_REMAP, br)) return r;
   h->remap_set = br != preset;
   if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_BLOCK, bb)) return r;
-  if (best_block) *best_block = step_workgroup(h);
+  if (best_block) *best_block = step_workgroup(h, h->tune_block);
   if (best_remap) *best_remap = br;
   return 0;
 }

@@ -165,13 +165,13 @@ class Lattice:
         call("aslhip_set_tuning", self.h, int(knob), int(value))
 
     def tuning(self):
-        """The current launch settings: (workgroup size, XCD run length)."""
+        """The launch settings: (workgroup size, XCD run length); (512, 4 or 64) stand for the automatic ones."""
         b, r = ctypes.c_int(0), ctypes.c_int(0)
         call("aslhip_get_tuning", self.h, ctypes.byref(b), ctypes.byref(r))
         return b.value, r.value
 
     def tuning_value(self, knob):
-        """The value a tuning knob has now (TUNE_CPL: the cells per lane the step kernel runs with)."""
+        """What a single step runs with now (TUNE_BLOCK: its workgroup size, TUNE_CPL: its cells per lane)."""
         v = ctypes.c_int(0)
         call("aslhip_tuning_value", self.h, int(knob), ctypes.byref(v))
         return v.value
@@ -184,7 +184,8 @@ class Lattice:
 
     def time_steps(self, nsteps, write_macro=False, graph=False, each=False):
         """(ms of the whole call, summed ms of the step kernels; 0 with graph=True)
-        [, per-launch ms as a numpy array if each]."""
+        [, per-launch ms as a numpy array if each].  One launch per step, no
+        sweeps, unless graph=True."""
         tot = ctypes.c_double(0)
         ker = ctypes.c_double(0)
         per = np.zeros(int(nsteps)) if each else None

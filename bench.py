@@ -297,9 +297,10 @@ def precision_study(n, snapshots, u0=0.04, tau=0.5005):
 def cavity_study(no_cpu=False, steps=1000):
     """64^3 lid-driven cavity (tau 0.6, lid 0.05 on ZE executed first, no-slip
     elsewhere), FP32: GPU MLUPS and step-kernel bandwidth, CPU oracle MLUPS."""
+    from asl_amd import _lib
     n = 64
     L = batch_cavity(n, 0.6)
-    block, remap = L.autotune(20)
+    L.autotune(20)
     L.step(100, write_macro=False, graph=True)
     L.synchronize()
     t0 = time.perf_counter()
@@ -313,7 +314,7 @@ def cavity_study(no_cpu=False, steps=1000):
             "gpu_mlups": round(cells * steps / wall / 1e6, 1), "ms_per_step": round(wall * 1e3 / steps, 5),
             "kernel_ms_avg": round(kern_s * 1e3, 5),
             "kernel_gbps": round((152.0 * cells + cells) / kern_s / 1e9, 1),
-            "launch": {"workgroup": block, "xcd_run": remap}}
+            "launch": {"workgroup": L.tuning_value(_lib.TUNE_BLOCK), "xcd_run": L.tuning_value(_lib.TUNE_XCD_REMAP)}}
     if not no_cpu:
         import oracle
         from oracle.lbgk import set_threads
@@ -623,10 +624,10 @@ def main():
         L.set_tuning(_lib.TUNE_CPL, args.cpl)
     if args.lds >= 0:
         L.set_tuning(_lib.TUNE_LDS, args.lds)
-    block, remap = L.autotune(20) if args.autotune else L.tuning()
+    if args.autotune:
+        L.autotune(20)
     if args.remap >= 0:
         L.set_tuning(_lib.TUNE_XCD_REMAP, args.remap)
-        remap = args.remap
     cpl = L.tuning_value(_lib.TUNE_CPL)
     st = L.stats()
     counted = st["counted"]
@@ -678,8 +679,9 @@ def main():
                      "kernel_ms_avg": round(kern_s * 1e3, 5), "kernel_ms_min": round(float(np.min(each)), 5),
                      "kernel_ms_median": round(float(np.median(each)), 5), "kernel_launches_timed": KERNEL_LAUNCHES,
                      "bytes_per_launch": bytes_per_launch, "graph_ms_per_step": round(ms_graph / args.steps, 5),
-                     "launch": {"workgroup": L.tuning_value(_lib.TUNE_BLOCK), "xcd_run": remap,
-                                "cells_per_lane": cpl, "lds_tiles": L.tuning_value(_lib.TUNE_LDS)}},
+                     "launch": {"workgroup": L.tuning_value(_lib.TUNE_BLOCK),
+                                "xcd_run": L.tuning_value(_lib.TUNE_XCD_REMAP), "cells_per_lane": cpl,
+                                "lds_tiles": L.tuning_value(_lib.TUNE_LDS)}},
         "cpu_baseline": None,
     }
     if not args.no_cpu:

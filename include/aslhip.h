@@ -422,13 +422,18 @@ int aslhip_set_tuning(aslhip_lattice *h, int knob, int value);
  * numbers below 1, more launches than an int counts, on a periodic lattice more
  * steps than planes. */
 int aslhip_sweep_plan(int nx, int periodic, int planes, int steps, int nsteps, int *out, int cap);
-/* The value a tuning knob has now (ASLHIP_TUNE_CPL: the cells per lane the
- * step kernel runs with; ASLHIP_TUNE_LDS: 0, 1 or 2 as it runs LDS-staged
- * tiles on no step, every step or even steps). */
+/* What a single step runs with now (ASLHIP_TUNE_CPL: the cells per lane;
+ * ASLHIP_TUNE_LDS: 0, 1 or 2 as it runs LDS-staged tiles on no step, every step
+ * or even steps; ASLHIP_TUNE_BLOCK: the workgroup size, runs of 2 or 4 cells per
+ * lane at most 512, tiles on every step 256, tiles on even steps only the odd
+ * steps' workgroup; ASLHIP_TUNE_XCD_REMAP: the run length, chosen or automatic);
+ * ASLHIP_TUNE_SWEEP_KB: the setting. */
 int aslhip_tuning_value(aslhip_lattice *h, int knob, int *value);
-/* The workgroup size the step kernel runs with (runs of 2 or 4 cells per lane:
- * at most 512; LDS-staged tiles on every step: 256; tiles on even steps only:
- * the odd steps' workgroup) and the XCD run length (either may be NULL). */
+/* The settings of the workgroup size (with the limits of runs of cells and
+ * tiles, as in aslhip_tuning_value) and of the XCD run length (either may be
+ * NULL).  Until the caller or the autotuner chooses them: 512 and 4 (64 for FP16 /
+ * BF16 storage), which stand for the automatic ones; aslhip_tuning_value gives
+ * what runs. */
 int aslhip_get_tuning(aslhip_lattice *h, int *block, int *remap);
 
 /* The autotuner: times nsteps (rounded up to even) real steps of the lattice
@@ -443,8 +448,9 @@ int aslhip_autotune(aslhip_lattice *h, int nsteps, int *best_block, int *best_re
 
 /* Times nsteps steps with HIP events recorded on the lattice's stream.
  * ms_total: wall time of the whole call between the events; ms_kernel:
- * summed time of the step kernels (events around each launch; 0 with
- * ASLHIP_STEP_GRAPH, whose replays carry no events between launches);
+ * summed time of the step kernels (events around each launch, one launch per
+ * step of the whole lattice, no sweeps; 0 with ASLHIP_STEP_GRAPH, which steps
+ * as aslhip_step does, without events between launches);
  * ms_each: nsteps doubles, the duration of each launch (0 with
  * ASLHIP_STEP_GRAPH).  Any output may be NULL. */
 int aslhip_time_steps(aslhip_lattice *h, int nsteps, unsigned flags,

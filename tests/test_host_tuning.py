@@ -1,4 +1,6 @@
 """Launch settings and what is launched, over the stand-in for the HIP runtime (host_hip.py)."""
+import pytest
+
 import host_hip
 
 
@@ -16,4 +18,48 @@ for knob, value in ((_lib.TUNE_LDS, 1), (_lib.TUNE_CPL, 2), (_lib.TUNE_CPL, 4), 
         L.step(8)
         got = launches()
         assert len(got) > 8 and {b for _, b in got} == {block}, (knob, value, block, set(got))
+""")
+
+
+@pytest.mark.parametrize("size,kw,lanes", [
+    ((1, 1, 5), {}, 128), ((32, 32, 32), {}, 128), ((33, 32, 32), {}, 256), ((64, 32, 32), {}, 256),
+    ((65, 32, 32), {}, 512), ((33, 32, 32), {"q": 27, "dtype": "f64"}, 256),
+    ((65, 64, 64), {"q": 27, "dtype": "f64", "periodic": True}, 256), ((32, 32, 32), {"q": 15}, 128)])
+def test_values_of_what_runs(size, kw, lanes):
+    """Small lattices take the smallest workgroup that gives every CU at most one, D3Q27 in FP64 256 lanes; the
+    values say so, the settings (512 and 4) until somebody chooses stand for it."""
+    host_hip.run("""
+L = cavity(%r, **%r)
+assert L.tuning() == (512, 4)
+L.step(1)
+launches()
+for choose in (None, 512, 1024, 64):
+    if choose:
+        L.set_tuning(_lib.TUNE_BLOCK, choose)
+        L.set_tuning(_lib.TUNE_XCD_REMAP, 3)
+    L.step(2)
+    (grid, block), again = launches()
+    assert again == (grid, block) and L.tuning_value(_lib.TUNE_BLOCK) == block, (choose, block)
+    most = 512 if (L.q, L.host_dtype) == (27, np.float64) else 1024
+    assert block == (min(choose, most) if choose else %d), (choose, block)
+    assert L.tuning_value(_lib.TUNE_XCD_REMAP) == (3 if choose else max(1, grid // 8))
+    if choose:
+        assert L.tuning() == (min(choose, most), 3)
+""" % (size, kw, lanes))
+
+
+def test_values_of_tiles_and_runs_of_cells():
+    host_hip.run("""
+for knob, value, want in ((_lib.TUNE_LDS, 1, 256), (_lib.TUNE_LDS, 2, 128), (_lib.TUNE_CPL, 2, 128), (_lib.TUNE_CPL, 4, 128)):
+    L = cavity((16, 16, 16))
+    L.set_tuning(knob, value)
+    L.step(2)
+    launches()
+    L.step(2)
+    got = [b for _, b in launches()]
+    assert L.tuning_value(_lib.TUNE_BLOCK) == want and want in got, (knob, value, got)
+    L.set_tuning(_lib.TUNE_BLOCK, 1024)
+    L.step(2)
+    got = [b for _, b in launches()]
+    assert L.tuning_value(_lib.TUNE_BLOCK) in got and L.tuning()[0] == L.tuning_value(_lib.TUNE_BLOCK), (knob, value, got)
 """)
