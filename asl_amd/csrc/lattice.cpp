@@ -1875,82 +1875,27 @@ int aslhip_tuning_value(aslhip_lattice *h, int knob, int *value) {
   }
 }
 
-int aslhip_autotune(aslhip_lattice *h, int nsteps, int *best_block, int *best_remap) {
-  if (int r = check(h)) return r;
-  if (nsteps < 1) return fail(ASLHIP_EINVAL, "ASL ERROR: autotune needs at least one step per candidate");
-  nsteps += nsteps & 1;
-  const int remaps[6] = {0, 2, 4, 8, 16, 64};
-  const int preset = h->selem == 2 ? 64 : 4;  // direct kernel: stands for the automatic order (xcd_run)
-  double best = 1e300;
-  int bb = h->tune_block, br = h->tune_remap, bc = h->tune_cpl, bl = effective_lds(h);
-  auto trial = [&](int lds, int cpl, int remap, int blk) -> int {
-    if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_LDS, lds)) return r;
-    if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_CPL, cpl)) return r;
-    if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_XCD_REMAP, remap)) return r;
-    h->remap_set = remap != preset;
-    if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_BLOCK, blk)) return r;
-    double tot = 0., ker = 0.;
-    if (int r = aslhip_time_steps(h, nsteps, 0u, &tot, &ker, nullptr)) return r;
-    if (ker < best) {
-      best = ker;
-      bb = blk;
-      br = remap;
-      bc = cpl;
-      bl = lds;
-    }
-    return 0;
-  };
-  // LDS-staged tiles where the lattice can run them: on every step (fixed
-  // workgroup), on even steps (workgroup of the odd steps' direct kernel)
-  if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_CPL, 0)) return r;
-  if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_LDS, 1)) return r;
-  if (effective_lds(h)) {
-    for (int remap : remaps)
-      if (int r = trial(1, 0, remap, h->tune_block)) return r;
-    for (int remap : remaps)
-      for (int blk : {256, 512, 1024})
-        if (int r = trial(2, 0, remap, blk)) return r;
-  }
-  // direct: the distinct cells-per-lane values this lattice can run
-  if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_LDS, 0)) return r;
-  std::vector<int> cpls;
-  for (int c : {1, 2, 4}) {
-    if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_CPL, c)) return r;
-    if (effective_cpl(h) == c) cpls.push_back(c);
-  }
-  for (int cpl : cpls)
-    for (int remap : remaps)
-      for (int blk : {256, 512, 1024})
-        if (int r = trial(0, cpl, remap, blk)) return r;
-  if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_LDS, bl)) return r;
-  if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_CPL, bc)) return r;
-  if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_XCD_REMAP, br)) return r;
-  h->remap_set = br != preset;
-  if (int r = aslhip_set_tuning(h, ASLHIP_TUNE_BLOCK, bb)) return r;
-  if (best_block) *best_block = step_workgroup(h, h->tune_block);
-  if (best_remap) *best_remap = br;
-  return 0;
-}
+}  // extern "C"
 
-int aslhip_time_steps(aslhip_lattice *h, int nsteps, unsigned flags, double *ms_total, double *ms_kernel,
-                      double *ms_each) {
-  if (int r = check(h)) return r;
+namespace {
+
+// Times nsteps steps between two events; each: with events around every launch,
+// one launch per step (no sweeps, no graphs).
+int time_run(aslhip_lattice *h, int nsteps, unsigned flags, bool each, double *ms_total, double *ms_kernel,
+             double *ms_each) {
   if (int r = flush_deferred(h)) return r;
   flags &= ~ASLHIP_STEP_DEFER;
-  if (nsteps < 1) return fail(ASLHIP_EINVAL, "ASL ERROR: time_steps needs at least one step");
   if (h->dirty || !h->pending.empty()) {
     int r = aslhip_finalize(h);
     if (r) return r;
   }
-  // replayed graphs have no events between their launches
-  const bool graph = (flags & ASLHIP_STEP_GRAPH) != 0;
-  std::vector<hipEvent_t> ev(graph ? 0 : 2 * (size_t)nsteps);
+  std::vector<hipEvent_t> ev(each ? 2 * (size_t)nsteps : 0);
   for (auto &e : ev) HIPCHK(hipEventCreate(&e));
   hipEvent_t t0, t1;
   HIPCHK(hipEventCreate(&t0));
   HIPCHK(hipEventCreate(&t1));
   HIPCHK(hipEventRecord(t0, h->stream));
-  int r = step_impl(h, nsteps, flags, graph ? nullptr : &ev);
+  int r = step_impl(h, nsteps, flags, each ? &ev : nullptr);
   HIPCHK(hipEventRecord(t1, h->stream));
   HIPCHK(hipEventSynchronize(t1));
   if (r == 0) {
@@ -1958,20 +1903,108 @@ int aslhip_time_steps(aslhip_lattice *h, int nsteps, unsigned flags, double *ms_
     HIPCHK(hipEventElapsedTime(&ms, t0, t1));
     if (ms_total) *ms_total = ms;
     double ksum = 0.;
-    for (int s = 0; s < (graph ? 0 : nsteps); ++s) {
+    for (int s = 0; s < nsteps; ++s) {
       float k = 0.f;
-      HIPCHK(hipEventElapsedTime(&k, ev[2 * s], ev[2 * s + 1]));
+      if (each) HIPCHK(hipEventElapsedTime(&k, ev[2 * s], ev[2 * s + 1]));
       ksum += k;
       if (ms_each) ms_each[s] = k;
     }
-    if (graph && ms_each)
-      for (int s = 0; s < nsteps; ++s) ms_each[s] = 0.;
     if (ms_kernel) *ms_kernel = ksum;
   }
   for (auto &e : ev) (void)hipEventDestroy(e);
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
   return r;
+}
+
+}  // namespace
+
+extern "C" {
+
+int aslhip_autotune(aslhip_lattice *h, int nsteps, int *best_block, int *best_remap) {
+  if (int r = check(h)) return r;
+  if (nsteps < 1) return fail(ASLHIP_EINVAL, "ASL ERROR: autotune needs at least one step per candidate");
+  nsteps += nsteps & 1;
+  if (int r = flush_deferred(h)) return r;
+  const int remaps[6] = {0, 2, 4, 8, 16, 64};
+  // Direct kernel: these stand for the automatic order (xcd_run) and workgroup
+  // (step_lanes), which small lattices and D3Q27 in FP64 run better with than with
+  // any fixed value here.
+  const int preset = h->selem == 2 ? 64 : 4, lanes = 512;
+  struct Candidate {
+    int lds, cpl, remap, block;
+  };
+  auto set = [&](const Candidate &c) {
+    drop_graphs(h);
+    h->tune_lds = c.lds;
+    h->tune_cpl = c.cpl;
+    h->tune_remap = c.remap;
+    h->remap_set = c.remap != preset;
+    h->tune_block = c.block;
+    h->block_set = c.block != lanes;
+  };
+  const Candidate automatic = {-1, 0, preset, lanes};
+  set(automatic);
+  const int auto_lds = effective_lds(h);
+  // Lattices whose runs of nsteps steps sweep, with the direct kernel at least:
+  // candidates are compared by whole runs, as aslhip_step takes them, others by
+  // the time of their launches.
+  int g = 0, t = 0;
+  set({0, 1, preset, lanes});
+  sweep_shape(h, nsteps, g, t);
+  const bool sweeping = t > 0;
+  // the distinct cells-per-lane values this lattice can run (sweeps take one)
+  std::vector<int> cpls;
+  for (int c : {1, 2, 4}) {
+    set({0, c, preset, lanes});
+    if (effective_cpl(h) == c && (c == 1 || !sweeping)) cpls.push_back(c);
+  }
+  set({1, 0, preset, lanes});
+  const bool tiles = effective_lds(h) != 0;
+  std::vector<Candidate> all;
+  if (sweeping) all.push_back(automatic);
+  // LDS-staged tiles where the lattice can run them: on every step (fixed
+  // workgroup), on even steps (workgroup of the odd steps' direct kernel; sweeps
+  // of such a lattice are those of the direct kernel)
+  if (tiles) {
+    for (int remap : remaps) all.push_back({1, 0, remap, lanes});
+    for (int remap : remaps)
+      for (int blk : {256, 512, 1024})
+        if (!sweeping) all.push_back({2, 0, remap, blk});
+  }
+  for (int cpl : cpls)
+    for (int remap : remaps)
+      for (int blk : {256, 512, 1024}) all.push_back({0, cpl, remap, blk});
+  double best = 1e300, auto_ms = 1e300;
+  Candidate win = automatic;
+  for (Candidate c : all) {
+    // what a lattice that does not sweep launches by itself
+    const bool is_auto = c.lds < 0 || (!sweeping && c.lds == auto_lds && c.cpl <= 1 && c.remap == preset && c.block == lanes);
+    if (is_auto) c = automatic;
+    set(c);
+    double tot = 0., ker = 0.;
+    if (int r = time_run(h, nsteps, 0u, !sweeping, &tot, &ker, nullptr)) return r;
+    const double ms = sweeping ? tot : ker;
+    if (is_auto) auto_ms = ms;
+    if (ms < best) {
+      best = ms;
+      win = c;
+    }
+  }
+  if (best > 0.98 * auto_ms) win = automatic;  // a fixed setting has to be worth it
+  set(win);
+  if (best_block) *best_block = step_workgroup(h, h->tune_block);
+  if (best_remap) *best_remap = win.remap;
+  return 0;
+}
+
+int aslhip_time_steps(aslhip_lattice *h, int nsteps, unsigned flags, double *ms_total, double *ms_kernel,
+                      double *ms_each) {
+  if (int r = check(h)) return r;
+  if (int r = flush_deferred(h)) return r;
+  if (nsteps < 1) return fail(ASLHIP_EINVAL, "ASL ERROR: time_steps needs at least one step");
+  // replayed graphs have no events between their launches
+  return time_run(h, nsteps, flags, (flags & ASLHIP_STEP_GRAPH) == 0, ms_total, ms_kernel, ms_each);
 }
 
 }  // extern "C"

@@ -441,8 +441,13 @@ int aslhip_get_tuning(aslhip_lattice *h, int *block, int *remap);
  * tiles on every step x XCD runs 0/2/4/8/16/64, tiles on even steps x XCD
  * runs x odd-step workgroup 256/512/1024; direct with cells per lane 1/2/4
  * where it can run them x XCD runs x workgroup 256/512/1024) with HIP
- * events, keeps the fastest and returns its workgroup size and XCD run
- * length (either pointer may be NULL; the variant: aslhip_tuning_value).
+ * events around its launches, keeps the fastest and returns its workgroup size
+ * and XCD run length as aslhip_get_tuning does (either pointer may be NULL; the
+ * variant: aslhip_tuning_value).  A workgroup of 512 and the initial run length
+ * stand for the automatic ones.  Lattices whose runs of nsteps steps sweep are
+ * timed by whole runs, the automatic settings among the candidates (runs of cells
+ * and tiles on even steps, whose sweeps are the direct kernel's, are left out).
+ * The automatic settings stay, or come back, unless a candidate is 2 % faster.
  * The trial steps advance the simulation like any other steps. */
 int aslhip_autotune(aslhip_lattice *h, int nsteps, int *best_block, int *best_remap);
 

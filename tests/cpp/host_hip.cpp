@@ -35,8 +35,8 @@ struct Event {
 };
 struct Cost {
   std::string part;
-  uint32_t block;
-  double ms;
+  uint32_t block, below;  // workgroup size, number of workgroups below this (0: any)
+  double ms;              // per workgroup
 };
 
 std::recursive_mutex mu;
@@ -93,7 +93,7 @@ void host_hip_device(int d) { device = d; }
 void host_hip_limit(size_t n) { limit = n; }
 size_t host_hip_used() { return used; }
 void host_hip_no_new(int on) { no_new = on != 0; }
-void host_hip_cost(const char *part, unsigned block, double ms) { costs.push_back({part, block, ms}); }
+void host_hip_cost(const char *part, unsigned block, unsigned below, double ms) { costs.push_back({part, block, below, ms}); }
 void host_hip_forget() {
   launches.clear();
   copies.clear();
@@ -252,7 +252,8 @@ int hipLaunchKernel(const void *f, Dim grid, Dim block, void **, size_t, void *s
   launches.push_back({name, grid.x, block.x, stream});
   double ms = 0.;
   for (const auto &c : costs)  // later rules win
-    if (name.find(c.part) != std::string::npos && (c.block == 0 || c.block == block.x)) ms = c.ms;
+    if (name.find(c.part) != std::string::npos && (!c.block || c.block == block.x) && (!c.below || grid.x < c.below))
+      ms = c.ms * grid.x;
   Stream *s = static_cast<Stream *>(stream);
   if (s && s->capturing)
     s->captured += ms;

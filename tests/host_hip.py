@@ -15,7 +15,7 @@ sys.path.insert(0, %r)
 H = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)  # before the library: its HIP calls bind to these
 H.host_hip_used.restype = ctypes.c_size_t
 H.host_hip_limit.argtypes = [ctypes.c_size_t]
-H.host_hip_cost.argtypes = [ctypes.c_char_p, ctypes.c_uint, ctypes.c_double]
+H.host_hip_cost.argtypes = [ctypes.c_char_p, ctypes.c_uint, ctypes.c_uint, ctypes.c_double]
 H.host_hip_launches.restype = H.host_hip_copies.restype = ctypes.c_char_p
 import numpy as np
 import asl_amd
@@ -27,6 +27,14 @@ def launches(part="k_step"):
     out = [l.rsplit(" ", 2) for l in H.host_hip_launches().decode().splitlines()]
     H.host_hip_forget()
     return [(int(g), int(b)) for n, g, b in out if part in n]
+
+
+DIRECT, TILE, RUN = b"6k_stepI", b"11k_step_tileI", b"10k_step_runI"
+
+
+def cost(kernel, ms, block=0, below=0):
+    # time of a launch per workgroup: of that size, in launches of fewer than `below` workgroups
+    H.host_hip_cost(kernel, block, below, ms)
 
 
 def copies():

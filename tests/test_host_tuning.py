@@ -63,3 +63,66 @@ for knob, value, want in ((_lib.TUNE_LDS, 1, 256), (_lib.TUNE_LDS, 2, 128), (_li
     got = [b for _, b in launches()]
     assert L.tuning_value(_lib.TUNE_BLOCK) in got and L.tuning()[0] == L.tuning_value(_lib.TUNE_BLOCK), (knob, value, got)
 """)
+
+
+def test_autotune_keeps_the_small_workgroups():
+    """16^3 runs fastest with the 128 lanes that no fixed candidate has: it stays automatic."""
+    host_hip.run("""
+for k in (TILE, RUN):
+    cost(k, 100.0)
+for block, ms in ((128, 1.0), (256, 1.1), (512, 1.3), (1024, 2.0)):
+    cost(DIRECT, ms * block / 128, block)
+L = cavity((16, 16, 16))
+L.step(2)
+assert L.autotune(10) == (512, 4) == L.tuning()
+launches()
+L.step(1)
+assert launches() == [(32, 128)]
+cost(DIRECT, 0.1, 1024)
+assert L.autotune(10)[0] == 1024
+launches()
+L.step(1)
+assert launches() == [(4, 1024)] and L.tuning_value(_lib.TUNE_BLOCK) == 1024
+""")
+
+
+def test_autotune_keeps_the_sweeps():
+    """A box whose single steps are fastest with tiles and whose runs are faster in sweeps (their launches of few
+    workgroups find the cache): runs still sweep, single steps still take tiles."""
+    host_hip.run("""
+L = cavity((256, 182, 180))
+assert 19 * 4 * L.len > 560 << 20
+whole = 256 * 182 * 180 // 512
+cost(DIRECT, 1.1, 512)
+cost(DIRECT, 1.3, 256)
+cost(DIRECT, 2.6, 1024)
+cost(TILE, 0.5)
+for block in (256, 512, 1024):
+    cost(DIRECT, 0.9 * block / 512, block, whole)
+L.step(2)
+L.autotune(20)
+launches()
+L.step(20)
+got = launches()
+assert len(got) > 20, got
+L.step(1)
+assert launches() == [(len(range(0, 182 * 182, 256)) * 256, 256)]
+assert L.tuning_value(_lib.TUNE_LDS) == 1 and L.tuning_value(_lib.TUNE_SWEEP_KB) == -1
+cost(TILE, 0.1)  # tiles better than any sweep: chosen for runs too
+L.autotune(20)
+launches()
+L.step(20)
+assert len(launches()) == 20
+""")
+
+
+def test_autotune_steps_as_often_as_before():
+    """The trial steps advance the simulation: 60 candidates on a small box, 24 on a periodic lattice."""
+    host_hip.run("""
+for kw, n in ((dict(), 6 + 6 * 3 + 2 * 6 * 3), (dict(periodic=True), 6 * 3)):
+    L = cavity((24, 20, 22), **kw)
+    L.step(2)
+    launches()
+    L.autotune(9)
+    assert len(launches()) == 10 * n
+""")
