@@ -160,8 +160,8 @@ struct aslhip_lattice {
   bool closure_mfma = true;  // evaluate the network with BF16 matrix instructions
   ClosureParams *d_cl = nullptr;
   float *d_feat = nullptr;  // closure features scratch (7 per interior cell)
-  void *d_view = nullptr;     // one view of the populations (read_f, write_f), kept up to VIEW_KEEP bytes
-  void *d_surface = nullptr;  // surface force / flux: result (3 len macroscopic values), then the map (len floats)
+  Scratch view;     // one view of the populations (read_f, write_f): Q len macroscopic values
+  Scratch surface;  // surface force / flux: result (3 len macroscopic values), then the map (len floats)
   double dx = 1., pos0[3] = {0., 0., 0.};
   // a stream reading rho / u through aslhip_macro_device: the next work that
   // writes them waits for what it has queued by then
@@ -225,8 +225,10 @@ void drop_graphs(aslhip_lattice *h) {
 
 void free_all(aslhip_lattice *h) {
   drop_graphs(h);
+  scratch_drop(h->view);
+  scratch_drop(h->surface);
   void *ptrs[] = {h->f,  h->rho,  h->u,           h->code,         h->pat, h->rec, h->mode,
-                  h->val, h->vl, h->vlbc, h->red_partial, h->red_out, h->d_args, h->d_cl, h->d_feat, h->d_view, h->d_surface};
+                  h->val, h->vl, h->vlbc, h->red_partial, h->red_out, h->d_args, h->d_cl, h->d_feat};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (auto &v : h->vis)
@@ -1131,25 +1133,6 @@ int step_impl(aslhip_lattice *h, int nsteps, unsigned flags, std::vector<hipEven
   return run_steps(h, nsteps, first, raw, (flags & ASLHIP_STEP_WRITE_MACRO) != 0, ev, graph);
 }
 
-// A device buffer for one view of the populations (Q len macroscopic values).
-// Views of up to VIEW_KEEP bytes keep it: allocating and freeing 45 MB took 0.4
-// ms of a read or write of 1.6.
-constexpr size_t VIEW_KEEP = 256u << 20;
-int view_buffer(aslhip_lattice *h, void **buf, size_t *bytes) {
-  *bytes = (size_t)h->len * h->Q * h->melem;
-  if (h->d_view) {
-    *buf = h->d_view;
-    return 0;
-  }
-  HIPCHK(device_alloc(buf, *bytes));
-  if (*bytes <= VIEW_KEEP) h->d_view = *buf;
-  return 0;
-}
-int view_done(aslhip_lattice *h, void *buf) {
-  if (buf != h->d_view) HIPCHK(hipFree(buf));
-  return 0;
-}
-
 int copy_out(aslhip_lattice *h, const void *dev, void *host, size_t bytes) {
   HIPCHK(to_host(host, dev, bytes, h->stream));
   return 0;
@@ -1479,9 +1462,9 @@ int aslhip_write_f(aslhip_lattice *h, const void *f) {
   if (int r = flush_deferred(h)) return r;
   if (int r = order_after_consumer(h)) return r;
   void *d = nullptr;
-  size_t bytes = 0;
-  if (int r = view_buffer(h, &d, &bytes)) return r;
-  HIPCHK(to_device(d, f, bytes, h->stream));
+  const size_t bytes = (size_t)h->len * h->Q * h->melem;
+  HIPCHK(scratch_take(h->view, bytes, &d));
+  hipError_t e = to_device(d, f, bytes, h->stream);
   WriteFArgs a;
   a.f = h->f;
   a.qs_bytes = h->qs_bytes;
@@ -1490,9 +1473,9 @@ int aslhip_write_f(aslhip_lattice *h, const void *f) {
   a.in = d;
   a.rho = h->rho;
   a.u = h->u;
-  HIPCHK(launch_write_f(h->Q, h->dtype, a, h->stream));
-  if (d != h->d_view) HIPCHK(hipStreamSynchronize(h->stream));  // before it is freed
-  if (int r = view_done(h, d)) return r;
+  if (e == hipSuccess) e = launch_write_f(h->Q, h->dtype, a, h->stream);
+  const hipError_t done = scratch_give(h->view, bytes, d, h->stream);
+  HIPCHK(e != hipSuccess ? e : done);
   h->initialized = true;
   h->fresh = true;
   h->bc_since_init = false;
@@ -1688,12 +1671,14 @@ int aslhip_read_f(aslhip_lattice *h, void *out) {
   if (!out) return fail(ASLHIP_EINVAL, "ASL ERROR: read_f needs an output buffer");
   if (int r = flush_deferred(h)) return r;
   void *d = nullptr;
-  size_t bytes = 0;
-  if (int r = view_buffer(h, &d, &bytes)) return r;
+  const size_t bytes = (size_t)h->len * h->Q * h->melem;
+  HIPCHK(scratch_take(h->view, bytes, &d));
   int r = aslhip::read_f_through(h, out, d, bytes, true);
   (void)hipStreamSynchronize(h->stream);
-  if (int r2 = view_done(h, d)) return r2;
-  return r;
+  const hipError_t done = scratch_give(h->view, bytes, d);
+  if (r) return r;
+  HIPCHK(done);
+  return 0;
 }
 
 }  // extern "C"
@@ -1701,8 +1686,8 @@ int aslhip_read_f(aslhip_lattice *h, void *out) {
 namespace {
 
 // ComputeSurfaceForceMap / ComputeSurfaceFluxMap on the device.  The map and
-// the result go through a buffer that the lattice keeps (allocating and freeing
-// on each call took longer than the kernel).
+// the result go through a kept buffer (allocating and freeing on each call took
+// longer than the kernel).
 int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   if (int r = check(h)) return r;
   if (!map || !out) return fail(ASLHIP_EINVAL, "ASL ERROR: surface force/flux needs a map and an output field");
@@ -1712,23 +1697,23 @@ int surface_impl(aslhip_lattice *h, const float *map, void *out, bool flux) {
   if (int r = prepare(h, false)) return r;
   if (int r = upload_args(h)) return r;
   const size_t len = (size_t)h->len, outb = len * 3 * h->melem, mapb = len * sizeof(float);
-  if (!h->d_surface) {
-    if (device_alloc(&h->d_surface, outb + mapb) != hipSuccess) {
-      h->d_surface = nullptr;
-      return fail(ASLHIP_EHIP, "ASL ERROR: surface force/flux: out of memory");
-    }
-  }
+  void *d = nullptr;
+  if (scratch_take(h->surface, outb + mapb, &d) != hipSuccess)
+    return fail(ASLHIP_EHIP, "ASL ERROR: surface force/flux: out of memory");
   SurfaceArgs s;
-  s.out = h->d_surface;
-  float *dmap = reinterpret_cast<float *>(static_cast<char *>(h->d_surface) + outb);
+  s.out = d;
+  float *dmap = reinterpret_cast<float *>(static_cast<char *>(d) + outb);
   s.map = dmap;
   s.len = h->len;
   s.per = h->periodic ? 1 : 0;
   s.after_odd = h->next_odd ? 0 : 1;
   s.flux = flux ? 1 : 0;
-  HIPCHK(to_device(dmap, map, mapb, h->stream));
-  HIPCHK(launch_surface(h->Q, h->dtype, s, h->h_direct, h->d_args, h->stream));
-  return copy_out(h, h->d_surface, out, flux ? len * h->melem : outb);
+  hipError_t e = to_device(dmap, map, mapb, h->stream);
+  if (e == hipSuccess) e = launch_surface(h->Q, h->dtype, s, h->h_direct, h->d_args, h->stream);
+  const int r = e == hipSuccess ? copy_out(h, d, out, flux ? len * h->melem : outb) : 0;
+  const hipError_t done = scratch_give(h->surface, outb + mapb, d, e == hipSuccess && r == 0 ? nullptr : h->stream);
+  HIPCHK(e != hipSuccess ? e : done);
+  return r;
 }
 
 }  // namespace

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/aslhip.h"
+#include "memory.hpp"
 
 namespace aslhip {
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
@@ -13,19 +14,6 @@ int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 // buffer buf (a deferred step runs first).  staged: through the pinned ring
 // (which allocates on its first use), else by the runtime's copies.
 int read_f_through(aslhip_lattice *h, void *out, void *buf, size_t buf_bytes, bool staged);
-
-// Device memory.  A failed allocation is reported by its return value alone:
-// the runtime would also keep it as the thread's last error, which the next
-// launch on this thread would report as its own.
-template <class T>
-hipError_t device_alloc(T **p, size_t n) {
-  const hipError_t e = hipMalloc(reinterpret_cast<void **>(p), n);
-  if (e != hipSuccess) {
-    *p = nullptr;
-    (void)hipGetLastError();
-  }
-  return e;
-}
 }  // namespace aslhip
 
 #define HIPCHK(expr)                                                                                        \

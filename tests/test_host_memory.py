@@ -66,3 +66,60 @@ B.set_tuning(_lib.TUNE_BLOCK, 256)
 B.step(1)
 assert launches("k_step_batch")[0] == (3 * 24**3 // 256, 256)
 """)
+
+
+def test_kept_buffers_are_bounded():
+    """Views and surface buffers stay with their lattices up to 512 MiB in all and 256 MiB each."""
+    host_hip.run("""
+def held(L, call):
+    before = H.host_hip_used()
+    call(L)
+    call(L)
+    return H.host_hip_used() - before
+
+
+view, surface = (lambda L: L.f()), (lambda L: L.surface_force(np.ones(L.S, np.float32)))
+Ls = [asl_amd.Lattice((100, 100, 100), 19, nu=0.1, periodic=True) for _ in range(10)]
+for L in Ls:
+    L.init_equilibrium()
+    L.step(1)
+kept = [held(L, view) for L in Ls]  # 81 MB each
+assert kept == [76 * Ls[0].len] * 6 + [0] * 4, kept
+for L in Ls[:6]:
+    L.write_f(np.ones((19,) + L.S, np.float32))
+used = H.host_hip_used()
+del L, Ls[:6]
+assert held(Ls[0], view) == 76 * Ls[0].len and held(Ls[0], surface) == 16 * Ls[0].len
+big = asl_amd.Lattice((260, 260, 260), 15, nu=0.1, periodic=True)
+big.init_equilibrium()
+big.step(1)
+assert 16 * big.len > 256 << 20 and held(big, surface) == 0
+""")
+
+
+def test_kept_buffers_make_room():
+    """A lattice that fits only without the kept buffers of others fits; they are allocated again when needed."""
+    host_hip.run("""
+A = cavity((100, 100, 100))
+B = cavity((60, 60, 60))
+f = np.ones((19,) + A.S, np.float32)
+A.step(1)
+B.step(1)
+want = H.host_hip_used()
+A.surface_force(np.ones(A.S, np.float32))
+A.write_f(f)
+B.f()
+assert H.host_hip_used() > want + 76 * A.len
+H.host_hip_limit(H.host_hip_used() + 1000)
+C = cavity((80, 80, 80))
+C.step(1)
+H.host_hip_limit(0)
+A.f()
+A.write_f(f)
+B.f()
+del C
+H.host_hip_limit(H.host_hip_used() + 1000)
+M = asl_amd.Mlp(np.zeros(_lib.CLOSURE_NPARAM, np.float32))
+M.set_data(np.zeros((10000, 7), np.float32), np.zeros(10000, np.float32))
+M.gradient()
+""")
