@@ -1415,13 +1415,11 @@ int aslhip_init_equilibrium_field(aslhip_lattice *h, const void *rho, const void
   if (!u) return fail(ASLHIP_EINVAL, "ASL ERROR: initF needs a velocity field");
   void *drho = nullptr, *du = nullptr;
   const size_t n = (size_t)h->len * h->melem;
-  HIPCHK(device_alloc(&du, 3 * n));
+  hipError_t e = device_alloc(&du, 3 * n);
+  if (e == hipSuccess && rho) e = device_alloc(&drho, n);
   // the stream is waited for below, before the caller may change the fields
-  HIPCHK(to_device(du, u, 3 * n, h->stream, false));
-  if (rho) {
-    HIPCHK(device_alloc(&drho, n));
-    HIPCHK(to_device(drho, rho, n, h->stream, false));
-  }
+  if (e == hipSuccess) e = to_device(du, u, 3 * n, h->stream, false);
+  if (e == hipSuccess && rho) e = to_device(drho, rho, n, h->stream, false);
   InitArgs a;
   a.f = h->f;
   a.qs_bytes = h->qs_bytes;
@@ -1432,10 +1430,12 @@ int aslhip_init_equilibrium_field(aslhip_lattice *h, const void *rho, const void
   a.u_in = du;
   a.rho = h->rho;
   a.u = h->u;
-  HIPCHK(launch_init(h->Q, h->dtype, a, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  HIPCHK(hipFree(du));
-  if (drho) HIPCHK(hipFree(drho));
+  if (e == hipSuccess) e = launch_init(h->Q, h->dtype, a, h->stream);
+  const hipError_t done = hipStreamSynchronize(h->stream);
+  if (du) (void)hipFree(du);
+  if (drho) (void)hipFree(drho);
+  if (e != hipSuccess || done != hipSuccess)
+    return fail(ASLHIP_EHIP, "ASL ERROR: initial fields: %s", hipGetErrorString(e != hipSuccess ? e : done));
   h->initialized = true;
   h->fresh = true;
   h->bc_since_init = false;

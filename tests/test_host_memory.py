@@ -123,3 +123,23 @@ M = asl_amd.Mlp(np.zeros(_lib.CLOSURE_NPARAM, np.float32))
 M.set_data(np.zeros((10000, 7), np.float32), np.zeros(10000, np.float32))
 M.gradient()
 """)
+
+
+def test_initial_fields_that_do_not_fit():
+    """The first field's buffer goes back when the second has no room."""
+    host_hip.run("""
+L = asl_amd.Lattice((40, 40, 40), 19, nu=0.1, periodic=True)
+rho, u = np.ones(L.S, np.float32), np.zeros((3,) + L.S, np.float32)
+used = H.host_hip_used()
+for room in (13, 5):  # bytes a cell, of 16
+    H.host_hip_limit(used + room * L.len)
+    for _ in range(2):
+        try:
+            L.init_equilibrium(rho, u)
+            raise SystemExit("it fitted")
+        except asl_amd.ASLError:
+            assert H.host_hip_used() == used, H.host_hip_used() - used
+H.host_hip_limit(used + 17 * L.len)
+L.init_equilibrium(rho, u)
+assert H.host_hip_used() == used
+""")
