@@ -39,6 +39,17 @@ __device__ __forceinline__ constexpr int drow(int r, int h) { return 8 * (r / 4)
 // register r in half h holds unit 2 r + h.
 __device__ __forceinline__ int unit_at(int q) { return 2 * (4 * (q >> 3) + (q & 3)) + ((q >> 2) & 1); }
 
+// The sample within the batch of a lane's column: 32-bit unsigned, since the last
+// workgroup of a batch near 2^31 goes past it (as a signed number it would count as
+// one before the first sample, and be read).
+__device__ __host__ constexpr unsigned sample_of(unsigned block, int spw, int it, int w, int col) {
+  return ((block * static_cast<unsigned>(spw) + static_cast<unsigned>(it)) * NWAVE + static_cast<unsigned>(w)) * 32u +
+         static_cast<unsigned>(col);
+}
+constexpr unsigned MAX_BATCH = 0x7fffffffu;
+static_assert(sample_of((MAX_BATCH - 1) / (64 * NWAVE), 2, 1, NWAVE - 1, 31) >= MAX_BATCH,
+              "a lane past the largest batch must not count as one of its samples");
+
 // Forward and backward on the FP32 matrix instructions: every wavefront takes
 // 32 samples at a time, one per column, as five products
 //   H1 = relu(W1 x + b1),   H2 = relu(W2 H1 + b2),
@@ -104,8 +115,8 @@ __global__ __launch_bounds__(MLP_GRAD_BLOCK) void k_mlp_grad(const MlpGradArgs a
 #pragma unroll 1
   for (int it = 0; it < SPW; ++it) {
     // this column's sample within the batch
-    const int k = ((static_cast<int>(blockIdx.x) * SPW + it) * NWAVE + w) * 32 + col;
-    const bool live = k < a.count;
+    const unsigned k = sample_of(blockIdx.x, SPW, it, w, col);
+    const bool live = k < static_cast<unsigned>(a.count);
     long long s = 0;
     if (live)
       s = a.seed ? static_cast<long long>(mix64(a.seed + (static_cast<unsigned long long>(k) + 1ull) *
