@@ -198,8 +198,9 @@ struct Division {
 };
 
 // Whether Quotient(r) gives the terms of an equilibrium (4.5 a^2 / r and
-// 1.5 m^2 / r = mm / r) as a division would.  r lies in [2^-16, 2^16] and
-// x <= 2^42: no overflow, and no underflow for x >= 2^-100 (q >= 2^-116, its
+// 1.5 m^2 / r = mm / r) as a division would.  r lies in [2^-16, 2^16] and x is at
+// most 9 mm < 2^44 (4.5 a^2 of a corner direction, a^2 <= 3 m^2): no overflow (q <
+// 2^60), and no underflow for x >= 2^-100 (q >= 2^-116, its
 // remainder a multiple of 2^-146).  A smaller x may be off in its last bits,
 // but then it is below 2^-84 and is added to or subtracted from a value of at
 // least r / 2 >= 2^-17 (a < 2^-50 there), whose rounding it cannot reach.
@@ -433,23 +434,22 @@ __device__ __forceinline__ unsigned on_entry(const StepHot &g, unsigned fb, int 
   return static_cast<unsigned>(__builtin_amdgcn_sbfe(static_cast<int>(fb), (g.fpos >> (4 * j)) & 15u, 1u));
 }
 
-// Bounce-back and constant links of a cell on the faces fb: entry by entry,
-// later ones over earlier ones.  Four vector instructions per entry, in place
+// Bounce-back links of a cell on the faces fb: entry by entry, later ones over
+// earlier ones.  Three vector instructions per entry, in place
 // of a search over three faces per link that was about 800 instructions in
 // every wavefront with a face cell, that is in nearly every wavefront where a
 // row is not much longer than one.  us per step of a closed box before and
 // after (256 x 128 x 128): D3Q19 FP32 126.2 -> 120.3, FP16 67.6 -> 62.4, FP64
 // 230 -> 211, D3Q27 FP16 111 -> 91.5, FP64 382 -> 328; 64^3: D3Q19 FP32 12.1
 // -> 9.6, FP16 10.8 -> 7.7.
-__device__ __forceinline__ void face_masks(const StepHot &g, unsigned fb, unsigned &bounce, unsigned &cnst) {
-  bounce = cnst = 0u;
+__device__ __forceinline__ unsigned face_masks(const StepHot &g, unsigned fb) {
+  unsigned bounce = 0u;
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     const unsigned m = on_entry(g, fb, j) & g.flinks[j];
-    const bool b = (g.fbounce >> j) & 1u;
-    bounce = (bounce & ~m) | (b ? m : 0u);
-    cnst = (cnst & ~m) | (b ? 0u : m);
+    bounce = (bounce & ~m) | ((g.fbounce >> j) & 1u ? m : 0u);
   }
+  return bounce;
 }
 
 // Links that enter through face f.
@@ -559,7 +559,7 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
   // on z faces only (all wavefronts, where rows are short) choose a slot for
   // the links through those only.
   const bool raw = (g.flags & STEP_F_RAW) != 0;
-  unsigned fb = 0, bmask = 0, cmask = 0;
+  unsigned fb = 0, bmask = 0;
   bool faces = false, xyfaces = false;
   if constexpr (!PER) {
     const bool bxy = (it.x == 1) | (it.x == g.nx) | (it.y == 1) | (it.y == g.ny);
@@ -568,7 +568,7 @@ __device__ __forceinline__ void step_body(const StepHot &g, const StepArgs &a, c
     faces = __any((bxy | bz) & !raw);
     if (xyfaces) {
       fb = face_bits(g, it.x, it.y, it.z);
-      face_masks(g, fb, bmask, cmask);
+      bmask = face_masks(g, fb);
     } else if (faces) {
       fb = (it.z == 1 ? 16u : 0u) | (it.z == g.nz ? 32u : 0u);
     }
@@ -710,8 +710,7 @@ __device__ __forceinline__ void step_body_run(const StepHot &g, const StepArgs &
   const unsigned fxy = raw_links ? 0u : face_bits(g, x, y, 0);
   const bool zlo = !raw_links && z0 == 1, zhi = !raw_links && z0 + CPL - 1 == g.nz;
   const bool xyf = __any(fxy != 0u), zf = __any(zlo || zhi);  // wavefront-uniform
-  unsigned bxy = 0, cxy = 0;  // bounce-back links of the x and y faces
-  if (xyf) face_masks(g, fxy, bxy, cxy);
+  const unsigned bxy = xyf ? face_masks(g, fxy) : 0u;  // bounce-back links of the x and y faces
   // the other slot of link k's pair for the cell at byte offset ibc
   auto other = [&](int k, unsigned ibc) -> unsigned {
     const unsigned o = ES * static_cast<unsigned>(offc<Q>(k, g.sx, g.sy));
@@ -744,9 +743,7 @@ __device__ __forceinline__ void step_body_run(const StepHot &g, const StepArgs &
     for (int k = 0; k < Q; ++k) v[c][k] = CD::dec(raw[k][c]);
   if (zf) {
     // bounce-back links with a z share of the end cells, whichever face they bounce at
-    unsigned blo, bhi, unused;
-    face_masks(g, fxy | (zlo ? 16u : 0u), blo, unused);
-    face_masks(g, fxy | (zhi ? 32u : 0u), bhi, unused);
+    const unsigned blo = face_masks(g, fxy | (zlo ? 16u : 0u)), bhi = face_masks(g, fxy | (zhi ? 32u : 0u));
 #pragma unroll
     for (int k = 1; k < Q; ++k) {
       const int cz = Lat<Q>::c[k][2];
@@ -1003,8 +1000,7 @@ __device__ __forceinline__ void step_body_tile(const StepHot &g, const StepArgs 
   const bool raw = (g.flags & STEP_F_RAW) != 0;
   const unsigned fb = (!column || raw) ? 0u : face_bits(g, x, y, zi);
   const bool faces = __any(fb != 0u);
-  unsigned bmask = 0, cmask = 0;
-  if (faces) face_masks(g, fb, bmask, cmask);
+  const unsigned bmask = faces ? face_masks(g, fb) : 0u;
   // the other slot of link k's pair: the outgoing row of k at column t - (offset of c_k)
   auto other_col = [&](int k) -> int { return t - offc<Q>(k, g.sx, g.sy); };
   auto other_in_tile = [&](int k) -> bool {

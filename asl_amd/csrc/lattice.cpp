@@ -662,13 +662,15 @@ int step_workgroup(const aslhip_lattice *h, int lanes) {
 // Lanes per workgroup of the direct kernel: tune_block, unless nobody chose it
 // and the lattice is small.  A step of one workgroup per CU or less takes as
 // long as one workgroup, and smaller ones start and end sooner: 16^3 D3Q19
-// FP32 in a graph 4.29 us (512 lanes), 3.71 (256), 3.55 (128); 16^3 D3Q27 FP64
-// 6.79, 5.62, 5.09; 32^3 4.61, 4.14, 4.26; 40^3 5.33, 5.08, 5.70; from 48^3 up
-// 512 is level or better.  So the smallest of 128, 256 lanes that gives every
-// CU at most one workgroup.  D3Q27 in FP64, of which a CU holds 12 wavefronts,
-// takes 256 lanes throughout, so that all 12 find room: 64^3 periodic 18.6 (512)
-// -> 17.8, 97^3 63.4 -> 61.4, beside two more 75.5 -> 73.9.  The matrix-core closure
-// kernel shares one copy of the weights per workgroup and keeps the large ones.
+// FP32 box in a graph 4.45 us (512 lanes), 3.84 (256), 3.69 (128); 16^3 D3Q27 FP64
+// 7.14, 5.83, 5.37; 32^3 4.74, 4.15, 4.01; 40^3 5.19, 4.54, 5.08; 48^3 5.66, 5.60, 5.61.
+// So the smallest of 128, 256 lanes that gives every CU at most one workgroup.
+// (Above, 256 gain where they fill the last round of workgroups better, 56^3 8.0 ->
+// 7.1, and are level elsewhere, 64^3 8.46 -> 8.34: not automatic.)  D3Q27 in FP64, of
+// which a CU holds 12 wavefronts, takes 256 lanes throughout, so that all 12 find
+// room: 64^3 periodic 18.5 (512) -> 17.8, 97^3 63.4 -> 61.4, beside two more 75.5 ->
+// 73.9.  The matrix-core closure kernel shares one copy of the weights per workgroup
+// and keeps the large ones.
 int step_lanes(const aslhip_lattice *h) {
   const bool tall = step_block(h->Q, static_cast<int>(h->selem)) < STEP_BLOCK;
   if (!h->block_set && !h->has_closure)

@@ -5,7 +5,8 @@
 //
 // Loss: half the mean squared error over the batch.  Adam: Kingma & Ba,
 // "Adam: A Method for Stochastic Optimization" (ICLR 2015), Algorithm 1.
-// All FP32 except the cross-wavefront gradient and loss sums (FP64).
+// All FP32 except the sums over wavefronts and over workgroups (FP64, a workgroup's
+// own sum stored as FP32 between the two).
 #include <hip/hip_runtime.h>
 
 #include "closure.hpp"
@@ -51,8 +52,8 @@ static_assert(sample_of((MAX_BATCH - 1) / (64 * NWAVE), 2, 1, NWAVE - 1, 31) >= 
               "a lane past the largest batch must not count as one of its samples");
 
 // Forward and backward on the FP32 matrix instructions: every wavefront takes
-// 32 samples at a time, one per column, as five products
-//   H1 = relu(W1 x + b1),   H2 = relu(W2 H1 + b2),
+// 32 samples at a time, one per column, as six products
+//   H1 = relu(W1 x + b1),   H2 = relu(W2 H1 + b2),   y = w3 H2 + b3,
 //   dH1 = W2^T dH2 [H1 > 0],   gW2 += dH2 H1^T,   (gW1, gb1) += dH1 (x, 1)^T.
 // v_mfma_f32_32x32x2f32 takes A[l % 32][l / 32] and B[l / 32][l % 32] from lane
 // l; with the units in unit_at's order k-step r uses units 2 r and 2 r + 1, which
@@ -65,11 +66,13 @@ static_assert(sample_of((MAX_BATCH - 1) / (64 * NWAVE), 2, 1, NWAVE - 1, 31) >= 
 // The two gradients contract over samples; their operands go through LDS once,
 // transposed.  g_b2, g_w3, g_b3 and the loss are sums per lane, added up at the
 // end.  Sums of at most 64 samples (SPW blocks of 32) are kept in FP32, as few
-// roundings as 64-sample blocks on the vector ALUs had; everything beyond is
+// roundings as 64-sample blocks on the vector ALUs had; the four wavefronts' are
+// added in FP64 and stored as the workgroup's FP32 sum, which k_mlp_reduce adds in
 // FP64.
 //
 // Bound by latency: 16384 samples are 118 MFLOP (1 us of the matrix cores) in
-// one block per wavefront, 76 dependent instructions of 64 cycles; before, on
+// one block per wavefront, 84 matrix instructions of 64 cycles in a chain of 68 (gW2
+// and gW1 are independent of each other); before, on
 // the vector ALUs with the weight products summed from LDS one sample after the
 // other, 91 us.  20 training steps of 16384 samples: 3370 -> 300 us with the
 // reduction below (270 without the order of the sums).
