@@ -160,6 +160,7 @@ struct aslhip_lattice {
   bool closure_mfma = true;  // evaluate the network with BF16 matrix instructions
   ClosureParams *d_cl = nullptr;
   float *d_feat = nullptr;  // closure features scratch (7 per interior cell)
+  int queued = 0;   // step launches since the host last waited for the stream
   Scratch view;     // one view of the populations (read_f, write_f): Q len macroscopic values
   Scratch surface;  // surface force / flux: result (3 len macroscopic values), then the map (len floats)
   double dx = 1., pos0[3] = {0., 0., 0.};
@@ -857,6 +858,7 @@ int launch_planes(aslhip_lattice *h, bool odd, unsigned fl, int p0, int np) {
     a.hot.remap = xcd_run(h, a.hot.nchunks, false);
     a.hot.mspan = udiv_magic(8u * static_cast<unsigned>(a.hot.remap));
   }
+  ++h->queued;
   HIPCHK(launch_step(h->Q, h->dtype, odd, h->periodic, is_wide(h), a, h->stream));
   return 0;
 }
@@ -1136,7 +1138,7 @@ int step_impl(aslhip_lattice *h, int nsteps, unsigned flags, std::vector<hipEven
 }
 
 int copy_out(aslhip_lattice *h, const void *dev, void *host, size_t bytes) {
-  HIPCHK(to_host(host, dev, bytes, h->stream));
+  HIPCHK(to_host(host, dev, bytes, h->stream, &h->queued));
   return 0;
 }
 
@@ -1609,6 +1611,7 @@ int aslhip_synchronize(aslhip_lattice *h) {
   if (int r = check(h)) return r;
   if (int r = flush_deferred(h)) return r;
   HIPCHK(hipStreamSynchronize(h->stream));
+  h->queued = 0;
   return 0;
 }
 
@@ -1677,6 +1680,7 @@ int aslhip_read_f(aslhip_lattice *h, void *out) {
   HIPCHK(scratch_take(h->view, bytes, &d));
   int r = aslhip::read_f_through(h, out, d, bytes, true);
   (void)hipStreamSynchronize(h->stream);
+  h->queued = 0;
   const hipError_t done = scratch_give(h->view, bytes, d);
   if (r) return r;
   HIPCHK(done);

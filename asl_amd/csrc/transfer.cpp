@@ -16,11 +16,16 @@
 //   to the host     70 KB 11.1 / 17.9, 512 KB 29 / 35, 1 MB 59 / 66, 2 MB 118 /
 //                   115, 3 MB 178 / 153, 8 MB 465 / 315, 32 MB 1890 / 930
 //   to the device   70 KB 10.5 / 17.8, 1 MB 51 / 59, 4 MB 131 / 183, 8 MB 240 /
-//                   315, 24 MB 680 / 708, 32 MB 910 / 905, 48 MB 1757 / 1323
+//                   315, 24 MB 680 / 708, 32 MB 910 / 905, 48 MB 1757 / 1323; writes of
+//                   the populations of three lattices in turn: 10.7 MB 345 / 425,
+//                   15.5 MB 566 / 540, 25.5 MB 920 / 805
 // - memory that the runtime knows (pinned, on a device): its own path; 3.4 MB
 //   into pinned memory take 69 us there and 157 through the ring;
 // - to the host, one chunk or less: one buffer and a wait for the stream in
-//   place of an event (23 KB 9.5, 70 KB 12, 443 KB 26);
+//   place of an event (23 KB 9.5, 70 KB 12, 443 KB 26), unless the host has not
+//   waited for more launches than WAIT_STREAM, which makes such a wait dear.  16^3
+//   steps and a read of rho, stream / event: 1 step 23.8 / 31.2, 6 steps 39 / 46, 8
+//   steps 70 / 53, 40 steps 190 / 165;
 // - to the device, less than RING_FROM: the runtime's path.
 //
 // One ring for the process (RING buffers of CHUNK bytes), held while some
@@ -42,7 +47,8 @@ constexpr size_t CHUNK = 2u << 20;
 constexpr int RING = 8;                      // buffers: chunks in flight and chunks being copied
 constexpr int COPIERS = 4;                   // copy threads
 constexpr size_t THREADS_FROM = 4u << 20;    // smaller transfers end before a thread would pay
-constexpr size_t RING_FROM = 30u << 20;      // to the device: smaller transfers take the runtime's path
+constexpr int WAIT_STREAM = 6;               // launches up to which waiting for the stream beats an event
+constexpr size_t RING_FROM = 14u << 20;      // to the device: smaller transfers take the runtime's path
 constexpr int MAX_DEVICES = 64;
 
 std::mutex ring_mu;   // held during a transfer
@@ -169,7 +175,7 @@ void transfer_drop() {
   if (--holders == 0) release_ring();
 }
 
-hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s) {
+hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s, int *launches) {
   if (n == 0) return hipStreamSynchronize(s);
   std::unique_lock<std::mutex> lock(ring_mu, std::defer_lock);
   hipEvent_t *ev = pageable(dst) && lock.try_lock() ? ring_ready(s) : nullptr;
@@ -179,7 +185,10 @@ hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s) {
   }
   if (n <= CHUNK) {
     hipError_t e = hipMemcpyAsync(ring, src, n, hipMemcpyDeviceToHost, s);
-    const hipError_t w = hipStreamSynchronize(s);
+    const bool event = launches && *launches > WAIT_STREAM;
+    if (e == hipSuccess && event) e = hipEventRecord(ev[0], s);
+    const hipError_t w = e == hipSuccess && event ? hipEventSynchronize(ev[0]) : hipStreamSynchronize(s);
+    if (launches && !event) *launches = 0;
     if (e == hipSuccess) e = w;
     if (e == hipSuccess) std::memcpy(dst, ring, n);
     return e;

@@ -12,7 +12,8 @@ void transfer_hold();
 void transfer_drop();
 
 // Copies n bytes after the work queued on s; returns when dst holds them.
-hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s);
+// launches: those queued since the host last waited for s, 0 after this call has.
+hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s, int *launches = nullptr);
 // Copies n bytes; returns when src may change (wait false: once s has been
 // waited for, which is the caller's to do), work queued on s afterwards sees dst.
 hipError_t to_device(void *dst, const void *src, size_t n, hipStream_t s, bool wait = true);

@@ -43,7 +43,7 @@ std::recursive_mutex mu;
 std::map<const void *, std::string> names;
 std::map<void *, size_t> allocated;
 size_t used = 0, limit = 0;
-int device = 0, last = 0;
+int device = 0, last = 0, event_waits = 0;
 double now = 0.;
 bool no_new = false;
 std::vector<Launch> launches;
@@ -92,6 +92,7 @@ extern "C" {
 void host_hip_device(int d) { device = d; }
 void host_hip_limit(size_t n) { limit = n; }
 size_t host_hip_used() { return used; }
+int host_hip_event_waits() { return event_waits; }
 void host_hip_no_new(int on) { no_new = on != 0; }
 void host_hip_cost(const char *part, unsigned block, unsigned below, double ms) { costs.push_back({part, block, below, ms}); }
 void host_hip_forget() {
@@ -239,7 +240,11 @@ int hipEventRecord(void *e, void *s) {
   static_cast<Event *>(e)->at = now;
   return 0;
 }
-int hipEventSynchronize(void *) { return 0; }
+int hipEventSynchronize(void *) {
+  LOCK;
+  ++event_waits;
+  return 0;
+}
 int hipEventElapsedTime(float *ms, void *a, void *b) {
   *ms = static_cast<float>(static_cast<Event *>(b)->at - static_cast<Event *>(a)->at);
   return 0;

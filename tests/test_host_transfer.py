@@ -20,14 +20,14 @@ assert copies() == [("d", "p", view)]
 
 
 def test_small_transfers():
-    """To the device without the ring up to 30 MiB, to the host through one buffer up to 2 MiB; all bytes arrive."""
+    """To the device without the ring below 14 MiB, to the host through one buffer up to 2 MiB; all bytes arrive."""
     host_hip.run("""
 MB = 1 << 20
 M = asl_amd.Mlp(np.arange(_lib.CLOSURE_NPARAM, dtype=np.float32))
 H.host_hip_forget()
 assert np.array_equal(M.params(), np.arange(_lib.CLOSURE_NPARAM))
 assert copies() == [("p", "d", 4 * _lib.CLOSURE_NPARAM)]
-for n, direct in ((3, True), (30 * MB // 28 - 1, True), (30 * MB // 28 + 1, False)):
+for n, direct in ((3, True), (14 * MB // 28 - 1, True), (14 * MB // 28 + 1, False)):
     x = np.zeros((n, 7), np.float32)
     M.set_data(x, np.zeros(n, np.float32))
     got = [c for c in copies() if c[0] == "d"]
@@ -43,7 +43,7 @@ L = asl_amd.Lattice((80, 80, 80), 19, nu=0.05, periodic=True)
 L.init_equilibrium()
 M = asl_amd.Mlp(np.zeros(_lib.CLOSURE_NPARAM, np.float32))
 f = np.ones((19,) + L.S, np.float32)
-assert f.nbytes >= 30 << 20
+assert f.nbytes >= 14 << 20
 L.velocity()
 for device in (1, 0, 1):
     H.host_hip_device(device)
@@ -68,4 +68,24 @@ H.host_hip_no_new(1)
 r = lib.aslhip_read_velocity(L.h, p)
 H.host_hip_no_new(0)
 assert r == 0 and want.tobytes() == out.tobytes()
+""")
+
+
+def test_small_reads_wait_for_an_event_after_many_launches():
+    host_hip.run("""
+L = cavity((16, 16, 16))
+L.step(1)
+
+
+def waits(read):
+    before = H.host_hip_event_waits()
+    read()
+    return H.host_hip_event_waits() - before
+
+
+for steps, want in ((0, 0), (3, 0), (6, 0), (7, 1), (0, 1), (1, 1)):
+    L.step(steps)
+    assert waits(L.rho) == want, (steps, want)
+L.synchronize()
+assert waits(L.velocity) == 0
 """)
