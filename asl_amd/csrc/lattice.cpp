@@ -668,12 +668,15 @@ int step_workgroup(const aslhip_lattice *h, int lanes) {
 // So the smallest of 128, 256 lanes that gives every CU at most one workgroup.
 // (Above, 256 gain where they fill the last round of workgroups better, 56^3 8.0 ->
 // 7.1, and are level elsewhere, 64^3 8.46 -> 8.34: not automatic.)  D3Q27 in FP64, of
-// which a CU holds 12 wavefronts, takes 256 lanes throughout, so that all 12 find
-// room: 64^3 periodic 18.5 (512) -> 17.8, 97^3 63.4 -> 61.4, beside two more 75.5 ->
-// 73.9.  The matrix-core closure kernel shares one copy of the weights per workgroup
+// which a CU holds 12 wavefronts, takes 256 lanes, so that all 12 find room: 64^3
+// periodic 18.5 (512) -> 17.8, 97^3 63.4 -> 61.4, beside two more 75.5 -> 73.9; in sweeps
+// 200^3 631 -> 611, 300^3 2195 -> 2076.  Launches over a whole lattice that streams from
+// HBM keep 512: 200^3 (1.8 GB) 671 (512), 675 (256), 120 x 400 x 300 1269, 1311, 300^3 2418,
+// 2563.  The matrix-core closure kernel shares one copy of the weights per workgroup
 // and keeps the large ones.
-int step_lanes(const aslhip_lattice *h) {
-  const bool tall = step_block(h->Q, static_cast<int>(h->selem)) < STEP_BLOCK;
+constexpr long long TALL_BYTES = 1536LL << 20;
+int step_lanes(const aslhip_lattice *h, bool sweep) {
+  const bool tall = step_block(h->Q, static_cast<int>(h->selem)) < STEP_BLOCK && (sweep || h->qs_bytes * h->Q <= TALL_BYTES);
   if (!h->block_set && !h->has_closure)
     for (int lanes : {128, 256})
       if ((tall && lanes == 256) || 1LL * h->n[0] * h->n[1] * h->n[2] <= 256LL * lanes)
@@ -760,7 +763,7 @@ StepArgs step_args(const aslhip_lattice *h, int block = 0, int cpl = 0, bool odd
   g.nz = h->n[2];
   a.len = h->len;
   a.cpl = cpl > 0 ? cpl : effective_cpl(h);
-  g.block = block > 0 ? block : step_lanes(h);
+  g.block = block > 0 ? block : step_lanes(h, false);
   if (a.cpl > 1 && g.block > STEP_RUN_BLOCK) g.block = STEP_RUN_BLOCK;
   g.block = direct_block(h, g.block);
   const int lds = effective_lds(h);
@@ -821,7 +824,7 @@ int upload_args(aslhip_lattice *h) {
   if (!h->h_args.empty()) {
     if (std::memcmp(base, h->h_args.data(), sizeof base) == 0) {
       // tiles and runs of cells do not show every change of the workgroup size that the sweeps take
-      if (h->h_direct.block != direct_block(h, step_lanes(h))) h->h_direct = step_args(h, step_lanes(h), 1).g;
+      if (h->h_direct.block != direct_block(h, step_lanes(h, true))) h->h_direct = step_args(h, step_lanes(h, true), 1).g;
       return 0;
     }
     for (int p = 0; p < 2; ++p)
@@ -830,7 +833,7 @@ int upload_args(aslhip_lattice *h) {
     HIPCHK(hipStreamSynchronize(h->stream));
   }
   h->h_args.assign(base, base + 2);
-  h->h_direct = step_args(h, step_lanes(h), 1).g;
+  h->h_direct = step_args(h, step_lanes(h, true), 1).g;
   // stream-ordered: steps queued before still see the previous arguments
   HIPCHK(hipMemcpyAsync(h->d_args, h->h_args.data(), sizeof base, hipMemcpyHostToDevice, h->stream));
   return 0;
@@ -1857,7 +1860,7 @@ int aslhip_tuning_value(aslhip_lattice *h, int knob, int *value) {
   if (!value) return fail(ASLHIP_EINVAL, "ASL ERROR: tuning_value needs an output");
   switch (knob) {
     case ASLHIP_TUNE_XCD_REMAP: *value = h->remap_set ? h->tune_remap : step_args(h).g.remap; return 0;
-    case ASLHIP_TUNE_BLOCK: *value = step_workgroup(h, step_lanes(h)); return 0;
+    case ASLHIP_TUNE_BLOCK: *value = step_workgroup(h, step_lanes(h, false)); return 0;
     case ASLHIP_TUNE_WIDE: *value = is_wide(h) ? 1 : 0; return 0;
     case ASLHIP_TUNE_CPL: *value = effective_cpl(h); return 0;
     case ASLHIP_TUNE_LDS: *value = effective_lds(h); return 0;
@@ -2291,7 +2294,10 @@ int aslhip_batch_create(aslhip_batch **out, aslhip_lattice *const *lattices, int
   b->wide = is_wide(lattices[0]);
   // D3Q27 in FP64 (see step_lanes), 512 -> 256 lanes: 10 lattices of 40^3..70^3 in
   // groups 160 -> 153 us per step, 12 of 24^3 18.1 -> 16.3
-  if (step_block(b->Q, static_cast<int>(lattices[0]->selem)) < STEP_BLOCK) b->block = 256;
+  long long largest = 0;
+  for (int l = 0; l < n; ++l)
+    if (lattices[l]) largest = std::max(largest, lattices[l]->qs_bytes * lattices[l]->Q);
+  if (step_block(b->Q, static_cast<int>(lattices[0]->selem)) < STEP_BLOCK && largest <= TALL_BYTES) b->block = 256;
   for (int l = 0; l < n; ++l) {
     aslhip_lattice *h = lattices[l];
     if (!h || h->Q != b->Q || h->dtype != b->dtype || h->periodic != b->periodic || is_wide(h) != b->wide) {

@@ -375,7 +375,7 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  *   512); a workgroup takes that many consecutive interior cells.  D3Q27 in FP64
  *   runs with at most 512; as long as neither the caller nor the autotuner has
  *   set it, lattices of at most 65536 cells run with 128 or 256 and D3Q27 in FP64
- *   with 256. */
+ *   with 256 (but for whole-lattice launches over 1.5 GiB of populations). */
 #define ASLHIP_TUNE_XCD_REMAP 1
 #define ASLHIP_TUNE_BLOCK 2
 /* Batches only: the steps of a graph chunk, or 8 eager steps and more, go
@@ -521,7 +521,7 @@ int aslhip_batch_step(aslhip_batch *b, int nsteps, unsigned flags);
 /* As aslhip_batch_step, timed with HIP events on the batch's stream. */
 int aslhip_batch_time_steps(aslhip_batch *b, int nsteps, unsigned flags, double *ms_total);
 /* Workgroup size (ASLHIP_TUNE_BLOCK, default 1024; 256 for D3Q27
- * in FP64), LDS-staged tiles (ASLHIP_TUNE_LDS 1 or 0; default: D3Q19 FP32 groups
+ * in FP64 with no lattice over 1.5 GiB), LDS-staged tiles (ASLHIP_TUNE_LDS 1 or 0; default: D3Q19 FP32 groups
  * over 256 MiB) or group size (ASLHIP_TUNE_GROUP_MB) of the batch's launches; the
  * autotuners choose between tiles and the direct kernel's workgroup size
  * (256/512/1024, tiles by default as above, timing nsteps real eager steps each;

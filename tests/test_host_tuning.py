@@ -126,3 +126,21 @@ for kw, n in ((dict(), 6 + 6 * 3 + 2 * 6 * 3), (dict(periodic=True), 6 * 3)):
     L.autotune(9)
     assert len(launches()) == 10 * n
 """)
+
+
+def test_large_fp64_d3q27_lattices():
+    """Whole-lattice launches that stream from HBM take 512 lanes, sweeps and smaller lattices 256."""
+    host_hip.run("""
+for n, lanes in ((180, 256), (210, 512)):
+    L = cavity((n, n, n), 27, dtype="f64", periodic=True)
+    L.step(2)
+    launches()
+    L.step(2)
+    assert {b for _, b in launches()} == {lanes} and L.tuning_value(_lib.TUNE_BLOCK) == lanes
+    L.step(8)
+    got = launches()
+    assert len(got) > 8 and {b for _, b in got} == {256}
+    B = asl_amd.Batch([L])
+    B.step(1)
+    assert {b for _, b in launches("k_step_batch")} == {lanes}
+""")
