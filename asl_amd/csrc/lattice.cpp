@@ -896,17 +896,26 @@ constexpr int SWEEP_STEPS = 16, SWEEP_MIN_STEPS = 4, SWEEP_TILED_MIN_STEPS = 6, 
 // Whether a window of wp planes pays.  Every launch of a window costs some 5 us
 // of its own and a sweep takes wp / 2 steps, so thick planes lose, more so in
 // boxes (the direct kernel's own reuse, odd steps from the other end, is worth
-// 256 MiB a step).  us per step of 20 alone, launch per step -> sweeps: 16 planes
-// and more at least level but for FP64 (above); 12 planes, D3Q19 FP64 400 x 300:
-// 20 planes 121 -> 132, 60 403 -> 396, box 402 -> 408; 11, D3Q19 FP32 512 x 512: 24
-// 165 -> 179, 80 604 -> 587; 8, D3Q27 FP32 512 x 512: 40 439 -> 474, 200 2276 ->
-// 2243, box 2257 -> 2366; 10, FP16 750 x 750: 80 708 -> 720, box 711 -> 753; 4,
-// D3Q27 FP32 700 x 700: 300 6490 -> 6990; FP64 500 x 500: 20 408 -> 429, 200 4925 ->
-// 4309, box 4665 -> 4601; D3Q19 FP64 512 x 512 (5): 300 4937 -> 4528, box 4685 -> 4837.
+// 256 MiB a step); the larger the lattice, the less.  us per step of 20 alone,
+// launch per step -> sweeps: 16 planes and more at least level but for FP64
+// (above).  Periodic: 12 planes, D3Q19 FP64 400 x 300: 20 planes 121 -> 132, 60 403 ->
+// 396, 80 559 -> 531; 11, D3Q19 FP32 512 x 512: 24 165 -> 179, 80 604 -> 587; 8, D3Q27
+// FP32 512 x 512: 40 439 -> 474, 200 2276 -> 2243; 10, FP16 750 x 750: 80 708 -> 720;
+// 4, D3Q27 FP32 700 x 700: 300 6490 -> 6990, FP64 500 x 500: 20 408 -> 429, 60 1345 ->
+// 1282, 200 4925 -> 4309; 5, D3Q19 FP64 512 x 512: 300 4937 -> 4528.  Boxes: 12 planes,
+// D3Q19 FP64 400 x 300: 60 402 -> 408, 90 638 -> 648, 150 1059 -> 1024, 300 2150 -> 2055;
+// 11, D3Q19 FP32 512 x 512: 40 292 -> 309, 150 1235 -> 1149, 300 2376 -> 2306; 8, D3Q27
+// FP32 512 x 512: 200 2257 -> 2366, FP64 400 x 300: 40 392 -> 408, 120 1267 -> 1227; 10,
+// FP16 750 x 750: 80 711 -> 753, 300 2730 -> 2876; 4, D3Q27 FP64 500 x 500: 60 1287 ->
+// 1384, 200 4665 -> 4601; 5, D3Q19 FP64 512 x 512: 300 4685 -> 4837.
 bool sweep_pays(const aslhip_lattice *h, long long wp, long long bytes) {
+  constexpr long long MIB = 1LL << 20;
+  const bool f64 = h->selem == 8;
   if (wp >= 16) return true;
-  if (wp >= 8) return h->periodic && h->selem >= 4 && bytes >= 1536LL << 20;
-  return h->selem == 8 && (h->periodic || h->Q == 27) && bytes >= 8LL << 30;
+  if (h->selem < 4) return false;
+  if (wp >= 8)
+    return h->periodic ? bytes >= 1536 * MIB : (wp >= 9 && bytes >= 2048 * MIB) || (f64 && bytes >= 2816 * MIB);
+  return f64 && (h->periodic || h->Q == 27) && bytes >= (h->periodic && h->Q == 27 ? 3072 : 8192) * MIB;
 }
 
 void sweep_shape(const aslhip_lattice *h, int n, int &g, int &t) {

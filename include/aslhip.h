@@ -411,7 +411,7 @@ int aslhip_stats(aslhip_lattice *h, int64_t out[4]);
  * ASLHIP_STEP_GRAPH; one cell per lane).  0: off, -1: automatic (default:
  * lattices over 256 MiB of populations in runs of at least 4 steps; those that
  * run tiles by default over 560 MiB and 6 steps; FP64 below 768 MiB from 8 steps
- * on; planes of more than 14 MiB on large periodic lattices only).  Lattices with
+ * on; planes of more than 14 MiB on lattices of several GiB only).  Lattices with
  * velocity-map BCs do not sweep.  Results are bit for bit the same for every
  * value. */
 #define ASLHIP_TUNE_SWEEP_KB 7

@@ -10,7 +10,8 @@ import host_hip
     ((20, 400, 300), 19, "f64", True, 20, False), ((20, 400, 300), 19, "f64", False, 20, False),
     ((24, 512, 512), 19, "f32", True, 20, False), ((40, 700, 700), 27, "f32", True, 20, False),
     ((40, 500, 500), 27, "f64", True, 20, False), ((30, 750, 750), 19, "f16", True, 20, False),
-    ((80, 512, 512), 19, "f32", True, 20, True),
+    ((80, 512, 512), 19, "f32", True, 20, True), ((80, 400, 300), 19, "f64", False, 20, False),
+    ((130, 400, 300), 19, "f64", False, 20, True),
     # 16 planes and more
     ((160, 150, 150), 19, "f64", True, 20, True), ((160, 150, 150), 19, "f64", True, 8, True),
     ((160, 150, 150), 19, "f64", True, 7, False), ((170, 170, 170), 27, "f16", False, 4, True),
