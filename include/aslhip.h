@@ -520,9 +520,9 @@ int aslhip_batch_destroy(aslhip_batch *b);
 int aslhip_batch_step(aslhip_batch *b, int nsteps, unsigned flags);
 /* As aslhip_batch_step, timed with HIP events on the batch's stream. */
 int aslhip_batch_time_steps(aslhip_batch *b, int nsteps, unsigned flags, double *ms_total);
-/* Workgroup size (ASLHIP_TUNE_BLOCK, default 1024; 256 for D3Q27
- * in FP64 with no lattice over 1.5 GiB), LDS-staged tiles (ASLHIP_TUNE_LDS 1 or 0; default: D3Q19 FP32 groups
- * over 256 MiB) or group size (ASLHIP_TUNE_GROUP_MB) of the batch's launches; the
+/* Workgroup size (ASLHIP_TUNE_BLOCK, default 1024; 256 for D3Q27 in FP64 with no
+ * lattice over 1.5 GiB), LDS-staged tiles (ASLHIP_TUNE_LDS 1 or 0; default: D3Q19
+ * FP32 groups over 256 MiB) or group size (ASLHIP_TUNE_GROUP_MB) of the batch's launches; the
  * autotuners choose between tiles and the direct kernel's workgroup size
  * (256/512/1024, tiles by default as above, timing nsteps real eager steps each;
  * returns 256 for tiles) and the group
